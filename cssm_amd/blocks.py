@@ -186,10 +186,13 @@ class CSSMSHViTBlock:
         """x + Mlp(norm2(x)) per frame (cssm_shvit.py:231-266; Mlp shvit.py:156-182)."""
         shp = x.shape
         H, W, C = shp[-3:]
-        x5 = x if x.dim() == 5 else x.unsqueeze(1)
         n2 = p["norm2"]
-        h = S.block_norm_posconv(x5, S.block_norm_stats(x5, "layer"), "layer", n2["scale"], n2["bias"], None, None,
-                                 x5.shape[1]).float()
+        if S.layer_norm_supported(C):
+            h = S.layer_norm(x, n2["scale"], n2["bias"]).float()
+        else:
+            x5 = x if x.dim() == 5 else x.unsqueeze(1)
+            h = S.block_norm_posconv(x5, S.block_norm_stats(x5, "layer"), "layer", n2["scale"], n2["bias"], None, None,
+                                     x5.shape[1]).float()
         m = p["mlp"]
         h = Fn.gelu(torch.addmm(m["fc1"]["bias"], h.reshape(-1, C), m["fc1"]["kernel"]), approximate="tanh")
         hid = h.shape[-1]

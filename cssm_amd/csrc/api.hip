@@ -808,6 +808,22 @@ int cssm_block_norm_posconv(const void* x, int dtype, int B, int T_in, int T_out
                     "cssm_block_norm_posconv");
 }
 
+int cssm_layer_norm(const void* x, int dtype, long long M, int C, float eps, const float* scale, const float* bias,
+                    int pre_act, int post_act, void* out, void* stream) {
+  if (!x || !scale || !bias || !out)
+    return fail(CSSM_ERR_NULL, "cssm_layer_norm: x, scale, bias and out must be non-null");
+  if (M <= 0 || M > 0x7fffffffLL || C <= 0) return fail(CSSM_ERR_SHAPE, "cssm_layer_norm: M=%lld C=%d", M, C);
+  if (!dtype_ok(dtype)) return fail(CSSM_ERR_ARG, "cssm_layer_norm: dtype=%d", dtype);
+  if (pre_act < 0 || pre_act > 3 || post_act < 0 || post_act > 3)
+    return fail(CSSM_ERR_ARG, "cssm_layer_norm: pre_act=%d post_act=%d", pre_act, post_act);
+  if (!(eps >= 0.0f)) return fail(CSSM_ERR_ARG, "cssm_layer_norm: eps must be >= 0");
+  if (!cssm::layer_norm_supported(dtype, C, x, scale, bias, out))
+    return fail(CSSM_ERR_UNSUPPORTED, "cssm_layer_norm: C=%d is too wide for one row in registers", C);
+  return hip_status(cssm::launch_layer_norm(x, dtype, M, C, eps, scale, bias, pre_act, post_act, out,
+                                            static_cast<hipStream_t>(stream)),
+                    "cssm_layer_norm");
+}
+
 int cssm_block_residual(const void* res, int T_res, const void* y, int T_y, int dtype, int B, int T_out, int H,
                         int W, int C, int act, void* out, void* stream) {
   if (!res || !y || !out) return fail(CSSM_ERR_NULL, "cssm_block_residual: res, y and out must be non-null");

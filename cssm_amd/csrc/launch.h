@@ -223,6 +223,11 @@ hipError_t launch_block_norm_stats(const void* x, int dtype, int B, int T, int H
 hipError_t launch_block_norm_posconv(const void* x, int dtype, int B, int T_in, int T_out, int H, int W, int C,
                                      int mode, const float* stats, const float* scale, const float* bias,
                                      const float* pk, const float* pb, void* out, hipStream_t s);
+// LayerNorm over the rows of (M, C) with an activation before and / or after (0 none, 1 gelu, 2 relu,
+// 3 softplus); hipErrorInvalidValue where layer_norm_supported is false
+bool layer_norm_supported(int dtype, int C, const void* x, const float* scale, const float* bias, const void* out);
+hipError_t launch_layer_norm(const void* x, int dtype, long long M, int C, float eps, const float* scale,
+                             const float* bias, int pre, int post, void* out, hipStream_t s);
 hipError_t launch_block_residual(const void* res, int T_res, const void* y, int T_y, int dtype, int B, int T_out,
                                  int H, int W, int C, int act, void* out, hipStream_t s);
 

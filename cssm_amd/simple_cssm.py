@@ -196,6 +196,8 @@ class SimpleCSSM:
     def _layer_norm(x, p, mode):
         """flax LayerNorm on the HIP block-norm kernels: mode 'layer' per pixel over C,
         'temporal_layer' over (T, C), 'global_layer' over (T, H, W, C) of a (B, T, H, W, C) x."""
+        if mode == "layer" and S.layer_norm_supported(x.shape[-1]):
+            return S.layer_norm(x.contiguous(), p["scale"], p["bias"])
         shape = x.shape
         x5 = x.reshape(shape[0], 1, 1, 1, shape[-1]) if x.dim() == 2 else (x.unsqueeze(1) if x.dim() == 4 else x)
         x5 = x5.contiguous()
@@ -242,6 +244,19 @@ class SimpleCSSM:
         xp = Fn.pad(x.permute(0, 3, 1, 2), (lo, hi, lo, hi))
         return Fn.conv2d(xp, k.permute(3, 2, 0, 1).contiguous(), p["bias"]).permute(0, 2, 3, 1).contiguous()
 
+    def _norm_act(self, v, kind, order, name, p, bs, training):
+        """act(norm(v)) for order 'pre', norm(act(v)) for 'post' (simple_cssm.py:247-255, 510-535); the
+        per-pixel LayerNorm with its activation is one kernel."""
+        on_pixels = kind not in ("batch", "instance") and not (v.dim() == 5 and (kind == "global_instance"
+                                                                                 or kind in _LN_MODES))
+        if on_pixels and S.layer_norm_supported(v.shape[-1]):
+            act = self.act_type if self.act_type in ("gelu", "relu") else "softplus"
+            return S.layer_norm(v.contiguous(), p[name]["scale"], p[name]["bias"],
+                                **({"post": act} if order == "pre" else {"pre": act}))
+        if order == "pre":
+            return self._act(self._norm(v, kind, name, p, bs, training))
+        return self._norm(self._act(v), kind, name, p, bs, training)
+
     def apply(self, variables: Params, x: torch.Tensor, training: bool = False, return_spatial: bool = False,
               return_features: bool = False, injected_features: Optional[torch.Tensor] = None,
               injected_qkv_spatial=None, injected_post_cssm: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -256,9 +271,7 @@ class SimpleCSSM:
         x = x.reshape(B * T, H, W, C).contiguous()
 
         def norm_act(v, name):                                              # :247-255
-            if self.stem_norm_order == "pre":
-                return self._act(self._norm(v, stem_norm, name, p, bs, training))
-            return self._norm(self._act(v), stem_norm, name, p, bs, training)
+            return self._norm_act(v, stem_norm, self.stem_norm_order, name, p, bs, training)
         if self.stem_mode == "pathtracker":                                 # :257-264
             if self.stem_norm_order == "pre":
                 x = self._conv(norm_act(x, "norm1"), p["conv1"])
@@ -285,7 +298,7 @@ class SimpleCSSM:
             y = cell.apply({"params": p[f"cssm_{i}"]}, x, injected_qkv_spatial=injected_qkv_spatial)
             x = S.block_residual(x, y, x.shape[1], "none")                  # x + cssm(x), :482
             if self.depth > 1 and i < self.depth - 1:                       # :486-496
-                x = self._act(self._norm(x, body_norm, f"body_norm_{i}", p, bs, training))
+                x = self._norm_act(x, body_norm, "pre", f"body_norm_{i}", p, bs, training)
                 if self.inter_mlp_ratio > 0:
                     h = self._act(Fn.linear(x, p[f"mlp_{i}_up"]["kernel"].t(), p[f"mlp_{i}_up"]["bias"]))
                     x = x + Fn.linear(h, p[f"mlp_{i}_down"]["kernel"].t(), p[f"mlp_{i}_down"]["bias"])
@@ -299,17 +312,11 @@ class SimpleCSSM:
         x = x.contiguous()
         head = p["head"]
         if return_spatial:                                                  # :510-521
-            if self.readout_norm == "pre":
-                x = self._act(self._norm(x, body_norm, "norm_pre", p, bs, training))
-            else:
-                x = self._norm(self._act(x), body_norm, "norm_pre", p, bs, training)
+            x = self._norm_act(x, body_norm, self.readout_norm, "norm_pre", p, bs, training)
             return Fn.linear(x, head["kernel"].t(), head["bias"])
         if self.frame_readout == "last":                                    # :524-527
             x = x[:, -1].contiguous()
-        if self.readout_norm == "pre":                                      # :530-535
-            x = self._act(self._norm(x, body_norm, "norm_pre", p, bs, training))
-        else:
-            x = self._norm(self._act(x), body_norm, "norm_pre", p, bs, training)
+        x = self._norm_act(x, body_norm, self.readout_norm, "norm_pre", p, bs, training)   # :530-535
         axes = (1, 2) if self.frame_readout == "last" else (1, 2, 3)        # :538-549
         x = x.amax(dim=axes) if self.pool_type == "max" else x.mean(dim=axes)
         x = self._norm(x.contiguous(), body_norm, "norm_post", p, bs, training)   # :552

@@ -932,6 +932,33 @@ def block_norm_posconv(x: torch.Tensor, stats: torch.Tensor, block_norm: str, sc
     return out
 
 
+LN_ACTS = {"none": 0, "gelu": 1, "relu": 2, "softplus": 3}
+
+
+def layer_norm(x: torch.Tensor, scale: torch.Tensor, bias: torch.Tensor, eps: float = 1e-6, pre: str = "none",
+               post: str = "none") -> torch.Tensor:
+    """post(LayerNorm(pre(x))) over the last axis (simple_cssm.py:192-255, cssm_shvit.py:231), of x's
+    shape and dtype; the same values as :func:`block_norm_stats` ('layer') with
+    :func:`block_norm_posconv` on the activated x."""
+    _dev(x, "x")
+    if x.dtype not in _DTYPES:
+        raise ValueError(f"unsupported dtype {x.dtype}")
+    _dev(scale, "scale", torch.float32)
+    _dev(bias, "bias", torch.float32)
+    C = x.shape[-1]
+    if scale.shape != (C,) or bias.shape != (C,):
+        raise ValueError(f"scale {tuple(scale.shape)} / bias {tuple(bias.shape)} do not match C={C}")
+    out = torch.empty_like(x)
+    _lib.call("cssm_layer_norm", x.data_ptr(), _DTYPES[x.dtype], x.numel() // C, C, float(eps), scale.data_ptr(),
+              bias.data_ptr(), LN_ACTS[pre], LN_ACTS[post], out.data_ptr(), _stream())
+    return out
+
+
+def layer_norm_supported(C: int) -> bool:
+    """Rows :func:`layer_norm` takes whatever the alignment of its tensors."""
+    return C <= 512
+
+
 def block_residual(res: torch.Tensor, y: torch.Tensor, T_out: int, output_act: str = "none") -> torch.Tensor:
     """res + act(y) (cssm_shvit.py:211-228): the last frame of each when T_out = 1,
     frame by frame otherwise; (B, T_out, H, W, C)."""

@@ -709,6 +709,19 @@ int cssm_block_norm_posconv(const void* x, int dtype, int B, int T_in, int T_out
                             const float* pos_bias, void* out, void* stream);
 
 /*
+ * out = post(LayerNorm(pre(x))) over the last axis of x (M, C): the 'layer' norm
+ * of SimpleCSSM with its activation (simple_cssm.py:192-255) and the block's
+ * norm2 (cssm_shvit.py:231) in one pass, the same values as
+ * cssm_block_norm_stats (mode 2) followed by cssm_block_norm_posconv.
+ *   x, out  (M, C) of dtype (out may be x); scale, bias (C) float32
+ *   pre_act / post_act  0 none, 1 gelu (tanh form), 2 relu, 3 softplus
+ * C up to 2048 where C % 4 == 0 and x / out are 4-element and scale / bias 16-byte
+ * aligned, else up to 512; CSSM_ERR_UNSUPPORTED beyond.
+ */
+int cssm_layer_norm(const void* x, int dtype, long long M, int C, float eps, const float* scale, const float* bias,
+                    int pre_act, int post_act, void* out, void* stream);
+
+/*
  * out = res + act(y) (cssm_shvit.py:211-228): T_out = 1 takes the last frame
  * of res (T_res frames) and of y (T_y frames), T_out > 1 frame by frame
  * (keep_time; T_res = T_y = T_out).  act 0 none, 1 gelu (tanh form, as
