@@ -342,7 +342,7 @@ int cssm_short_conv(const void* x, int in_dtype, int B, int T, int C, int H, int
     return fail(CSSM_ERR_SHAPE, "cssm_short_conv: B=%d T=%d C=%d H=%d W=%d ks=%d kt=%d", B, T, C, H, W, ks, kt);
   if ((in_dtype != CSSM_F32 && in_dtype != CSSM_BF16) || (out_dtype != CSSM_F32 && out_dtype != CSSM_BF16))
     return fail(CSSM_ERR_ARG, "cssm_short_conv: dtypes %d/%d", in_dtype, out_dtype);
-  return hip_status(cssm::launch_short_conv(x, in_dtype, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, out_dtype, ctx,
+  return hip_status(cssm::launch_short_conv(x, in_dtype, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, out_dtype, ctx, 0,
                                             static_cast<hipStream_t>(stream)),
                     "cssm_short_conv");
 }

@@ -120,7 +120,8 @@ hipError_t launch_ctx_reduce(const float* partial, int F, int HW, int tile_rows,
 
 hipError_t launch_short_conv(const void* x, int in_dtype, int B, int T, int C, int H, int W, int ks, const float* ws,
                              const float* bs, int kt, const float* wt, const float* bt, void* u, int out_dtype,
-                             float* ctx, hipStream_t s);
+                             float* ctx, int pre, hipStream_t s);   // pre: store the pre-activation
+bool short_conv_planes_supported(int T, int H, int W, int ks, int kt);
 
 // ---- GatedDeltaNetCSSM
 // gate weights: index 0 alpha, 1 beta, 2 B_k, 3 B_v; kind 0 dense, 1 factored, 2 channel, 3 scalar.

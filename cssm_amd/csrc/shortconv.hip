@@ -3,9 +3,10 @@
 //   o_t   = sum_{j < kt} w_t[j] s_{t - kt + 1 + j} + b_t (zeros for t < 0; cssm.py:494-500)
 //   u_t   = SiLU(o_t)                                   (cssm.py:502)
 //   ctx_t = mean_{h,w} u_t                              (cssm.py:536)
-// Either convolution may be absent (ks = 0 / kt = 0).  One block per (b, c)
-// plane sequence; threads stride over pixels, the T loop is outermost so the
-// spatial mean of every step reduces inside the block.
+// Either convolution may be absent (ks = 0 / kt = 0).  short_conv_planes runs the
+// cell's own sizes (ks 0 or 3, kt <= 4, planes up to 128 x 128); short_conv_kernel,
+// one block per (b, c) plane sequence with threads striding over pixels and every tap
+// read from global memory, takes the rest.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -84,9 +85,202 @@ short_conv_kernel(const TI* __restrict__ x, int T, int C, int H, int W, int ks, 
   }
 }
 
+// Whole planes per workgroup, LP threads (a power of two) per plane with PX pixels each,
+// walking a chunk of the frames in order.  A frame's plane goes through LDS with a zero
+// border (NB buffers; the next frame's loads are in flight meanwhile), its 3 x 3 sums s_t are
+// taken once and the last three frames' kept in registers for the temporal taps.  The
+// one-pass-per-tap kernel above reads 9 kt values per output through L1 instead, and a
+// block per plane leaves most CUs idle at small B C: frames are therefore dealt in chunks of
+// tlen to gridDim.y (each starts kt - 1 frames early, spatial sums only).  Same sums in the
+// same order as the kernel above, so the same results.  One read and one write of x: 1024
+// frames x 256 planes of 16 x 16 in 216 us (2.5 TB/s; the kernel above 5.75 ms), 512 frames x
+// 128 planes of 14 x 14 in 49 us (331 us), 512 x 32 of 32 x 32 in 57 us (436 us).
+// pre != 0 stores o_t instead of u_t (ctx stays the mean of u_t).
+template <int KS, int PX, int NT, int NB, int LDSF, class TI, class TO>
+__global__ void __launch_bounds__(NT)
+short_conv_planes(const TI* __restrict__ x, long long P, int T, int C, int H, int W, const float* __restrict__ ws,
+                  const float* __restrict__ bs, int kt, const float* __restrict__ wt, const float* __restrict__ bt,
+                  TO* __restrict__ u, float* __restrict__ ctx, int LP, int tlen, int pre) {
+  __shared__ float buf[KS ? NB * LDSF : 1];
+  __shared__ float red[2][NT / 64];
+  const int tid = threadIdx.x, NPL = NT / LP, pl = tid / LP, li = tid % LP;
+  const int HW = H * W, RS = W + 2, PS = (H + 2) * RS;
+  const long long plane = (long long)blockIdx.x * NPL + pl;
+  const bool live = plane < P;
+  const long long b = live ? plane / C : 0;
+  const int c = live ? int(plane % C) : 0;
+  const size_t base = (size_t(b) * T * C + c) * HW, tstep = size_t(C) * HW;
+  float k9[9], kt4[4], bsc = 0.0f, btc = 0.0f;
+  if (KS) {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) k9[i] = ws[i * C + c];
+    bsc = bs[c];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) kt4[j] = j < kt ? wt[(kt - 1 - j) * C + c] : 0.0f;   // by lag
+  if (kt > 0) btc = bt[c];
+  int off[PX];     // LDS slot of the pixel's upper left neighbour
+#pragma unroll
+  for (int k = 0; k < PX; ++k) {
+    const int p = li + k * LP;
+    off[k] = pl * PS + (p / W) * RS + p % W;
+  }
+  if (KS) {
+    for (int i = tid; i < NB * LDSF; i += NT) buf[i] = 0.0f;
+    __syncthreads();
+  }
+  const int t0 = int(blockIdx.y) * tlen, t1 = t0 + tlen < T ? t0 + tlen : T;
+  const int ts = kt > 1 ? (t0 - (kt - 1) > 0 ? t0 - (kt - 1) : 0) : t0;
+  float nx[PX], h1[PX], h2[PX], h3[PX];
+  auto load = [&](int t) {
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+      const int p = li + k * LP;
+      nx[k] = live && p < HW ? sc_ld(x, base + size_t(t) * tstep + p) : 0.0f;
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < PX; ++k) h1[k] = h2[k] = h3[k] = 0.0f;
+  load(ts);
+  // the mean of frame t from the waves' sums (LP > 64), one barrier after they were written
+  auto finish_ctx = [&](int t) {
+    if (ctx != nullptr && LP > 64 && li == 0 && live) {
+      float sum = 0.0f;
+      for (int i = 0; i < LP / 64; ++i) sum += red[t & 1][tid / 64 + i];
+      ctx[(size_t(b) * T + t) * C + c] = sum / float(HW);
+    }
+  };
+  for (int t = ts; t < t1; ++t) {
+    float* bt_ = buf + (NB == 2 ? (t & 1) * LDSF : 0);
+    float s[PX];
+    if (KS) {
+#pragma unroll
+      for (int k = 0; k < PX; ++k)
+        if (li + k * LP < HW) bt_[off[k] + RS + 1] = nx[k];
+    } else {
+#pragma unroll
+      for (int k = 0; k < PX; ++k) s[k] = nx[k];
+    }
+    if (KS || LP > 64) __syncthreads();
+    if (t > t0) finish_ctx(t - 1);
+    if (t + 1 < t1) load(t + 1);
+    if (KS) {
+#pragma unroll
+      for (int k = 0; k < PX; ++k) {
+        float acc = bsc;
+        const float* q = bt_ + (li + k * LP < HW ? off[k] : 0);
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) acc = fmaf(q[i * RS + j], k9[i * 3 + j], acc);
+        s[k] = acc;
+      }
+    }
+    if (t >= t0) {
+      float csum = 0.0f;
+      TO* ut = u + base + size_t(t) * tstep;
+#pragma unroll
+      for (int k = 0; k < PX; ++k) {
+        const int p = li + k * LP;
+        float o = s[k];
+        if (kt > 0) {   // oldest frame first; frames before the first are left out
+          o = btc;
+          if (kt > 3 && t >= 3) o = fmaf(kt4[3], h3[k], o);
+          if (kt > 2 && t >= 2) o = fmaf(kt4[2], h2[k], o);
+          if (kt > 1 && t >= 1) o = fmaf(kt4[1], h1[k], o);
+          o = fmaf(kt4[0], s[k], o);
+        }
+        const float v = o / (1.0f + expf(-o));
+        if (live && p < HW) {
+          sc_st(ut, size_t(p), pre ? o : v);
+          csum += v;
+        }
+      }
+      if (ctx != nullptr) {
+        for (int o = (LP < 64 ? LP : 64) / 2; o > 0; o >>= 1) csum += __shfl_xor(csum, o, 64);
+        if (LP <= 64) {
+          if (li == 0 && live) ctx[(size_t(b) * T + t) * C + c] = csum / float(HW);
+        } else if ((tid & 63) == 0) {
+          red[t & 1][tid / 64] = csum;
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+      h3[k] = h2[k];
+      h2[k] = h1[k];
+      h1[k] = s[k];
+    }
+    if (KS && NB == 1) __syncthreads();   // one buffer: its readers are done
+  }
+  if (LP > 64) {
+    __syncthreads();
+    finish_ctx(t1 - 1);
+  }
+}
+
+// LDS floats of a plane with its border, per kernel class
+constexpr int kScSmall = 4096, kScMid = 4400, kScLarge = 16900;
+
+template <int PX, int NT, int NB, int LDSF, class TI, class TO>
+static void run_short_conv_planes(const TI* x, int B, int T, int C, int H, int W, int ks, const float* ws,
+                                  const float* bs, int kt, const float* wt, const float* bt, TO* u, float* ctx,
+                                  int LP, int pre, hipStream_t s) {
+  const long long P = (long long)B * C, groups = (P + NT / LP - 1) / (NT / LP);
+  // frames per workgroup: all of them when the planes alone give every CU its waves (16 per CU),
+  // else chunks of at least 8 (a chunk reads kt - 1 frames more)
+  const long long want = 256LL * 1024 / NT;
+  long long chunks = groups >= want ? 1 : (want + groups - 1) / groups;
+  if (chunks > (T + 7) / 8) chunks = (T + 7) / 8;
+  const int tlen = int((T + chunks - 1) / chunks);
+  const dim3 grid(unsigned(groups), unsigned((T + tlen - 1) / tlen));
+  if (ks == 3)
+    hipLaunchKernelGGL((short_conv_planes<3, PX, NT, NB, LDSF, TI, TO>), grid, dim3(NT), 0, s, x, P, T, C, H, W, ws,
+                       bs, kt, wt, bt, u, ctx, LP, tlen, pre);
+  else
+    hipLaunchKernelGGL((short_conv_planes<0, PX, NT, NB, LDSF, TI, TO>), grid, dim3(NT), 0, s, x, P, T, C, H, W, ws,
+                       bs, kt, wt, bt, u, ctx, LP, tlen, pre);
+}
+
+template <class TI, class TO>
+static void run_short_conv(const TI* x, int B, int T, int C, int H, int W, int ks, const float* ws, const float* bs,
+                           int kt, const float* wt, const float* bt, TO* u, float* ctx, int pre, hipStream_t s) {
+  const long long HW = (long long)H * W, ps = (long long)(H + 2) * (W + 2);
+  int LP = 1;
+  while (LP < 256 && LP * 4 < HW) LP *= 2;
+  if (HW <= 1024 && (256 / LP) * ps <= kScSmall)
+    run_short_conv_planes<4, 256, 2, kScSmall>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, LP, pre, s);
+  else if (HW <= 4096 && ps <= kScMid)
+    run_short_conv_planes<4, 1024, 2, kScMid>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, 1024, pre, s);
+  else
+    run_short_conv_planes<16, 1024, 1, kScLarge>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, 1024, pre, s);
+}
+
+// where short_conv_planes applies (else the general kernel, which has no pre form)
+bool short_conv_planes_supported(int T, int H, int W, int ks, int kt) {
+  return (ks == 0 || ks == 3) && kt <= 4 && (long long)H * W <= 16384 && (long long)(H + 2) * (W + 2) <= kScLarge &&
+         T <= 65535 * 8;
+}
+
 hipError_t launch_short_conv(const void* x, int in_dtype, int B, int T, int C, int H, int W, int ks, const float* ws,
                              const float* bs, int kt, const float* wt, const float* bt, void* u, int out_dtype,
-                             float* ctx, hipStream_t s) {
+                             float* ctx, int pre, hipStream_t s) {
+  if (short_conv_planes_supported(T, H, W, ks, kt)) {
+    if (in_dtype == 0 && out_dtype == 0)
+      run_short_conv(static_cast<const float*>(x), B, T, C, H, W, ks, ws, bs, kt, wt, bt, static_cast<float*>(u), ctx,
+                     pre, s);
+    else if (in_dtype == 0)
+      run_short_conv(static_cast<const float*>(x), B, T, C, H, W, ks, ws, bs, kt, wt, bt, static_cast<uint16_t*>(u),
+                     ctx, pre, s);
+    else if (out_dtype == 0)
+      run_short_conv(static_cast<const uint16_t*>(x), B, T, C, H, W, ks, ws, bs, kt, wt, bt, static_cast<float*>(u),
+                     ctx, pre, s);
+    else
+      run_short_conv(static_cast<const uint16_t*>(x), B, T, C, H, W, ks, ws, bs, kt, wt, bt,
+                     static_cast<uint16_t*>(u), ctx, pre, s);
+    return hipGetLastError();
+  }
+  if (pre) return hipErrorInvalidValue;
   const dim3 grid(unsigned(B * C)), block(256);
   if (in_dtype == 0 && out_dtype == 0)
     hipLaunchKernelGGL((short_conv_kernel<float, float>), grid, block, 0, s, static_cast<const float*>(x), T, C, H, W,
