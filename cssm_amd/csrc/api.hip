@@ -194,6 +194,23 @@ int cssm_gated_scan_fwd(const void* u, const void* z, void* y, int dtype, int B,
   return hip_status(e, "cssm_gated_scan_fwd");
 }
 
+int cssm_gated_scan_bins(float* spec, const float* gates, const float* khat, float* state, int first, int B, int T,
+                         int C, int H, int W, float c_scale, void* stream) {
+  if (!spec || !gates || !khat || (!state && !first))
+    return fail(CSSM_ERR_NULL, "cssm_gated_scan_bins: spec, gates and khat (and state after the first frames)");
+  if (B <= 0 || T <= 0 || C <= 0 || H <= 0 || W <= 0 || B > 65535 || !(c_scale > 0.0f) ||
+      (long long)C * H * (W / 2 + 1) > 0x7fffffffLL - 64)
+    return fail(CSSM_ERR_SHAPE, "cssm_gated_scan_bins: B=%d T=%d C=%d H=%d W=%d c_scale=%g", B, T, C, H, W,
+                double(c_scale));
+  if (!aligned(gates, 16) || !aligned(spec, 8) || !aligned(khat, 8) || !aligned(state, 8))
+    return fail(CSSM_ERR_ALIGN, "cssm_gated_scan_bins: gates 16-byte aligned, complex tensors 8");
+  return hip_status(cssm::launch_gated_scan_fwd_bins(
+                        reinterpret_cast<float2*>(spec), reinterpret_cast<const float4*>(gates),
+                        reinterpret_cast<const float2*>(khat), reinterpret_cast<float2*>(state), first ? 1 : 0, B, T,
+                        C, H, W, c_scale, static_cast<hipStream_t>(stream)),
+                    "cssm_gated_scan_bins");
+}
+
 int cssm_gated_scan_bwd(const float* uspec, const float* dspec, const float* gates, const float* khat, int B, int T,
                         int C, int H, int W, float c_scale, float* yspec, float* sdu, float* dgates, float* dkhat,
                         void* stream) {

@@ -188,6 +188,10 @@ hipError_t launch_gdn_scan_bins_train(const float2* spec, const float2* ab, long
 hipError_t launch_gated_scan_bwd_bins(const float2* uspec, const float2* dspec, const float4* gates,
                                       const float2* khat, int B, int T, int C, int H, int W, float c_scale,
                                       float2* yspec, float2* sdu, float4* dgates, float2* dkhat, hipStream_t s);
+// forward recurrence of the gated scan on spectra (B, T, C, H, WF), in place: rfft2(u) -> C h; state
+// (B, C, H, WF) carries h between calls on consecutive frames (read unless first; may be null)
+hipError_t launch_gated_scan_fwd_bins(float2* spec, const float4* gates, const float2* khat, float2* state, int first,
+                                      int B, int T, int C, int H, int W, float c_scale, hipStream_t s);
 // the GDN spectral core in one kernel (32 x 32 planes, d_k = 4): rfft2 -> norms -> delta rule -> irfft2
 bool gdn_core_fused_supported(int H, int W, int dk);
 hipError_t launch_gdn_core_fused(const float* qkv, int use_l2, const float2* ab, long long ab_frame, int ab_head,

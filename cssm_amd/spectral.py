@@ -177,8 +177,51 @@ def gated_scan(u: torch.Tensor, z: torch.Tensor, gates: torch.Tensor, khat: torc
     if out is None:
         out = torch.empty_like(u)
     _dev(out, "out", u.dtype)
+    if u.dtype == torch.float32 and not (u_silu or z_silu) and gated_split_rule(B * C, T, H, W):
+        return _gated_scan_split(u, z, gates, khat, out)
     _lib.call("cssm_gated_scan_fwd", u.data_ptr(), z.data_ptr(), out.data_ptr(), _DTYPES[u.dtype],
               B, T, C, H, W, gates.data_ptr(), khat.data_ptr(), int(u_silu), int(z_silu), _stream())
+    return out
+
+
+# microseconds per step of the fused scan while its plane groups fit the chip at once, per plane side
+_FUSED_STEP_US = {8: 7.6, 16: 7.1, 32: 7.3, 64: 13.0, 128: 11.4}
+
+
+def gated_split_rule(planes: int, T: int, H: int, W: int) -> bool:
+    """Whether :func:`gated_scan` of ``planes`` = B C planes runs as batched transforms around the per-bin
+    recurrence instead of the fused kernel.  The fused kernel keeps a plane group on one workgroup for all T,
+    so while the groups fit the chip at once a step takes a fixed latency whatever their number (the table:
+    measured at 64 planes, T = 16..1024); the split form takes three launches (24 us) and its traffic, 6.2e-6
+    us per sample (measured at 8..128, 64..4096 planes).  Split where that estimate is at least a tenth lower;
+    measured fused / split us: 16x16, 256 planes, T = 8 58 / 25, T = 1024 7830 / 570; 32x32, 512 planes, T = 8
+    61 / 38; 64x64, 256 planes, T = 8 108 / 65; 128x128, 64 planes, T = 8 91 / 61; and on the other side of
+    the line 16x16, 4096 planes, T = 16 131 / 127; 32x32, 2048 planes, T = 8 78 / 106; 128x128, 128 planes,
+    T = 8 100 / 107."""
+    step = _FUSED_STEP_US.get(H) if H == W else None
+    return step is not None and 24.0 + 6.2e-6 * planes * T * H * W < 0.9 * step * T
+
+
+def _gated_scan_split(u, z, gates, khat, out, max_bytes: int = 1 << 30):
+    """:func:`gated_scan` as batched rfft2 -> recurrence per bin (cssm_gated_scan_bins) -> irfft2 x z
+    through spectra in HBM, at most ``max_bytes`` of them at a time: batch elements in groups, or one
+    element's frames in pieces with the state carried over.  (1024 frames x 256 planes of 16x16 in pieces of
+    64 / 128 / 256 / 512 MiB: 640 / 588 / 585 / 566 us.)"""
+    B, T, C, H, W = u.shape
+    Wf = W // 2 + 1
+    frames = max(1, max_bytes // (C * H * Wf * 8))
+    nb, nt = (min(B, frames // T), T) if T <= frames else (1, frames)
+    state = torch.empty((1, C, H, Wf), dtype=torch.complex64, device=u.device) if nt < T else None
+    whole = nb == B and nt == T
+    for b in range(0, B, nb):
+        for t in range(0, T, nt):
+            k, m = min(nb, B - b), min(nt, T - t)
+            us, zs, os = ((v if whole else v[b:b + k, t:t + m]).view(k * m, C, H * W) for v in (u, z, out))
+            spec = rfft2_ex(us, H, W)
+            _lib.call("cssm_gated_scan_bins", spec.data_ptr(), (gates if whole else gates[b, t]).data_ptr(),
+                      khat.data_ptr(), state.data_ptr() if state is not None else None, int(t == 0), k, m, C, H, W,
+                      scan_c_scale(H, W), _stream())
+            irfft2_ex(spec, W, os, m=zs)
     return out
 
 

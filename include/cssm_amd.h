@@ -190,6 +190,17 @@ int cssm_gated_scan_fwd(const void* u, const void* z, void* y, int dtype, int B,
                         int z_act, void* stream);
 
 /*
+ * Forward recurrence of the gated scan on spectra, in place: spec (B, T, C, H,
+ * W/2+1) complex holds rfft2(u) (natural order, as cssm_rfft2 writes it) and
+ * receives C_t h_t, whose irfft2 times z is what cssm_gated_scan_fwd stores
+ * (cssm.py:559-577).  gates (B, T, H, W/2+1, 4) and khat as that function reads
+ * them, c_scale the gates' own.  state (B, C, H, W/2+1) complex carries h to the
+ * next call on the following frames: read unless first != 0, written if not NULL.
+ */
+int cssm_gated_scan_bins(float* spec, const float* gates, const float* khat, float* state, int first, int B, int T,
+                         int C, int H, int W, float c_scale, void* stream);
+
+/*
  * Backward of cssm_gated_scan_fwd (with u_act = z_act = identity): the
  * spectral-domain reverse recurrence.  Replaces the gradient jax.value_and_grad
  * takes through cssm.py:531-581 (main.py:283; the log-space scan's custom VJPs,

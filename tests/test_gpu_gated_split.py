@@ -1,0 +1,53 @@
+"""The gated scan through spectra in HBM (cssm_gated_scan_bins between the batched transforms) against
+the fused kernel and, with a plane of zeros on the floor, at the edges of its frame and batch pieces."""
+import pytest
+
+from tests.gpu_util import print_case
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def S():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from cssm_amd import spectral
+    return spectral
+
+
+def _case(S, B, T, C, H, seed=0):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    u = torch.randn((B, T, C, H, H), generator=gen, device="cuda")
+    u[:, T // 2, 0] = 0.0                                   # floored bins
+    z = torch.randn(u.shape, generator=gen, device="cuda")
+    ctx = torch.randn((B, T, C), generator=gen, device="cuda")
+    Wf = H // 2 + 1
+    p = {n: {"kernel": 0.2 * torch.randn((C, H * Wf), generator=gen, device="cuda"),
+             "bias": 0.5 * torch.randn(H * Wf, generator=gen, device="cuda")}
+         for n in ("delta_proj", "B_proj", "C_proj")}
+    gates = S.gated_gates(ctx, p, H, H, "dense", "softplus", S.scan_c_scale(H, H))
+    k = 0.3 * torch.randn((C, 5, 5), generator=gen, device="cuda")
+    return u, z, gates, S.spectral_kernel(k, H, H, scan_order=True)
+
+
+# T around the eight frames held in flight; 128: the scan's column and K_hat orders
+@pytest.mark.parametrize("B,T,C,H", [(2, 1, 32, 8), (1, 7, 40, 16), (1, 8, 8, 16), (3, 9, 8, 16), (1, 17, 6, 32),
+                                     (2, 3, 3, 64), (1, 5, 2, 128)])
+@pytest.mark.parametrize("pieces", [None, "batch", "frames"])
+def test_split_scan_equals_fused(S, monkeypatch, B, T, C, H, pieces):
+    print_case(test="split_scan", B=B, T=T, C=C, H=H, pieces=pieces)
+    u, z, gates, khat = _case(S, B, T, C, H)
+    monkeypatch.setattr(S, "gated_split_rule", lambda *a: False)
+    ref = S.gated_scan(u, z, gates, khat)
+    frame = C * H * (H // 2 + 1) * 8
+    kw = {None: {}, "batch": {"max_bytes": frame * T}, "frames": {"max_bytes": frame * 3}}[pieces]
+    got = S._gated_scan_split(u, z, gates, khat, torch.empty_like(u), **kw)
+    # both are fp32 transforms of <= 2^14 samples around the same recurrence: a few 1e-6 of RMS
+    assert (got - ref).abs().max() <= 2e-5 * ref.pow(2).mean().sqrt()
+
+
+def test_rule_picks_the_split_form_for_few_planes(S):
+    assert S.gated_split_rule(256, 1024, 16, 16) and S.gated_split_rule(64, 8, 128, 128)
+    assert not S.gated_split_rule(8192, 8, 128, 128) and not S.gated_split_rule(1024, 1, 32, 32)
+    assert not S.gated_split_rule(64, 64, 7, 7)
