@@ -583,18 +583,21 @@ int cssm_im2col_same(const void* x, int dtype, int F, int H, int W, int C, int k
                     "cssm_im2col_same");
 }
 
-static bool plane_set_ok(const float* p, int fs, int C) { return p == nullptr || (fs >= C && aligned(p, 16)); }
+// power-of-two planes move as 4-element vectors, the others as elements
+static bool plane_set_ok(const float* p, int fs, int C, int H) {
+  return p == nullptr || (fs >= C && aligned(p, (H & (H - 1)) == 0 ? 16 : 4));
+}
 
 int cssm_rfft2_ex(const float* x, int x_fs, int x_act, const float* a, int a_fs, int a_act, int C, long long P,
                   int H, int W, float* spec, void* stream) {
   if (!x || !spec) return fail(CSSM_ERR_NULL, "cssm_rfft2_ex: x and spec must be non-null");
   if (P <= 0 || C <= 0 || P % C) return fail(CSSM_ERR_SHAPE, "cssm_rfft2_ex: P=%lld C=%d (P a multiple of C)", P, C);
   if (!cssm::fft_ex_supported(H, W))
-    return fail(CSSM_ERR_UNSUPPORTED, "cssm_rfft2_ex: %dx%d planes (square powers of two 4..128)", H, W);
+    return fail(CSSM_ERR_UNSUPPORTED, "cssm_rfft2_ex: %dx%d planes (square, powers of two to 128 or 3..15)", H, W);
   if ((x_act != CSSM_LOAD_IDENTITY && x_act != CSSM_LOAD_SILU) || (a_act != CSSM_LOAD_IDENTITY && a_act != CSSM_LOAD_SILU))
     return fail(CSSM_ERR_ARG, "cssm_rfft2_ex: x_act=%d a_act=%d", x_act, a_act);
-  if (!plane_set_ok(x, x_fs, C) || !plane_set_ok(a, a_fs, C) || !aligned(spec, 8))
-    return fail(CSSM_ERR_ALIGN, "cssm_rfft2_ex: plane sets need fs >= C and 16-byte alignment, spec 8");
+  if (!plane_set_ok(x, x_fs, C, H) || !plane_set_ok(a, a_fs, C, H) || !aligned(spec, 8))
+    return fail(CSSM_ERR_ALIGN, "cssm_rfft2_ex: plane sets need fs >= C and 16-byte alignment (powers of two), spec 8");
   cssm::FftEx e{};
   e.x = {x, x_fs};
   e.a = {a, a_fs};
@@ -614,9 +617,9 @@ int cssm_irfft2_ex(const float* spec, long long P, int H, int W, int C, float* y
     return fail(CSSM_ERR_UNSUPPORTED, "cssm_irfft2_ex: plane sums of %lld %dx%d planes", P, H, W);
   if (P <= 0 || C <= 0 || P % C) return fail(CSSM_ERR_SHAPE, "cssm_irfft2_ex: P=%lld C=%d (P a multiple of C)", P, C);
   if (!cssm::fft_ex_supported(H, W))
-    return fail(CSSM_ERR_UNSUPPORTED, "cssm_irfft2_ex: %dx%d planes (square powers of two 4..128)", H, W);
-  if (!plane_set_ok(y, y_fs, C) || !plane_set_ok(m, m_fs, C) || !plane_set_ok(d, d_fs, C) || !aligned(spec, 8))
-    return fail(CSSM_ERR_ALIGN, "cssm_irfft2_ex: plane sets need fs >= C and 16-byte alignment, spec 8");
+    return fail(CSSM_ERR_UNSUPPORTED, "cssm_irfft2_ex: %dx%d planes (square, powers of two to 128 or 3..15)", H, W);
+  if (!plane_set_ok(y, y_fs, C, H) || !plane_set_ok(m, m_fs, C, H) || !plane_set_ok(d, d_fs, C, H) || !aligned(spec, 8))
+    return fail(CSSM_ERR_ALIGN, "cssm_irfft2_ex: plane sets need fs >= C and 16-byte alignment (powers of two), spec 8");
   cssm::FftEx e{};
   e.m = {m, m_fs};
   e.d = {d, d_fs};

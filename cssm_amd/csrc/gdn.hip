@@ -849,6 +849,94 @@ irfft2_planes_ex(const float2* __restrict__ spec, long long P, const FftEx e) {
   }
 }
 
+// The same on the direct transforms of small planes that are not powers of two (rfft2_small,
+// irfft2_small), NP consecutive planes per workgroup, each plane's set offset taken once into LDS.
+template <int H>
+__global__ void __launch_bounds__((SmallGeom<H, H>::NT))
+rfft2_small_ex(const FftEx e, long long P, float2* __restrict__ spec) {
+  using G = SmallGeom<H, H>;
+  constexpr int W = H, WF = G::WF, HW = G::HW, NT = G::NT, NP = G::NP;
+  __shared__ float xs[NP * HW];
+  __shared__ float2 rs[NP * G::PS];
+  __shared__ size_t xo[NP], ao[NP];
+  const int tid = int(threadIdx.x);
+  const long long p0 = (long long)blockIdx.x * NP;
+  const int np = int(P - p0 < NP ? P - p0 : NP);
+  for (int pl = tid; pl < np; pl += NT) {
+    xo[pl] = e.x.off(p0 + pl, e.C, HW);
+    ao[pl] = e.a.p ? e.a.off(p0 + pl, e.C, HW) : 0;
+  }
+  __syncthreads();
+  for (int i = tid; i < np * HW; i += NT) {
+    const int pl = i / HW, r = i % HW;
+    float v = e.x.p[xo[pl] + r];
+    if (e.x_act) v = silu1(v);
+    if (e.a.p) {
+      const float u = e.a.p[ao[pl] + r];
+      v *= e.a_act ? silu1(u) : u;
+    }
+    xs[i] = v;
+  }
+  __syncthreads();
+  for (int j = tid; j < np * H; j += NT) small_row_r2c<W>(xs + j * W, rs + (j / H) * G::PS + (j % H) * G::RSP);
+  __syncthreads();
+  const int cpl = tid / WF, cv = tid % WF;
+  if (tid < G::NCJ && cpl < np) {
+    float2 r[H], X[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) r[h] = rs[cpl * G::PS + h * G::RSP + cv];
+    dft_sym<H, false>(r, X);
+    float2* out = spec + size_t(p0 + cpl) * (H * WF) + cv;
+#pragma unroll
+    for (int u = 0; u < H; ++u) out[u * WF] = X[u];
+  }
+}
+
+template <int H>
+__global__ void __launch_bounds__((SmallGeom<H, H>::NT))
+irfft2_small_ex(const float2* __restrict__ spec, long long P, const FftEx e) {
+  using G = SmallGeom<H, H>;
+  constexpr int W = H, WF = G::WF, HW = G::HW, NT = G::NT, NP = G::NP;
+  __shared__ float xs[NP * HW];
+  __shared__ float2 rs[NP * G::PS];
+  __shared__ size_t yo[NP], mo[NP], dof[NP];
+  const int tid = int(threadIdx.x);
+  const long long p0 = (long long)blockIdx.x * NP;
+  const int np = int(P - p0 < NP ? P - p0 : NP);
+  const PlaneSet ys{e.y, e.y_fs};
+  for (int pl = tid; pl < np; pl += NT) {
+    yo[pl] = ys.off(p0 + pl, e.C, HW);
+    mo[pl] = e.m.p ? e.m.off(p0 + pl, e.C, HW) : 0;
+    dof[pl] = e.d.p ? e.d.off(p0 + pl, e.C, HW) : 0;
+  }
+  for (int i = tid; i < np * H * WF; i += NT) {
+    const int pl = i / (H * WF), r = i % (H * WF);
+    rs[pl * G::PS + (r / WF) * G::RSP + r % WF] = spec[size_t(p0) * (H * WF) + i];
+  }
+  __syncthreads();
+  const int cpl = tid / WF, cv = tid % WF;
+  if (tid < G::NCJ && cpl < np) {
+    float2 r[H], Z[H];
+#pragma unroll
+    for (int u = 0; u < H; ++u) r[u] = rs[cpl * G::PS + u * G::RSP + cv];
+    dft_sym<H, true>(r, Z);
+    constexpr float inv = 1.0f / float(HW);
+#pragma unroll
+    for (int h = 0; h < H; ++h) rs[cpl * G::PS + h * G::RSP + cv] = cscale(Z[h], inv);
+  }
+  __syncthreads();
+  for (int j = tid; j < np * H; j += NT) small_row_c2r<W>(rs + (j / H) * G::PS + (j % H) * G::RSP, xs + j * W);
+  __syncthreads();
+  for (int i = tid; i < np * HW; i += NT) {
+    const int pl = i / HW, r = i % HW;
+    float v = xs[i];
+    if (e.add) v += e.add[p0 + pl];
+    if (e.m.p) v *= e.m.p[mo[pl] + r];
+    if (e.d.p) v *= dsilu1(e.d.p[dof[pl] + r]);
+    e.y[yo[pl] + r] = v;
+  }
+}
+
 namespace {
 template <int LH, int NP, int PPT>
 hipError_t run_fwd_ex(const FftEx& e, long long P, float2* spec, hipStream_t s) {
@@ -923,10 +1011,40 @@ hipError_t launch_im2col_same(const void* x, int dtype, long long rows, int H, i
   return hipGetLastError();
 }
 
-bool fft_ex_supported(int H, int W) { return H == W && H >= 4 && H <= 128 && (H & (H - 1)) == 0; }
+static bool fft_ex_pow2(int H, int W) { return H == W && H >= 4 && H <= 128 && (H & (H - 1)) == 0; }
+bool fft_ex_supported(int H, int W) { return fft_ex_pow2(H, W) || small_plane(H, W); }
+
+static hipError_t small_fwd_ex(const FftEx& e, long long P, int H, float2* spec, hipStream_t s) {
+#define CSSM_SMALL_EX(N)                                                                                          \
+  case N:                                                                                                         \
+    hipLaunchKernelGGL(rfft2_small_ex<N>, dim3(unsigned((P + SmallGeom<N, N>::NP - 1) / SmallGeom<N, N>::NP)),    \
+                       dim3(SmallGeom<N, N>::NT), 0, s, e, P, spec);                                              \
+    break;
+  switch (H) {
+    CSSM_SMALL_EX(3) CSSM_SMALL_EX(5) CSSM_SMALL_EX(6) CSSM_SMALL_EX(7) CSSM_SMALL_EX(9) CSSM_SMALL_EX(10)
+    CSSM_SMALL_EX(11) CSSM_SMALL_EX(12) CSSM_SMALL_EX(13) CSSM_SMALL_EX(14) CSSM_SMALL_EX(15)
+    default: return hipErrorInvalidValue;
+  }
+#undef CSSM_SMALL_EX
+  return hipGetLastError();
+}
+static hipError_t small_inv_ex(const float2* spec, long long P, int H, const FftEx& e, hipStream_t s) {
+#define CSSM_SMALL_EX(N)                                                                                          \
+  case N:                                                                                                         \
+    hipLaunchKernelGGL(irfft2_small_ex<N>, dim3(unsigned((P + SmallGeom<N, N>::NP - 1) / SmallGeom<N, N>::NP)),   \
+                       dim3(SmallGeom<N, N>::NT), 0, s, spec, P, e);                                              \
+    break;
+  switch (H) {
+    CSSM_SMALL_EX(3) CSSM_SMALL_EX(5) CSSM_SMALL_EX(6) CSSM_SMALL_EX(7) CSSM_SMALL_EX(9) CSSM_SMALL_EX(10)
+    CSSM_SMALL_EX(11) CSSM_SMALL_EX(12) CSSM_SMALL_EX(13) CSSM_SMALL_EX(14) CSSM_SMALL_EX(15)
+    default: return hipErrorInvalidValue;
+  }
+#undef CSSM_SMALL_EX
+  return hipGetLastError();
+}
 
 bool irfft2_ex_sums_supported(long long P, int H, int W) {
-  if (!fft_ex_supported(H, W) || P <= 0) return false;
+  if (!fft_ex_pow2(H, W) || P <= 0) return false;
 #define CSSM_SUMS_CASE(LH, NP_, PPT_) \
   if (np == NP_) return Geom<LH, LH, NP_, PPT_>::V4_LINEAR;
   CSSM_FFT_TABLE(CSSM_SUMS_CASE, 32)
@@ -936,6 +1054,7 @@ bool irfft2_ex_sums_supported(long long P, int H, int W) {
 
 hipError_t launch_rfft2_ex(const FftEx& e, long long P, int H, int W, float2* spec, hipStream_t s) {
   if (!fft_ex_supported(H, W)) return hipErrorInvalidValue;
+  if (small_plane(H, W)) return small_fwd_ex(e, P, H, spec, s);
 #define CSSM_FWD_EX_CASE(LH, NP_, PPT_) \
   if (np == NP_) return run_fwd_ex<LH, NP_, PPT_>(e, P, spec, s);
   CSSM_FFT_TABLE(CSSM_FWD_EX_CASE, 64)
@@ -945,6 +1064,7 @@ hipError_t launch_rfft2_ex(const FftEx& e, long long P, int H, int W, float2* sp
 
 hipError_t launch_irfft2_ex(const float2* spec, long long P, int H, int W, const FftEx& e, hipStream_t s) {
   if (!fft_ex_supported(H, W)) return hipErrorInvalidValue;
+  if (small_plane(H, W)) return small_inv_ex(spec, P, H, e, s);
 #define CSSM_INV_EX_CASE(LH, NP_, PPT_) \
   if (np == NP_) return run_inv_ex<LH, NP_, PPT_>(spec, P, e, s);
   CSSM_FFT_TABLE(CSSM_INV_EX_CASE, 32)

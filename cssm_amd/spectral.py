@@ -185,7 +185,8 @@ def gated_scan(u: torch.Tensor, z: torch.Tensor, gates: torch.Tensor, khat: torc
 
 
 # microseconds per step of the fused scan while its plane groups fit the chip at once, per plane side
-_FUSED_STEP_US = {8: 7.6, 16: 7.1, 32: 7.3, 64: 13.0, 128: 11.4}
+_FUSED_STEP_US = {3: 1.0, 4: 1.1, 5: 5.4, 6: 2.2, 7: 2.7, 8: 7.5, 9: 8.6, 10: 7.9, 11: 9.3, 12: 11.2, 13: 13.0,
+                  14: 4.1, 15: 4.8, 16: 7.1, 32: 7.3, 64: 13.0, 128: 11.4}
 
 
 def gated_split_rule(planes: int, T: int, H: int, W: int) -> bool:
@@ -193,13 +194,16 @@ def gated_split_rule(planes: int, T: int, H: int, W: int) -> bool:
     recurrence instead of the fused kernel.  The fused kernel keeps a plane group on one workgroup for all T,
     so while the groups fit the chip at once a step takes a fixed latency whatever their number (the table:
     measured at 64 planes, T = 16..1024); the split form takes three launches (24 us) and its traffic, 6.2e-6
-    us per sample (measured at 8..128, 64..4096 planes).  Split where that estimate is at least a tenth lower;
-    measured fused / split us: 16x16, 256 planes, T = 8 58 / 25, T = 1024 7830 / 570; 32x32, 512 planes, T = 8
-    61 / 38; 64x64, 256 planes, T = 8 108 / 65; 128x128, 64 planes, T = 8 91 / 61; and on the other side of
-    the line 16x16, 4096 planes, T = 16 131 / 127; 32x32, 2048 planes, T = 8 78 / 106; 128x128, 128 planes,
-    T = 8 100 / 107."""
+    us per sample of a power-of-two plane from 8x8 up and 12e-6 of the others (measured at 3..128, 64..4096
+    planes).  Split where that estimate is at least a tenth lower; measured fused / split us: 16x16, 256
+    planes, T = 8 58 / 25, T = 1024 7830 / 570; 32x32, 512 planes, T = 8 61 / 38; 64x64, 256 planes, T = 8
+    108 / 65; 128x128, 64 planes, T = 8 91 / 61; 13x13, 4096 planes, T = 8 124 / 71; 14x14, 512 planes, T = 32
+    137 / 44; and on the other side of the line 16x16, 4096 planes, T = 16 131 / 127; 32x32, 2048 planes, T = 8
+    78 / 106; 128x128, 128 planes, T = 8 100 / 107; 14x14, 4096 planes, T = 32 155 / 322; 7x7, 512 planes, T = 8
+    23 / 21."""
     step = _FUSED_STEP_US.get(H) if H == W else None
-    return step is not None and 24.0 + 6.2e-6 * planes * T * H * W < 0.9 * step * T
+    per_sample = 6.2e-6 if H >= 8 and (H & (H - 1)) == 0 else 12e-6
+    return step is not None and 24.0 + per_sample * planes * T * H * W < 0.9 * step * T
 
 
 def _gated_scan_split(u, z, gates, khat, out, max_bytes: int = 1 << 30):

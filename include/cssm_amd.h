@@ -490,8 +490,8 @@ int cssm_fft_min_group(int H, int W);
  * phases.  float32 planes are addressed as strided sets: plane p = f*C + c of
  * a set (ptr, fs) starts at ptr + (f*fs + c)*H*W, so the halves of a
  * plane-major (F, 2C, H*W) tensor are sets with fs = 2C.  P planes, a
- * multiple of C; H = W a power of two 4..128 (cssm_fft_ex_supported); sets
- * 16-byte aligned with fs >= C; spec (P, H, W/2+1) complex64, 8-byte aligned.
+ * multiple of C; H = W a power of two 4..128 or any of 3..15
+ * (cssm_fft_ex_supported); sets 16-byte aligned (powers of two) with fs >= C; spec (P, H, W/2+1) complex64, 8-byte aligned.
  *   cssm_rfft2_ex   spec = rfft2(x_act(x) * a_act(a)); a may be NULL (factor 1)
  *                   (x_act, a_act: cssm_load_act)
  *   cssm_irfft2_ex  y = (irfft2(spec) + add[p]) * m * SiLU'(d), each of add

@@ -33,7 +33,8 @@ def _case(S, B, T, C, H, seed=0):
 
 # T around the eight frames held in flight; 128: the scan's column and K_hat orders
 @pytest.mark.parametrize("B,T,C,H", [(2, 1, 32, 8), (1, 7, 40, 16), (1, 8, 8, 16), (3, 9, 8, 16), (1, 17, 6, 32),
-                                     (2, 3, 3, 64), (1, 5, 2, 128)])
+                                     (2, 3, 3, 64), (1, 5, 2, 128), (2, 9, 7, 7), (1, 5, 40, 3), (3, 4, 11, 14),
+                                     (1, 11, 19, 13), (2, 3, 32, 4)])
 @pytest.mark.parametrize("pieces", [None, "batch", "frames"])
 def test_split_scan_equals_fused(S, monkeypatch, B, T, C, H, pieces):
     print_case(test="split_scan", B=B, T=T, C=C, H=H, pieces=pieces)
@@ -50,4 +51,32 @@ def test_split_scan_equals_fused(S, monkeypatch, B, T, C, H, pieces):
 def test_rule_picks_the_split_form_for_few_planes(S):
     assert S.gated_split_rule(256, 1024, 16, 16) and S.gated_split_rule(64, 8, 128, 128)
     assert not S.gated_split_rule(8192, 8, 128, 128) and not S.gated_split_rule(1024, 1, 32, 32)
-    assert not S.gated_split_rule(64, 64, 7, 7)
+    assert S.gated_split_rule(64, 64, 7, 7) and not S.gated_split_rule(64, 4, 7, 7)
+    assert not S.gated_split_rule(64, 64, 16, 32)
+
+
+@pytest.mark.parametrize("H", [3, 7, 12, 14, 15])
+def test_small_plane_transforms_with_fused_work(S, H):
+    """cssm_rfft2_ex / cssm_irfft2_ex on small planes: strided halves of a (F, 2C, HW) tensor, activations,
+    the factor, the per-plane addend and SiLU', against torch in float64 (a few fp32 roundings: 2e-6 of RMS)."""
+    print_case(test="small_ex", H=H)
+    gen = torch.Generator(device="cuda").manual_seed(H)
+    F, C, HW = 3, 13, H * H
+    xz, m = (torch.randn((F, n, HW), generator=gen, device="cuda") for n in (2 * C, C))
+    x, a = xz[:, :C], xz[:, C:]
+    add = torch.randn((F, C), generator=gen, device="cuda")
+    sil = torch.nn.functional.silu
+
+    def close(got, ref):
+        assert (got - ref).abs().max() <= 1e-5 * ref.abs().pow(2).mean().sqrt()
+    spec = S.rfft2_ex(x, H, H, x_silu=True, a=a, a_silu=True)
+    ref = torch.fft.rfft2((sil(x.double()) * sil(a.double())).view(F, C, H, H))
+    close(spec.to(torch.complex128), ref)
+    close(S.rfft2_ex(a, H, H).to(torch.complex128), torch.fft.rfft2(a.double().reshape(F, C, H, H)))
+    out = torch.zeros_like(xz)
+    S.irfft2_ex(spec, H, out[:, C:], add=add, m=m, d=x)
+    s = torch.sigmoid(x.double())
+    want = ((torch.fft.irfft2(ref, s=(H, H)).view(F, C, HW) + add.double()[..., None]) * m.double()
+            * s * (1 + x.double() * (1 - s)))
+    close(out[:, C:].double(), want)
+    assert not out[:, :C].any()
