@@ -111,6 +111,14 @@ SIGNATURES = {
     "cssm_depthwise_conv_wgrad_supported": (_I, [_I, _I, _I]),
     "cssm_gdn_scan_bins_train": (_I, [_P, _P, _LL, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P]),
     "cssm_gdn_scan_bins_bwd": (_I, [_P, _P, _LL, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P]),
+    "cssm_gdn_core_train": (_I, [_P, _P, _P, _LL, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P]),
+    "cssm_gdn_core_bwd": (_I, [_P, _P, _P, _LL, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P]),
+    "cssm_gdn_qkv_act": (_I, [_P, _LL, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P]),
+    "cssm_gdn_qkv_act_bwd_blocks": (_I, [_I, _I, _I]),
+    "cssm_gdn_qkv_act_bwd": (_I, [_P, _LL, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P, _LL, _P, _P, _P]),
+    "cssm_gdn_norm_gate": (_I, [_P, _P, _LL, _I, _I, _I, _I, _I, _P, _P, _P, _P]),
+    "cssm_gdn_norm_gate_blocks": (_I, [_I, _I]),
+    "cssm_gdn_norm_gate_bwd": (_I, [_P, _P, _LL, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _LL, _P, _P]),
     "cssm_gdn_proj_out": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P]),
     "cssm_gdn_proj_out_xgate": (_I, [_P, _I, _P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P, _P, _P, _I, _P]),
     "cssm_gdn_proj_out_xgate_supported": (_I, [_I, _I, _I]),

@@ -677,10 +677,10 @@ int cssm_gdn_scan_bins_train(const float* spec, const float* ab, long long ab_fr
   if (!aligned(spec, 8) || !aligned(ab, 8) || !aligned(what, 8) || !aligned(ohat, 8) || !aligned(states, 8))
     return fail(CSSM_ERR_ALIGN, "cssm_gdn_scan_bins_train: complex tensors must be 8-byte aligned");
   return hip_status(cssm::launch_gdn_scan_bins_train(
-                        reinterpret_cast<const float2*>(spec), reinterpret_cast<const float2*>(ab), ab_frame, ab_head,
-                        ab_bin, reinterpret_cast<const float2*>(what), B, T, C, H, W, dk, scan_variant,
+                        reinterpret_cast<const float2*>(spec), nullptr, reinterpret_cast<const float2*>(ab), ab_frame,
+                        ab_head, ab_bin, reinterpret_cast<const float2*>(what), B, T, C, H, W, dk, scan_variant,
                         reinterpret_cast<float2*>(ohat), reinterpret_cast<float2*>(states), nullptr, nullptr, nullptr,
-                        nullptr, false, static_cast<hipStream_t>(stream)),
+                        nullptr, false, false, static_cast<hipStream_t>(stream)),
                     "cssm_gdn_scan_bins_train");
 }
 
@@ -695,13 +695,141 @@ int cssm_gdn_scan_bins_bwd(const float* spec, const float* ab, long long ab_fram
       !aligned(dspec, 8) || !aligned(dab, 8) || !aligned(dwhat, 8))
     return fail(CSSM_ERR_ALIGN, "cssm_gdn_scan_bins_bwd: complex tensors must be 8-byte aligned");
   return hip_status(cssm::launch_gdn_scan_bins_train(
-                        reinterpret_cast<const float2*>(spec), reinterpret_cast<const float2*>(ab), ab_frame, ab_head,
-                        ab_bin, reinterpret_cast<const float2*>(what), B, T, C, H, W, dk, scan_variant, nullptr,
+                        reinterpret_cast<const float2*>(spec), nullptr, reinterpret_cast<const float2*>(ab), ab_frame,
+                        ab_head, ab_bin, reinterpret_cast<const float2*>(what), B, T, C, H, W, dk, scan_variant, nullptr,
                         const_cast<float2*>(reinterpret_cast<const float2*>(states)),
                         reinterpret_cast<const float2*>(dohat), reinterpret_cast<float2*>(dspec),
-                        reinterpret_cast<float2*>(dab), reinterpret_cast<float2*>(dwhat), true,
+                        reinterpret_cast<float2*>(dab), reinterpret_cast<float2*>(dwhat), true, false,
                         static_cast<hipStream_t>(stream)),
                     "cssm_gdn_scan_bins_bwd");
+}
+
+int cssm_gdn_core_train(const float* spec, const float* norms, const float* ab, long long ab_frame, int ab_head,
+                        int ab_bin, const float* what, int B, int T, int C, int H, int W, int dk, int scan_variant,
+                        float* ohat, float* states, void* stream) {
+  if (!spec || !ab || !what || !ohat || !states)
+    return fail(CSSM_ERR_NULL, "cssm_gdn_core_train: spec, ab, what, ohat and states must be non-null");
+  if (int e = gdn_train_check("cssm_gdn_core_train", B, T, C, H, W, dk, ab_frame, ab_head, ab_bin)) return e;
+  if (int e = gdn_variant_check("cssm_gdn_core_train", scan_variant)) return e;
+  if (!aligned(spec, 8) || !aligned(ab, 8) || !aligned(what, 8) || !aligned(ohat, 8) || !aligned(states, 8))
+    return fail(CSSM_ERR_ALIGN, "cssm_gdn_core_train: complex tensors must be 8-byte aligned");
+  return hip_status(cssm::launch_gdn_scan_bins_train(
+                        reinterpret_cast<const float2*>(spec), norms, reinterpret_cast<const float2*>(ab), ab_frame,
+                        ab_head, ab_bin, reinterpret_cast<const float2*>(what), B, T, C, H, W, dk, scan_variant,
+                        reinterpret_cast<float2*>(ohat), reinterpret_cast<float2*>(states), nullptr, nullptr, nullptr,
+                        nullptr, false, true, static_cast<hipStream_t>(stream)),
+                    "cssm_gdn_core_train");
+}
+
+int cssm_gdn_core_bwd(const float* spec, const float* norms, const float* ab, long long ab_frame, int ab_head,
+                      int ab_bin, const float* what, const float* states, const float* dospec, int B, int T, int C,
+                      int H, int W, int dk, int scan_variant, float* dspec, float* dab, float* dwhat, void* stream) {
+  if (!spec || !ab || !what || !states || !dospec || !dspec || !dab || !dwhat)
+    return fail(CSSM_ERR_NULL, "cssm_gdn_core_bwd: null argument");
+  if (int e = gdn_train_check("cssm_gdn_core_bwd", B, T, C, H, W, dk, ab_frame, ab_head, ab_bin)) return e;
+  if (int e = gdn_variant_check("cssm_gdn_core_bwd", scan_variant)) return e;
+  if ((long long)B * T * 2 * C > 0x7fffffffLL)
+    return fail(CSSM_ERR_SHAPE, "cssm_gdn_core_bwd: B=%d T=%d C=%d", B, T, C);
+  if (!aligned(spec, 8) || !aligned(ab, 8) || !aligned(what, 8) || !aligned(states, 8) || !aligned(dospec, 8) ||
+      !aligned(dspec, 8) || !aligned(dab, 8) || !aligned(dwhat, 8))
+    return fail(CSSM_ERR_ALIGN, "cssm_gdn_core_bwd: complex tensors must be 8-byte aligned");
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  hipError_t e = cssm::launch_gdn_scan_bins_train(
+      reinterpret_cast<const float2*>(spec), norms, reinterpret_cast<const float2*>(ab), ab_frame, ab_head, ab_bin,
+      reinterpret_cast<const float2*>(what), B, T, C, H, W, dk, scan_variant, nullptr,
+      const_cast<float2*>(reinterpret_cast<const float2*>(states)), reinterpret_cast<const float2*>(dospec),
+      reinterpret_cast<float2*>(dspec), reinterpret_cast<float2*>(dab), reinterpret_cast<float2*>(dwhat), true, true,
+      st);
+  if (e == hipSuccess && norms)
+    e = cssm::launch_spec_norm_bwd(reinterpret_cast<const float2*>(spec), norms, reinterpret_cast<float2*>(dspec),
+                                   B * T, C, H, W, st);
+  return hip_status(e, "cssm_gdn_core_bwd");
+}
+
+static int qkv_act_args(const char* fn, const float* raw, long long raw_fs, int B, int T, int C, int HW, int kt,
+                        const float* const* conv_kernel, const float* const* conv_bias, int gate_mode,
+                        const float* gates, cssm::QkvActArgs& a) {
+  if (!raw || (kt > 0 && (!conv_kernel || !conv_bias)) || (gate_mode && !gates))
+    return fail(CSSM_ERR_NULL, "%s: null argument", fn);
+  if (B <= 0 || T <= 0 || C <= 0 || HW <= 0 || B > 65535 || kt < 0 || kt > 8 || raw_fs < 3LL * C * HW ||
+      (long long)B * T > 0x7fffffffLL || (3 * ((C + 7) / 8) + 3) / 4 > 65535)
+    return fail(CSSM_ERR_SHAPE, "%s: B=%d T=%d C=%d HW=%d kt=%d", fn, B, T, C, HW, kt);
+  if (gate_mode < 0 || gate_mode > 3) return fail(CSSM_ERR_ARG, "%s: gate_mode=%d", fn, gate_mode);
+  if (HW % 4 == 0 && (!aligned(raw, 16) || raw_fs % 4 || (gate_mode && !aligned(gates, 16))))
+    return fail(CSSM_ERR_ALIGN, "%s: planes and gates must be 16-byte aligned", fn);
+  a = cssm::QkvActArgs{raw, raw_fs, B, T, C, HW, {}, gate_mode, gates};
+  for (int i = 0; i < 3 && kt > 0; ++i) {
+    if (!conv_kernel[i] || !conv_bias[i]) return fail(CSSM_ERR_NULL, "%s: short conv %d", fn, i);
+    a.sc.w[i] = conv_kernel[i];
+    a.sc.b[i] = conv_bias[i];
+  }
+  return CSSM_OK;
+}
+
+int cssm_gdn_qkv_act(const float* raw, long long raw_fs, int B, int T, int C, int HW, int kt,
+                     const float* const* conv_kernel, const float* const* conv_bias, int gate_mode,
+                     const float* gates, float* out, void* stream) {
+  cssm::QkvActArgs a;
+  if (int e = qkv_act_args("cssm_gdn_qkv_act", raw, raw_fs, B, T, C, HW, kt, conv_kernel, conv_bias, gate_mode, gates,
+                           a))
+    return e;
+  if (!out) return fail(CSSM_ERR_NULL, "cssm_gdn_qkv_act: out must be non-null");
+  if (HW % 4 == 0 && !aligned(out, 16)) return fail(CSSM_ERR_ALIGN, "cssm_gdn_qkv_act: out must be 16-byte aligned");
+  return hip_status(cssm::launch_qkv_act_fwd(a, kt, out, static_cast<hipStream_t>(stream)), "cssm_gdn_qkv_act");
+}
+
+int cssm_gdn_qkv_act_bwd_blocks(int B, int C, int HW) {
+  return B > 0 && C > 0 && HW > 0 ? cssm::qkv_act_bwd_blocks(B, C, HW) : 0;
+}
+
+int cssm_gdn_qkv_act_bwd(const float* raw, long long raw_fs, int B, int T, int C, int HW, int kt,
+                         const float* const* conv_kernel, const float* const* conv_bias, int gate_mode,
+                         const float* gates, const float* dout, float* draw, long long draw_fs, float* dgates,
+                         float* sums, void* stream) {
+  cssm::QkvActArgs a;
+  if (int e = qkv_act_args("cssm_gdn_qkv_act_bwd", raw, raw_fs, B, T, C, HW, kt, conv_kernel, conv_bias, gate_mode,
+                           gates, a))
+    return e;
+  if (!dout || !draw || !sums || (gate_mode && !dgates))
+    return fail(CSSM_ERR_NULL, "cssm_gdn_qkv_act_bwd: dout, draw, sums (and dgates with gates) must be non-null");
+  if (draw_fs < 3LL * C * HW) return fail(CSSM_ERR_SHAPE, "cssm_gdn_qkv_act_bwd: draw_fs=%lld", draw_fs);
+  if (HW % 4 == 0 && (!aligned(dout, 16) || !aligned(draw, 16) || draw_fs % 4 || !aligned(dgates, 16)))
+    return fail(CSSM_ERR_ALIGN, "cssm_gdn_qkv_act_bwd: planes must be 16-byte aligned");
+  return hip_status(cssm::launch_qkv_act_bwd(a, kt, dout, draw, draw_fs, dgates, sums,
+                                             static_cast<hipStream_t>(stream)),
+                    "cssm_gdn_qkv_act_bwd");
+}
+
+static int norm_gate_args(const char* fn, const float* o, const float* g, long long g_fs, int F, int C, int HW,
+                          int norm, int act) {
+  if (!o || !g) return fail(CSSM_ERR_NULL, "%s: null argument", fn);
+  if (F <= 0 || C <= 0 || HW <= 0 || g_fs < (long long)C * HW)
+    return fail(CSSM_ERR_SHAPE, "%s: F=%d C=%d HW=%d g_fs=%lld", fn, F, C, HW, g_fs);
+  if (norm < 0 || norm > 2 || act < 1 || act > 2) return fail(CSSM_ERR_ARG, "%s: norm=%d act=%d", fn, norm, act);
+  if (!cssm::norm_gate_train_supported(C)) return fail(CSSM_ERR_UNSUPPORTED, "%s: C=%d > 128", fn, C);
+  return CSSM_OK;
+}
+
+int cssm_gdn_norm_gate(const float* o, const float* g, long long g_fs, int F, int C, int HW, int norm, int act,
+                       const float* scale, const float* shift, float* y, void* stream) {
+  if (int e = norm_gate_args("cssm_gdn_norm_gate", o, g, g_fs, F, C, HW, norm, act)) return e;
+  if (!y) return fail(CSSM_ERR_NULL, "cssm_gdn_norm_gate: y must be non-null");
+  cssm::NormGateArgs a{o, g, g_fs, scale, shift, norm, act, y, nullptr, nullptr, 0, nullptr, C, HW};
+  return hip_status(cssm::launch_norm_gate_train(a, (long long)F * HW, false, static_cast<hipStream_t>(stream)),
+                    "cssm_gdn_norm_gate");
+}
+
+int cssm_gdn_norm_gate_blocks(int F, int HW) { return F > 0 && HW > 0 ? cssm::norm_gate_blocks((long long)F * HW) : 0; }
+
+int cssm_gdn_norm_gate_bwd(const float* o, const float* g, long long g_fs, int F, int C, int HW, int norm, int act,
+                           const float* scale, const float* shift, const float* dy, float* d_o, float* dg,
+                           long long dg_fs, float* sums, void* stream) {
+  if (int e = norm_gate_args("cssm_gdn_norm_gate_bwd", o, g, g_fs, F, C, HW, norm, act)) return e;
+  if (!dy || !d_o || !dg || !sums) return fail(CSSM_ERR_NULL, "cssm_gdn_norm_gate_bwd: null argument");
+  if (dg_fs < (long long)C * HW) return fail(CSSM_ERR_SHAPE, "cssm_gdn_norm_gate_bwd: dg_fs=%lld", dg_fs);
+  cssm::NormGateArgs a{o, g, g_fs, scale, shift, norm, act, d_o, dy, dg, dg_fs, sums, C, HW};
+  return hip_status(cssm::launch_norm_gate_train(a, (long long)F * HW, true, static_cast<hipStream_t>(stream)),
+                    "cssm_gdn_norm_gate_bwd");
 }
 
 int cssm_depthwise_conv_wgrad_supported(int W, int C, int ks) { return cssm::dwconv_wgrad_supported(W, C, ks) ? 1 : 0; }

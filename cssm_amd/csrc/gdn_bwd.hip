@@ -22,6 +22,10 @@
 // entry; the log-eps scan's map f(x) = x (1 + 1e-8 / |x|) stretches the
 // tangential part of the gradient, df^T g = g + (1e-8 / |x|) Re(conj(g) i u) i u
 // with u = x / |x| (its constant 1e-8 at x = 0 passes none).
+// s_t for dq is the state entering step t + 1, already loaded there (only the last step's is advanced
+// again), and where the forward's rank-1 form applies (no mapped entry) the adjoint takes it too, without
+// M's entries: about a third of the arithmetic of the entry-by-entry form, which bounded the reverse pass
+// (32 x 8 frames, 16 heads, 32 x 32, d_k = 4: 627 -> 308 us, 2.5 TB/s).
 // The key normalisation's backward is
 //   dk = n dk' - n^3 k Re(sum_l dk'_l conj(k_l)),   n = (|k|^2 + 1e-6)^(-1/2).
 #include <hip/hip_runtime.h>
@@ -34,7 +38,8 @@
 namespace cssm {
 
 struct GdnTrainArgs {
-  const float2* spec;    // (B, T, 3C, H, WF): q and k with the spectral norms applied, v
+  const float2* spec;    // (B, T, 3C, H, WF): q and k (with the spectral norms applied if norms is null), v
+  const float* norms;    // (B, T, 3C) sums |X|^2 of the planes of spec, or null
   const float2* ab;      // (alpha, beta) at (b T + t) ab_frame + head ab_head + bin ab_bin
   long long ab_frame;
   int ab_head, ab_bin;
@@ -47,7 +52,16 @@ struct GdnTrainArgs {
   float2* dwhat;         // (B, n_h, H WF) reverse out: dW_hat summed over t, per batch element
   int T, C, HWF;
   int variant;           // kScanGoom / kScanLinear / kScanLogEps (gdn_step.h)
+  // planes: dohat is rfft2 of the output planes' gradient and dspec's planes go into irfft2, so the
+  // transforms' adjoint factors c_v / (H W) and H W / c_v are applied here (W > 0), the latter to q and
+  // k only without norms (else spec_norm_bwd applies it)
+  int H, W;
 };
+
+// the spectral L2 norm's factor of plane ch (cssm.py:4890-4897)
+__device__ __forceinline__ float spec_rnorm(const GdnTrainArgs& a, size_t ch) {
+  return a.norms ? 1.0f / sqrtf(a.norms[ch] + 1e-6f) : 1.0f;
+}
 
 template <int DK>
 __device__ __forceinline__ size_t state_at(const GdnTrainArgs& a, int b, int t, int head, int i, int c, int bin) {
@@ -76,6 +90,13 @@ __global__ void __launch_bounds__(256) gdn_scan_bins_save(const GdnTrainArgs a) 
       q[j] = a.spec[(ch0 + j) * HWF + bin];
       k[j] = a.spec[(ch0 + C + j) * HWF + bin];
       v[j] = a.spec[(ch0 + 2 * C + j) * HWF + bin];
+    }
+    if (a.norms) {
+#pragma unroll
+      for (int j = 0; j < DK; ++j) {
+        q[j] = cscale(q[j], spec_rnorm(a, ch0 + j));
+        k[j] = cscale(k[j], spec_rnorm(a, ch0 + C + j));
+      }
     }
 #pragma unroll
     for (int i = 0; i < DK; ++i)
@@ -142,6 +163,11 @@ __global__ void __launch_bounds__(256) gdn_scan_bins_bwd(const GdnTrainArgs a) {
 #pragma unroll
     for (int j = 0; j < DK; ++j) carry[i][j] = make_float2(0.f, 0.f);
   float2 dwh = make_float2(0.f, 0.f);
+  const int col = a.W > 0 ? bin % (a.W / 2 + 1) : 0;
+  const float cv = col == 0 || 2 * col == a.W ? 1.0f : 2.0f, hw = float(a.H) * float(a.W);
+  const float in_w = a.W > 0 ? cv / hw : 1.0f, out_w = a.W > 0 ? hw / cv : 1.0f;
+  const float qk_w = a.norms ? 1.0f : out_w;
+  float2 st[DK][DK];   // s_t: the state leaving step t, which is the one entering step t + 1
   for (int t = a.T - 1; t >= 0; --t) {
     const size_t fr = size_t(b) * a.T + t;
     const size_t ch0 = fr * 3 * C + size_t(head) * DK;
@@ -159,17 +185,34 @@ __global__ void __launch_bounds__(256) gdn_scan_bins_bwd(const GdnTrainArgs a) {
       for (int c = 0; c < DK; ++c) sp[i][c] = a.states[state_at<DK>(a, b, t, head, i, c, bin)];
     const float2 g2 = a.ab[fr * a.ab_frame + size_t(head) * a.ab_head + size_t(bin) * a.ab_bin];
     const float alpha = g2.x, beta = g2.y;
-    // key-vector normalisation, as gdn_bin_step
+#pragma unroll
+    for (int j = 0; j < DK; ++j) {
+      if (a.norms) {
+        q[j] = cscale(q[j], spec_rnorm(a, ch0 + j));
+        kr[j] = cscale(kr[j], spec_rnorm(a, ch0 + C + j));
+      }
+      dov[j] = cscale(dov[j], in_w);
+    }
+    // key-vector normalisation and the form of the step, as gdn_bin_step
     float kk = 0.0f;
 #pragma unroll
     for (int j = 0; j < DK; ++j) kk = fmaf(kr[j].x, kr[j].x, fmaf(kr[j].y, kr[j].y, kk));
     const float kn = 1.0f / sqrtf(kk + 1e-6f);
     float2 k[DK];
 #pragma unroll
-    for (int j = 0; j < DK; ++j) k[j] = cscale(kr[j], kn);
-    const float2 aw = cscale(wh, alpha);
+    for (int j = 0; j < DK; ++j) k[j] = kr[j];
+    const GdnBinPre<DK> pre = gdn_bin_prep<DK>(k, v, wh, alpha, beta, variant);
+    const float2 aw = pre.aw;
+    if (t == a.T - 1) {
+#pragma unroll
+      for (int i = 0; i < DK; ++i) {
+#pragma unroll
+        for (int c = 0; c < DK; ++c) st[i][c] = sp[i][c];
+        gdn_bin_row<DK>(st[i], v[i], q, k, pre, beta, variant);
+      }
+    }
 
-    // s_t (recomputed from s_{t-1}) for dq; g = carry + do conj(q)
+    // dq_r = sum_i do_i conj(s_t[i][r]); g = carry + do conj(q)
     float2 dq[DK], g[DK][DK];
 #pragma unroll
     for (int r = 0; r < DK; ++r) dq[r] = make_float2(0.f, 0.f);
@@ -177,69 +220,90 @@ __global__ void __launch_bounds__(256) gdn_scan_bins_bwd(const GdnTrainArgs a) {
     for (int i = 0; i < DK; ++i)
 #pragma unroll
       for (int r = 0; r < DK; ++r) {
-        bool fl;
-        float2 xd;
-        float2 st = d_entry(beta, v[i], k[r], variant, xd, fl);
-#pragma unroll
-        for (int c = 0; c < DK; ++c) {
-          float2 m, xm;
-          bool fm;
-          const float2 M = m_entry(aw, beta, k[r], k[c], r == c, variant, m, xm, fm);
-          st = cadd(st, cmul(M, sp[i][c]));
-        }
-        dq[r] = cadd(dq[r], cmulc(dov[i], st));
+        dq[r] = cadd(dq[r], cmulc(dov[i], st[i][r]));
         g[i][r] = cadd(carry[i][r], cmulc(dov[i], q[r]));
+        st[i][r] = sp[i][r];
       }
 
-    // through M: carry' = M^H g, and the inputs of the entries the floor left alone
     float2 dk[DK], dv[DK];
 #pragma unroll
     for (int j = 0; j < DK; ++j) dk[j] = dv[j] = make_float2(0.f, 0.f);
     float2 daw = make_float2(0.f, 0.f);
     float dbeta = 0.0f;
+    if (pre.rank1) {
+      // no entry of M or D is mapped: row i of the step is s_i <- aW (s_i - beta k p_i) + beta v_i k^H with
+      // p_i = k^H s_i, whose adjoint needs no entry of M (with a_i = conj(aW) g_i, e_i = k^H a_i):
+      //   carry_i = a_i - beta k e_i,  daW += g_i . conj(s_i - beta k p_i),  dv_i = beta g_i . k,
+      //   dbeta += Re(conj(g_i . k) v_i) - Re(conj(e_i) p_i),
+      //   dk += beta (conj(g_i) v_i - conj(p_i) a_i - conj(e_i) s_i)
 #pragma unroll
-    for (int i = 0; i < DK; ++i)
+      for (int i = 0; i < DK; ++i) {
+        float2 ar[DK], e = make_float2(0.f, 0.f), p = e, gk = e;
 #pragma unroll
-      for (int c = 0; c < DK; ++c) carry[i][c] = make_float2(0.f, 0.f);
-#pragma unroll
-    for (int r = 0; r < DK; ++r)
-#pragma unroll
-      for (int c = 0; c < DK; ++c) {
-        float2 m, xm;
-        bool fm;
-        const float2 M = m_entry(aw, beta, k[r], k[c], r == c, variant, m, xm, fm);
-        float2 dM = make_float2(0.f, 0.f);
-#pragma unroll
-        for (int i = 0; i < DK; ++i) {
-          carry[i][c] = cadd(carry[i][c], cmulc(g[i][r], M));   // conj(M) g
-          dM = cadd(dM, cmulc(g[i][r], sp[i][c]));             // g conj(s_{t-1})
+        for (int r = 0; r < DK; ++r) {
+          ar[r] = cmulc(g[i][r], aw);
+          e = cadd(e, cmulc(ar[r], k[r]));
+          p = cadd(p, cmulc(sp[i][r], k[r]));
+          gk = cadd(gk, cmul(g[i][r], k[r]));
         }
-        if (!fm) {
-          dM = entry_adjoint(dM, xm, variant);                 // dL/d(aW m)
-          daw = cadd(daw, cmulc(dM, m));                       // dM conj(m)
-          const float2 dm = cmulc(dM, aw);                     // dM conj(aW)
-          // m = delta - beta k_r conj(k_c)
-          const float2 kk_rc = cmulc(k[r], k[c]);
-          dbeta -= dm.x * kk_rc.x + dm.y * kk_rc.y;            // Re(conj(dm) k_r conj(k_c))
-          dk[r] = cadd(dk[r], cscale(cmul(dm, k[c]), -beta));
-          dk[c] = cadd(dk[c], cscale(cmul(make_float2(dm.x, -dm.y), k[r]), -beta));
+        dbeta += gk.x * v[i].x + gk.y * v[i].y - (e.x * p.x + e.y * p.y);
+        dv[i] = cscale(gk, beta);
+        const float2 bp = cscale(p, beta), be = cscale(e, beta), bv = cscale(v[i], beta);
+#pragma unroll
+        for (int r = 0; r < DK; ++r) {
+          const float2 kp = cmul(k[r], bp), ke = cmul(k[r], be);
+          daw = cadd(daw, cmulc(g[i][r], make_float2(sp[i][r].x - kp.x, sp[i][r].y - kp.y)));
+          carry[i][r] = make_float2(ar[r].x - ke.x, ar[r].y - ke.y);
+          const float2 x = cmulc(bv, g[i][r]), y = cmulc(ar[r], bp), z = cmulc(sp[i][r], be);
+          dk[r] = make_float2(dk[r].x + (x.x - y.x - z.x), dk[r].y + (x.y - y.y - z.y));
         }
       }
-    // through D[i][r] = beta v_i conj(k_r)
+    } else {
+      // through M: carry' = M^H g, and the inputs of the entries the floor left alone
 #pragma unroll
-    for (int i = 0; i < DK; ++i)
+      for (int i = 0; i < DK; ++i)
 #pragma unroll
-      for (int r = 0; r < DK; ++r) {
-        bool fl;
-        float2 xd;
-        d_entry(beta, v[i], k[r], variant, xd, fl);
-        if (fl) continue;
-        const float2 dD = entry_adjoint(g[i][r], xd, variant);
-        const float2 vk = cmulc(v[i], k[r]);
-        dbeta += dD.x * vk.x + dD.y * vk.y;                    // Re(conj(dD) v_i conj(k_r))
-        dv[i] = cadd(dv[i], cscale(cmul(dD, k[r]), beta));
-        dk[r] = cadd(dk[r], cscale(cmul(make_float2(dD.x, -dD.y), v[i]), beta));
-      }
+        for (int c = 0; c < DK; ++c) carry[i][c] = make_float2(0.f, 0.f);
+#pragma unroll
+      for (int r = 0; r < DK; ++r)
+#pragma unroll
+        for (int c = 0; c < DK; ++c) {
+          float2 m, xm;
+          bool fm;
+          const float2 M = m_entry(aw, beta, k[r], k[c], r == c, variant, m, xm, fm);
+          float2 dM = make_float2(0.f, 0.f);
+#pragma unroll
+          for (int i = 0; i < DK; ++i) {
+            carry[i][c] = cadd(carry[i][c], cmulc(g[i][r], M));   // conj(M) g
+            dM = cadd(dM, cmulc(g[i][r], sp[i][c]));             // g conj(s_{t-1})
+          }
+          if (!fm) {
+            dM = entry_adjoint(dM, xm, variant);                 // dL/d(aW m)
+            daw = cadd(daw, cmulc(dM, m));                       // dM conj(m)
+            const float2 dm = cmulc(dM, aw);                     // dM conj(aW)
+            // m = delta - beta k_r conj(k_c)
+            const float2 kk_rc = cmulc(k[r], k[c]);
+            dbeta -= dm.x * kk_rc.x + dm.y * kk_rc.y;            // Re(conj(dm) k_r conj(k_c))
+            dk[r] = cadd(dk[r], cscale(cmul(dm, k[c]), -beta));
+            dk[c] = cadd(dk[c], cscale(cmul(make_float2(dm.x, -dm.y), k[r]), -beta));
+          }
+        }
+      // through D[i][r] = beta v_i conj(k_r)
+#pragma unroll
+      for (int i = 0; i < DK; ++i)
+#pragma unroll
+        for (int r = 0; r < DK; ++r) {
+          bool fl;
+          float2 xd;
+          d_entry(beta, v[i], k[r], variant, xd, fl);
+          if (fl) continue;
+          const float2 dD = entry_adjoint(g[i][r], xd, variant);
+          const float2 vk = cmulc(v[i], k[r]);
+          dbeta += dD.x * vk.x + dD.y * vk.y;                    // Re(conj(dD) v_i conj(k_r))
+          dv[i] = cadd(dv[i], cscale(cmul(dD, k[r]), beta));
+          dk[r] = cadd(dk[r], cscale(cmul(make_float2(dD.x, -dD.y), v[i]), beta));
+        }
+    }
     // aW = alpha W_hat
     const float dalpha = daw.x * wh.x + daw.y * wh.y;          // Re(daW conj(W_hat))
     dwh = cadd(dwh, cscale(daw, alpha));
@@ -251,21 +315,22 @@ __global__ void __launch_bounds__(256) gdn_scan_bins_bwd(const GdnTrainArgs a) {
 #pragma unroll
     for (int j = 0; j < DK; ++j) {
       const float2 dkr = make_float2(kn * dk[j].x - kn3 * kr[j].x * red, kn * dk[j].y - kn3 * kr[j].y * red);
-      a.dspec[(ch0 + j) * HWF + bin] = dq[j];
-      a.dspec[(ch0 + C + j) * HWF + bin] = dkr;
-      a.dspec[(ch0 + 2 * C + j) * HWF + bin] = dv[j];
+      a.dspec[(ch0 + j) * HWF + bin] = cscale(dq[j], qk_w);
+      a.dspec[(ch0 + C + j) * HWF + bin] = cscale(dkr, qk_w);
+      a.dspec[(ch0 + 2 * C + j) * HWF + bin] = cscale(dv[j], out_w);
     }
     a.dab[(fr * nh + head) * HWF + bin] = make_float2(dalpha, dbeta);
   }
   a.dwhat[(size_t(b) * nh + head) * HWF + bin] = dwh;
 }
 
-hipError_t launch_gdn_scan_bins_train(const float2* spec, const float2* ab, long long ab_frame, int ab_head,
-                                      int ab_bin, const float2* what, int B, int T, int C, int H, int W, int dk,
-                                      int variant, float2* ohat, float2* states, const float2* dohat, float2* dspec,
-                                      float2* dab, float2* dwhat, bool backward, hipStream_t s) {
-  GdnTrainArgs a{spec, ab, ab_frame, ab_head, ab_bin, what, ohat, states, dohat, dspec, dab, dwhat, T, C,
-                 H * (W / 2 + 1), variant};
+hipError_t launch_gdn_scan_bins_train(const float2* spec, const float* norms, const float2* ab, long long ab_frame,
+                                      int ab_head, int ab_bin, const float2* what, int B, int T, int C, int H, int W,
+                                      int dk, int variant, float2* ohat, float2* states, const float2* dohat,
+                                      float2* dspec, float2* dab, float2* dwhat, bool backward, bool planes,
+                                      hipStream_t s) {
+  GdnTrainArgs a{spec, norms, ab, ab_frame, ab_head, ab_bin, what, ohat, states, dohat, dspec, dab, dwhat, T, C,
+                 H * (W / 2 + 1), variant, H, planes ? W : 0};
   const dim3 grid(unsigned((a.HWF + 255) / 256), unsigned(C / dk), unsigned(B));
 #define CSSM_GDN_TRAIN(D)                                                                   \
   if (backward) hipLaunchKernelGGL(gdn_scan_bins_bwd<D>, grid, dim3(256), 0, s, a);         \

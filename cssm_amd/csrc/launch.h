@@ -180,10 +180,45 @@ hipError_t launch_dwconv_wgrad(const float* x, const float* dy, int F, int H, in
                                int blocks, hipStream_t s);
 // training: forward with the state entering every step saved (backward = false), or the reverse
 // pass from those states (backward = true); gdn_bwd.hip
-hipError_t launch_gdn_scan_bins_train(const float2* spec, const float2* ab, long long ab_frame, int ab_head,
-                                      int ab_bin, const float2* what, int B, int T, int C, int H, int W, int dk,
-                                      int variant, float2* ohat, float2* states, const float2* dohat, float2* dspec,
-                                      float2* dab, float2* dwhat, bool backward, hipStream_t s);
+hipError_t launch_gdn_scan_bins_train(const float2* spec, const float* norms, const float2* ab, long long ab_frame,
+                                      int ab_head, int ab_bin, const float2* what, int B, int T, int C, int H, int W,
+                                      int dk, int variant, float2* ohat, float2* states, const float2* dohat,
+                                      float2* dspec, float2* dab, float2* dwhat, bool backward, bool planes,
+                                      hipStream_t s);
+// adjoint of the spectral L2 norm of q and k in place on dspec, with rfft2's adjoint factors; gdn_train.hip
+hipError_t launch_spec_norm_bwd(const float2* spec, const float* norms, float2* dspec, int F, int C, int H, int W,
+                                hipStream_t s);
+// training: short conv + SiLU + input gates of q | k | v and their adjoint (gdn_train.hip)
+struct QkvActArgs {
+  const float* raw;      // (F, 3C, HW) projections, frame stride raw_fs floats
+  long long raw_fs;
+  int B, T, C, HW;
+  GdnShortConv sc;
+  int gate_mode;         // 0 none, 1 gates (2, F, HW), 2 (2, F), 3 (F, 2C, HW)
+  const float* gates;
+};
+int qkv_act_bwd_blocks(int B, int C, int HW);
+hipError_t launch_qkv_act_fwd(const QkvActArgs& a, int kt, float* out, hipStream_t s);
+hipError_t launch_qkv_act_bwd(const QkvActArgs& a, int kt, const float* dout, float* draw, long long draw_fs,
+                              float* gpart, float* wpart, hipStream_t s);
+// training: y = (norm(o) scale + shift) act(g) per pixel, and its adjoint (y = do, part (blocks, 3, C))
+struct NormGateArgs {
+  const float* o;        // (F, C, HW)
+  const float* g;        // gate pre-activation, frame stride g_fs floats
+  long long g_fs;
+  const float* scale;
+  const float* shift;
+  int norm, act;         // 0 none, 1 rms, 2 layer; 1 SiLU, 2 sigmoid
+  float* y;              // forward: y (F, C, HW); adjoint: do
+  const float* dy;
+  float* dg;             // frame stride dg_fs floats
+  long long dg_fs;
+  float* part;
+  int C, HW;
+};
+bool norm_gate_train_supported(int C);
+int norm_gate_blocks(long long M);
+hipError_t launch_norm_gate_train(const NormGateArgs& a, long long M, bool bwd, hipStream_t s);
 // backward of the gated scan: the spectral-domain reverse recurrence per (b, bin), T <= 32
 hipError_t launch_gated_scan_bwd_bins(const float2* uspec, const float2* dspec, const float4* gates,
                                       const float2* khat, int B, int T, int C, int H, int W, float c_scale,

@@ -853,6 +853,137 @@ def gdn_scan_bins_backward(spec: torch.Tensor, ab: torch.Tensor, gate_type: str,
     return dspec, dab, dwhat
 
 
+def gdn_core_train(spec: torch.Tensor, norms: Optional[torch.Tensor], ab: torch.Tensor, gate_type: str,
+                   what: torch.Tensor, delta_key_dim: int, W: int, scan_variant: str = "goom"):
+    """Training forward of the delta rule on the planes' own spectra (cssm_gdn_core_train): spec
+    (B, T, 3C, H, Wf) and norms (B, T, 3C) or None from :func:`rfft2`.  Returns (ohat, states) as
+    :func:`gdn_scan_bins_train`."""
+    _dev(spec, "spec", torch.complex64)
+    _dev(ab, "ab", torch.float32)
+    _dev(what, "what", torch.complex64)
+    B, T, C3, H, Wf = spec.shape
+    C, dk = C3 // 3, delta_key_dim
+    fs, hs, bs = _ab_strides(ab, gate_type)
+    ohat = torch.empty((B, T, C, H, Wf), dtype=torch.complex64, device=spec.device)
+    states = torch.empty((B, T, C // dk, dk, dk, H * Wf), dtype=torch.complex64, device=spec.device)
+    _lib.call("cssm_gdn_core_train", spec.data_ptr(), norms.data_ptr() if norms is not None else None, ab.data_ptr(),
+              fs, hs, bs, what.data_ptr(), B, T, C, H, W, dk, _variant(scan_variant), ohat.data_ptr(),
+              states.data_ptr(), _stream())
+    return ohat, states
+
+
+def gdn_core_backward(spec: torch.Tensor, norms: Optional[torch.Tensor], ab: torch.Tensor, gate_type: str,
+                      what: torch.Tensor, states: torch.Tensor, dospec: torch.Tensor, delta_key_dim: int, W: int,
+                      scan_variant: str = "goom"):
+    """Reverse pass of :func:`gdn_core_train` (cssm_gdn_core_bwd) from dospec = rfft2 of the output planes'
+    gradient: (dspec, whose irfft2 is the gradient of the q, k, v planes; dab; dwhat) as
+    :func:`gdn_scan_bins_backward`."""
+    for t, n in ((spec, "spec"), (what, "what"), (states, "states"), (dospec, "dospec")):
+        _dev(t, n, torch.complex64)
+    _dev(ab, "ab", torch.float32)
+    B, T, C3, H, Wf = spec.shape
+    C, dk = C3 // 3, delta_key_dim
+    if tuple(dospec.shape) != (B, T, C, H, Wf) or tuple(states.shape) != (B, T, C // dk, dk, dk, H * Wf):
+        raise ValueError("dospec / states shapes do not match spec")
+    fs, hs, bs = _ab_strides(ab, gate_type)
+    dspec = torch.empty_like(spec)
+    dab = torch.empty((B, T, C // dk, H * Wf, 2), dtype=torch.float32, device=spec.device)
+    dwhat = torch.empty((B, C // dk, H, Wf), dtype=torch.complex64, device=spec.device)
+    _lib.call("cssm_gdn_core_bwd", spec.data_ptr(), norms.data_ptr() if norms is not None else None, ab.data_ptr(), fs,
+              hs, bs, what.data_ptr(), states.data_ptr(), dospec.data_ptr(), B, T, C, H, W, dk,
+              _variant(scan_variant), dspec.data_ptr(), dab.data_ptr(), dwhat.data_ptr(), _stream())
+    return dspec, dab, dwhat
+
+
+def _frames(t: torch.Tensor, name: str, C: int, HW: int) -> int:
+    """Frame stride in floats of a float32 (F, C, HW) channel slice of a plane-major tensor."""
+    if not isinstance(t, torch.Tensor) or t.device.type != "cuda" or t.dtype != torch.float32:
+        raise ValueError(f"{name} must be a float32 GPU tensor")
+    if t.dim() != 3 or t.shape[1:] != (C, HW) or t.stride(2) != 1 or t.stride(1) != HW or t.stride(0) < C * HW:
+        raise ValueError(f"{name}: a (F, {C}, {HW}) channel slice of a plane-major tensor is needed")
+    return t.stride(0)
+
+
+def _conv_ptrs(convs):
+    if not convs:
+        return 0, None, None
+    ks = [_dev(convs[2 * i], "short_conv.kernel", torch.float32) for i in range(3)]
+    bs = [_dev(convs[2 * i + 1], "short_conv.bias", torch.float32) for i in range(3)]
+    return (ks[0].shape[0], (ctypes.c_void_p * 3)(*[k.data_ptr() for k in ks]),
+            (ctypes.c_void_p * 3)(*[b.data_ptr() for b in bs]))
+
+
+def gdn_qkv_act(raw: torch.Tensor, B: int, T: int, convs, gate_mode: int, gates: Optional[torch.Tensor]):
+    """out (F, 3C, HW) = gate SiLU(short conv(raw)) of raw (F, 3C, HW), a channel slice of a plane-major tensor
+    (cssm_gdn_qkv_act); convs = (kernel_q, bias_q, kernel_k, ...) or (), gates as the entry point's modes."""
+    F, C3, HW = raw.shape
+    fs = _frames(raw, "raw", C3, HW)
+    kt, kern, cb = _conv_ptrs(convs)
+    out = torch.empty((F, C3, HW), dtype=torch.float32, device=raw.device)
+    gp = _dev(gates, "gates", torch.float32).data_ptr() if gate_mode else None
+    _lib.call("cssm_gdn_qkv_act", raw.data_ptr(), fs, B, T, C3 // 3, HW, kt, kern, cb, gate_mode, gp, out.data_ptr(),
+              _stream())
+    return out
+
+
+def gdn_qkv_act_backward(raw: torch.Tensor, B: int, T: int, convs, gate_mode: int, gates: Optional[torch.Tensor],
+                         dout: torch.Tensor, draw: torch.Tensor):
+    """Adjoint of :func:`gdn_qkv_act`: writes draw (F, 3C, HW) (a channel slice allowed) and returns (dgates of
+    gates' shape or None, sums (3C, kt + 2): the taps', the conv bias's and draw's sums)."""
+    F, C3, HW = raw.shape
+    C = C3 // 3
+    fs, dfs = _frames(raw, "raw", C3, HW), _frames(draw, "draw", C3, HW)
+    _dev(dout, "dout", torch.float32)
+    kt, kern, cb = _conv_ptrs(convs)
+    n = int(_lib.load().cssm_gdn_qkv_act_bwd_blocks(B, C, HW))
+    sums = torch.empty((B, n, C3, kt + 2), dtype=torch.float32, device=raw.device)
+    dg = None
+    if gate_mode:
+        _dev(gates, "gates", torch.float32)
+        dg = torch.empty((F, 2 * C, HW) if gate_mode == 3 else (2, (C + 7) // 8, F, HW), dtype=torch.float32,
+                         device=raw.device)
+    _lib.call("cssm_gdn_qkv_act_bwd", raw.data_ptr(), fs, B, T, C, HW, kt, kern, cb, gate_mode,
+              gates.data_ptr() if gate_mode else None, dout.data_ptr(), draw.data_ptr(), dfs,
+              dg.data_ptr() if dg is not None else None, sums.data_ptr(), _stream())
+    if gate_mode in (1, 2):
+        dg = dg.sum(dim=1) if gate_mode == 1 else dg.sum(dim=(1, 3))
+    return dg, sums.sum(dim=(0, 1))
+
+
+def gdn_norm_gate_supported(C: int) -> bool:
+    return C <= 128
+
+
+def gdn_norm_gate(o: torch.Tensor, g: torch.Tensor, norm: str, scale: Optional[torch.Tensor],
+                  shift: Optional[torch.Tensor], act: str) -> torch.Tensor:
+    """y = (norm(o) scale + shift) act(g) per pixel over the channels of plane-major o, g (F, C, HW), g a channel
+    slice allowed (cssm_gdn_norm_gate)."""
+    _dev(o, "o", torch.float32)
+    F, C, HW = o.shape
+    y = torch.empty_like(o)
+    _lib.call("cssm_gdn_norm_gate", o.data_ptr(), g.data_ptr(), _frames(g, "g", C, HW), F, C, HW, _NORMS[norm],
+              _ACTS[act], scale.data_ptr() if scale is not None else None,
+              shift.data_ptr() if shift is not None else None, y.data_ptr(), _stream())
+    return y
+
+
+def gdn_norm_gate_backward(o: torch.Tensor, g: torch.Tensor, norm: str, scale: Optional[torch.Tensor],
+                           shift: Optional[torch.Tensor], act: str, dy: torch.Tensor, dg: torch.Tensor):
+    """Adjoint of :func:`gdn_norm_gate`: writes dg (a channel slice allowed) and returns (do, sums (3, C): the
+    gradients of scale and shift, and the sum of dg)."""
+    _dev(o, "o", torch.float32)
+    _dev(dy, "dy", torch.float32)
+    F, C, HW = o.shape
+    do = torch.empty_like(o)
+    n = int(_lib.load().cssm_gdn_norm_gate_blocks(F, HW))
+    sums = torch.empty((n, 3, C), dtype=torch.float32, device=o.device)
+    _lib.call("cssm_gdn_norm_gate_bwd", o.data_ptr(), g.data_ptr(), _frames(g, "g", C, HW), F, C, HW, _NORMS[norm],
+              _ACTS[act], scale.data_ptr() if scale is not None else None,
+              shift.data_ptr() if shift is not None else None, dy.data_ptr(), do.data_ptr(), dg.data_ptr(),
+              _frames(dg, "dg", C, HW), sums.data_ptr(), _stream())
+    return do, sums.sum(dim=0)
+
+
 def gdn_core_fused_supported(H: int, W: int, delta_key_dim: int) -> bool:
     return bool(_lib.load().cssm_gdn_core_fused_supported(H, W, delta_key_dim))
 

@@ -475,34 +475,161 @@ def _temporal_encoding(T: int, C: int, base: float, device) -> torch.Tensor:
     return torch.stack([torch.sin(th), torch.cos(th)], -1).reshape(T, C).float()
 
 
-def _gdn_gate(p, name, gate_type, ctx, x, H, W, nh, bounded=False, spatial=False):
+def _gate_products(p, names, gate_type, ctx):
+    """{parameter name: ctx kernel + bias} of the named gates' Dense layers as one product (their kernels side
+    by side: one GEMM forward and two backward instead of up to eight of each)."""
+    keys = [f"{n}_{a}" for n in names for a in "hw"] if gate_type == "factored" else list(names)
+    out = torch.addmm(torch.cat([p[k]["bias"] for k in keys]), ctx.reshape(-1, ctx.shape[-1]),
+                      torch.cat([p[k]["kernel"] for k in keys], dim=1)).view(*ctx.shape[:-1], -1)
+    return dict(zip(keys, out.split([p[k]["bias"].shape[0] for k in keys], dim=-1)))
+
+
+def _gdn_gate(p, name, gate_type, ctx, x, H, W, nh, bounded=False, spatial=False, products=None):
     """_gate (cssm.py:4798-4842).  Spatial gates come back broadcastable against plane-major
-    (B, T, C, H, W); the others as the (B, T, n_ab) alpha / beta planes the bins kernel reads."""
+    (B, T, C, H, W); the others as the (B, T, n_ab) alpha / beta planes the bins kernel reads.
+    ``products`` (:func:`_gate_products`) stands in for the Dense layers of ctx."""
     B, T, C = ctx.shape
     Wf = W // 2 + 1
 
-    def dense(z, q):
-        return z @ q["kernel"] + q["bias"]
+    def dense(z, name):
+        if products is not None:
+            return products[name]
+        return z @ p[name]["kernel"] + p[name]["bias"]
     if gate_type == "channel":
         if spatial:
             q = p[name]
             g = torch.sigmoid(x @ q["kernel"].reshape(C, C) + q["bias"])     # (B, T, H, W, C)
             return g.permute(0, 1, 4, 2, 3)
-        raw = torch.sigmoid(dense(ctx, p[name]))                             # (B, T, n_h)
+        raw = torch.sigmoid(dense(ctx, name))                             # (B, T, n_h)
     elif gate_type == "factored":
-        raw = torch.sigmoid(dense(ctx, p[f"{name}_h"])[..., :, None] + dense(ctx, p[f"{name}_w"])[..., None, :])
+        raw = torch.sigmoid(dense(ctx, f"{name}_h")[..., :, None] + dense(ctx, f"{name}_w")[..., None, :])
         if spatial:
             return raw[:, :, None]                                           # (B, T, 1, H, W)
         raw = raw.reshape(B, T, H * Wf)
     elif gate_type == "scalar":
-        raw = torch.sigmoid(dense(ctx, p[name]))                             # (B, T, 1)
+        raw = torch.sigmoid(dense(ctx, name))                             # (B, T, 1)
         if spatial:
             return raw[..., None, None]
     else:
-        raw = torch.sigmoid(dense(ctx, p[name]))
+        raw = torch.sigmoid(dense(ctx, name))
         if spatial:
             return raw.view(B, T, 1, H, W)
     return 0.1 + 0.89 * raw if bounded else raw
+
+
+class _GdnFn(torch.autograd.Function):
+    """qkv_proj and gate_proj -> short conv + SiLU + input gates -> rfft2 -> spectral norms and delta rule ->
+    irfft2 -> norm x gate of the GDN cell (cssm.py:4753-5137 up to output_proj), as one autograd node on HIP
+    kernels both ways.  xq2 is qkv_proj's input where it is not x2 (the qkv depthwise conv), or None: then both
+    projections run side by side, forward and in their gradients.  gkv holds the input gates in
+    cssm_gdn_qkv_act's layout of gate_mode."""
+
+    @staticmethod
+    def forward(ctx, x2, xq2, w_qkv, b_qkv, w_g, b_g, what, ab, gkv, scale, shift, meta, *convs):
+        B, T, H, W, C, dk, gate_mode, gate_type, l2, variant, norm, act = meta
+        F, HW = B * T, H * W
+        if xq2 is None:
+            planes = S.proj_planes(x2, torch.cat([w_qkv, w_g], dim=1), torch.cat([b_qkv, b_g]), F, HW,
+                                   out_dtype=torch.float32)
+            raw, g = planes[:, :3 * C], planes[:, 3 * C:]
+        else:
+            raw = S.proj_planes(xq2, w_qkv, b_qkv, F, HW, out_dtype=torch.float32)
+            g = S.proj_planes(x2, w_g, b_g, F, HW, out_dtype=torch.float32)
+        qkv = S.gdn_qkv_act(raw, B, T, convs, gate_mode, gkv)
+        spec, norms = S.rfft2(qkv.view(B, T, 3 * C, H, W), want_norms=l2)
+        del qkv
+        ohat, states = S.gdn_core_train(spec, norms, ab, gate_type, what, dk, W, variant)
+        o = S.irfft2(ohat, W).view(F, C, HW)
+        ctx.save_for_backward(x2, xq2, w_qkv, w_g, what, ab, gkv, scale, shift, raw, g, spec, norms, states, o, *convs)
+        ctx.meta = meta
+        return S.gdn_norm_gate(o, g, norm, scale, shift, act)
+
+    @staticmethod
+    def backward(ctx, dy):
+        (x2, xq2, w_qkv, w_g, what, ab, gkv, scale, shift, raw, g, spec, norms, states, o,
+         *convs) = ctx.saved_tensors
+        B, T, H, W, C, dk, gate_mode, gate_type, l2, variant, norm, act = ctx.meta
+        F, HW = B * T, H * W
+        dall = torch.empty((F, 4 * C, HW), dtype=torch.float32, device=dy.device) if xq2 is None else None
+        draw = dall[:, :3 * C] if xq2 is None else torch.empty_like(raw)
+        dg = dall[:, 3 * C:] if xq2 is None else torch.empty_like(g)
+        do, ng_sums = S.gdn_norm_gate_backward(o, g, norm, scale, shift, act, dy.contiguous(), dg)
+        dospec, _ = S.rfft2(do.view(B, T, C, H, W))
+        del do
+        dspec, dab, dwhat = S.gdn_core_backward(spec, norms, ab, gate_type, what, states, dospec, dk, W, variant)
+        del dospec
+        if gate_type in ("dense", "factored"):      # one (alpha, beta) per bin, shared by the heads
+            dab = dab.sum(dim=2)
+        elif gate_type == "channel":                # one per head, shared by the bins
+            dab = dab.sum(dim=3)
+        else:                                       # one per frame
+            dab = dab.sum(dim=(2, 3)).unsqueeze(2)
+        dqkv = S.irfft2(dspec, W).view(F, 3 * C, HW)
+        del dspec
+        dgkv, sums = S.gdn_qkv_act_backward(raw, B, T, convs, gate_mode, gkv, dqkv, draw)
+        del dqkv
+        kt = convs[0].shape[0] if convs else 0
+        d_convs = []
+        for i in range(3 if convs else 0):
+            part = sums[i * C:(i + 1) * C]
+            d_convs += [part[:, :kt].t().unsqueeze(1), part[:, kt]]
+
+        def d_proj(d, w, x):                        # gradients of x and of the (K, N) kernel
+            K = w.shape[0]
+            dx = S.proj_out(d, w.t().contiguous(), w.new_zeros(K), out_dtype=torch.float32)
+            return dx, torch.bmm(d, x.view(F, HW, K)).sum(dim=0).t()
+        if xq2 is None:
+            dxq = None
+            dx, dw = d_proj(dall, torch.cat([w_qkv, w_g], dim=1), x2)
+            dw_qkv, dw_g = dw[:, :3 * C], dw[:, 3 * C:]
+        else:
+            dx, dw_g = d_proj(dg, w_g, x2)
+            dxq, dw_qkv = d_proj(draw, w_qkv, xq2)
+        return (dx, dxq, dw_qkv, sums[:, kt + 1], dw_g, ng_sums[2], dwhat.sum(dim=0), dab, dgkv,
+                ng_sums[0] if scale is not None else None, ng_sums[1] if shift is not None else None, None, *d_convs)
+
+
+def _gdn_fused_apply(cell, p, x, ctx, what, dims):
+    """gdn_train_apply through _GdnFn: the gates and W_hat on torch (small), the rest on the one node."""
+    B, T, H, W, C, dk, nh = dims
+    F, HW = B * T, H * W
+    x2 = x.reshape(-1, C).contiguous()
+    xq2 = None
+    if cell.qkv_conv_size > 1:
+        xq2 = _dwconv_cl(x.reshape(F, H, W, C), p["qkv_dw"]).reshape(-1, C).contiguous()
+
+    names = ["alpha", "beta"] + (["B_k", "B_v"] if cell.use_input_gates and cell.gate_type != "channel" else [])
+    products = _gate_products(p, names, cell.gate_type, ctx)
+
+    def gate(name, **kw):
+        prods = products if name in names else None
+        return _gdn_gate(p, name, cell.gate_type, ctx, x, H, W, nh, products=prods, **kw)
+    ab = torch.stack([gate("alpha", bounded=True), gate("beta")], dim=-1).contiguous()
+    gate_mode, gkv = 0, None
+    if cell.use_input_gates:
+        bk, bv = gate("B_k", spatial=True), gate("B_v", spatial=True)
+        if cell.gate_type == "channel":             # (B, T, C, H, W) each, side by side
+            gate_mode, gkv = 3, torch.cat([bk, bv], dim=2).reshape(F, 2 * C, HW)
+        elif cell.gate_type == "scalar":
+            gate_mode, gkv = 2, torch.stack([bk, bv]).reshape(2, F)
+        else:
+            gate_mode, gkv = 1, torch.stack([bk, bv]).reshape(2, F, HW)
+        gkv = gkv.contiguous()
+    convs = []
+    if cell.short_conv_size > 0:
+        for n in "qkv":
+            convs += [p[f"short_conv_{n}"]["kernel"].contiguous(), p[f"short_conv_{n}"]["bias"].contiguous()]
+    scale = shift = None
+    if cell.output_norm == "rms":
+        scale = p["rms_scale"]
+    elif cell.output_norm == "layer":
+        scale, shift = p["output_layernorm"]["scale"], p["output_layernorm"]["bias"]
+    meta = (B, T, H, W, C, dk, gate_mode, cell.gate_type, cell.use_spectral_l2_norm, cell.scan_variant,
+            cell.output_norm, "silu" if cell.output_gate_act == "silu" else "sigmoid")
+    y = _GdnFn.apply(x2, xq2, p["qkv_proj"]["kernel"], p["qkv_proj"]["bias"], p["gate_proj"]["kernel"],
+                     p["gate_proj"]["bias"], what, ab, gkv, scale, shift, meta, *convs)
+    out = _ProjOutFn.apply(y, p["output_proj"]["kernel"], p["output_proj"]["bias"])
+    return out.view(B, T, H, W, C)
 
 
 def gdn_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tensor:
@@ -519,8 +646,10 @@ def gdn_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tens
     ctx = x.mean(dim=(2, 3))
     if not cell.position_independent_gates:
         ctx = ctx + _temporal_encoding(T, C, cell.rope_base, x.device)[None]
-    xq = x.reshape(F, H, W, C)
     ks = cell.qkv_conv_size
+    if not (ks > 1 and not cell.qkv_conv_separable) and S.gdn_norm_gate_supported(C) and cell.short_conv_size <= 8:
+        return _gdn_fused_apply(cell, p, x, ctx, what, (B, T, H, W, C, dk, nh))
+    xq = x.reshape(F, H, W, C)
     if ks > 1 and not cell.qkv_conv_separable:
         # full-channel SAME conv (cssm.py:4750-4753), lo = (ks - 1) // 2 rows / columns of zeros before
         # and ks // 2 after, as lax pads; torch's conv2d correlates like lax does

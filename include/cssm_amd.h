@@ -612,6 +612,60 @@ int cssm_gdn_scan_bins_bwd(const float* spec, const float* ab, long long ab_fram
                            void* stream);
 
 /*
+ * The same pair on the planes' own spectra (training path of the whole core,
+ * cssm.py:4875-5025): norms (B, T, 3C) = the sums |X|^2 cssm_rfft2 returns, or
+ * NULL without the spectral L2 norm (:4890-4897), applied to q and k on load.
+ * The reverse takes dospec = cssm_rfft2 of the output planes' gradient and
+ * returns dspec such that cssm_irfft2 of it is the gradient of the q, k, v
+ * planes: the transforms' adjoint factors and the norm's adjoint included.
+ * Other arguments as above (W may be odd).
+ */
+int cssm_gdn_core_train(const float* spec, const float* norms, const float* ab, long long ab_frame, int ab_head,
+                        int ab_bin, const float* what, int B, int T, int C, int H, int W, int delta_key_dim,
+                        int scan_variant, float* ohat, float* states, void* stream);
+int cssm_gdn_core_bwd(const float* spec, const float* norms, const float* ab, long long ab_frame, int ab_head,
+                      int ab_bin, const float* what, const float* states, const float* dospec, int B, int T, int C,
+                      int H, int W, int delta_key_dim, int scan_variant, float* dspec, float* dab, float* dwhat,
+                      void* stream);
+
+/*
+ * Training form of cssm_gdn_qkv_post (cssm.py:4763-4848), out of place in float32:
+ * out (F, 3C, HW) = gate * SiLU(causal short conv of raw) (F = B T), raw (F, 3C, HW)
+ * with a frame stride of raw_fs floats.  kt = 0 skips conv and SiLU; kt <= 8.
+ *   gate_mode 0 none; 1 gates (2, F, HW): B_k, B_v per pixel; 2 gates (2, F) per frame;
+ *   3 gates (F, 2C, HW) per channel and pixel
+ * The adjoint writes draw (frame stride draw_fs floats), dgates -- mode 3 (F, 2C, HW);
+ * else partial sums (2, (C + 7) / 8, F, HW) for the caller to add over axis 1 (and,
+ * mode 2, the pixels) -- and sums (B, blocks, 3C, kt + 2), blocks =
+ * cssm_gdn_qkv_act_bwd_blocks: the taps' gradients (kernel order), the conv bias's and
+ * the sum of draw, to add over the first two axes.
+ */
+int cssm_gdn_qkv_act(const float* raw, long long raw_fs, int B, int T, int C, int HW, int kt,
+                     const float* const* conv_kernel, const float* const* conv_bias, int gate_mode,
+                     const float* gates, float* out, void* stream);
+int cssm_gdn_qkv_act_bwd_blocks(int B, int C, int HW);
+int cssm_gdn_qkv_act_bwd(const float* raw, long long raw_fs, int B, int T, int C, int HW, int kt,
+                         const float* const* conv_kernel, const float* const* conv_bias, int gate_mode,
+                         const float* gates, const float* dout, float* draw, long long draw_fs, float* dgates,
+                         float* sums, void* stream);
+
+/*
+ * Training form of the output path before output_proj (cssm.py:4853-4859,
+ * 5026-5137): y (F, C, HW) = (norm(o) scale + shift) act(g) per pixel over the
+ * channels, norm 0 none, 1 rms, 2 layer (eps 1e-6), act 1 SiLU, 2 sigmoid, g
+ * the gate's pre-activation (frame stride g_fs floats), scale / shift (C) or
+ * NULL; C <= 128.  The adjoint writes d_o (F, C, HW), dg (frame stride dg_fs) and
+ * sums (blocks, 3, C), blocks = cssm_gdn_norm_gate_blocks: the gradients of
+ * scale, of shift, and the sum of dg, to add over the first axis.
+ */
+int cssm_gdn_norm_gate(const float* o, const float* g, long long g_fs, int F, int C, int HW, int norm, int act,
+                       const float* scale, const float* shift, float* y, void* stream);
+int cssm_gdn_norm_gate_blocks(int F, int HW);
+int cssm_gdn_norm_gate_bwd(const float* o, const float* g, long long g_fs, int F, int C, int HW, int norm, int act,
+                           const float* scale, const float* shift, const float* dy, float* d_o, float* dg,
+                           long long dg_fs, float* sums, void* stream);
+
+/*
  * The GDN spectral core as one kernel where a workgroup can hold a (batch,
  * head)'s state for all T (32 x 32 planes, delta_key_dim 4: the video-shaped
  * config): per step it reads the head's q, k, v planes once, runs their rfft2,
