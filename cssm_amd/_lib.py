@@ -91,6 +91,12 @@ SIGNATURES = {
                                        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
                                        ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                        ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
+    "cssm_short_conv_train_supported": (_I, [_I, _I, _I, _I, _I]),
+    "cssm_short_conv_train": (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P, _P, _P]),
+    "cssm_short_conv_bwd_chunks": (_I, [_I, _I, _I, _I, _I]),
+    "cssm_short_conv_bwd": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _LL, _P, _P]),
+    "cssm_spectral_kernel_bwd_supported": (_I, [_I, _I, _I]),
+    "cssm_spectral_kernel_bwd": (_I, [_P, _I, _I, _I, _I, _I, ctypes.c_float, _I, _I, _I, _P, _P, _P]),
     "cssm_proj_planes": (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P]),
     "cssm_frame_mean": (_I, [_P, _I, _I, _I, _I, _P, _P]),
     "cssm_depthwise_conv": (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _I, _P]),

@@ -79,6 +79,24 @@ int cssm_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, 
   return hip_status(e, "cssm_spectral_kernel");
 }
 
+int cssm_spectral_kernel_bwd_supported(int K, int H, int W) {
+  return cssm::spectral_kernel_bwd_supported(K, H, W) ? 1 : 0;
+}
+
+int cssm_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, float rho, int squash, int goom_floor,
+                             int scan_order, const float* dkhat, float* dk, void* stream) {
+  if (!k || !dkhat || !dk) return fail(CSSM_ERR_NULL, "cssm_spectral_kernel_bwd: k, dkhat and dk must be non-null");
+  if (B <= 0 || C <= 0 || K <= 0 || H <= 0 || W <= 0)
+    return fail(CSSM_ERR_SHAPE, "cssm_spectral_kernel_bwd: B=%d C=%d K=%d H=%d W=%d must be positive", B, C, K, H, W);
+  if (!aligned(dkhat, 8)) return fail(CSSM_ERR_ALIGN, "cssm_spectral_kernel_bwd: dkhat must be 8-byte aligned");
+  if (!cssm::spectral_kernel_bwd_supported(K, H, W))
+    return fail(CSSM_ERR_UNSUPPORTED, "cssm_spectral_kernel_bwd: K=%d, %dx%d planes", K, H, W);
+  return hip_status(cssm::launch_spectral_kernel_bwd(k, B, C, K, H, W, rho, squash, goom_floor, scan_order ? 1 : 0,
+                                                     reinterpret_cast<const float2*>(dkhat), dk,
+                                                     static_cast<hipStream_t>(stream)),
+                    "cssm_spectral_kernel_bwd");
+}
+
 int cssm_plane_mean(const void* x, int dtype, long long nplanes, int H, int W, int act, float* out,
                     void* stream) {
   if (!x || !out) return fail(CSSM_ERR_NULL, "cssm_plane_mean: x and out must be non-null");
@@ -362,6 +380,45 @@ int cssm_short_conv(const void* x, int in_dtype, int B, int T, int C, int H, int
   return hip_status(cssm::launch_short_conv(x, in_dtype, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, out_dtype, ctx, 0,
                                             static_cast<hipStream_t>(stream)),
                     "cssm_short_conv");
+}
+
+int cssm_short_conv_train_supported(int T, int H, int W, int ks, int kt) {
+  return T > 0 && H > 0 && W > 0 && ks >= 0 && kt >= 0 && cssm::short_conv_planes_supported(T, H, W, ks, kt) ? 1 : 0;
+}
+
+static int short_conv_train_check(const char* fn, int B, int T, int C, int H, int W, int ks, const float* ws,
+                                  const float* bs, int kt, const float* wt) {
+  if (B <= 0 || T <= 0 || C <= 0 || H <= 0 || W <= 0 || ks < 0 || kt < 0)
+    return fail(CSSM_ERR_SHAPE, "%s: B=%d T=%d C=%d H=%d W=%d ks=%d kt=%d", fn, B, T, C, H, W, ks, kt);
+  if ((ks > 0 && (!ws || !bs)) || (kt > 0 && !wt))
+    return fail(CSSM_ERR_NULL, "%s: weights of an enabled convolution are missing", fn);
+  if (!cssm::short_conv_planes_supported(T, H, W, ks, kt))
+    return fail(CSSM_ERR_UNSUPPORTED, "%s: ks=%d kt=%d on %dx%d planes", fn, ks, kt, H, W);
+  return CSSM_OK;
+}
+
+int cssm_short_conv_train(const float* x, int B, int T, int C, int H, int W, int ks, const float* ws, const float* bs,
+                          int kt, const float* wt, const float* bt, float* o, float* ctx, void* stream) {
+  if (!x || !o || (kt > 0 && !bt)) return fail(CSSM_ERR_NULL, "cssm_short_conv_train: null argument");
+  if (int e = short_conv_train_check("cssm_short_conv_train", B, T, C, H, W, ks, ws, bs, kt, wt)) return e;
+  return hip_status(cssm::launch_short_conv(x, 0, B, T, C, H, W, ks, ws, bs, kt, wt, bt, o, 0, ctx, 1,
+                                            static_cast<hipStream_t>(stream)),
+                    "cssm_short_conv_train");
+}
+
+int cssm_short_conv_bwd_chunks(int B, int T, int C, int H, int W) {
+  return B > 0 && T > 0 && C > 0 && H > 0 && W > 0 ? cssm::short_conv_bwd_chunks(B, T, C, H, W) : 0;
+}
+
+int cssm_short_conv_bwd(const float* x, const float* d_o, int B, int T, int C, int H, int W, int ks, const float* ws,
+                        const float* bs, int kt, const float* wt, float* dx, long long dx_fs, float* sums,
+                        void* stream) {
+  if (!x || !d_o || !dx || !sums) return fail(CSSM_ERR_NULL, "cssm_short_conv_bwd: null argument");
+  if (int e = short_conv_train_check("cssm_short_conv_bwd", B, T, C, H, W, ks, ws, bs, kt, wt)) return e;
+  if (dx_fs < (long long)C * H * W) return fail(CSSM_ERR_SHAPE, "cssm_short_conv_bwd: dx_fs=%lld", dx_fs);
+  return hip_status(cssm::launch_short_conv_bwd(x, d_o, B, T, C, H, W, ks, ws, bs, kt, wt, dx, dx_fs, sums,
+                                                static_cast<hipStream_t>(stream)),
+                    "cssm_short_conv_bwd");
 }
 
 }  // extern "C"
@@ -840,7 +897,7 @@ int cssm_depthwise_conv_wgrad(const float* x, const float* dy, int F, int H, int
   if (F <= 0 || H <= 0 || W <= 0 || C <= 0 || blocks <= 0 || blocks > 65535)
     return fail(CSSM_ERR_SHAPE, "cssm_depthwise_conv_wgrad: F=%d H=%d W=%d C=%d blocks=%d", F, H, W, C, blocks);
   if (!cssm::dwconv_wgrad_supported(W, C, ks))
-    return fail(CSSM_ERR_UNSUPPORTED, "cssm_depthwise_conv_wgrad: ks=%d C=%d W=%d (ks 3/5/7, C/4 dividing 64, W %% 8 == 0)",
+    return fail(CSSM_ERR_UNSUPPORTED, "cssm_depthwise_conv_wgrad: ks=%d C=%d W=%d (ks 3/5/7, C %% 4 == 0 up to 1024)",
                 ks, C, W);
   if (!aligned(x, 16) || !aligned(dy, 16) || !aligned(partial, 16))
     return fail(CSSM_ERR_ALIGN, "cssm_depthwise_conv_wgrad: tensors must be 16-byte aligned");

@@ -353,7 +353,10 @@ hipError_t launch_gdn_scan_bins_train(const float2* spec, const float* norms, co
 // owns 4 channels and strips of 8 pixels of a row: it loads the strip's dy and,
 // per tap row, the 8 + KS - 1 inputs it needs once, and keeps all KS^2 taps'
 // sums in registers.  Block partials (KS^2, C) are reduced in a fixed order
-// (lane shuffles, then across waves through LDS); the caller sums the blocks.
+// (lane shuffles, then across waves through LDS, or all through LDS where the quads do not
+// divide a wave); the caller sums the blocks.  A last strip past the row is masked.  (Rows that
+// are no multiple of 8, or C / 4 not dividing 64, went to the library's conv: the training
+// step of 960 frames of 14x14x128 with a 5 x 5 conv 48 ms.)
 namespace {
 template <int KS>
 __global__ void __launch_bounds__(256) dwconv_wgrad_cl(const float* __restrict__ x, const float* __restrict__ dy,
@@ -361,8 +364,8 @@ __global__ void __launch_bounds__(256) dwconv_wgrad_cl(const float* __restrict__
   constexpr int LO = (KS - 1) / 2, RW = 8, NCOL = RW + KS - 1;
   const int CQ = C / 4, SPB = 256 / CQ;                     // channel quads; strips per block pass
   const int tid = int(threadIdx.x), cq = tid % CQ, sl = tid / CQ;
-  const int c0 = cq * 4, WS = W / RW;
-  const long long strips = (long long)F * H * WS;
+  const int c0 = cq * 4, WS = (W + RW - 1) / RW;
+  const long long strips = sl < SPB ? (long long)F * H * WS : 0;   // threads past SPB CQ take none
   float4 acc[KS][KS];
 #pragma unroll
   for (int a = 0; a < KS; ++a)
@@ -378,7 +381,8 @@ __global__ void __launch_bounds__(256) dwconv_wgrad_cl(const float* __restrict__
     float4 g[RW];
 #pragma unroll
     for (int q = 0; q < RW; ++q)
-      g[q] = *reinterpret_cast<const float4*>(dy + ((f * H + h) * W + w0 + q) * C + c0);
+      g[q] = w0 + q < W ? *reinterpret_cast<const float4*>(dy + ((f * H + h) * W + w0 + q) * C + c0)
+                        : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int a = 0; a < KS; ++a) {
       const int hh = h + a - LO;
@@ -400,6 +404,26 @@ __global__ void __launch_bounds__(256) dwconv_wgrad_cl(const float* __restrict__
           acc[a][b].w = fmaf(xin[q + b].w, g[q].w, acc[a][b].w);
         }
     }
+  }
+  if (64 % CQ != 0) {   // uniform: the block's strips of each quad added in order
+    __shared__ float4 all[256];
+#pragma unroll
+    for (int a = 0; a < KS; ++a)
+#pragma unroll
+      for (int b = 0; b < KS; ++b) {
+        all[tid] = acc[a][b];
+        __syncthreads();
+        if (tid < CQ) {
+          float4 t = all[tid];
+          for (int q = 1; q < SPB; ++q) {
+            const float4 v = all[q * CQ + tid];
+            t = make_float4(t.x + v.x, t.y + v.y, t.z + v.z, t.w + v.w);
+          }
+          *reinterpret_cast<float4*>(partial + (size_t(blockIdx.x) * KS * KS + a * KS + b) * C + tid * 4) = t;
+        }
+        __syncthreads();
+      }
+    return;
   }
   // threads of one channel quad: lanes l, l + CQ, ... of a wave, then the waves
   __shared__ float4 red[4][64];
@@ -434,7 +458,7 @@ __global__ void __launch_bounds__(256) dwconv_wgrad_cl(const float* __restrict__
 
 bool dwconv_wgrad_supported(int W, int C, int ks) {
   const int cq = C / 4;
-  return (ks == 3 || ks == 5 || ks == 7) && C % 4 == 0 && cq >= 1 && cq <= 64 && 64 % cq == 0 && W % 8 == 0;
+  return (ks == 3 || ks == 5 || ks == 7) && C % 4 == 0 && cq >= 1 && cq <= 256 && W >= 1;
 }
 
 hipError_t launch_dwconv_wgrad(const float* x, const float* dy, int F, int H, int W, int C, int ks, float* partial,

@@ -75,6 +75,9 @@ __device__ __forceinline__ float ctx_tile_sum(const float* __restrict__ partial,
 
 hipError_t launch_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, int squash,
                                   int goom_floor, int scan_order, float2* khat, hipStream_t s);
+bool spectral_kernel_bwd_supported(int K, int H, int W);
+hipError_t launch_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, float rho, int squash,
+                                      int goom_floor, int scan_order, const float2* d, float* dk, hipStream_t s);
 hipError_t launch_plane_mean(const void* x, int dtype, long long nplanes, int HW, int act, float* out,
                              hipStream_t s);
 hipError_t launch_gated_gates(const float* ctx, const CtxPartials& cp, int BT, int C, int H, int W, int factored,
@@ -122,6 +125,11 @@ hipError_t launch_short_conv(const void* x, int in_dtype, int B, int T, int C, i
                              const float* bs, int kt, const float* wt, const float* bt, void* u, int out_dtype,
                              float* ctx, int pre, hipStream_t s);   // pre: store the pre-activation
 bool short_conv_planes_supported(int T, int H, int W, int ks, int kt);
+// adjoint of its convolutions: dx (frame stride dx_fs floats) and sums (chunks, B C, 16)
+int short_conv_bwd_chunks(int B, int T, int C, int H, int W);
+hipError_t launch_short_conv_bwd(const float* x, const float* dout, int B, int T, int C, int H, int W, int ks,
+                                 const float* ws, const float* bs, int kt, const float* wt, float* dx,
+                                 long long dx_fs, float* sums, hipStream_t s);
 
 // ---- GatedDeltaNetCSSM
 // gate weights: index 0 alpha, 1 beta, 2 B_k, 3 B_v; kind 0 dense, 1 factored, 2 channel, 3 scalar.

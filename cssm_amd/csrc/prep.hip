@@ -20,67 +20,144 @@ namespace cssm {
 // in double precision.  One block per channel.
 // out: (C, H, W/2+1) complex, optionally GOOM-floored (|x| < 1e-7 -> 1e-7+0j).
 // ---------------------------------------------------------------------------
-__global__ void spectral_kernel_prep(const float* __restrict__ k, int K, int H, int W, float rho,
-                                     int squash, int goom_floor, int scan_order, float2* __restrict__ out) {
-  extern __shared__ double sm_d[];   // rows x WF complex (re, im)
-  const int c = blockIdx.x;
-  const int WF = W / 2 + 1;
-  // taps that survive: rows [r0, r0+nr) of k land on padded rows [oh, oh+nr)
+// The twiddles cos / sin (2 pi m / N) are taken once per workgroup into LDS (one sincospi per table entry
+// instead of one per tap and bin: 64 channels of 128 x 128 from 11 x 11 taps, four workgroups a channel: 127 -> 17 us, the same values).
+struct SpecTaps {
+  int r0, nr, oh, q0, nq, ow;   // rows [r0, r0 + nr) of k land on padded rows [oh, oh + nr); columns likewise
+};
+__host__ __device__ inline SpecTaps spec_taps(int K, int H, int W) {
   // (the host rejects K between H and W, which the reference cannot run either)
-  int r0, nr, oh, q0, nq, ow;
-  if (K > H || K > W) {   // centre crop of both axes
-    r0 = (K - H) / 2; nr = H; oh = 0;
-    q0 = (K - W) / 2; nq = W; ow = 0;
-  } else {                // zero pad, tap (i, j) -> (i + (H-K)//2, j + (W-K)//2)
-    r0 = 0; nr = K; oh = (H - K) / 2;
-    q0 = 0; nq = K; ow = (W - K) / 2;
-  }
-  const float* kc = k + size_t(c) * K * K;
-  // stage 1: R[i][v] = sum_j k[i][j] e^{-2 pi i v (j') / W}
-  for (int idx = threadIdx.x; idx < nr * WF; idx += blockDim.x) {
+  if (K > H || K > W) return {(K - H) / 2, H, 0, (K - W) / 2, W, 0};   // centre crop of both axes
+  return {0, K, (H - K) / 2, 0, K, (W - K) / 2};                       // zero pad
+}
+
+// LDS: tw (W), th (H) double2 tables, then R[i][v] = sum_j k[i][j] e^{-2 pi i v j' / W}
+__device__ __forceinline__ void spec_rows(const float* kc, int K, int H, int W, const SpecTaps& q, double2* tw,
+                                          double2* th, double2* R) {
+  const int WF = W / 2 + 1;
+  for (int m = threadIdx.x; m < W; m += blockDim.x) sincospi(2.0 * double(m) / double(W), &tw[m].y, &tw[m].x);
+  for (int m = threadIdx.x; m < H; m += blockDim.x) sincospi(2.0 * double(m) / double(H), &th[m].y, &th[m].x);
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < q.nr * WF; idx += blockDim.x) {
     const int i = idx / WF, v = idx % WF;
     double re = 0.0, im = 0.0;
-    for (int j = 0; j < nq; ++j) {
-      const int jp = j + ow;
-      const long long m = (long long)v * jp % W;
-      double sn, cs;
-      sincospi(2.0 * double(m) / double(W), &sn, &cs);
-      const double kv = double(kc[(r0 + i) * K + (q0 + j)]);
-      re += kv * cs;
-      im -= kv * sn;
+    int m = v * q.ow % W;                        // v (j + ow) mod W
+    for (int j = 0; j < q.nq; ++j, m = m + v < W ? m + v : m + v - W) {
+      const double2 w = tw[m];
+      const double kv = double(kc[(q.r0 + i) * K + (q.q0 + j)]);
+      re += kv * w.x;
+      im -= kv * w.y;
     }
-    sm_d[2 * idx] = re;
-    sm_d[2 * idx + 1] = im;
+    R[idx] = make_double2(re, im);
   }
   __syncthreads();
-  // stage 2: F[u][v] = sum_i R[i][v] e^{-2 pi i u (i') / H}, at position
-  // (u, p) of the output with v = scan_col(p) in the scan's column order, in
-  // the scan's slot khat_pos(u, p)
-  for (int idx = threadIdx.x; idx < H * WF; idx += blockDim.x) {
+}
+// F[u][v] = sum_i R[i][v] e^{-2 pi i u i' / H}
+__device__ __forceinline__ double2 spec_bin(const double2* R, const double2* th, const SpecTaps& q, int H, int WF,
+                                            int u, int v) {
+  double re = 0.0, im = 0.0;
+  int m = u * q.oh % H;                          // u (i + oh) mod H
+  for (int i = 0; i < q.nr; ++i, m = m + u < H ? m + u : m + u - H) {
+    const double2 w = th[m], a = R[i * WF + v];
+    // (ar + i ai)(cs - i sn)
+    re += a.x * w.x + a.y * w.y;
+    im += a.y * w.x - a.x * w.y;
+  }
+  return make_double2(re, im);
+}
+
+__global__ void spectral_kernel_prep(const float* __restrict__ k, int K, int H, int W, float rho,
+                                     int squash, int goom_floor, int scan_order, float2* __restrict__ out) {
+  extern __shared__ double2 sm_d[];
+  const int c = blockIdx.x, WF = W / 2 + 1;
+  const SpecTaps q = spec_taps(K, H, W);
+  double2 *tw = sm_d, *th = sm_d + W, *R = sm_d + W + H;
+  spec_rows(k + size_t(c) * K * K, K, H, W, q, tw, th, R);
+  // at position (u, p) of the output with v = scan_col(p) in the scan's column order, in the scan's
+  // slot khat_pos(u, p); gridDim.y workgroups share a channel's bins
+  for (int idx = int(blockIdx.y) * blockDim.x + threadIdx.x; idx < H * WF; idx += gridDim.y * blockDim.x) {
     const int u = idx / WF, v = scan_order ? scan_col(H, W, idx % WF) : idx % WF;
-    double re = 0.0, im = 0.0;
-    for (int i = 0; i < nr; ++i) {
-      const int ip = i + oh;
-      const long long m = (long long)u * ip % H;
-      double sn, cs;
-      sincospi(2.0 * double(m) / double(H), &sn, &cs);
-      const double ar = sm_d[2 * (i * WF + v)], ai = sm_d[2 * (i * WF + v) + 1];
-      // (ar + i ai)(cs - i sn)
-      re += ar * cs + ai * sn;
-      im += ai * cs - ar * sn;
-    }
+    double2 f = spec_bin(R, th, q, H, WF, u, v);
     if (squash) {
-      const double mag = sqrt(re * re + im * im);
-      const double f = double(rho) / (1.0 + mag);
-      re *= f;
-      im *= f;
+      const double mag = sqrt(f.x * f.x + f.y * f.y);
+      const double g = double(rho) / (1.0 + mag);
+      f.x *= g;
+      f.y *= g;
     }
-    float2 o = make_float2(float(re), float(im));
+    float2 o = make_float2(float(f.x), float(f.y));
     if (goom_floor) {
       const float m2 = o.x * o.x + o.y * o.y;
       if (m2 < 1e-14f) o = make_float2(1e-7f, 0.0f);
     }
     out[size_t(c) * H * WF + (scan_order ? khat_pos(H, W, u, idx % WF) : idx)] = o;
+  }
+}
+
+// Adjoint of the spectral kernel: dk (C, K, K) from d (B, C, H, WF), the gradient (dL/dRe + i dL/dIm) of
+// the kernel's bins per batch element, added over b in order.  With F the padded kernel's DFT and
+// K_hat = rho F / (1 + |F|):
+//   dF = rho (d / (1 + |F|) - F Re(conj(d) F) / (|F| (1 + |F|)^2)),
+// nothing through a floored bin (|K_hat| < 1e-7), and dk[i][j] = Re sum_{u,v} dF e^{+2 pi i (u i' / H +
+// v j' / W)}: over u for the nr kept rows, then over v.  One workgroup per channel; F in double as the
+// forward takes it, dF in LDS as float (fp32 gradients), the sums in double.
+__global__ void __launch_bounds__(512) spectral_kernel_bwd(const float* __restrict__ k, int B, int C, int K, int H,
+                                                           int W, float rho, int squash, int goom_floor,
+                                                           int scan_order, const float2* __restrict__ d,
+                                                           float* __restrict__ dk) {
+  extern __shared__ double2 sm_d[];
+  const int c = blockIdx.x, WF = W / 2 + 1, n = H * WF;
+  const SpecTaps q = spec_taps(K, H, W);
+  double2 *tw = sm_d, *th = sm_d + W, *R = sm_d + W + H;
+  float2* dF = reinterpret_cast<float2*>(R + q.nr * WF);
+  spec_rows(k + size_t(c) * K * K, K, H, W, q, tw, th, R);
+  for (int idx = threadIdx.x; idx < n; idx += blockDim.x) {
+    const int u = idx / WF, v = scan_order ? scan_col(H, W, idx % WF) : idx % WF;
+    const size_t pos = scan_order ? khat_pos(H, W, u, idx % WF) : idx;
+    float2 g = make_float2(0.0f, 0.0f);
+    for (int b = 0; b < B; ++b) {
+      const float2 e = d[(size_t(b) * C + c) * n + pos];
+      g.x += e.x;
+      g.y += e.y;
+    }
+    if (squash || goom_floor) {
+      const double2 f = spec_bin(R, th, q, H, WF, u, v);
+      const double mag = sqrt(f.x * f.x + f.y * f.y), s = squash ? 1.0 / (1.0 + mag) : 1.0;
+      const double kr = squash ? double(rho) * s : 1.0;
+      const float2 o = make_float2(float(f.x * kr), float(f.y * kr));
+      if (goom_floor && o.x * o.x + o.y * o.y < 1e-14f) {
+        g = make_float2(0.0f, 0.0f);
+      } else if (squash) {
+        const double t = mag > 0.0 ? double(rho) * s * s * (g.x * f.x + g.y * f.y) / mag : 0.0;
+        g = make_float2(float(kr * g.x - t * f.x), float(kr * g.y - t * f.y));
+      }
+    }
+    dF[u * WF + v] = g;
+  }
+  __syncthreads();
+  // P[i][v] = sum_u dF[u][v] e^{+2 pi i u i' / H} over R, then dk[i][j] = Re sum_v P[i][v] e^{+2 pi i v j' / W}
+  for (int idx = threadIdx.x; idx < q.nr * WF; idx += blockDim.x) {
+    const int i = idx / WF, v = idx % WF;
+    double re = 0.0, im = 0.0;
+    int m = 0;
+    const int step = i + q.oh;
+    for (int u = 0; u < H; ++u, m = m + step < H ? m + step : m + step - H) {
+      const double2 w = th[m];
+      const float2 g = dF[u * WF + v];
+      re += g.x * w.x - g.y * w.y;
+      im += g.x * w.y + g.y * w.x;
+    }
+    R[idx] = make_double2(re, im);
+  }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < K * K; idx += blockDim.x) {
+    const int i = idx / K - q.r0, j = idx % K - q.q0;
+    double a = 0.0;
+    if (i >= 0 && i < q.nr && j >= 0 && j < q.nq)
+      for (int v = 0, m = 0; v < WF; ++v, m = m + j + q.ow < W ? m + j + q.ow : m + j + q.ow - W) {
+        const double2 w = tw[m], pv = R[i * WF + v];
+        a += pv.x * w.x - pv.y * w.y;
+      }
+    dk[size_t(c) * K * K + idx] = float(a);
   }
 }
 
@@ -503,11 +580,41 @@ __global__ void plane_mean_kernel(const TIN* __restrict__ x, long long nplanes, 
 hipError_t launch_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, int squash,
                                   int goom_floor, int scan_order, float2* khat, hipStream_t s) {
   const int WF = W / 2 + 1;
-  const int rows = (K > H || K > W) ? H : K;
-  const size_t shm = size_t(rows) * WF * 2 * sizeof(double);
-  if (shm > 64 * 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(spectral_kernel_prep, dim3(C), dim3(256), shm, s, k, K, H, W, rho, squash,
-                     goom_floor, scan_order, khat);
+  const SpecTaps q = spec_taps(K, H, W);
+  if (size_t(q.nr) * WF * sizeof(double2) > 64 * 1024) return hipErrorInvalidValue;   // (as ever: planes refused)
+  const size_t shm = (size_t(q.nr) * WF + W + H) * sizeof(double2);
+  if (shm > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(spectral_kernel_prep),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, int(shm));
+    if (e != hipSuccess) return e;
+  }
+  // few channels: a channel's bins over several workgroups (each takes the rows' sums again)
+  int ny = (256 + C - 1) / C;
+  const int most = (H * WF + 255) / 256;
+  if (ny > most) ny = most;
+  hipLaunchKernelGGL(spectral_kernel_prep, dim3(C, ny), dim3(256), shm, s, k, K, H, W, rho, squash, goom_floor,
+                     scan_order, khat);
+  return hipGetLastError();
+}
+
+static size_t spec_bwd_lds(int K, int H, int W) {
+  const SpecTaps q = spec_taps(K, H, W);
+  const size_t WF = W / 2 + 1;
+  return (q.nr * WF + W + H) * sizeof(double2) + H * WF * sizeof(float2);
+}
+// planes whose bins and row sums fit a workgroup's LDS (128 x 128 with up to 31 taps)
+bool spectral_kernel_bwd_supported(int K, int H, int W) {
+  return K > 0 && H > 0 && W > 0 && !((K > H || K > W) && (K < H || K < W)) && spec_bwd_lds(K, H, W) <= 128 * 1024;
+}
+hipError_t launch_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, float rho, int squash,
+                                      int goom_floor, int scan_order, const float2* d, float* dk, hipStream_t s) {
+  if (!spectral_kernel_bwd_supported(K, H, W)) return hipErrorInvalidValue;
+  const size_t shm = spec_bwd_lds(K, H, W);
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(spectral_kernel_bwd),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(spectral_kernel_bwd, dim3(C), dim3(512), shm, s, k, B, C, K, H, W, rho, squash, goom_floor,
+                     scan_order, d, dk);
   return hipGetLastError();
 }
 

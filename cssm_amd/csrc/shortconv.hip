@@ -222,44 +222,238 @@ short_conv_planes(const TI* __restrict__ x, long long P, int T, int C, int H, in
 // LDS floats of a plane with its border, per kernel class
 constexpr int kScSmall = 4096, kScMid = 4400, kScLarge = 16900;
 
-template <int PX, int NT, int NB, int LDSF, class TI, class TO>
-static void run_short_conv_planes(const TI* x, int B, int T, int C, int H, int W, int ks, const float* ws,
-                                  const float* bs, int kt, const float* wt, const float* bt, TO* u, float* ctx,
-                                  int LP, int pre, hipStream_t s) {
-  const long long P = (long long)B * C, groups = (P + NT / LP - 1) / (NT / LP);
-  // frames per workgroup: all of them when the planes alone give every CU its waves (16 per CU),
-  // else chunks of at least 8 (a chunk reads kt - 1 frames more)
+// the kernel class of a call (0: 256 threads, 4 pixels each; 1: 1024, 4; 2: 1024, 16), threads per plane and
+// frames per workgroup: all of them when the planes alone give every CU its waves (16 per CU), else
+// chunks of at least 8 (a chunk reads kt - 1 frames more)
+struct ScShape {
+  int cls, LP, tlen;
+};
+static ScShape sc_shape(int B, int T, int C, int H, int W) {
+  const long long HW = (long long)H * W, ps = (long long)(H + 2) * (W + 2);
+  ScShape r{0, 1, T};
+  while (r.LP < 256 && r.LP * 4 < HW) r.LP *= 2;
+  if (!(HW <= 1024 && (256 / r.LP) * ps <= kScSmall)) {
+    r.cls = HW <= 4096 && ps <= kScMid ? 1 : 2;
+    r.LP = 1024;
+  }
+  const int NT = r.cls == 0 ? 256 : 1024;
+  const long long P = (long long)B * C, groups = (P + NT / r.LP - 1) / (NT / r.LP);
   const long long want = 256LL * 1024 / NT;
   long long chunks = groups >= want ? 1 : (want + groups - 1) / groups;
   if (chunks > (T + 7) / 8) chunks = (T + 7) / 8;
-  const int tlen = int((T + chunks - 1) / chunks);
-  const dim3 grid(unsigned(groups), unsigned((T + tlen - 1) / tlen));
+  r.tlen = int((T + chunks - 1) / chunks);
+  return r;
+}
+
+template <int PX, int NT, int NB, int LDSF, class TI, class TO>
+static void run_short_conv_planes(const TI* x, int B, int T, int C, int H, int W, int ks, const float* ws,
+                                  const float* bs, int kt, const float* wt, const float* bt, TO* u, float* ctx,
+                                  const ScShape& r, int pre, hipStream_t s) {
+  const long long P = (long long)B * C;
+  const dim3 grid(unsigned((P + NT / r.LP - 1) / (NT / r.LP)), unsigned((T + r.tlen - 1) / r.tlen));
   if (ks == 3)
     hipLaunchKernelGGL((short_conv_planes<3, PX, NT, NB, LDSF, TI, TO>), grid, dim3(NT), 0, s, x, P, T, C, H, W, ws,
-                       bs, kt, wt, bt, u, ctx, LP, tlen, pre);
+                       bs, kt, wt, bt, u, ctx, r.LP, r.tlen, pre);
   else
     hipLaunchKernelGGL((short_conv_planes<0, PX, NT, NB, LDSF, TI, TO>), grid, dim3(NT), 0, s, x, P, T, C, H, W, ws,
-                       bs, kt, wt, bt, u, ctx, LP, tlen, pre);
+                       bs, kt, wt, bt, u, ctx, r.LP, r.tlen, pre);
 }
 
 template <class TI, class TO>
 static void run_short_conv(const TI* x, int B, int T, int C, int H, int W, int ks, const float* ws, const float* bs,
                            int kt, const float* wt, const float* bt, TO* u, float* ctx, int pre, hipStream_t s) {
-  const long long HW = (long long)H * W, ps = (long long)(H + 2) * (W + 2);
-  int LP = 1;
-  while (LP < 256 && LP * 4 < HW) LP *= 2;
-  if (HW <= 1024 && (256 / LP) * ps <= kScSmall)
-    run_short_conv_planes<4, 256, 2, kScSmall>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, LP, pre, s);
-  else if (HW <= 4096 && ps <= kScMid)
-    run_short_conv_planes<4, 1024, 2, kScMid>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, 1024, pre, s);
+  const ScShape r = sc_shape(B, T, C, H, W);
+  if (r.cls == 0)
+    run_short_conv_planes<4, 256, 2, kScSmall>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, r, pre, s);
+  else if (r.cls == 1)
+    run_short_conv_planes<4, 1024, 2, kScMid>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, r, pre, s);
   else
-    run_short_conv_planes<16, 1024, 1, kScLarge>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, 1024, pre, s);
+    run_short_conv_planes<16, 1024, 1, kScLarge>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, r, pre, s);
 }
 
 // where short_conv_planes applies (else the general kernel, which has no pre form)
 bool short_conv_planes_supported(int T, int H, int W, int ks, int kt) {
   return (ks == 0 || ks == 3) && kt <= 4 && (long long)H * W <= 16384 && (long long)(H + 2) * (W + 2) <= kScLarge &&
          T <= 65535 * 8;
+}
+
+// Adjoint of short_conv_planes' convolutions: from do = dL/d(pre-activation) of every frame,
+//   ds_t = sum_l w_l do_{t+l} (w_l the tap of lag l),  dx_t = the 3 x 3 conv of ds_t with flipped taps,
+//   dw_l = sum s_t do_{t+l},  db_t = sum do,  dW[i][j] = sum ds x shifted,  db_s = sum ds
+// and the sum of dx (the projection's bias gradient).  The same plane groups and frame chunks, walked
+// backwards with do of the next three frames in registers (a chunk starts kt - 1 frames late); x_t and
+// ds_t go through LDS with zero borders, s_t is taken from x_t again.  Each plane's sixteen sums leave
+// once per chunk: sums (chunks, B C, 16) = [W 9, b_s, w_0..w_3 by lag, b_t, dx].  Reads x and do, writes
+// dx once: 256 frames x 64 planes of 32 x 32 in 72 us (2.8 TB/s; the library's depthwise conv, its im2col
+// weight gradient and the elementwise passes around them 4.5 ms).
+template <int KS, int PX, int NT, int LDSF>
+__global__ void __launch_bounds__(NT)
+short_conv_planes_bwd(const float* __restrict__ x, const float* __restrict__ dout, long long P, int T, int C, int H,
+                      int W, const float* __restrict__ ws, const float* __restrict__ bs, int kt,
+                      const float* __restrict__ wt, float* __restrict__ dx, long long dx_fs, float* __restrict__ sums,
+                      int LP, int tlen) {
+  __shared__ float bx[KS ? LDSF : 1], bd[KS ? LDSF : 1];
+  __shared__ float red[16][NT / 64];
+  const int tid = threadIdx.x, NPL = NT / LP, pl = tid / LP, li = tid % LP;
+  const int HW = H * W, RS = W + 2, PS = (H + 2) * RS;
+  const long long plane = (long long)blockIdx.x * NPL + pl;
+  const bool live = plane < P;
+  const long long b = live ? plane / C : 0;
+  const int c = live ? int(plane % C) : 0;
+  const size_t base = (size_t(b) * T * C + c) * HW, tstep = size_t(C) * HW;
+  float* dxp = dx + size_t(b) * T * dx_fs + size_t(c) * HW;
+  float k9[9], kt4[4], bsc = 0.0f;
+  if (KS) {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) k9[i] = ws[i * C + c];
+    bsc = bs[c];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) kt4[j] = j < kt ? wt[(kt - 1 - j) * C + c] : 0.0f;
+  int off[PX];
+#pragma unroll
+  for (int k = 0; k < PX; ++k) {
+    const int p = li + k * LP;
+    off[k] = pl * PS + (p < HW ? (p / W) * RS + p % W : 0);
+  }
+  if (KS) {
+    for (int i = tid; i < LDSF; i += NT) bx[i] = bd[i] = 0.0f;
+    __syncthreads();
+  }
+  const int t0 = int(blockIdx.y) * tlen, t1 = t0 + tlen < T ? t0 + tlen : T;
+  int te = t1 - 1 + (kt > 1 ? kt - 1 : 0);
+  if (te > T - 1) te = T - 1;
+  float acc[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
+  float d1[PX], d2[PX], d3[PX], nd[PX], nx[PX];   // do of frames t + 1, t + 2, t + 3; the next frame's loads
+#pragma unroll
+  for (int k = 0; k < PX; ++k) d1[k] = d2[k] = d3[k] = 0.0f;
+  auto load = [&](int t) {
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+      const int p = li + k * LP;
+      const bool ok = live && p < HW;
+      nd[k] = ok ? dout[base + size_t(t) * tstep + p] : 0.0f;
+      nx[k] = ok && t < t1 ? x[base + size_t(t) * tstep + p] : 0.0f;
+    }
+  };
+  load(te);
+  for (int t = te; t >= t0; --t) {
+    float d0[PX], ds[PX], xv[PX];
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+      d0[k] = nd[k];
+      xv[k] = nx[k];
+    }
+    if (t > t0) load(t - 1);
+    if (t < t1) {
+#pragma unroll
+      for (int k = 0; k < PX; ++k) {
+        ds[k] = d0[k];
+        if (kt > 0) {
+          ds[k] = kt4[0] * d0[k];
+          if (kt > 1) ds[k] = fmaf(kt4[1], d1[k], ds[k]);
+          if (kt > 2) ds[k] = fmaf(kt4[2], d2[k], ds[k]);
+          if (kt > 3) ds[k] = fmaf(kt4[3], d3[k], ds[k]);
+        }
+        if (KS && li + k * LP < HW) {
+          bx[off[k] + RS + 1] = xv[k];
+          bd[off[k] + RS + 1] = ds[k];
+        }
+      }
+      if (KS) __syncthreads();
+      float* dt = dxp + size_t(t) * dx_fs;
+#pragma unroll
+      for (int k = 0; k < PX; ++k) {
+        const int p = li + k * LP;
+        float s = xv[k], g = ds[k];
+        if (KS) {
+          s = bsc;
+          g = 0.0f;
+          const float* qx = bx + off[k];
+          const float* qd = bd + off[k];
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+              const float v = qx[i * RS + j];
+              s = fmaf(v, k9[i * 3 + j], s);
+              acc[i * 3 + j] = fmaf(ds[k], v, acc[i * 3 + j]);
+              g = fmaf(qd[(2 - i) * RS + 2 - j], k9[i * 3 + j], g);
+            }
+          acc[9] += ds[k];
+        }
+        if (!(live && p < HW)) s = g = 0.0f;
+        acc[10] = fmaf(s, d0[k], acc[10]);
+        acc[11] = fmaf(s, d1[k], acc[11]);
+        acc[12] = fmaf(s, d2[k], acc[12]);
+        acc[13] = fmaf(s, d3[k], acc[13]);
+        acc[14] += d0[k];
+        acc[15] += g;
+        if (live && p < HW) dt[p] = g;
+      }
+      if (KS) __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+      d3[k] = d2[k];
+      d2[k] = d1[k];
+      d1[k] = d0[k];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    for (int o = (LP < 64 ? LP : 64) / 2; o > 0; o >>= 1) acc[j] += __shfl_xor(acc[j], o, 64);
+  float* out = sums + (size_t(blockIdx.y) * P + (live ? plane : 0)) * 16;
+  if (LP <= 64) {
+    if (li == 0 && live)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) out[j] = acc[j];
+    return;
+  }
+  if ((tid & 63) == 0)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) red[j][tid / 64] = acc[j];
+  __syncthreads();
+  if (live && li < 16) {
+    float v = 0.0f;
+    for (int i = 0; i < LP / 64; ++i) v += red[li][pl * (LP / 64) + i];
+    out[li] = v;
+  }
+}
+
+int short_conv_bwd_chunks(int B, int T, int C, int H, int W) {
+  const ScShape r = sc_shape(B, T, C, H, W);
+  return (T + r.tlen - 1) / r.tlen;
+}
+
+template <int KS, int PX, int NT, int LDSF>
+static void run_short_conv_bwd(const float* x, const float* dout, int B, int T, int C, int H, int W, const float* ws,
+                               const float* bs, int kt, const float* wt, float* dx, long long dx_fs, float* sums,
+                               const ScShape& r, hipStream_t s) {
+  const long long P = (long long)B * C;
+  const dim3 grid(unsigned((P + NT / r.LP - 1) / (NT / r.LP)), unsigned((T + r.tlen - 1) / r.tlen));
+  hipLaunchKernelGGL((short_conv_planes_bwd<KS, PX, NT, LDSF>), grid, dim3(NT), 0, s, x, dout, P, T, C, H, W, ws, bs,
+                     kt, wt, dx, dx_fs, sums, r.LP, r.tlen);
+}
+
+hipError_t launch_short_conv_bwd(const float* x, const float* dout, int B, int T, int C, int H, int W, int ks,
+                                 const float* ws, const float* bs, int kt, const float* wt, float* dx,
+                                 long long dx_fs, float* sums, hipStream_t s) {
+  if (!short_conv_planes_supported(T, H, W, ks, kt)) return hipErrorInvalidValue;
+  const ScShape r = sc_shape(B, T, C, H, W);
+#define CSSM_SCB(KS_)                                                                                                \
+  if (r.cls == 0) run_short_conv_bwd<KS_, 4, 256, kScSmall>(x, dout, B, T, C, H, W, ws, bs, kt, wt, dx, dx_fs, sums, r, s); \
+  else if (r.cls == 1) run_short_conv_bwd<KS_, 4, 1024, kScMid>(x, dout, B, T, C, H, W, ws, bs, kt, wt, dx, dx_fs, sums, r, s); \
+  else run_short_conv_bwd<KS_, 16, 1024, kScLarge>(x, dout, B, T, C, H, W, ws, bs, kt, wt, dx, dx_fs, sums, r, s);
+  if (ks == 3) {
+    CSSM_SCB(3)
+  } else {
+    CSSM_SCB(0)
+  }
+#undef CSSM_SCB
+  return hipGetLastError();
 }
 
 hipError_t launch_short_conv(const void* x, int in_dtype, int B, int T, int C, int H, int W, int ks, const float* ws,

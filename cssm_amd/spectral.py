@@ -55,6 +55,23 @@ def spectral_kernel(k: torch.Tensor, H: int, W: int, rho: float = 0.999, squash:
     return out
 
 
+def spectral_kernel_bwd_supported(K: int, H: int, W: int) -> bool:
+    return bool(_lib.load().cssm_spectral_kernel_bwd_supported(K, H, W))
+
+
+def spectral_kernel_backward(k: torch.Tensor, dkhat: torch.Tensor, W: int, rho: float, squash: bool, goom_floor: bool,
+                             scan_order: bool) -> torch.Tensor:
+    """dk (C, K, K) from dkhat (B, C, H, W//2+1), the bins' gradients per batch element
+    (cssm_spectral_kernel_bwd)."""
+    _dev(k, "k", torch.float32)
+    _dev(dkhat, "dkhat", torch.complex64)
+    B, C, H, _ = dkhat.shape
+    dk = torch.empty_like(k)
+    _lib.call("cssm_spectral_kernel_bwd", k.data_ptr(), B, C, k.shape[1], H, W, float(rho), int(squash),
+              int(goom_floor), int(scan_order), dkhat.data_ptr(), dk.data_ptr(), _stream())
+    return dk
+
+
 def scan_col_order(H: int, W: int) -> List[int]:
     """Column order of the per-bin planes :func:`gated_scan` reads (gates, K_hat):
     entry p is the frequency column stored at position p of a row (the identity
@@ -393,6 +410,47 @@ def short_conv(x: torch.Tensor, spatial: Optional[Dict[str, torch.Tensor]],
     _lib.call("cssm_short_conv", x.data_ptr(), _DTYPES[x.dtype], B, T, C, H, W, ks, ws, bs, kt, wt, bt,
               u.data_ptr(), _DTYPES[od], ctx.data_ptr() if ctx is not None else None, _stream())
     return u, ctx
+
+
+def short_conv_train_supported(T: int, H: int, W: int, ks: int, kt: int) -> bool:
+    return bool(_lib.load().cssm_short_conv_train_supported(T, H, W, ks, kt))
+
+
+def _short_conv_ptrs(spatial, temporal):
+    (ws, bs), (wt, bt) = spatial or (None, None), temporal or (None, None)
+    for t, n in ((ws, "spatial kernel"), (bs, "spatial bias"), (wt, "temporal kernel"), (bt, "temporal bias")):
+        if t is not None:
+            _dev(t, f"short_conv {n}", torch.float32)
+    return (ws.shape[0] if ws is not None else 0, ws.data_ptr() if ws is not None else None,
+            bs.data_ptr() if bs is not None else None, wt.shape[0] if wt is not None else 0,
+            wt.data_ptr() if wt is not None else None, bt.data_ptr() if bt is not None else None)
+
+
+def short_conv_train(x: torch.Tensor, spatial, temporal):
+    """(o, ctx): the pre-activation of :func:`short_conv` and the spatial mean of its SiLU (cssm_short_conv_train);
+    spatial / temporal = (kernel, bias) or None."""
+    _dev(x, "x", torch.float32)
+    B, T, C, H, W = x.shape
+    ks, ws, bs, kt, wt, bt = _short_conv_ptrs(spatial, temporal)
+    o = torch.empty_like(x)
+    ctx = torch.empty((B, T, C), dtype=torch.float32, device=x.device)
+    _lib.call("cssm_short_conv_train", x.data_ptr(), B, T, C, H, W, ks, ws, bs, kt, wt, bt, o.data_ptr(),
+              ctx.data_ptr(), _stream())
+    return o, ctx
+
+
+def short_conv_backward(x: torch.Tensor, do: torch.Tensor, spatial, temporal, dx: torch.Tensor) -> torch.Tensor:
+    """Adjoint of :func:`short_conv_train`'s convolutions for the gradient do of o: writes dx (F, C, HW) (a channel
+    slice of a plane-major tensor allowed) and returns the sums (C, 16) of cssm_short_conv_bwd."""
+    _dev(x, "x", torch.float32)
+    _dev(do, "do", torch.float32)
+    B, T, C, H, W = x.shape
+    ks, ws, bs, kt, wt, bt = _short_conv_ptrs(spatial, temporal)
+    n = int(_lib.load().cssm_short_conv_bwd_chunks(B, T, C, H, W))
+    sums = torch.empty((n * B, C, 16), dtype=torch.float32, device=x.device)
+    _lib.call("cssm_short_conv_bwd", x.data_ptr(), do.data_ptr(), B, T, C, H, W, ks, ws, bs, kt, wt, dx.data_ptr(),
+              _frames(dx, "dx", C, H * W), sums.data_ptr(), _stream())
+    return sums.sum(dim=0)
 
 
 # ----------------------------------------------------------------- GDN cell
@@ -796,7 +854,7 @@ def depthwise_conv_wgrad(x: torch.Tensor, dy: torch.Tensor, ks: int, blocks: int
     F = 1
     for d in lead:
         F *= d
-    blocks = max(1, min(blocks, (F * H * (W // 8) + 63) // 64))
+    blocks = max(1, min(blocks, (F * H * ((W + 7) // 8) + 63) // 64))
     partial = torch.empty((blocks, ks, ks, C), dtype=torch.float32, device=x.device)
     _lib.call("cssm_depthwise_conv_wgrad", x.data_ptr(), dy.data_ptr(), F, H, W, C, ks, partial.data_ptr(), blocks,
               _stream())

@@ -155,7 +155,7 @@ class _DwConvFn(torch.autograd.Function):
 
 def _dwconv_cl(x4, q):
     """Depthwise SAME conv of channels-last (F, H, W, C) frames: the HIP kernels where they apply
-    (odd ks in 3..7, C / 4 dividing 64, W % 8 == 0), else torch's conv."""
+    (odd ks in 3..7, C a multiple of 4 up to 1024), else torch's conv."""
     ks = q["kernel"].shape[0]
     F, H, W, C = x4.shape
     if ks % 2 == 1 and S.depthwise_conv_wgrad_supported(W, C, ks):
@@ -253,45 +253,50 @@ def _gate_leaves(p: Dict[str, Any], gate_type: str):
 
 
 class _GatedInScanFn(torch.autograd.Function):
-    """in_proj -> SiLU -> ctx -> gates -> fused scan -> x SiLU(z) of the gated cell without short
-    convolutions (cssm.py:480-581 up to out_proj), as one autograd node whose backward runs on HIP
+    """in_proj [-> short convolutions] -> SiLU -> ctx -> gates -> fused scan -> x SiLU(z) of the gated cell
+    (cssm.py:480-581 up to out_proj), as one autograd node whose backward runs on HIP
     kernels end to end: in_proj stores the pre-activations and takes ctx as the mean of their
-    SiLU in the same pass (CSSM_PROJ_STORE_PRE_CTX_SILU); the scan applies both SiLUs on load.
+    SiLU in the same pass (CSSM_PROJ_STORE_PRE_CTX_SILU; with short convolutions cssm_short_conv_train does,
+    from in_proj's plain output); the scan applies both SiLUs on load.
     Backward: rfft2 of SiLU(x_main) and of dy * SiLU(z) (cssm_rfft2_ex), the reverse recurrence
     (cssm_gated_scan_bwd), the gates' adjoint (cssm_gated_gates_bwd) with the gate projections'
-    gradients as GEMMs over frames, K_hat's construction differentiated by torch on its small
-    tensors, then cssm_irfft2_ex writes the two pre-activation gradients straight into one
+    gradients as GEMMs over frames, K_hat's adjoint (cssm_spectral_kernel_bwd), then cssm_irfft2_ex writes the two pre-activation gradients straight into one
     plane-major (F, 2C, HW) tensor: dz = irfft2(Y) * dy * SiLU'(z) and
     dx_main = (irfft2(dU) + dctx / HW) * SiLU'(x_main), the ctx term being the spatial mean's
-    gradient; in_proj's gradients follow from that tensor (dx on the projection kernel with W^T,
-    dW as one batched GEMM over frames)."""
+    gradient; short convolutions take that half through cssm_short_conv_bwd first; in_proj's gradients
+    follow from that tensor (dx on the projection kernel with W^T, dW as one batched GEMM over
+    frames).  convs: (spatial kernel, bias, temporal kernel, bias), None where absent."""
 
     @staticmethod
-    def forward(ctx, x2, w_in, b_in, kernel, meta, *gate_params):
+    def forward(ctx, x2, w_in, b_in, kernel, meta, ws, bs, wt, bt, *gate_params):
         B, T, H, W, Ci, gate_type, activation, rho, rebuild = meta
         F, HW = B * T, H * W
-        xm, z, cx = S.proj_in(x2, w_in, b_in, F, HW, want_ctx=True, out_dtype=torch.float32, ctx_of_silu=True)
+        spatial, temporal = (ws, bs) if ws is not None else None, (wt, bt) if wt is not None else None
+        raw = None
+        if spatial or temporal:
+            raw, z, _ = S.proj_in(x2, w_in, b_in, F, HW, out_dtype=torch.float32)
+            xm, cx = S.short_conv_train(raw.view(B, T, Ci, H, W), spatial, temporal)
+        else:
+            xm, z, cx = S.proj_in(x2, w_in, b_in, F, HW, want_ctx=True, out_dtype=torch.float32, ctx_of_silu=True)
         c_scale = S.scan_c_scale(H, W)
         gates = S.gated_gates(cx.view(B, T, Ci), rebuild(list(gate_params)), H, W, gate_type, activation, c_scale)
         khat = S.spectral_kernel(kernel, H, W, rho, goom_floor=True, scan_order=True)
         y = S.gated_scan(xm.view(B, T, Ci, H, W), z.view(B, T, Ci, H, W), gates, khat, u_silu=True, z_silu=True)
-        ctx.save_for_backward(x2, w_in, xm, z, cx, kernel, khat, *gate_params)
+        ctx.save_for_backward(x2, w_in, raw, xm, z, cx, kernel, khat, ws, bs, wt, bt, *gate_params)
         ctx.meta = meta
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        x2, w_in, xm, z, cx, kernel, khat_f, *gate_params = ctx.saved_tensors
+        x2, w_in, raw, xm, z, cx, kernel, khat, ws, bs, wt, bt, *gate_params = ctx.saved_tensors
         B, T, H, W, Ci, gate_type, activation, rho, rebuild = ctx.meta
         F, HW, Wf = B * T, H * W, W // 2 + 1
         K = x2.shape[1]
         dy = dy.contiguous().view(F, Ci, HW)
+        xm = xm.view(F, Ci, HW)
         c_scale = S.scan_c_scale(H, W)
         gps = rebuild(list(gate_params))
         cx3 = cx.view(B, T, Ci)
-        with torch.enable_grad():
-            k_l = kernel.detach().requires_grad_(True)
-            khat = khat_planes(k_l, H, W, rho)
         gates_c = S.gated_gates(cx3, gps, H, W, gate_type, activation, c_scale)
         uspec = S.rfft2_ex(xm, H, W, x_silu=True)
         dspec = S.rfft2_ex(dy, H, W, a=z, a_silu=True)
@@ -299,10 +304,9 @@ class _GatedInScanFn(torch.autograd.Function):
         sdu = torch.empty_like(uspec)
         dgates = torch.empty_like(gates_c)
         dkh = torch.empty((B, Ci, H, Wf), dtype=torch.complex64, device=dy.device)
-        # the reverse recurrence on the forward's own K_hat; torch's construction only differentiates it
-        S.gated_scan_bwd_bins(uspec, dspec, gates_c, khat_f, B, T, Ci, H, W, c_scale, yspec, sdu, dgates, dkh)
+        S.gated_scan_bwd_bins(uspec, dspec, gates_c, khat, B, T, Ci, H, W, c_scale, yspec, sdu, dgates, dkh)
         del uspec, dspec, gates_c
-        (dk,) = torch.autograd.grad([khat], [k_l], [dkh.sum(dim=0)])
+        dk = _khat_adjoint(kernel, dkh, H, W, rho)
         # the gate pre-activations' gradients (cssm_gated_gates_bwd), then the projections' as GEMMs
         # over frames: every gate kernel side by side is one (Ci, 3 n) matrix, the layout of dfac
         dfac = S.gated_gates_backward(cx3, gps, H, W, dgates, gate_type, activation, c_scale).view(F, -1)
@@ -321,13 +325,54 @@ class _GatedInScanFn(torch.autograd.Function):
         sums = (torch.empty((2, F, Ci), dtype=torch.float32, device=dy.device)
                 if S.irfft2_ex_sums_supported(F * Ci, H, W) else None)
         S.irfft2_ex(yspec, W, dxz[:, Ci:], m=dy, d=z, sums=sums[1] if sums is not None else None)
-        S.irfft2_ex(sdu, W, dxz[:, :Ci], add=(dcx.reshape(F, Ci) * (1.0 / HW)).contiguous(), d=xm,
-                    sums=sums[0] if sums is not None else None)
+        do = dxz[:, :Ci] if raw is None else torch.empty((F, Ci, HW), dtype=torch.float32, device=dy.device)
+        S.irfft2_ex(sdu, W, do, add=(dcx.reshape(F, Ci) * (1.0 / HW)).contiguous(), d=xm,
+                    sums=sums[0] if sums is not None and raw is None else None)
         del yspec, sdu
+        conv_grads = [None] * 4
+        if raw is None:
+            db = sums.sum(dim=1).reshape(-1) if sums is not None else dxz.sum(dim=(0, 2))
+        else:
+            spatial, temporal = (ws, bs) if ws is not None else None, (wt, bt) if wt is not None else None
+            cs = S.short_conv_backward(raw.view(B, T, Ci, H, W), do.view(B, T, Ci, H, W), spatial, temporal,
+                                       dxz[:, :Ci])
+            del do
+            if spatial:
+                conv_grads[:2] = [cs[:, :9].t().reshape(ws.shape), cs[:, 9]]
+            if temporal:                            # sums by lag: tap j has lag kt - 1 - j
+                conv_grads[2:] = [cs[:, 10:10 + wt.shape[0]].flip(1).t().reshape(wt.shape), cs[:, 14]]
+            db = torch.cat([cs[:, 15], sums[1].sum(dim=0) if sums is not None else dxz[:, Ci:].sum(dim=(0, 2))])
         dx = S.proj_out(dxz, w_in.t().contiguous(), w_in.new_zeros(K), out_dtype=torch.float32)
         dw = torch.bmm(dxz, x2.view(F, HW, K)).sum(dim=0).t()
-        db = sums.sum(dim=1).reshape(-1) if sums is not None else dxz.sum(dim=(0, 2))
-        return (dx, dw, db, dk, None, *gp_grads)
+        return (dx, dw, db, dk, None, *conv_grads, *gp_grads)
+
+
+def _khat_adjoint(kernel, dkh, H, W, rho):
+    """Gradient of the spectral kernel parameter from K_hat's per batch element, (B, C, H, Wf) in the scan layout."""
+    if S.spectral_kernel_bwd_supported(kernel.shape[-1], H, W):
+        return S.spectral_kernel_backward(kernel, dkh, W, rho, squash=True, goom_floor=True, scan_order=True)
+    with torch.enable_grad():
+        k_l = kernel.detach().requires_grad_(True)
+        khat = khat_planes(k_l, H, W, rho)
+    return torch.autograd.grad([khat], [k_l], [dkh.sum(dim=0)])[0]
+
+
+class _WhatFn(torch.autograd.Function):
+    """W_hat = rho F / (1 + |F|) (or F) of the GDN cell's kernel parameter on the HIP kernels
+    (cssm_spectral_kernel and its adjoint)."""
+
+    @staticmethod
+    def forward(ctx, k, H, W, rho, squash):
+        ctx.save_for_backward(k)
+        ctx.args = (W, rho, squash)
+        return S.spectral_kernel(k, H, W, rho, squash=squash, goom_floor=False)
+
+    @staticmethod
+    def backward(ctx, g):
+        (k,) = ctx.saved_tensors
+        W, rho, squash = ctx.args
+        return (S.spectral_kernel_backward(k, g.contiguous().unsqueeze(0), W, rho, squash, False, False), None, None,
+                None, None)
 
 
 def gated_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tensor:
@@ -340,12 +385,16 @@ def gated_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Te
     if not S.gated_scan_supported(H, W):
         raise NotImplementedError(f"no fused scan kernel for {H}x{W} planes")
     no_convs = cell.short_conv_spatial_size == 0 and cell.short_conv_size == 0
-    if no_convs and S.fft_ex_supported(H, W):
+    if S.fft_ex_supported(H, W) and (no_convs or S.short_conv_train_supported(T, H, W, cell.short_conv_spatial_size,
+                                                                               cell.short_conv_size)):
         # in_proj through the scan as one node whose backward runs on the fused HIP transforms
         gps, rebuild = _gate_leaves(p, cell.gate_type)
         meta = (B, T, H, W, Ci, cell.gate_type, cell.gate_activation, cell.spectral_rho, rebuild)
+        convs = []
+        for n, size in (("short_conv_spatial", cell.short_conv_spatial_size), ("short_conv_temporal", cell.short_conv_size)):
+            convs += [p[n]["kernel"].contiguous(), p[n]["bias"].contiguous()] if size > 0 else [None, None]
         y = _GatedInScanFn.apply(x.reshape(-1, cin).float().contiguous(), p["in_proj"]["kernel"],
-                                 p["in_proj"]["bias"], p["kernel"], meta, *gps)
+                                 p["in_proj"]["bias"], p["kernel"], meta, *convs, *gps)
         out = _ProjOutFn.apply(y.view(B * T, Ci, H * W), p["out_proj"]["kernel"], p["out_proj"]["bias"])
         return out.view(B, T, H, W, cell.channels)
     xz = _ProjPlanesFn.apply(x.reshape(-1, cin).float().contiguous(), p["in_proj"]["kernel"], p["in_proj"]["bias"],
@@ -642,7 +691,11 @@ def gdn_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tens
     if not S.fft_supported(H, W):
         raise NotImplementedError(f"no spectral transform kernel for {H}x{W} planes")
     x = x.float()
-    what = what_planes(p["kernel"], H, W, cell.spectral_rho, not cell.no_spectral_clamp).contiguous()
+    squash = not cell.no_spectral_clamp
+    if S.spectral_kernel_bwd_supported(p["kernel"].shape[-1], H, W):
+        what = _WhatFn.apply(p["kernel"].contiguous(), H, W, cell.spectral_rho, squash)
+    else:
+        what = what_planes(p["kernel"], H, W, cell.spectral_rho, squash).contiguous()
     ctx = x.mean(dim=(2, 3))
     if not cell.position_independent_gates:
         ctx = ctx + _temporal_encoding(T, C, cell.rope_base, x.device)[None]

@@ -115,6 +115,17 @@ int cssm_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, 
                          int goom_floor, int scan_order, float* khat, void* stream);
 
 /*
+ * Adjoint of cssm_spectral_kernel: dk (C, K, K) from dkhat (B, C, H, W/2+1)
+ * complex, the gradients (dL/dRe + i dL/dIm) of the kernel's bins per batch
+ * element, added over B; the other arguments as the forward call's.  Nothing
+ * passes a floored bin.  The bins and the kernel's row sums must fit 128 KB of LDS
+ * (cssm_spectral_kernel_bwd_supported).
+ */
+int cssm_spectral_kernel_bwd_supported(int K, int H, int W);
+int cssm_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, float rho, int squash, int goom_floor,
+                             int scan_order, const float* dkhat, float* dk, void* stream);
+
+/*
  * Spatial mean of every H x W plane: out[i] = mean(act(x[i, :, :])).
  * Replaces cssm.py:536 (ctx = x_main.mean(axis=(2, 3))) for plane-major x.
  *   x (nplanes, H, W) of dtype; out (nplanes) float32; act = cssm_load_act.
@@ -317,6 +328,24 @@ int cssm_proj_out(const void* y, int in_dtype, int F, int HW, int K, int N, cons
 int cssm_short_conv(const void* x, int in_dtype, int B, int T, int C, int H, int W, int ks,
                     const float* ws, const float* bs, int kt, const float* wt, const float* bt,
                     void* u, int out_dtype, float* ctx, void* stream);
+
+/*
+ * Training form of cssm_short_conv in float32: o = the pre-activation the SiLU
+ * takes, ctx (B, T, C) = the spatial mean of SiLU(o) or NULL; ks 0 or 3, kt <= 4,
+ * planes up to 128 x 128 (cssm_short_conv_train_supported).  The adjoint of its two
+ * convolutions takes d_o (B, T, C, H, W) and writes dx (frame stride dx_fs
+ * floats) and sums (chunks, B, C, 16), chunks = cssm_short_conv_bwd_chunks: the
+ * gradients of the 3 x 3 taps (9, kernel order), the spatial bias, the temporal
+ * taps by lag (4: lag l is tap kt - 1 - l), the temporal bias, and the sum of dx, to
+ * add over the first two axes.
+ */
+int cssm_short_conv_train_supported(int T, int H, int W, int ks, int kt);
+int cssm_short_conv_train(const float* x, int B, int T, int C, int H, int W, int ks, const float* ws, const float* bs,
+                          int kt, const float* wt, const float* bt, float* o, float* ctx, void* stream);
+int cssm_short_conv_bwd_chunks(int B, int T, int C, int H, int W);
+int cssm_short_conv_bwd(const float* x, const float* d_o, int B, int T, int C, int H, int W, int ks, const float* ws,
+                        const float* bs, int kt, const float* wt, float* dx, long long dx_fs, float* sums,
+                        void* stream);
 
 /*
  * Dense projection of channels-last rows into ONE plane-major tensor.
@@ -569,7 +598,7 @@ int cssm_gdn_scan_bins(const float* spec, const float* norms, const float* ab, l
  * x[h + a - (ks-1)/2][w + b - (ks-1)/2][c] dy[h][w][c], zero outside the frame.
  *   x, dy    (F, H, W, C) float32 channels-last
  *   partial  (blocks, ks, ks, C) float32 out: per-block partial sums (add them over blocks)
- * ks in {3, 5, 7}, C / 4 dividing 64, W a multiple of 8 (cssm_depthwise_conv_wgrad_supported);
+ * ks in {3, 5, 7}, C a multiple of 4 up to 1024 (cssm_depthwise_conv_wgrad_supported);
  * 16-byte aligned tensors; blocks <= 65535.
  */
 int cssm_depthwise_conv_wgrad(const float* x, const float* dy, int F, int H, int W, int C, int ks, float* partial,
