@@ -95,7 +95,9 @@ SIGNATURES = {
     "cssm_short_conv_train": (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P, _P, _P]),
     "cssm_short_conv_bwd_chunks": (_I, [_I, _I, _I, _I, _I]),
     "cssm_short_conv_bwd": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _LL, _P, _P]),
-    "cssm_spectral_kernel_bwd_supported": (_I, [_I, _I, _I]),
+    "cssm_spectral_kernel_bwd_parts": (_I, [_I, _I, _I, _I]),
+    "cssm_gated_scan_bwd_groups": (_I, [_I, _I, _I, _I]),
+    "cssm_gated_scan_bwd_split": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, ctypes.c_float, _P, _P, _I, _P, _P, _P]),
     "cssm_spectral_kernel_bwd": (_I, [_P, _I, _I, _I, _I, _I, ctypes.c_float, _I, _I, _I, _P, _P, _P]),
     "cssm_proj_planes": (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P]),
     "cssm_frame_mean": (_I, [_P, _I, _I, _I, _I, _P, _P]),

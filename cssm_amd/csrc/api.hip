@@ -79,8 +79,8 @@ int cssm_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, 
   return hip_status(e, "cssm_spectral_kernel");
 }
 
-int cssm_spectral_kernel_bwd_supported(int K, int H, int W) {
-  return cssm::spectral_kernel_bwd_supported(K, H, W) ? 1 : 0;
+int cssm_spectral_kernel_bwd_parts(int C, int K, int H, int W) {
+  return cssm::spectral_kernel_bwd_supported(C, K, H, W) ? cssm::spectral_kernel_bwd_parts(C, W) : 0;
 }
 
 int cssm_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, float rho, int squash, int goom_floor,
@@ -89,7 +89,7 @@ int cssm_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, 
   if (B <= 0 || C <= 0 || K <= 0 || H <= 0 || W <= 0)
     return fail(CSSM_ERR_SHAPE, "cssm_spectral_kernel_bwd: B=%d C=%d K=%d H=%d W=%d must be positive", B, C, K, H, W);
   if (!aligned(dkhat, 8)) return fail(CSSM_ERR_ALIGN, "cssm_spectral_kernel_bwd: dkhat must be 8-byte aligned");
-  if (!cssm::spectral_kernel_bwd_supported(K, H, W))
+  if (!cssm::spectral_kernel_bwd_supported(C, K, H, W))
     return fail(CSSM_ERR_UNSUPPORTED, "cssm_spectral_kernel_bwd: K=%d, %dx%d planes", K, H, W);
   return hip_status(cssm::launch_spectral_kernel_bwd(k, B, C, K, H, W, rho, squash, goom_floor, scan_order ? 1 : 0,
                                                      reinterpret_cast<const float2*>(dkhat), dk,
@@ -229,25 +229,36 @@ int cssm_gated_scan_bins(float* spec, const float* gates, const float* khat, flo
                     "cssm_gated_scan_bins");
 }
 
-int cssm_gated_scan_bwd(const float* uspec, const float* dspec, const float* gates, const float* khat, int B, int T,
-                        int C, int H, int W, float c_scale, float* yspec, float* sdu, float* dgates, float* dkhat,
-                        void* stream) {
+int cssm_gated_scan_bwd_split(const float* uspec, const float* dspec, const float* gates, const float* khat, int B,
+                              int T, int C, int H, int W, float c_scale, float* yspec, float* sdu, int groups,
+                              float* dgates, float* dkhat, void* stream) {
   if (!uspec || !dspec || !gates || !khat || !yspec || !sdu || !dgates || !dkhat)
-    return fail(CSSM_ERR_NULL, "cssm_gated_scan_bwd: null argument");
-  if (B <= 0 || T <= 0 || C <= 0 || H <= 0 || W <= 0 || !(c_scale > 0.0f))
-    return fail(CSSM_ERR_SHAPE, "cssm_gated_scan_bwd: B=%d T=%d C=%d H=%d W=%d c_scale=%g", B, T, C, H, W,
+    return fail(CSSM_ERR_NULL, "cssm_gated_scan_bwd_split: null argument");
+  if (B <= 0 || T <= 0 || C <= 0 || H <= 0 || W <= 0 || groups <= 0 || groups > C || !(c_scale > 0.0f))
+    return fail(CSSM_ERR_SHAPE, "cssm_gated_scan_bwd_split: B=%d T=%d C=%d H=%d W=%d c_scale=%g", B, T, C, H, W,
                 double(c_scale));
-  if (T > 32) return fail(CSSM_ERR_UNSUPPORTED, "cssm_gated_scan_bwd: T=%d (the reverse pass holds T <= 32 states)", T);
+  if (T > 32) return fail(CSSM_ERR_UNSUPPORTED, "cssm_gated_scan_bwd_split: T=%d (the reverse pass holds T <= 32 states)", T);
   if (!aligned(gates, 16) || !aligned(dgates, 16) || !aligned(uspec, 8) || !aligned(dspec, 8) || !aligned(khat, 8) ||
       !aligned(yspec, 8) || !aligned(sdu, 8) || !aligned(dkhat, 8))
-    return fail(CSSM_ERR_ALIGN, "cssm_gated_scan_bwd: gates 16-byte aligned, complex tensors 8");
+    return fail(CSSM_ERR_ALIGN, "cssm_gated_scan_bwd_split: gates 16-byte aligned, complex tensors 8");
   return hip_status(cssm::launch_gated_scan_bwd_bins(
                         reinterpret_cast<const float2*>(uspec), reinterpret_cast<const float2*>(dspec),
                         reinterpret_cast<const float4*>(gates), reinterpret_cast<const float2*>(khat), B, T, C, H, W,
                         c_scale, reinterpret_cast<float2*>(yspec), reinterpret_cast<float2*>(sdu),
-                        reinterpret_cast<float4*>(dgates), reinterpret_cast<float2*>(dkhat),
+                        reinterpret_cast<float4*>(dgates), reinterpret_cast<float2*>(dkhat), groups,
                         static_cast<hipStream_t>(stream)),
-                    "cssm_gated_scan_bwd");
+                    "cssm_gated_scan_bwd_split");
+}
+
+int cssm_gated_scan_bwd_groups(int B, int C, int H, int W) {
+  return B > 0 && C > 0 && H > 0 && W > 0 ? cssm::gated_bwd_groups(B, C, H, W) : 0;
+}
+
+int cssm_gated_scan_bwd(const float* uspec, const float* dspec, const float* gates, const float* khat, int B, int T,
+                        int C, int H, int W, float c_scale, float* yspec, float* sdu, float* dgates, float* dkhat,
+                        void* stream) {
+  return cssm_gated_scan_bwd_split(uspec, dspec, gates, khat, B, T, C, H, W, c_scale, yspec, sdu, 1, dgates, dkhat,
+                                   stream);
 }
 
 size_t cssm_proj_in_workspace_size(int F, int HW, int K, int N) {

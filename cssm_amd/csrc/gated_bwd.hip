@@ -18,8 +18,9 @@
 //   dY = rfft2(dy) c_v / (H W)         (y = irfft2(Y), C2R rule; c_v = 2 for
 //                                       0 < v < W/2, else 1)
 //   du = irfft2(dU H W / c_v)          (U = rfft2(u))
-// One thread owns one bin of one batch element and walks every channel, so
-// the channel sums of the gate gradients need no cross-thread reduction.
+// One thread owns one bin of one batch element and walks its group's channels, so
+// a group's channel sums of the gate gradients need no cross-thread reduction; the
+// groups' sums are added by the caller.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -35,7 +36,7 @@ struct GatedBwdArgs {
   const float2* khat;     // (C, H, WF) floored K_hat, scan layout (khat_pos)
   float2* yspec;          // (B, T, C, H, WF) out: Y_t = C h_t (irfft2 -> y_pre), natural order
   float2* sdu;            // (B, T, C, H, WF) out: dU_t H W / c_v (irfft2 -> du), natural order
-  float4* dgates;         // (B, T, H, WF) out: (dE, dDB, dVF2, dGCs) summed over channels, scan order
+  float4* dgates;         // (groups, B, T, H, WF) out: (dE, dDB, dVF2, dGCs) summed over a group's channels, scan order
   float2* dkhat;          // (B, C, H, WF) out: sum over t of E_t dA_t per batch element, khat's layout
   int T, C, H, W;
   float c_scale;          // the GCs = C c_scale of the gate planes
@@ -46,7 +47,8 @@ __global__ void __launch_bounds__(256) gated_scan_bwd_bins(const GatedBwdArgs a)
   const int H = a.H, W = a.W, WF = W / 2 + 1, HWF = H * WF;
   const int i = int(blockIdx.x) * 256 + int(threadIdx.x);
   if (i >= HWF) return;
-  const int b = blockIdx.y, T = a.T, C = a.C;
+  const int b = blockIdx.y, T = a.T, C = a.C, per = (C + int(gridDim.z) - 1) / int(gridDim.z);
+  const int c0 = int(blockIdx.z) * per, c1 = c0 + per < C ? c0 + per : C;
   const int u = i / WF, p = i % WF, v = scan_col(H, W, p);
   const int nat = u * WF + v;                       // spectra: natural column order
   const int kpos = khat_pos(H, W, u, p);            // K_hat and its gradient: the scan's slot
@@ -81,8 +83,9 @@ __global__ void __launch_bounds__(256) gated_scan_bwd_bins(const GatedBwdArgs a)
   constexpr bool AHEAD = MAXT <= 8;
   float2 kn;
   float2 Un[AHEAD ? MAXT : 1], Dn[AHEAD ? MAXT : 1];
-  if constexpr (AHEAD) fetch(0, kn, Un, Dn);
-  for (int c = 0; c < C; ++c) {
+  if constexpr (AHEAD)
+    if (c0 < c1) fetch(c0, kn, Un, Dn);
+  for (int c = c0; c < c1; ++c) {
     float2 h[MAXT], U[MAXT], D[MAXT];
     if constexpr (AHEAD) {
 #pragma unroll
@@ -95,7 +98,7 @@ __global__ void __launch_bounds__(256) gated_scan_bwd_bins(const GatedBwdArgs a)
     }
     const float2 kf = kn;
     if constexpr (AHEAD) {
-      if (c + 1 < C) fetch(c + 1, kn, Un, Dn);
+      if (c + 1 < c1) fetch(c + 1, kn, Un, Dn);
     }
     float2 hp = make_float2(0.f, 0.f);
 #pragma unroll
@@ -141,15 +144,29 @@ __global__ void __launch_bounds__(256) gated_scan_bwd_bins(const GatedBwdArgs a)
   }
 #pragma unroll
   for (int t = 0; t < MAXT; ++t)
-    if (t < T) a.dgates[(size_t(b) * T + t) * HWF + i] = gs[t];
+    if (t < T) a.dgates[((size_t(blockIdx.z) * gridDim.y + b) * T + t) * HWF + i] = gs[t];
+}
+
+// channel groups for about four workgroups per CU where all channels in one give fewer than the two that
+// fit (32 elements x 64 channels of 32 x 32: 144 -> 69 us with 11 groups), at least four channels each.
+// With the chip filled the groups gain nothing (16 elements of 128 x 128, 528 workgroups: 673 us, 684 in
+// four groups, and 30 us to add them).
+int gated_bwd_groups(int B, int C, int H, int W) {
+  const long long blocks = (long long)B * ((H * (W / 2 + 1) + 255) / 256);
+  if (blocks >= 512) return 1;
+  long long g = (1024 + blocks - 1) / blocks;
+  if (g > (C + 3) / 4) g = (C + 3) / 4;
+  const int per = int((C + g - 1) / g);
+  return (C + per - 1) / per;
 }
 
 hipError_t launch_gated_scan_bwd_bins(const float2* uspec, const float2* dspec, const float4* gates,
                                       const float2* khat, int B, int T, int C, int H, int W, float c_scale,
-                                      float2* yspec, float2* sdu, float4* dgates, float2* dkhat, hipStream_t s) {
+                                      float2* yspec, float2* sdu, float4* dgates, float2* dkhat, int groups,
+                                      hipStream_t s) {
   GatedBwdArgs a{uspec, dspec, gates, khat, yspec, sdu, dgates, dkhat, T, C, H, W, c_scale};
   const int hwf = H * (W / 2 + 1);
-  const dim3 grid(unsigned((hwf + 255) / 256), unsigned(B));
+  const dim3 grid(unsigned((hwf + 255) / 256), unsigned(B), unsigned(groups));
   if (T <= 8) hipLaunchKernelGGL(gated_scan_bwd_bins<8>, grid, dim3(256), 0, s, a);
   else if (T <= 32) hipLaunchKernelGGL(gated_scan_bwd_bins<32>, grid, dim3(256), 0, s, a);
   else return hipErrorInvalidValue;

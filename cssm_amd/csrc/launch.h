@@ -75,7 +75,8 @@ __device__ __forceinline__ float ctx_tile_sum(const float* __restrict__ partial,
 
 hipError_t launch_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, int squash,
                                   int goom_floor, int scan_order, float2* khat, hipStream_t s);
-bool spectral_kernel_bwd_supported(int K, int H, int W);
+bool spectral_kernel_bwd_supported(int C, int K, int H, int W);
+int spectral_kernel_bwd_parts(int C, int W);   // dk (parts, C, K, K)
 hipError_t launch_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, float rho, int squash,
                                       int goom_floor, int scan_order, const float2* d, float* dk, hipStream_t s);
 hipError_t launch_plane_mean(const void* x, int dtype, long long nplanes, int HW, int act, float* out,
@@ -228,9 +229,12 @@ bool norm_gate_train_supported(int C);
 int norm_gate_blocks(long long M);
 hipError_t launch_norm_gate_train(const NormGateArgs& a, long long M, bool bwd, hipStream_t s);
 // backward of the gated scan: the spectral-domain reverse recurrence per (b, bin), T <= 32
+// (channels in groups: dgates (groups, B, T, H, WF) partial sums)
+int gated_bwd_groups(int B, int C, int H, int W);
 hipError_t launch_gated_scan_bwd_bins(const float2* uspec, const float2* dspec, const float4* gates,
                                       const float2* khat, int B, int T, int C, int H, int W, float c_scale,
-                                      float2* yspec, float2* sdu, float4* dgates, float2* dkhat, hipStream_t s);
+                                      float2* yspec, float2* sdu, float4* dgates, float2* dkhat, int groups,
+                                      hipStream_t s);
 // forward recurrence of the gated scan on spectra (B, T, C, H, WF), in place: rfft2(u) -> C h; state
 // (B, C, H, WF) carries h between calls on consecutive frames (read unless first; may be null)
 hipError_t launch_gated_scan_fwd_bins(float2* spec, const float4* gates, const float2* khat, float2* state, int first,

@@ -31,15 +31,16 @@ __host__ __device__ inline SpecTaps spec_taps(int K, int H, int W) {
   return {0, K, (H - K) / 2, 0, K, (W - K) / 2};                       // zero pad
 }
 
-// LDS: tw (W), th (H) double2 tables, then R[i][v] = sum_j k[i][j] e^{-2 pi i v j' / W}
-__device__ __forceinline__ void spec_rows(const float* kc, int K, int H, int W, const SpecTaps& q, double2* tw,
-                                          double2* th, double2* R) {
-  const int WF = W / 2 + 1;
+// LDS: tw (W), th (H) double2 tables, then R[i][j] = sum_j' k[i][j'] e^{-2 pi i v j'' / W} for the nc columns
+// v = col(j)
+template <class Col>
+__device__ __forceinline__ void spec_rows(const float* kc, int K, int H, int W, const SpecTaps& q, int nc, Col col,
+                                          double2* tw, double2* th, double2* R) {
   for (int m = threadIdx.x; m < W; m += blockDim.x) sincospi(2.0 * double(m) / double(W), &tw[m].y, &tw[m].x);
   for (int m = threadIdx.x; m < H; m += blockDim.x) sincospi(2.0 * double(m) / double(H), &th[m].y, &th[m].x);
   __syncthreads();
-  for (int idx = threadIdx.x; idx < q.nr * WF; idx += blockDim.x) {
-    const int i = idx / WF, v = idx % WF;
+  for (int idx = threadIdx.x; idx < q.nr * nc; idx += blockDim.x) {
+    const int i = idx / nc, v = col(idx % nc);
     double re = 0.0, im = 0.0;
     int m = v * q.ow % W;                        // v (j + ow) mod W
     for (int j = 0; j < q.nq; ++j, m = m + v < W ? m + v : m + v - W) {
@@ -52,13 +53,13 @@ __device__ __forceinline__ void spec_rows(const float* kc, int K, int H, int W, 
   }
   __syncthreads();
 }
-// F[u][v] = sum_i R[i][v] e^{-2 pi i u i' / H}
-__device__ __forceinline__ double2 spec_bin(const double2* R, const double2* th, const SpecTaps& q, int H, int WF,
-                                            int u, int v) {
+// F[u][v] = sum_i R[i][j] e^{-2 pi i u i' / H}, j the column's slot of nc
+__device__ __forceinline__ double2 spec_bin(const double2* R, const double2* th, const SpecTaps& q, int H, int nc,
+                                            int u, int j) {
   double re = 0.0, im = 0.0;
   int m = u * q.oh % H;                          // u (i + oh) mod H
   for (int i = 0; i < q.nr; ++i, m = m + u < H ? m + u : m + u - H) {
-    const double2 w = th[m], a = R[i * WF + v];
+    const double2 w = th[m], a = R[i * nc + j];
     // (ar + i ai)(cs - i sn)
     re += a.x * w.x + a.y * w.y;
     im += a.y * w.x - a.x * w.y;
@@ -72,7 +73,7 @@ __global__ void spectral_kernel_prep(const float* __restrict__ k, int K, int H, 
   const int c = blockIdx.x, WF = W / 2 + 1;
   const SpecTaps q = spec_taps(K, H, W);
   double2 *tw = sm_d, *th = sm_d + W, *R = sm_d + W + H;
-  spec_rows(k + size_t(c) * K * K, K, H, W, q, tw, th, R);
+  spec_rows(k + size_t(c) * K * K, K, H, W, q, WF, [](int j) { return j; }, tw, th, R);
   // at position (u, p) of the output with v = scan_col(p) in the scan's column order, in the scan's
   // slot khat_pos(u, p); gridDim.y workgroups share a channel's bins
   for (int idx = int(blockIdx.y) * blockDim.x + threadIdx.x; idx < H * WF; idx += gridDim.y * blockDim.x) {
@@ -98,29 +99,34 @@ __global__ void spectral_kernel_prep(const float* __restrict__ k, int K, int H, 
 // K_hat = rho F / (1 + |F|):
 //   dF = rho (d / (1 + |F|) - F Re(conj(d) F) / (|F| (1 + |F|)^2)),
 // nothing through a floored bin (|K_hat| < 1e-7), and dk[i][j] = Re sum_{u,v} dF e^{+2 pi i (u i' / H +
-// v j' / W)}: over u for the nr kept rows, then over v.  One workgroup per channel; F in double as the
-// forward takes it, dF in LDS as float (fp32 gradients), the sums in double.
-__global__ void __launch_bounds__(512) spectral_kernel_bwd(const float* __restrict__ k, int B, int C, int K, int H,
+// v j' / W)}: over u for the nr kept rows, then over v.  The columns (positions p of
+// the layout) are dealt in gridDim.y runs of nc, each with its own part of the sum: dk (gridDim.y, C, K, K) for
+// the caller to add.  F in double as the forward takes it, dF in LDS as float (fp32 gradients), the sums in
+// double.  (One workgroup per channel: 149 us for 64 channels of 128 x 128 and 16 batch elements.)
+__global__ void __launch_bounds__(256) spectral_kernel_bwd(const float* __restrict__ k, int B, int C, int K, int H,
                                                            int W, float rho, int squash, int goom_floor,
-                                                           int scan_order, const float2* __restrict__ d,
+                                                           int scan_order, int nc, const float2* __restrict__ d,
                                                            float* __restrict__ dk) {
   extern __shared__ double2 sm_d[];
-  const int c = blockIdx.x, WF = W / 2 + 1, n = H * WF;
+  const int c = blockIdx.x, WF = W / 2 + 1, n = H * WF, p0 = int(blockIdx.y) * nc;
+  if (p0 + nc > WF) nc = WF - p0;
   const SpecTaps q = spec_taps(K, H, W);
   double2 *tw = sm_d, *th = sm_d + W, *R = sm_d + W + H;
-  float2* dF = reinterpret_cast<float2*>(R + q.nr * WF);
-  spec_rows(k + size_t(c) * K * K, K, H, W, q, tw, th, R);
-  for (int idx = threadIdx.x; idx < n; idx += blockDim.x) {
-    const int u = idx / WF, v = scan_order ? scan_col(H, W, idx % WF) : idx % WF;
-    const size_t pos = scan_order ? khat_pos(H, W, u, idx % WF) : idx;
+  float2* dF = reinterpret_cast<float2*>(R + q.nr * nc);
+  auto col = [&](int j) { return scan_order ? scan_col(H, W, p0 + j) : p0 + j; };
+  spec_rows(k + size_t(c) * K * K, K, H, W, q, nc, col, tw, th, R);
+  for (int idx = threadIdx.x; idx < H * nc; idx += blockDim.x) {
+    const int u = idx / nc, j = idx % nc;
+    const size_t pos = scan_order ? khat_pos(H, W, u, p0 + j) : u * WF + p0 + j;
     float2 g = make_float2(0.0f, 0.0f);
+#pragma unroll 8
     for (int b = 0; b < B; ++b) {
       const float2 e = d[(size_t(b) * C + c) * n + pos];
       g.x += e.x;
       g.y += e.y;
     }
     if (squash || goom_floor) {
-      const double2 f = spec_bin(R, th, q, H, WF, u, v);
+      const double2 f = spec_bin(R, th, q, H, nc, u, j);
       const double mag = sqrt(f.x * f.x + f.y * f.y), s = squash ? 1.0 / (1.0 + mag) : 1.0;
       const double kr = squash ? double(rho) * s : 1.0;
       const float2 o = make_float2(float(f.x * kr), float(f.y * kr));
@@ -131,18 +137,17 @@ __global__ void __launch_bounds__(512) spectral_kernel_bwd(const float* __restri
         g = make_float2(float(kr * g.x - t * f.x), float(kr * g.y - t * f.y));
       }
     }
-    dF[u * WF + v] = g;
+    dF[idx] = g;
   }
   __syncthreads();
-  // P[i][v] = sum_u dF[u][v] e^{+2 pi i u i' / H} over R, then dk[i][j] = Re sum_v P[i][v] e^{+2 pi i v j' / W}
-  for (int idx = threadIdx.x; idx < q.nr * WF; idx += blockDim.x) {
-    const int i = idx / WF, v = idx % WF;
+  // P[i][j] = sum_u dF[u][j] e^{+2 pi i u i' / H} over R, then dk[i][j'] = Re sum_j P[i][j] e^{+2 pi i v j'' / W}
+  for (int idx = threadIdx.x; idx < q.nr * nc; idx += blockDim.x) {
+    const int i = idx / nc, j = idx % nc, step = i + q.oh;
     double re = 0.0, im = 0.0;
     int m = 0;
-    const int step = i + q.oh;
     for (int u = 0; u < H; ++u, m = m + step < H ? m + step : m + step - H) {
       const double2 w = th[m];
-      const float2 g = dF[u * WF + v];
+      const float2 g = dF[u * nc + j];
       re += g.x * w.x - g.y * w.y;
       im += g.x * w.y + g.y * w.x;
     }
@@ -153,11 +158,11 @@ __global__ void __launch_bounds__(512) spectral_kernel_bwd(const float* __restri
     const int i = idx / K - q.r0, j = idx % K - q.q0;
     double a = 0.0;
     if (i >= 0 && i < q.nr && j >= 0 && j < q.nq)
-      for (int v = 0, m = 0; v < WF; ++v, m = m + j + q.ow < W ? m + j + q.ow : m + j + q.ow - W) {
-        const double2 w = tw[m], pv = R[i * WF + v];
+      for (int l = 0; l < nc; ++l) {
+        const double2 w = tw[col(l) * (j + q.ow) % W], pv = R[i * nc + l];
         a += pv.x * w.x - pv.y * w.y;
       }
-    dk[size_t(c) * K * K + idx] = float(a);
+    dk[(size_t(blockIdx.y) * C + c) * K * K + idx] = float(a);
   }
 }
 
@@ -318,19 +323,17 @@ constexpr int kGateThreads = 512, kGateKW = 32;
 // Few frames (a small batch): each frame's rows are split over gridDim.y workgroups of nr rows
 // (blockIdx.y), each computing its rows' products and all column products (the latter in every
 // workgroup of the frame) and writing its rows' bins; ctx is written by the first of them.
-template <bool FACTORED, bool WLDS>
+template <bool WLDS>
 __global__ void __launch_bounds__(kGateThreads, 4) gated_gates_kernel(const float* __restrict__ ctx, CtxPartials cp, int C,
                                                               int H, int W, int act, GateWeights gw, float c_scale,
                                                               float4* __restrict__ out, int nr_split) {
-  constexpr bool factored = FACTORED;
-  static_assert(!WLDS || FACTORED, "weights in LDS for the factored products");
   extern __shared__ float sm_f[];
   const int WF = W / 2 + 1;
   const int bt = blockIdx.x;
   const int nbin = H * WF;
   float* cx = sm_f;                                    // C
   float* fac = sm_f + C;                               // 3 (H + WF) factored vectors
-  float* scratch = fac + (factored ? 3 * (H + WF) : 0);
+  float* scratch = fac + 3 * (H + WF);
   if constexpr (WLDS) {
     const int nt = blockDim.x, tid = threadIdx.x;
     const int nv = 3 * (H + WF);
@@ -382,7 +385,7 @@ __global__ void __launch_bounds__(kGateThreads, 4) gated_gates_kernel(const floa
       const float d = gate_act(gr[0], act), dd = d + 1e-8f;
       out[size_t(bt) * nbin + o] = make_float4(expf(-d), dd * gr[1], dd * 2e-7f, gr[2] * c_scale);
     }
-  } else if constexpr (factored) {
+  } else {
     const int u0 = int(blockIdx.y) * nr_split;
     const int nr = H - u0 < nr_split ? H - u0 : nr_split;
     CtxPartials cpb = cp;
@@ -398,20 +401,57 @@ __global__ void __launch_bounds__(kGateThreads, 4) gated_gates_kernel(const floa
       const float d = gate_act(gr[0], act), dd = d + 1e-8f;
       out[size_t(bt) * nbin + o] = make_float4(expf(-d), dd * gr[1], dd * 2e-7f, gr[2] * c_scale);
     }
+  }
+}
+
+// Dense gates of FB frames: G_x[u, v] = ctx . kernel[:, u WF + v] + bias, one thread per bin (gridDim.y
+// runs of them) with the FB frames' three sums in registers, so a weight is read once for FB frames
+// (one 512-thread workgroup a frame read the whole kernel, 3 C H WF floats, from L2 for each).  The sums run
+// over the channels in order whatever FB.
+constexpr int kDenseNT = 256;
+template <int FB>
+__global__ void __launch_bounds__(kDenseNT) gated_gates_dense(const float* __restrict__ ctx, CtxPartials cp, int BT,
+                                                              int C, int H, int W, int act, GateWeights gw,
+                                                              float c_scale, float4* __restrict__ out) {
+  extern __shared__ float sm_f[];   // ctx of the frames, [c][FB] (and 256 floats of scratch for FB = 1)
+  const int WF = W / 2 + 1, nbin = H * WF, f0 = int(blockIdx.x) * FB;
+  const int nf = BT - f0 < FB ? BT - f0 : FB;
+  float* cx = sm_f;
+  if constexpr (FB == 1) {
+    if (blockIdx.y != 0) cp.ctx = nullptr;   // written once
+    frame_ctx(ctx, cp, f0, C, cx, cx + C);
   } else {
-    frame_ctx(ctx, cp, bt, C, cx, scratch);
-    for (int o = threadIdx.x; o < nbin; o += blockDim.x) {
-      const int bin = (o / WF) * WF + scan_col(H, W, o % WF);
-      float gr[3];
-      for (int g = 0; g < 3; ++g) {
-        float acc = gw.bd[g][bin];
-        const float* kk = gw.kd[g] + bin;
-#pragma unroll 8
-        for (int c = 0; c < C; ++c) acc = fmaf(cx[c], kk[size_t(c) * nbin], acc);
-        gr[g] = acc;
+    for (int i = threadIdx.x; i < C * FB; i += kDenseNT) {
+      const int j = i / C, c = i % C;
+      cx[c * FB + j] = j < nf ? ctx[size_t(f0 + j) * C + c] : 0.0f;
+    }
+    __syncthreads();
+  }
+  for (int o = int(blockIdx.y) * kDenseNT + threadIdx.x; o < nbin; o += gridDim.y * kDenseNT) {
+    const int bin = (o / WF) * WF + scan_col(H, W, o % WF);
+    float g[3][FB];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      const float b0 = gw.bd[x][bin];
+#pragma unroll
+      for (int j = 0; j < FB; ++j) g[x][j] = b0;
+    }
+    const float *k0 = gw.kd[0] + bin, *k1 = gw.kd[1] + bin, *k2 = gw.kd[2] + bin;
+#pragma unroll 4
+    for (int c = 0; c < C; ++c) {
+      const float w0 = k0[size_t(c) * nbin], w1 = k1[size_t(c) * nbin], w2 = k2[size_t(c) * nbin];
+#pragma unroll
+      for (int j = 0; j < FB; ++j) {
+        const float x = cx[c * FB + j];
+        g[0][j] = fmaf(x, w0, g[0][j]);
+        g[1][j] = fmaf(x, w1, g[1][j]);
+        g[2][j] = fmaf(x, w2, g[2][j]);
       }
-      const float d = gate_act(gr[0], act), dd = d + 1e-8f;
-      out[size_t(bt) * nbin + o] = make_float4(expf(-d), dd * gr[1], dd * 2e-7f, gr[2] * c_scale);
+    }
+#pragma unroll
+    for (int j = 0; j < FB; ++j) {
+      const float d = gate_act(g[0][j], act), dd = d + 1e-8f;
+      if (j < nf) out[size_t(f0 + j) * nbin + o] = make_float4(expf(-d), dd * g[1][j], dd * 2e-7f, g[2][j] * c_scale);
     }
   }
 }
@@ -597,24 +637,31 @@ hipError_t launch_spectral_kernel(const float* k, int C, int K, int H, int W, fl
   return hipGetLastError();
 }
 
-static size_t spec_bwd_lds(int K, int H, int W) {
-  const SpecTaps q = spec_taps(K, H, W);
-  const size_t WF = W / 2 + 1;
-  return (q.nr * WF + W + H) * sizeof(double2) + H * WF * sizeof(float2);
+// columns per workgroup of the adjoint: two workgroups per CU or more, at least four columns each
+static int spec_bwd_cols(int C, int W) {
+  const int WF = W / 2 + 1;
+  int ny = (512 + C - 1) / C;
+  if (ny > (WF + 3) / 4) ny = (WF + 3) / 4;
+  return (WF + ny - 1) / ny;
 }
-// planes whose bins and row sums fit a workgroup's LDS (128 x 128 with up to 31 taps)
-bool spectral_kernel_bwd_supported(int K, int H, int W) {
-  return K > 0 && H > 0 && W > 0 && !((K > H || K > W) && (K < H || K < W)) && spec_bwd_lds(K, H, W) <= 128 * 1024;
+int spectral_kernel_bwd_parts(int C, int W) {
+  const int nc = spec_bwd_cols(C, W);
+  return (W / 2 + nc) / nc;
+}
+static size_t spec_bwd_lds(int nc, int K, int H, int W) {
+  return (size_t(spec_taps(K, H, W).nr) * nc + W + H) * sizeof(double2) + size_t(H) * nc * sizeof(float2);
+}
+// planes whose bins and row sums fit a workgroup's 64 KB of LDS
+bool spectral_kernel_bwd_supported(int C, int K, int H, int W) {
+  return C > 0 && K > 0 && H > 0 && W > 0 && W < 32768 && !((K > H || K > W) && (K < H || K < W)) &&
+         spec_bwd_lds(spec_bwd_cols(C, W), K, H, W) <= 64 * 1024;
 }
 hipError_t launch_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, float rho, int squash,
                                       int goom_floor, int scan_order, const float2* d, float* dk, hipStream_t s) {
-  if (!spectral_kernel_bwd_supported(K, H, W)) return hipErrorInvalidValue;
-  const size_t shm = spec_bwd_lds(K, H, W);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(spectral_kernel_bwd),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(spectral_kernel_bwd, dim3(C), dim3(512), shm, s, k, B, C, K, H, W, rho, squash, goom_floor,
-                     scan_order, d, dk);
+  if (!spectral_kernel_bwd_supported(C, K, H, W)) return hipErrorInvalidValue;
+  const int nc = spec_bwd_cols(C, W);
+  hipLaunchKernelGGL(spectral_kernel_bwd, dim3(C, spectral_kernel_bwd_parts(C, W)), dim3(256),
+                     spec_bwd_lds(nc, K, H, W), s, k, B, C, K, H, W, rho, squash, goom_floor, scan_order, nc, d, dk);
   return hipGetLastError();
 }
 
@@ -650,7 +697,7 @@ hipError_t launch_gated_gates(const float* ctx, const CtxPartials& cp, int BT, i
     for (int g = 0; g < 3; ++g)
       wlds = wlds && (reinterpret_cast<uintptr_t>(w.kd[g]) % 16) == 0 && (reinterpret_cast<uintptr_t>(w.kw[g]) % 16) == 0;
     if (wlds) {
-      hipLaunchKernelGGL((gated_gates_kernel<true, true>), dim3(BT), dim3(NT), shm_w, s, ctx, cp, C, H, W, act, w,
+      hipLaunchKernelGGL((gated_gates_kernel<true>), dim3(BT), dim3(NT), shm_w, s, ctx, cp, C, H, W, act, w,
                          c_scale, gates, H);
     } else {
       // fewer frames than two per CU: split each frame's rows over more workgroups
@@ -662,12 +709,32 @@ hipError_t launch_gated_gates(const float* ctx, const CtxPartials& cp, int BT, i
       if (splits > H) splits = H;
       const int nr = (H + splits - 1) / splits;
       splits = (H + nr - 1) / nr;
-      hipLaunchKernelGGL((gated_gates_kernel<true, false>), dim3(BT, splits), dim3(NT), shm, s, ctx, cp, C, H, W,
+      hipLaunchKernelGGL((gated_gates_kernel<false>), dim3(BT, splits), dim3(NT), shm, s, ctx, cp, C, H, W,
                          act, w, c_scale, gates, nr);
     }
   } else {
-    hipLaunchKernelGGL((gated_gates_kernel<false, false>), dim3(BT), dim3(NT), shm, s, ctx, cp, C, H, W, act, w,
-                       c_scale, gates, H);
+    // eight frames a workgroup while that leaves every CU two of them, else fewer: below that the sums'
+    // latency shows, above it the weights' reads.  us at FB = 1 / 2 / 4 / 8 (one workgroup a frame):
+    // 256 frames, C = 64, 32 x 32 8.1 / 7.8 / 9.0 / 12.1 (12.0); 1024, C = 64, 64 x 64 74 / 45 / 32 / 29 (81);
+    // 256, C = 64, 128 x 128 148 / 82 / 50 / 35 (167); 1024, C = 256, 16 x 16 24 / 20 / 23 / 31 (27)
+    const int WF = W / 2 + 1, runs = (H * WF + kDenseNT - 1) / kDenseNT;
+    int fb = 8;
+    while (fb > 1 && (long long)((BT + fb - 1) / fb) * runs < 512) fb /= 2;
+    if (size_t(C) * fb * sizeof(float) > 64 * 1024 || (cp.partial && !cp.ctx)) fb = 1;
+    if (fb > 1 && cp.partial) {   // several frames share a workgroup: their means first (the same values)
+      const hipError_t e = launch_ctx_reduce(cp.partial, BT, cp.HW, cp.TM, cp.slots, C, cp.ctx, s);
+      if (e != hipSuccess) return e;
+      ctx = cp.ctx;
+    }
+    const size_t sh = size_t(C * fb + (fb == 1 ? 256 : 0)) * sizeof(float);
+    const dim3 grid(unsigned((BT + fb - 1) / fb), unsigned(runs));
+#define CSSM_DENSE(FB_) \
+  hipLaunchKernelGGL(gated_gates_dense<FB_>, grid, dim3(kDenseNT), sh, s, ctx, cp, BT, C, H, W, act, w, c_scale, gates)
+    if (fb == 1) CSSM_DENSE(1);
+    else if (fb == 2) CSSM_DENSE(2);
+    else if (fb == 4) CSSM_DENSE(4);
+    else CSSM_DENSE(8);
+#undef CSSM_DENSE
   }
   return hipGetLastError();
 }

@@ -55,8 +55,8 @@ def spectral_kernel(k: torch.Tensor, H: int, W: int, rho: float = 0.999, squash:
     return out
 
 
-def spectral_kernel_bwd_supported(K: int, H: int, W: int) -> bool:
-    return bool(_lib.load().cssm_spectral_kernel_bwd_supported(K, H, W))
+def spectral_kernel_bwd_supported(C: int, K: int, H: int, W: int) -> bool:
+    return bool(_lib.load().cssm_spectral_kernel_bwd_parts(C, K, H, W))
 
 
 def spectral_kernel_backward(k: torch.Tensor, dkhat: torch.Tensor, W: int, rho: float, squash: bool, goom_floor: bool,
@@ -66,10 +66,12 @@ def spectral_kernel_backward(k: torch.Tensor, dkhat: torch.Tensor, W: int, rho: 
     _dev(k, "k", torch.float32)
     _dev(dkhat, "dkhat", torch.complex64)
     B, C, H, _ = dkhat.shape
-    dk = torch.empty_like(k)
-    _lib.call("cssm_spectral_kernel_bwd", k.data_ptr(), B, C, k.shape[1], H, W, float(rho), int(squash),
+    K = k.shape[1]
+    dk = torch.empty((int(_lib.load().cssm_spectral_kernel_bwd_parts(C, K, H, W)), C, K, K), dtype=torch.float32,
+                     device=k.device)
+    _lib.call("cssm_spectral_kernel_bwd", k.data_ptr(), B, C, K, H, W, float(rho), int(squash),
               int(goom_floor), int(scan_order), dkhat.data_ptr(), dk.data_ptr(), _stream())
-    return dk
+    return dk.sum(dim=0)
 
 
 def scan_col_order(H: int, W: int) -> List[int]:
@@ -273,15 +275,19 @@ def gated_scan_backward(u: torch.Tensor, z: torch.Tensor, gates: torch.Tensor, k
 
 def gated_scan_bwd_bins(uspec, dspec, gates, khat, B: int, T: int, C: int, H: int, W: int, c_scale: float,
                         yspec, sdu, dgates, dkh) -> None:
-    """The per-bin reverse recurrence of the gated scan (cssm_gated_scan_bwd) on contiguous spectra
+    """The per-bin reverse recurrence of the gated scan (cssm_gated_scan_bwd_split) on contiguous spectra
     (B, T, C, H, W//2+1) laid out as the batched transforms write them; outputs written in place."""
     for t_, n in ((uspec, "uspec"), (dspec, "dspec"), (yspec, "yspec"), (sdu, "sdu"), (khat, "khat"), (dkh, "dkh")):
         _dev(t_, n, torch.complex64)
     _dev(gates, "gates", torch.float32)
     _dev(dgates, "dgates", torch.float32)
-    _lib.call("cssm_gated_scan_bwd", uspec.data_ptr(), dspec.data_ptr(), gates.data_ptr(), khat.data_ptr(),
-              B, T, C, H, W, float(c_scale), yspec.data_ptr(), sdu.data_ptr(), dgates.data_ptr(), dkh.data_ptr(),
-              _stream())
+    groups = int(_lib.load().cssm_gated_scan_bwd_groups(B, C, H, W))
+    parts = dgates if groups == 1 else torch.empty((groups, *dgates.shape), dtype=torch.float32, device=dgates.device)
+    _lib.call("cssm_gated_scan_bwd_split", uspec.data_ptr(), dspec.data_ptr(), gates.data_ptr(), khat.data_ptr(),
+              B, T, C, H, W, float(c_scale), yspec.data_ptr(), sdu.data_ptr(), groups, parts.data_ptr(),
+              dkh.data_ptr(), _stream())
+    if groups > 1:
+        torch.sum(parts, dim=0, out=dgates)
 
 
 def gated_scan_supported(H: int, W: int) -> bool:

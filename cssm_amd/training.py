@@ -96,6 +96,11 @@ def _col_sums(x: torch.Tensor) -> torch.Tensor:
     return S.frame_mean(x.view(M // R, R, 1, N)).sum(dim=0) * R
 
 
+def _plane_sums(x: torch.Tensor, H: int, W: int) -> torch.Tensor:
+    """(F, C) sums over the planes of a contiguous float32 (F, C, H*W) tensor, on the plane-mean kernel."""
+    return S.plane_mean(x.view(*x.shape[:2], H, W)) * float(H * W)
+
+
 class _PermuteIndex(torch.autograd.Function):
     """x.index_select(dim, idx) for a permutation idx, with the gradient gathered back through the
     inverse permutation (instead of index_select's scatter-add into a zeroed tensor)."""
@@ -331,7 +336,7 @@ class _GatedInScanFn(torch.autograd.Function):
         del yspec, sdu
         conv_grads = [None] * 4
         if raw is None:
-            db = sums.sum(dim=1).reshape(-1) if sums is not None else dxz.sum(dim=(0, 2))
+            db = sums.sum(dim=1).reshape(-1) if sums is not None else _plane_sums(dxz, H, W).sum(dim=0)
         else:
             spatial, temporal = (ws, bs) if ws is not None else None, (wt, bt) if wt is not None else None
             cs = S.short_conv_backward(raw.view(B, T, Ci, H, W), do.view(B, T, Ci, H, W), spatial, temporal,
@@ -341,7 +346,8 @@ class _GatedInScanFn(torch.autograd.Function):
                 conv_grads[:2] = [cs[:, :9].t().reshape(ws.shape), cs[:, 9]]
             if temporal:                            # sums by lag: tap j has lag kt - 1 - j
                 conv_grads[2:] = [cs[:, 10:10 + wt.shape[0]].flip(1).t().reshape(wt.shape), cs[:, 14]]
-            db = torch.cat([cs[:, 15], sums[1].sum(dim=0) if sums is not None else dxz[:, Ci:].sum(dim=(0, 2))])
+            db = torch.cat([cs[:, 15], sums[1].sum(dim=0) if sums is not None
+                            else _plane_sums(dxz, H, W)[:, Ci:].sum(dim=0)])
         dx = S.proj_out(dxz, w_in.t().contiguous(), w_in.new_zeros(K), out_dtype=torch.float32)
         dw = torch.bmm(dxz, x2.view(F, HW, K)).sum(dim=0).t()
         return (dx, dw, db, dk, None, *conv_grads, *gp_grads)
@@ -349,7 +355,7 @@ class _GatedInScanFn(torch.autograd.Function):
 
 def _khat_adjoint(kernel, dkh, H, W, rho):
     """Gradient of the spectral kernel parameter from K_hat's per batch element, (B, C, H, Wf) in the scan layout."""
-    if S.spectral_kernel_bwd_supported(kernel.shape[-1], H, W):
+    if S.spectral_kernel_bwd_supported(kernel.shape[0], kernel.shape[-1], H, W):
         return S.spectral_kernel_backward(kernel, dkh, W, rho, squash=True, goom_floor=True, scan_order=True)
     with torch.enable_grad():
         k_l = kernel.detach().requires_grad_(True)
@@ -692,7 +698,7 @@ def gdn_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tens
         raise NotImplementedError(f"no spectral transform kernel for {H}x{W} planes")
     x = x.float()
     squash = not cell.no_spectral_clamp
-    if S.spectral_kernel_bwd_supported(p["kernel"].shape[-1], H, W):
+    if S.spectral_kernel_bwd_supported(nh, p["kernel"].shape[-1], H, W):
         what = _WhatFn.apply(p["kernel"].contiguous(), H, W, cell.spectral_rho, squash)
     else:
         what = what_planes(p["kernel"], H, W, cell.spectral_rho, squash).contiguous()

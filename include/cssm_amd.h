@@ -115,13 +115,14 @@ int cssm_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, 
                          int goom_floor, int scan_order, float* khat, void* stream);
 
 /*
- * Adjoint of cssm_spectral_kernel: dk (C, K, K) from dkhat (B, C, H, W/2+1)
+ * Adjoint of cssm_spectral_kernel: the gradient of k from dkhat (B, C, H, W/2+1)
  * complex, the gradients (dL/dRe + i dL/dIm) of the kernel's bins per batch
  * element, added over B; the other arguments as the forward call's.  Nothing
- * passes a floored bin.  The bins and the kernel's row sums must fit 128 KB of LDS
- * (cssm_spectral_kernel_bwd_supported).
+ * passes a floored bin.  dk (parts, C, K, K) holds partial sums to add over the first
+ * axis, parts = cssm_spectral_kernel_bwd_parts (0: the sizes have no kernel, they do not fit
+ * a workgroup's LDS).
  */
-int cssm_spectral_kernel_bwd_supported(int K, int H, int W);
+int cssm_spectral_kernel_bwd_parts(int C, int K, int H, int W);
 int cssm_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, float rho, int squash, int goom_floor,
                              int scan_order, const float* dkhat, float* dk, void* stream);
 
@@ -233,6 +234,16 @@ int cssm_gated_scan_bins(float* spec, const float* gates, const float* khat, flo
 int cssm_gated_scan_bwd(const float* uspec, const float* dspec, const float* gates, const float* khat, int B, int T,
                         int C, int H, int W, float c_scale, float* yspec, float* sdu, float* dgates, float* dkhat,
                         void* stream);
+
+/*
+ * The same with the channels in groups that run side by side: dgates
+ * (groups, B, T, H, W/2+1, 4) holds each group's sums, to add over the first axis.
+ * groups in 1..C; cssm_gated_scan_bwd_groups gives the count that fills the chip (1 where one does).
+ */
+int cssm_gated_scan_bwd_groups(int B, int C, int H, int W);
+int cssm_gated_scan_bwd_split(const float* uspec, const float* dspec, const float* gates, const float* khat, int B,
+                              int T, int C, int H, int W, float c_scale, float* yspec, float* sdu, int groups,
+                              float* dgates, float* dkhat, void* stream);
 
 /*
  * Input projection with the layout change to plane-major fused in.

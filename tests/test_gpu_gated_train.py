@@ -81,7 +81,7 @@ def test_spectral_kernel_adjoint(S, C, K, H, squash, floor, order):
     k[0] = 0.0                                             # a floored channel
     B, Wf = 3, H // 2 + 1
     d = torch.complex(randn(gen, B, C, H, Wf), randn(gen, B, C, H, Wf))
-    assert S.spectral_kernel_bwd_supported(K, H, H)
+    assert S.spectral_kernel_bwd_supported(C, K, H, H)
     dk = S.spectral_kernel_backward(k, d, H, 0.999, squash, floor, order)
     kd = k.double().requires_grad_(True)
     if order:
