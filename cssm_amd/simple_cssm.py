@@ -265,10 +265,13 @@ class SimpleCSSM:
         bs = variables.get("batch_stats", {})
         stem_norm, body_norm = self._norms()
         x = x.float()
-        if x.dim() == 4:                                                    # :239-240
-            x = x.unsqueeze(1).expand(-1, self.seq_len, -1, -1, -1)
-        B, T, H, W, C = x.shape
-        x = x.reshape(B * T, H, W, C).contiguous()
+        # an image is repeated to seq_len frames (:239-240); the stem works frame by frame, so it runs once
+        # per image and its output is repeated
+        T = self.seq_len if x.dim() == 4 else x.shape[1]
+        if x.dim() == 4:
+            x = x.unsqueeze(1)
+        B, T_in, H, W, C = x.shape
+        x = x.reshape(B * T_in, H, W, C).contiguous()
 
         def norm_act(v, name):                                              # :247-255
             return self._norm_act(v, stem_norm, self.stem_norm_order, name, p, bs, training)
@@ -285,7 +288,7 @@ class SimpleCSSM:
                     x = norm_act(self._conv(x, p[f"conv{i + 1}"]), f"norm{i + 1}")
                 x = Fn.max_pool2d(x.permute(0, 3, 1, 2), 2, 2, ceil_mode=True).permute(0, 2, 3, 1)
         _, Hn, Wn, D = x.shape
-        x = x.reshape(B, T, Hn, Wn, D)                                      # :277-278
+        x = x.reshape(B, T_in, Hn, Wn, D).expand(B, T, Hn, Wn, D)           # :277-278
         if self.pos_embed == "learnable":                                   # :281-285
             x = x + p["pos_embed"]
         nreg = self.n_register_tokens
