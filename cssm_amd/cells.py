@@ -455,8 +455,8 @@ class GatedDeltaNetCSSM:
             gv = S.proj_planes(x, p["gate_proj"]["kernel"], p["gate_proj"]["bias"], F, HW, act=gact, out_dtype=f32)
         del xq, gates
         # spectral core: rfft2 -> delta-rule recurrence -> irfft2, in one kernel where a workgroup
-        # holds a head's state (32 x 32, d_k = 4), else through spectra in HBM
-        if S.gdn_core_fused_supported(H, W, dk):
+        # holds a head's state (32 x 32, d_k = 4) and there are enough of them, else through spectra in HBM
+        if S.gdn_core_fused_supported(H, W, dk) and S.gdn_core_fused_pays(B, T, C, dk):
             o = S.gdn_core_fused(qkv, self.use_spectral_l2_norm, ab, self.gate_type, what, dk, self.scan_variant)
             del qkv
         else:

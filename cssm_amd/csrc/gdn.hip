@@ -1096,8 +1096,11 @@ struct GdnBinArgs {
   int variant;          // kScanGoom / kScanLinear / kScanLogEps (gdn_step.h)
 };
 
-template <int DK>
-__global__ void __launch_bounds__(256) gdn_scan_bins(const GdnBinArgs a) {
+// AHEAD (few bins): the next step's spectra and gates are loaded while the current step runs, by 64-thread
+// workgroups that reach more CUs, so a step does not wait through its loads' latency.  With the chip full the
+// extra registers cost a wave per SIMD and more than that (3.48 -> 3.53 ms at 128 elements of 128 x 128).
+template <int DK, bool AHEAD>
+__global__ void __launch_bounds__(AHEAD ? 64 : 256) gdn_scan_bins(const GdnBinArgs a) {
   const int bin = blockIdx.x * blockDim.x + threadIdx.x;
   if (bin >= a.HWF) return;
   const int head = blockIdx.y, b = blockIdx.z;
@@ -1109,26 +1112,40 @@ __global__ void __launch_bounds__(256) gdn_scan_bins(const GdnBinArgs a) {
 #pragma unroll
     for (int j = 0; j < DK; ++j) s[i][j] = make_float2(0.f, 0.f);
 
-  for (int t = 0; t < a.T; ++t) {
+  float2 qn[DK], kn[DK], vn[DK], gn;
+  float rq[DK], rk[DK];
+  auto fetch = [&](int t) {
     const size_t fr = size_t(b) * a.T + t;
     const size_t ch0 = fr * 3 * C + size_t(head) * DK;   // q block; k at + C, v at + 2C
-    float2 q[DK], k[DK], v[DK];
 #pragma unroll
     for (int j = 0; j < DK; ++j) {
-      q[j] = a.spec[(ch0 + j) * HWF + bin];
-      k[j] = a.spec[(ch0 + C + j) * HWF + bin];
-      v[j] = a.spec[(ch0 + 2 * C + j) * HWF + bin];
-    }
-    if (a.norms) {
-#pragma unroll
-      for (int j = 0; j < DK; ++j) {
-        const float nq = 1.0f / sqrtf(a.norms[ch0 + j] + 1e-6f);
-        const float nk = 1.0f / sqrtf(a.norms[ch0 + C + j] + 1e-6f);
-        q[j] = cscale(q[j], nq);
-        k[j] = cscale(k[j], nk);
+      qn[j] = a.spec[(ch0 + j) * HWF + bin];
+      kn[j] = a.spec[(ch0 + C + j) * HWF + bin];
+      vn[j] = a.spec[(ch0 + 2 * C + j) * HWF + bin];
+      if (a.norms) {
+        rq[j] = a.norms[ch0 + j];
+        rk[j] = a.norms[ch0 + C + j];
       }
     }
-    const float2 g = a.ab[fr * a.ab_frame + size_t(head) * a.ab_head + size_t(bin) * a.ab_bin];
+    gn = a.ab[fr * a.ab_frame + size_t(head) * a.ab_head + size_t(bin) * a.ab_bin];
+  };
+  if (AHEAD) fetch(0);
+  for (int t = 0; t < a.T; ++t) {
+    const size_t fr = size_t(b) * a.T + t;
+    if (!AHEAD) fetch(t);
+    float2 q[DK], k[DK], v[DK];
+    const float2 g = gn;
+#pragma unroll
+    for (int j = 0; j < DK; ++j) {
+      q[j] = qn[j];
+      k[j] = kn[j];
+      v[j] = vn[j];
+      if (a.norms) {
+        q[j] = cscale(q[j], 1.0f / sqrtf(rq[j] + 1e-6f));
+        k[j] = cscale(k[j], 1.0f / sqrtf(rk[j] + 1e-6f));
+      }
+    }
+    if (AHEAD && t + 1 < a.T) fetch(t + 1);
     float2 o[DK];
     gdn_bin_step<DK>(s, q, k, v, wh, g.x, g.y, a.variant, o);
 #pragma unroll
@@ -1463,13 +1480,19 @@ hipError_t launch_gdn_scan_bins(const float2* spec, const float* norms, const fl
   a.HWF = H * (W / 2 + 1);
   a.variant = variant;
   const dim3 grid(unsigned((a.HWF + 255) / 256), unsigned(C / dk), unsigned(B));
+  // up to two 256-thread workgroups per CU: the latency of a step bounds the scan
+  const bool ahead = T > 1 && (long long)grid.x * grid.y * grid.z <= 512;
+  const dim3 grid64(unsigned((a.HWF + 63) / 64), grid.y, grid.z);
+#define CSSM_BINS(D)                                                                       \
+  case D:                                                                                  \
+    if (ahead) hipLaunchKernelGGL((gdn_scan_bins<D, true>), grid64, dim3(64), 0, s, a);    \
+    else hipLaunchKernelGGL((gdn_scan_bins<D, false>), grid, dim3(256), 0, s, a);          \
+    break;
   switch (dk) {
-    case 1: hipLaunchKernelGGL(gdn_scan_bins<1>, grid, dim3(256), 0, s, a); break;
-    case 2: hipLaunchKernelGGL(gdn_scan_bins<2>, grid, dim3(256), 0, s, a); break;
-    case 3: hipLaunchKernelGGL(gdn_scan_bins<3>, grid, dim3(256), 0, s, a); break;
-    case 4: hipLaunchKernelGGL(gdn_scan_bins<4>, grid, dim3(256), 0, s, a); break;
+    CSSM_BINS(1) CSSM_BINS(2) CSSM_BINS(3) CSSM_BINS(4)
     default: return hipErrorInvalidValue;
   }
+#undef CSSM_BINS
   return hipGetLastError();
 }
 
@@ -1554,6 +1577,16 @@ __device__ float dot_col(const float* ctx, const float* k, int C, int n, int col
 // FB frames per block (factored gates, host-chosen): each weight is loaded once and applied to the
 // FB frames' contexts (the per-frame sums keep their order, so the result does not depend on FB)
 constexpr int kGatesMaxFB = 4;
+// the context's temporal term: 0 none, 1 E[t, 2j] = sin(t / base^(2j / C)), E[t, 2j + 1] = cos(.), 2 a table
+__device__ __forceinline__ float ctx_term(int temporal, const float* ttable, float rope_base, int t, int c, int C) {
+  if (temporal == 1) {
+    const int j2 = c & ~1;
+    const double th = double(t) / pow(double(rope_base), double(j2) / double(C));
+    return float((c & 1) ? cos(th) : sin(th));
+  }
+  return temporal == 2 ? ttable[size_t(t) * C + c] : 0.0f;
+}
+
 __global__ void __launch_bounds__(1024)
 gdn_gates_kernel(const float* __restrict__ ctx_in, int T, int C, int H, int W, int nh, GdnGateWeights w,
                  int temporal, float rope_base, const float* __restrict__ ttable, float2* __restrict__ ab,
@@ -1569,17 +1602,8 @@ gdn_gates_kernel(const float* __restrict__ ctx_in, int T, int C, int H, int W, i
   float* cols = rows + FB * 4 * H;     // FB x 4 x max(W, WF)
   float* part = cols + FB * 4 * CW;    // factored: FB x P partial sums of each of the 4 (H + CW) products
   for (int e = threadIdx.x; e < FB * C; e += blockDim.x) {
-    const int fl = e / C, c = e % C, bt = f0 + fl, t = bt % T;
-    float v = ctx_in[size_t(bt) * C + c];
-    if (temporal == 1) {
-      // E[t, 2j] = sin(t / base^(2j / C)), E[t, 2j + 1] = cos(.)
-      const int j2 = c & ~1;
-      const double th = double(t) / pow(double(rope_base), double(j2) / double(C));
-      v += float((c & 1) ? cos(th) : sin(th));
-    } else if (temporal == 2) {
-      v += ttable[size_t(t) * C + c];
-    }
-    cx[e] = v;
+    const int fl = e / C, c = e % C, bt = f0 + fl;
+    cx[e] = ctx_in[size_t(bt) * C + c] + ctx_term(temporal, ttable, rope_base, bt % T, c, C);
   }
   __syncthreads();
   // gate g in {0 alpha, 1 beta, 2 B_k, 3 B_v}; spectral gates span (H, WF), spatial (H, W).
@@ -1645,10 +1669,70 @@ gdn_gates_kernel(const float* __restrict__ ctx_in, int T, int C, int H, int W, i
   }
 }
 
+// Dense gates of FB frames: one thread per output (the H WF alpha / beta pairs, then the H W input-gate
+// pairs; gridDim.y runs of them) with the FB frames' two sums in registers, so a weight is read once for FB
+// frames instead of once for each (as gated_gates_dense of prep.hip; the same sums in the same order).
+template <int FB>
+__global__ void __launch_bounds__(256) gdn_gates_dense(const float* __restrict__ ctx_in, int F, int T, int C, int H,
+                                                       int W, GdnGateWeights w, int temporal, float rope_base,
+                                                       const float* __restrict__ ttable, float2* __restrict__ ab,
+                                                       float2* __restrict__ bkv) {
+  extern __shared__ float sm[];   // ctx [c][FB]
+  const int n_ab = H * (W / 2 + 1), n = n_ab + (bkv ? H * W : 0), f0 = int(blockIdx.x) * FB;
+  for (int e = threadIdx.x; e < FB * C; e += 256) {
+    const int fl = e / C, c = e % C, bt = f0 + fl;
+    sm[c * FB + fl] = bt < F ? ctx_in[size_t(bt) * C + c] + ctx_term(temporal, ttable, rope_base, bt % T, c, C) : 0.0f;
+  }
+  __syncthreads();
+  for (int o = int(blockIdx.y) * 256 + threadIdx.x; o < n; o += gridDim.y * 256) {
+    const bool sp = o < n_ab;
+    const int g = sp ? 0 : 2, i = sp ? o : o - n_ab, m = sp ? n_ab : H * W;
+    const float *k0 = w.kd[g] + i, *k1 = w.kd[g + 1] + i;
+    float a0[FB], a1[FB];
+#pragma unroll
+    for (int j = 0; j < FB; ++j) a0[j] = a1[j] = 0.0f;
+#pragma unroll 4
+    for (int c = 0; c < C; ++c) {
+      const float w0 = k0[size_t(c) * m], w1 = k1[size_t(c) * m];
+#pragma unroll
+      for (int j = 0; j < FB; ++j) {
+        const float x = sm[c * FB + j];
+        a0[j] = fmaf(x, w0, a0[j]);
+        a1[j] = fmaf(x, w1, a1[j]);
+      }
+    }
+    const float b0 = w.bd[g][i], b1 = w.bd[g + 1][i];
+#pragma unroll
+    for (int j = 0; j < FB; ++j) {
+      if (f0 + j >= F) break;
+      const float x = sigmoid_f(a0[j] + b0), y = sigmoid_f(a1[j] + b1);
+      if (sp) ab[size_t(f0 + j) * n_ab + i] = make_float2(0.1f + 0.89f * x, y);
+      else bkv[size_t(f0 + j) * m + i] = make_float2(x, y);
+    }
+  }
+}
+
 hipError_t launch_gdn_gates(const float* ctx, int B, int T, int C, int H, int W, int nh, const GdnGateWeights& w,
                             int temporal, float rope_base, const float* ttable, float2* ab, float2* bkv,
                             hipStream_t s) {
   const int WF = W / 2 + 1, CW = W > WF ? W : WF;
+  const bool kv = bkv && w.kd[2];
+  if (w.kind == 0 && sizeof(float) * (size_t(C) + 4 * size_t(H) + 4 * size_t(CW)) <= 64 * 1024) {
+    // the frames per workgroup as for the gated cell's dense gates (launch_gated_gates)
+    const int F = B * T, runs = (H * WF + (kv ? H * W : 0) + 255) / 256;
+    int fb = 8;
+    while (fb > 1 && ((long long)((F + fb - 1) / fb) * runs < 512 || size_t(C) * fb * sizeof(float) > 64 * 1024)) fb /= 2;
+    const dim3 grid(unsigned((F + fb - 1) / fb), unsigned(runs));
+#define CSSM_DENSE(FB_)                                                                                          \
+  hipLaunchKernelGGL(gdn_gates_dense<FB_>, grid, dim3(256), size_t(C) * FB_ * sizeof(float), s, ctx, F, T, C, H, \
+                     W, w, temporal, rope_base, ttable, ab, kv ? bkv : nullptr)
+    if (fb == 1) CSSM_DENSE(1);
+    else if (fb == 2) CSSM_DENSE(2);
+    else if (fb == 4) CSSM_DENSE(4);
+    else CSSM_DENSE(8);
+#undef CSSM_DENSE
+    return hipGetLastError();
+  }
   constexpr int NT = 1024;
   const int NV = 4 * (H + CW), P = w.kind == 1 ? (NV >= NT ? 1 : NT / NV) : 0;
   const size_t per_frame = size_t(C) + 4 * size_t(H) + 4 * size_t(CW) + size_t(P) * NV;   // floats

@@ -2224,16 +2224,22 @@ hipError_t launch_gdn_qkv_proj(const void* X, int in_dtype, int B, int T, int HW
   const int M = B * T * HW, N = 3 * C;
   const QkvPost qp{{sc.w[0], sc.w[1], sc.w[2]}, {sc.b[0], sc.b[1], sc.b[2]}, kt, gate_mode, gates, T,
                    wg, bg, wg ? C : 0, gact, gv};
+  // Few (batch element, pixel block) sequences: the frame-sequential kernel walks T frames on a few CUs (3.5-4.5
+  // us a frame), so the projection of all frames at once and the post pass (about 1 us a frame) are faster, with
+  // the same results: up to 64 sequences and from 4 frames (64 -> 192 columns, us: 16 sequences, T = 8
+  // 37 / 21, T = 64 259 / 86; 64, T = 8 41 / 36; on the other side 128, T = 8 42 / 53; 4, T = 2 13.4 / 13.8).
+  // fp32 planes only: the post pass rereads them.
+  const bool two_step = T >= 4 && B * (long long)HW <= 64 * kFseqTM && out_dtype == 0 && wg == nullptr;
   // the frame-sequential kernel stores through buffer resources over one frame's planes
   const size_t esz = out_dtype == 0 ? 4 : 2;
-  if (qkv_fseq_supported(T, HW, K, kt) && kt <= 8 && size_t(N) * HW * esz < (size_t(1) << 31)) {
+  if (!two_step && qkv_fseq_supported(T, HW, K, kt) && kt <= 8 && size_t(N) * HW * esz < (size_t(1) << 31)) {
     if (in_dtype == 0 && out_dtype == 0) launch_qkv_fseq<float, float>(X, B, T, HW, K, N, W, b, out, qp, s);
     else if (in_dtype == 0) launch_qkv_fseq<float, uint16_t>(X, B, T, HW, K, N, W, b, out, qp, s);
     else if (out_dtype == 0) launch_qkv_fseq<uint16_t, float>(X, B, T, HW, K, N, W, b, out, qp, s);
     else launch_qkv_fseq<uint16_t, uint16_t>(X, B, T, HW, K, N, W, b, out, qp, s);
     return hipGetLastError();
   }
-  if (qkv_tiled_supported(T, HW, K, kt) && kt <= 8) {
+  if (!(two_step && qkv_fseq_supported(T, HW, K, kt)) && qkv_tiled_supported(T, HW, K, kt) && kt <= 8) {
     if (in_dtype == 0 && out_dtype == 0) qkv_fused_t<float, float>(X, T, M, K, N, W, b, HW, out, qp, s);
     else if (in_dtype == 0) qkv_fused_t<float, uint16_t>(X, T, M, K, N, W, b, HW, out, qp, s);
     else if (out_dtype == 0) qkv_fused_t<uint16_t, float>(X, T, M, K, N, W, b, HW, out, qp, s);

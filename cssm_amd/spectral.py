@@ -495,7 +495,9 @@ def frame_mean(x: torch.Tensor) -> torch.Tensor:
     if x.dtype not in _DTYPES:
         raise ValueError(f"unsupported dtype {x.dtype}")
     *lead, H, W, C = x.shape
-    F = int(torch.tensor(lead).prod()) if lead else 1
+    F = 1
+    for d in lead:
+        F *= d
     out = torch.empty((*lead, C), dtype=torch.float32, device=x.device)
     _lib.call("cssm_frame_mean", x.data_ptr(), _DTYPES[x.dtype], F, H * W, C, out.data_ptr(), _stream())
     return out
@@ -1050,6 +1052,15 @@ def gdn_norm_gate_backward(o: torch.Tensor, g: torch.Tensor, norm: str, scale: O
 
 def gdn_core_fused_supported(H: int, W: int, delta_key_dim: int) -> bool:
     return bool(_lib.load().cssm_gdn_core_fused_supported(H, W, delta_key_dim))
+
+
+def gdn_core_fused_pays(B: int, T: int, C: int, delta_key_dim: int) -> bool:
+    """Whether the fused core beats the batched transforms around the per-bin scan.  It gives each (batch
+    element, head) one workgroup for all T (about 13 us a step), so with few of them most CUs idle; measured
+    fused / three-kernel us: 16 workgroups, T = 8 115 / 43, T = 32 444 / 112; 64, T = 2 34 / 31; 256, T = 4
+    66 / 64, T = 32 459 / 423; and on the other side 128, T = 2 36 / 37; 512, T = 8 154 / 210; 16, T = 1 17 / 20."""
+    wgs = B * (C // delta_key_dim)
+    return not ((T >= 4 and wgs <= 256) or (T >= 2 and wgs <= 64))
 
 
 def gdn_core_fused(qkv: torch.Tensor, use_l2: bool, ab: torch.Tensor, gate_type: str, what: torch.Tensor,
