@@ -81,6 +81,10 @@ SIGNATURES = {
                                     ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
                                     ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cssm_gated_scan_bins": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, ctypes.c_float, _P]),
+    "cssm_gated_scan_bins_last": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, ctypes.c_float, _I, _P, _P]),
+    "cssm_gated_scan_last_supported": (_I, [_I, _I]),
+    "cssm_gated_scan_last": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P]),
+    "cssm_short_conv_still": (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P, _P, _P]),
     "cssm_gated_scan_bwd": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, ctypes.c_float, _P, _P, _P, _P, _P]),
     "cssm_proj_in_workspace_size": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "cssm_proj_in_noalloc": (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _P, _P]),

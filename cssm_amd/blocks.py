@@ -154,9 +154,16 @@ class CSSMSHViTBlock:
         n1 = p["norm1"]
         stats = S.block_norm_stats(x5, self.block_norm)
         pc = p.get("pos_conv") if self.use_pos_conv else None
+        # of an image's equal frames only the cell's last is kept (without the timestep gate): one frame in
+        still = (is_image and not self.timestep_gate and self.cssm_type != "gdn"
+                 and self.cell._still_pays(B, T, H, W))
         xc = S.block_norm_posconv(x5, stats, self.block_norm, n1["scale"], n1["bias"],
-                                  pc["kernel"] if pc is not None else None, pc["bias"] if pc is not None else None, T)
-        y = self.cell.apply({"params": p["cssm"]}, xc, out_dtype=out_dtype)
+                                  pc["kernel"] if pc is not None else None, pc["bias"] if pc is not None else None,
+                                  1 if still else T)
+        if still:
+            y = self.cell._apply_still({"params": p["cssm"]}, xc, T, out_dtype=out_dtype)
+        else:
+            y = self.cell.apply({"params": p["cssm"]}, xc, out_dtype=out_dtype)
         del xc
         res = x5 if x5.dtype == out_dtype else x5.to(out_dtype)
         if self.timestep_gate:

@@ -205,6 +205,50 @@ class GatedCSSM:
                          out_dtype=out_dtype or x.dtype)
         return out.view(B, T, H, W, self.channels)
 
+    def _still_pays(self, B: int, T: int, H: int, W: int) -> bool:
+        """Whether :meth:`_apply_still` covers B images of H x W (square planes that the batched transforms take,
+        a short convolution of at most 4 frames and 3 x 3 pixels) and is the faster form: always where the scan
+        itself ends in one frame (64 images of 14 x 14, C = 256, T = 2: 160 -> 123 us), behind the batched
+        transforms, two launches more, once the frames saved hold 2^20 samples (64 of 64 x 64, C = 64: T = 8
+        1405 -> 623 us, T = 2 439 -> 453; 512 of 4 x 4, C = 128: T = 8 130 -> 110, T = 5 99 -> 112; one of
+        64 x 64, C = 64, no taps, T = 2: 58 -> 64)."""
+        Ci = self.channels * self.expand
+        saved = T - min(T, max(1, self.short_conv_size))
+        if T <= 1 or not (S.gated_scan_last_supported(H, W) or B * Ci * H * W * saved > 1 << 20):
+            return False
+        return (S.gated_scan_supported(H, W) and Ci % S.gated_scan_min_group(H, W) == 0
+                and H >= 3 and S.fft_ex_supported(H, W) and B <= 65535
+                and S.short_conv_train_supported(1, H, W, self.short_conv_spatial_size, self.short_conv_size))
+
+    def _apply_still(self, variables: Params, x: torch.Tensor, T: int,
+                     out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+        """The last frame of :meth:`apply` on an image x (B, 1, H, W, C) repeated to T frames: (B, 1, H, W, C).
+        Behind the causal short convolution only its first few frames differ, so the projections run once per
+        image, the gates and forward transforms on the distinct frames, and the recurrence takes the last one
+        for the rest."""
+        p = variables["params"]
+        B, _, H, W, c_in = x.shape
+        Ci = self.channels * self.expand
+        HW, f32 = H * W, torch.float32
+        x = x.contiguous()
+        c_scale = S.scan_c_scale(H, W)
+        n = min(T, max(1, self.short_conv_size))
+        if self.short_conv_spatial_size > 0 or self.short_conv_size > 0:
+            xm, z, _ = S.proj_in(x, p["in_proj"]["kernel"], p["in_proj"]["bias"], B, HW, silu_hi=True, out_dtype=f32)
+            u, ctx = S.short_conv_still(xm.view(B, Ci, H, W), n,
+                                        p.get("short_conv_spatial") if self.short_conv_spatial_size > 0 else None,
+                                        p.get("short_conv_temporal") if self.short_conv_size > 0 else None)
+            gates = S.gated_gates(ctx, p, H, W, self.gate_type, self.gate_activation, c_scale=c_scale)
+        else:
+            u, z, _, gates = S.proj_in_gates(x, p["in_proj"]["kernel"], p["in_proj"]["bias"], B, 1, H, W, p,
+                                             self.gate_type, self.gate_activation, c_scale=c_scale, silu_lo=True,
+                                             silu_hi=True, out_dtype=f32)
+            u = u.view(B, 1, Ci, H, W)
+        y = S.gated_scan_last(u, z.view(B, Ci, H, W), gates, self.spectral_kernel(p, H, W), T - n + 1)
+        out = S.proj_out(y.view(B, Ci, HW), p["out_proj"]["kernel"], p["out_proj"]["bias"],
+                         out_dtype=out_dtype or x.dtype)
+        return out.view(B, 1, H, W, self.channels)
+
     __call__ = apply
 
 

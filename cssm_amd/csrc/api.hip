@@ -225,8 +225,40 @@ int cssm_gated_scan_bins(float* spec, const float* gates, const float* khat, flo
   return hip_status(cssm::launch_gated_scan_fwd_bins(
                         reinterpret_cast<float2*>(spec), reinterpret_cast<const float4*>(gates),
                         reinterpret_cast<const float2*>(khat), reinterpret_cast<float2*>(state), first ? 1 : 0, B, T,
-                        C, H, W, c_scale, static_cast<hipStream_t>(stream)),
+                        C, H, W, c_scale, nullptr, 1, static_cast<hipStream_t>(stream)),
                     "cssm_gated_scan_bins");
+}
+
+int cssm_gated_scan_bins_last(const float* spec, const float* gates, const float* khat, int B, int n, int C, int H,
+                              int W, float c_scale, int reps, float* last, void* stream) {
+  if (!spec || !gates || !khat || !last) return fail(CSSM_ERR_NULL, "cssm_gated_scan_bins_last: null argument");
+  if (B <= 0 || n <= 0 || C <= 0 || H <= 0 || W <= 0 || B > 65535 || reps <= 0 || !(c_scale > 0.0f) ||
+      (long long)C * H * (W / 2 + 1) > 0x7fffffffLL - 64)
+    return fail(CSSM_ERR_SHAPE, "cssm_gated_scan_bins_last: B=%d n=%d C=%d H=%d W=%d reps=%d", B, n, C, H, W, reps);
+  if (!aligned(gates, 16) || !aligned(spec, 8) || !aligned(khat, 8) || !aligned(last, 8))
+    return fail(CSSM_ERR_ALIGN, "cssm_gated_scan_bins_last: gates 16-byte aligned, complex tensors 8");
+  return hip_status(cssm::launch_gated_scan_fwd_bins(
+                        const_cast<float2*>(reinterpret_cast<const float2*>(spec)),
+                        reinterpret_cast<const float4*>(gates), reinterpret_cast<const float2*>(khat), nullptr, 1, B,
+                        n, C, H, W, c_scale, reinterpret_cast<float2*>(last), reps, static_cast<hipStream_t>(stream)),
+                    "cssm_gated_scan_bins_last");
+}
+
+int cssm_gated_scan_last_supported(int H, int W) { return cssm::gated_scan_last_has_kernel(H, W) ? 1 : 0; }
+
+int cssm_gated_scan_last(const float* u, const float* z, float* y, int B, int n, int C, int H, int W,
+                         const float* gates, const float* khat, int reps, void* stream) {
+  if (!u || !z || !y || !gates || !khat) return fail(CSSM_ERR_NULL, "cssm_gated_scan_last: null argument");
+  if (B <= 0 || n <= 0 || C <= 0 || H <= 0 || W <= 0 || reps <= 0)
+    return fail(CSSM_ERR_SHAPE, "cssm_gated_scan_last: B=%d n=%d C=%d H=%d W=%d reps=%d", B, n, C, H, W, reps);
+  if (!cssm::gated_scan_last_has_kernel(H, W))
+    return fail(CSSM_ERR_UNSUPPORTED, "cssm_gated_scan_last: no kernel for %dx%d planes", H, W);
+  if (!aligned(u, 4) || !aligned(z, 4) || !aligned(y, 4) || !aligned(gates, 16) || !aligned(khat, 8))
+    return fail(CSSM_ERR_ALIGN, "cssm_gated_scan_last: misaligned pointer");
+  return hip_status(cssm::launch_gated_scan_last(u, z, y, B, n, C, H, W, reinterpret_cast<const float4*>(gates),
+                                                 reinterpret_cast<const float2*>(khat), reps,
+                                                 static_cast<hipStream_t>(stream)),
+                    "cssm_gated_scan_last");
 }
 
 int cssm_gated_scan_bwd_split(const float* uspec, const float* dspec, const float* gates, const float* khat, int B,
@@ -415,6 +447,15 @@ int cssm_short_conv_train(const float* x, int B, int T, int C, int H, int W, int
   return hip_status(cssm::launch_short_conv(x, 0, B, T, C, H, W, ks, ws, bs, kt, wt, bt, o, 0, ctx, 1,
                                             static_cast<hipStream_t>(stream)),
                     "cssm_short_conv_train");
+}
+
+int cssm_short_conv_still(const float* x, int B, int T, int C, int H, int W, int ks, const float* ws, const float* bs,
+                          int kt, const float* wt, const float* bt, float* u, float* ctx, void* stream) {
+  if (!x || !u || (kt > 0 && !bt)) return fail(CSSM_ERR_NULL, "cssm_short_conv_still: null argument");
+  if (int e = short_conv_train_check("cssm_short_conv_still", B, T, C, H, W, ks, ws, bs, kt, wt)) return e;
+  return hip_status(cssm::launch_short_conv(x, 0, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, 0, ctx, 0,
+                                            static_cast<hipStream_t>(stream), true),
+                    "cssm_short_conv_still");
 }
 
 int cssm_short_conv_bwd_chunks(int B, int T, int C, int H, int W) {

@@ -23,9 +23,13 @@ namespace cssm {
 
 constexpr int kBinsAhead = 8;
 
+// last != nullptr: the final frame stands for reps steps and only its C h is wanted, (B, C, H, WF) in last
+// (spec is only read)
+
 __global__ void __launch_bounds__(64) gated_scan_fwd_bins(float2* __restrict__ spec, const float4* __restrict__ gates,
                                                           const float2* __restrict__ khat, float2* __restrict__ state,
-                                                          int first, int T, int C, int H, int W, float inv_cs) {
+                                                          int first, int T, int C, int H, int W, float inv_cs,
+                                                          float2* __restrict__ last, int reps) {
   const int WF = W / 2 + 1, HWF = H * WF;
   const int i = int(blockIdx.x) * 64 + int(threadIdx.x), b = blockIdx.y;
   if (i >= C * HWF) return;
@@ -63,18 +67,22 @@ __global__ void __launch_bounds__(64) gated_scan_fwd_bins(float2* __restrict__ s
       float2 V = make_float2(U[k].x * G[k].y, U[k].y * G[k].y);
       if (V.x * V.x + V.y * V.y < vf * vf) V = make_float2(vf, 0.f);
       const float2 A = cscale(kf, G[k].x);
-      h = make_float2(fmaf(A.x, h.x, fmaf(-A.y, h.y, V.x)), fmaf(A.x, h.y, fmaf(A.y, h.x, V.y)));
-      sp[size_t(t0 + k) * fs] = cscale(h, G[k].w * inv_cs);
+      const bool fin = last && t0 + k == T - 1;
+      for (int n = fin ? reps : 1; n > 0; --n)
+        h = make_float2(fmaf(A.x, h.x, fmaf(-A.y, h.y, V.x)), fmaf(A.x, h.y, fmaf(A.y, h.x, V.y)));
+      if (fin) last[(size_t(b) * C + c) * HWF + u * WF + scan_col(H, W, p)] = cscale(h, G[k].w * inv_cs);
+      else if (!last) sp[size_t(t0 + k) * fs] = cscale(h, G[k].w * inv_cs);
     }
   }
   if (state) state[size_t(b) * C * HWF + i] = h;
 }
 
 hipError_t launch_gated_scan_fwd_bins(float2* spec, const float4* gates, const float2* khat, float2* state, int first,
-                                      int B, int T, int C, int H, int W, float c_scale, hipStream_t s) {
+                                      int B, int T, int C, int H, int W, float c_scale, float2* last, int reps,
+                                      hipStream_t s) {
   const long long n = (long long)C * H * (W / 2 + 1);
   hipLaunchKernelGGL(gated_scan_fwd_bins, dim3(unsigned((n + 63) / 64), unsigned(B)), dim3(64), 0, s, spec, gates,
-                     khat, state, first, T, C, H, W, 1.0f / c_scale);
+                     khat, state, first, T, C, H, W, 1.0f / c_scale, last, reps);
   return hipGetLastError();
 }
 

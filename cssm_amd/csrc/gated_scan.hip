@@ -54,6 +54,7 @@ struct ScanArgs {
   const float4* gates;   // (B, T, H, WF) per-bin (E, DB, VF, GC), columns in scan_col order
   const float2* khat;    // (C, H, WF), GOOM-floored, scan layout (columns in scan_col order, slots khat_pos)
   int T, C, u_act, z_act;
+  int reps;              // LAST: steps the last frame stands for
 };
 
 
@@ -317,7 +318,11 @@ gated_scan_pow2(const ScanArgs a) {
 // under that bound, so the compiler may take up to 256, or 168 for 3 waves at T = 1 up to 14 x 14)
 // ONE (T = 1): the state enters at zero and is never read again, so h = V: no state registers,
 // no K_hat loads and no decay (A h = 0 exactly: A is finite), the same results as the general form.
-template <int H, int W, class IO, bool ONE>
+// LAST: the T frames are the distinct ones of a longer sequence whose last frame repeats reps times, and only
+// the final step's y is wanted: z and y hold one frame per (b, c) plane, earlier steps end with the recurrence
+// and the last frame's transform serves all its repeats (an image repeated to 8 steps behind a 4-tap short
+// convolution: 4 forward and 1 inverse transform instead of 8 and 8; 64 x 128 planes of 14 x 14 45 -> 24 us).
+template <int H, int W, class IO, bool ONE, bool LAST = false>
 __global__ void __launch_bounds__((SmallGeom<H, W>::NT), (H >= 8 ? (ONE && H <= 14 ? 3 : 2) : 512 / SmallGeom<H, W>::NT))
 gated_scan_small(const ScanArgs a, long long P) {
   using G = SmallGeom<H, W>;
@@ -372,6 +377,8 @@ gated_scan_small(const ScanArgs a, long long P) {
     asm volatile("" : "+v"(tl));
     const long long base0 = base_u[0] + (long long)t * tstride;
     const bool vec = VEC_OK && contig && ptr_ok && (base0 & 3) == 0;   // uniform over the group
+    const bool fin = !LAST || t == T - 1;                               // this step's y is wanted
+    const long long basez = LAST ? p0 * HW : base0;                     // (a multiple of 4 where VEC_OK)
     // The step's global loads are issued before any of them is used: u_t (doubled, act
     // applied: the recurrence runs on 2U as in the power-of-two kernel), on the vector path
     // z_t (read when y_t is stored), and the gates and K_hat of this thread's column (read
@@ -401,17 +408,19 @@ gated_scan_small(const ScanArgs a, long long P) {
     V4 zv[NEV];
     if (vec) {
       const V4* u4 = reinterpret_cast<const V4*>(up + base0);
-      const V4* z4 = reinterpret_cast<const V4*>(zp + base0);
+      const V4* z4 = reinterpret_cast<const V4*>(zp + basez);
       V4 uv[NEV];
 #pragma unroll
       for (int k = 0; k < NEV; ++k) {
         const int e = k * NT + tl;
         if (k * NT + NT <= NV || e < NV) uv[k] = u4[e];
       }
+      if (fin) {
 #pragma unroll
-      for (int k = 0; k < NEV; ++k) {
-        const int e = k * NT + tl;
-        if (k * NT + NT <= NV || e < NV) zv[k] = z4[e];
+        for (int k = 0; k < NEV; ++k) {
+          const int e = k * NT + tl;
+          if (k * NT + NT <= NV || e < NV) zv[k] = z4[e];
+        }
       }
 #pragma unroll
       for (int k = 0; k < NEV; ++k) {
@@ -463,6 +472,9 @@ gated_scan_small(const ScanArgs a, long long P) {
             float2 V = make_float2(sv[u].x * gq[u].y, sv[u].y * gq[u].y);
             if (V.x * V.x + V.y * V.y < gq[u].z * gq[u].z) V = make_float2(gq[u].z, 0.0f);
             sv[u] = make_float2(V.x * gq[u].w, V.y * gq[u].w);
+          } else if constexpr (LAST) {
+            const float2 x = sv[u];
+            for (int n = fin ? a.reps : 1; n > 0; --n) sv[u] = scan_bin(st[u], x, gq[u], kq[u]);
           } else {
             sv[u] = scan_bin(st[u], sv[u], gq[u], kq[u]);
           }
@@ -471,11 +483,14 @@ gated_scan_small(const ScanArgs a, long long P) {
 #pragma unroll
         for (int u = 0; u < H; ++u) sv[u] = make_float2(0.f, 0.f);
       }
-      dft_sym<H, true>(sv, r);
+      if (fin) {
+        dft_sym<H, true>(sv, r);
 #pragma unroll
-      for (int h = 0; h < H; ++h) rs[cpl * G::PS + h * G::RSP + cv] = r[h];
+        for (int h = 0; h < H; ++h) rs[cpl * G::PS + h * G::RSP + cv] = r[h];
+      }
     }
     __syncthreads();
+    if (!fin) continue;   // uniform: xs and rs are free for the next frame
     // C2R rows into xs
     for (int j = tid; j < G::NRJ; j += NT) {
       small_row_c2r<W>(rs + (j / H) * G::PS + (j % H) * G::RSP, xs + j * W);
@@ -483,7 +498,7 @@ gated_scan_small(const ScanArgs a, long long P) {
     __syncthreads();
     // x z_gate, store y_t
     if (vec) {
-      V4* y4 = reinterpret_cast<V4*>(yp + base0);
+      V4* y4 = reinterpret_cast<V4*>(yp + basez);
 #pragma unroll
       for (int k = 0; k < NEV; ++k) {
         const int e = k * NT + tl;
@@ -500,7 +515,9 @@ gated_scan_small(const ScanArgs a, long long P) {
         const int e = k * NT + tl;
         zg[k] = 0.0f;
         if (e < NP * HW) {
-          if (contig) {
+          if (LAST) {
+            if (gate_b[e / HW] >= 0) zg[k] = IO::to_f(zp[size_t(basez + e)]);
+          } else if (contig) {
             zg[k] = IO::to_f(zp[size_t(base0 + e)]);
           } else {
             const int pl = e / HW, px = e % HW;
@@ -513,7 +530,9 @@ gated_scan_small(const ScanArgs a, long long P) {
         const int e = k * NT + tl;
         if (e >= NP * HW) continue;
         const float g = a.z_act == 1 ? silu_f(zg[k]) : zg[k];
-        if (contig) {
+        if (LAST) {
+          if (gate_b[e / HW] >= 0) yp[size_t(basez + e)] = IO::from_f(xs[e] * g);
+        } else if (contig) {
           yp[size_t(base0 + e)] = IO::from_f(xs[e] * g);
         } else {
           const int pl = e / HW, px = e % HW;
@@ -835,6 +854,28 @@ int gated_scan_min_group(int H, int W) {
   }
 }
 
+bool gated_scan_last_has_kernel(int H, int W) { return H == W && H >= 5 && H <= 15 && H != 8; }
+
+hipError_t launch_gated_scan_last(const float* u, const float* z, float* y, int B, int n, int C, int H, int W,
+                                  const float4* gates, const float2* khat, int reps, hipStream_t s) {
+  ScanArgs a{u, z, y, gates, khat, n, C, 0, 0, reps};
+  const long long P = (long long)B * C;
+#define CSSM_LAST(N)                                                                                               \
+  case N:                                                                                                          \
+    hipLaunchKernelGGL((gated_scan_small<N, N, IoF32, false, true>),                                               \
+                       dim3(unsigned((P + SmallGeom<N, N>::NP - 1) / SmallGeom<N, N>::NP)),                        \
+                       dim3(SmallGeom<N, N>::NT), 0, s, a, P);                                                     \
+    break;
+  if (H != W) return hipErrorInvalidValue;
+  switch (H) {
+    CSSM_LAST(5) CSSM_LAST(6) CSSM_LAST(7) CSSM_LAST(9) CSSM_LAST(10) CSSM_LAST(11) CSSM_LAST(12) CSSM_LAST(13)
+    CSSM_LAST(14) CSSM_LAST(15)
+    default: return hipErrorInvalidValue;
+  }
+#undef CSSM_LAST
+  return hipGetLastError();
+}
+
 hipError_t launch_gated_scan(const void* u, const void* z, void* y, int dtype, int B, int T, int C, int H,
                              int W, const float4* gates, const float2* khat, int u_act, int z_act,
                              hipStream_t s) {
@@ -848,6 +889,7 @@ hipError_t launch_gated_scan(const void* u, const void* z, void* y, int dtype, i
   a.C = C;
   a.u_act = u_act;
   a.z_act = z_act;
+  a.reps = 1;
   if (dtype == 0) return dispatch_scan<IoF32>(a, B, H, W, s);
   return dispatch_scan<IoBF16>(a, B, H, W, s);
 }

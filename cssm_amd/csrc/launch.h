@@ -124,7 +124,8 @@ hipError_t launch_ctx_reduce(const float* partial, int F, int HW, int tile_rows,
 
 hipError_t launch_short_conv(const void* x, int in_dtype, int B, int T, int C, int H, int W, int ks, const float* ws,
                              const float* bs, int kt, const float* wt, const float* bt, void* u, int out_dtype,
-                             float* ctx, int pre, hipStream_t s);   // pre: store the pre-activation
+                             float* ctx, int pre, hipStream_t s,   // pre: store the pre-activation
+                             bool still = false);                   // still: x (B, 1, C, H, W), the same every frame
 bool short_conv_planes_supported(int T, int H, int W, int ks, int kt);
 // adjoint of its convolutions: dx (frame stride dx_fs floats) and sums (chunks, B C, 16)
 int short_conv_bwd_chunks(int B, int T, int C, int H, int W);
@@ -238,7 +239,12 @@ hipError_t launch_gated_scan_bwd_bins(const float2* uspec, const float2* dspec, 
 // forward recurrence of the gated scan on spectra (B, T, C, H, WF), in place: rfft2(u) -> C h; state
 // (B, C, H, WF) carries h between calls on consecutive frames (read unless first; may be null)
 hipError_t launch_gated_scan_fwd_bins(float2* spec, const float4* gates, const float2* khat, float2* state, int first,
-                                      int B, int T, int C, int H, int W, float c_scale, hipStream_t s);
+                                      int B, int T, int C, int H, int W, float c_scale, float2* last, int reps,
+                                      hipStream_t s);
+// the fused scan of n distinct frames whose last one repeats reps times, final y only: z, y (B, C, H, W)
+bool gated_scan_last_has_kernel(int H, int W);
+hipError_t launch_gated_scan_last(const float* u, const float* z, float* y, int B, int n, int C, int H, int W,
+                                  const float4* gates, const float2* khat, int reps, hipStream_t s);
 // the GDN spectral core in one kernel (32 x 32 planes, d_k = 4): rfft2 -> norms -> delta rule -> irfft2
 bool gdn_core_fused_supported(int H, int W, int dk);
 hipError_t launch_gdn_core_fused(const float* qkv, int use_l2, const float2* ab, long long ab_frame, int ab_head,

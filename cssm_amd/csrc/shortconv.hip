@@ -100,7 +100,7 @@ template <int KS, int PX, int NT, int NB, int LDSF, class TI, class TO>
 __global__ void __launch_bounds__(NT)
 short_conv_planes(const TI* __restrict__ x, long long P, int T, int C, int H, int W, const float* __restrict__ ws,
                   const float* __restrict__ bs, int kt, const float* __restrict__ wt, const float* __restrict__ bt,
-                  TO* __restrict__ u, float* __restrict__ ctx, int LP, int tlen, int pre) {
+                  TO* __restrict__ u, float* __restrict__ ctx, int LP, int tlen, int pre, int still) {
   __shared__ float buf[KS ? NB * LDSF : 1];
   __shared__ float red[2][NT / 64];
   const int tid = threadIdx.x, NPL = NT / LP, pl = tid / LP, li = tid % LP;
@@ -110,6 +110,7 @@ short_conv_planes(const TI* __restrict__ x, long long P, int T, int C, int H, in
   const long long b = live ? plane / C : 0;
   const int c = live ? int(plane % C) : 0;
   const size_t base = (size_t(b) * T * C + c) * HW, tstep = size_t(C) * HW;
+  const size_t xbase = still ? (size_t(b) * C + c) * HW : base, xstep = still ? 0 : tstep;   // one frame for all
   float k9[9], kt4[4], bsc = 0.0f, btc = 0.0f;
   if (KS) {
 #pragma unroll
@@ -136,7 +137,7 @@ short_conv_planes(const TI* __restrict__ x, long long P, int T, int C, int H, in
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
       const int p = li + k * LP;
-      nx[k] = live && p < HW ? sc_ld(x, base + size_t(t) * tstep + p) : 0.0f;
+      nx[k] = live && p < HW ? sc_ld(x, xbase + size_t(t) * xstep + p) : 0.0f;
     }
   };
 #pragma unroll
@@ -248,27 +249,27 @@ static ScShape sc_shape(int B, int T, int C, int H, int W) {
 template <int PX, int NT, int NB, int LDSF, class TI, class TO>
 static void run_short_conv_planes(const TI* x, int B, int T, int C, int H, int W, int ks, const float* ws,
                                   const float* bs, int kt, const float* wt, const float* bt, TO* u, float* ctx,
-                                  const ScShape& r, int pre, hipStream_t s) {
+                                  const ScShape& r, int pre, int still, hipStream_t s) {
   const long long P = (long long)B * C;
   const dim3 grid(unsigned((P + NT / r.LP - 1) / (NT / r.LP)), unsigned((T + r.tlen - 1) / r.tlen));
   if (ks == 3)
     hipLaunchKernelGGL((short_conv_planes<3, PX, NT, NB, LDSF, TI, TO>), grid, dim3(NT), 0, s, x, P, T, C, H, W, ws,
-                       bs, kt, wt, bt, u, ctx, r.LP, r.tlen, pre);
+                       bs, kt, wt, bt, u, ctx, r.LP, r.tlen, pre, still);
   else
     hipLaunchKernelGGL((short_conv_planes<0, PX, NT, NB, LDSF, TI, TO>), grid, dim3(NT), 0, s, x, P, T, C, H, W, ws,
-                       bs, kt, wt, bt, u, ctx, r.LP, r.tlen, pre);
+                       bs, kt, wt, bt, u, ctx, r.LP, r.tlen, pre, still);
 }
 
 template <class TI, class TO>
 static void run_short_conv(const TI* x, int B, int T, int C, int H, int W, int ks, const float* ws, const float* bs,
-                           int kt, const float* wt, const float* bt, TO* u, float* ctx, int pre, hipStream_t s) {
+                           int kt, const float* wt, const float* bt, TO* u, float* ctx, int pre, int still, hipStream_t s) {
   const ScShape r = sc_shape(B, T, C, H, W);
   if (r.cls == 0)
-    run_short_conv_planes<4, 256, 2, kScSmall>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, r, pre, s);
+    run_short_conv_planes<4, 256, 2, kScSmall>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, r, pre, still, s);
   else if (r.cls == 1)
-    run_short_conv_planes<4, 1024, 2, kScMid>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, r, pre, s);
+    run_short_conv_planes<4, 1024, 2, kScMid>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, r, pre, still, s);
   else
-    run_short_conv_planes<16, 1024, 1, kScLarge>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, r, pre, s);
+    run_short_conv_planes<16, 1024, 1, kScLarge>(x, B, T, C, H, W, ks, ws, bs, kt, wt, bt, u, ctx, r, pre, still, s);
 }
 
 // where short_conv_planes applies (else the general kernel, which has no pre form)
@@ -458,23 +459,23 @@ hipError_t launch_short_conv_bwd(const float* x, const float* dout, int B, int T
 
 hipError_t launch_short_conv(const void* x, int in_dtype, int B, int T, int C, int H, int W, int ks, const float* ws,
                              const float* bs, int kt, const float* wt, const float* bt, void* u, int out_dtype,
-                             float* ctx, int pre, hipStream_t s) {
+                             float* ctx, int pre, hipStream_t s, bool still) {
   if (short_conv_planes_supported(T, H, W, ks, kt)) {
     if (in_dtype == 0 && out_dtype == 0)
       run_short_conv(static_cast<const float*>(x), B, T, C, H, W, ks, ws, bs, kt, wt, bt, static_cast<float*>(u), ctx,
-                     pre, s);
+                     pre, still, s);
     else if (in_dtype == 0)
       run_short_conv(static_cast<const float*>(x), B, T, C, H, W, ks, ws, bs, kt, wt, bt, static_cast<uint16_t*>(u),
-                     ctx, pre, s);
+                     ctx, pre, still, s);
     else if (out_dtype == 0)
       run_short_conv(static_cast<const uint16_t*>(x), B, T, C, H, W, ks, ws, bs, kt, wt, bt, static_cast<float*>(u),
-                     ctx, pre, s);
+                     ctx, pre, still, s);
     else
       run_short_conv(static_cast<const uint16_t*>(x), B, T, C, H, W, ks, ws, bs, kt, wt, bt,
-                     static_cast<uint16_t*>(u), ctx, pre, s);
+                     static_cast<uint16_t*>(u), ctx, pre, still, s);
     return hipGetLastError();
   }
-  if (pre) return hipErrorInvalidValue;
+  if (pre || still) return hipErrorInvalidValue;
   const dim3 grid(unsigned(B * C)), block(256);
   if (in_dtype == 0 && out_dtype == 0)
     hipLaunchKernelGGL((short_conv_kernel<float, float>), grid, block, 0, s, static_cast<const float*>(x), T, C, H, W,

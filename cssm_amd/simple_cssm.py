@@ -288,7 +288,11 @@ class SimpleCSSM:
                     x = norm_act(self._conv(x, p[f"conv{i + 1}"]), f"norm{i + 1}")
                 x = Fn.max_pool2d(x.permute(0, 3, 1, 2), 2, 2, ceil_mode=True).permute(0, 2, 3, 1)
         _, Hn, Wn, D = x.shape
-        x = x.reshape(B, T_in, Hn, Wn, D).expand(B, T, Hn, Wn, D)           # :277-278
+        # one cell on an image's equal frames with the last one read out: the cell takes the image itself
+        still = (T_in == 1 and self.depth == 1 and self.cssm_type == "gated" and self.frame_readout == "last"
+                 and self.n_register_tokens == 0 and injected_features is None and injected_post_cssm is None
+                 and not return_features and not return_spatial and self.cells[0]._still_pays(B, T, Hn, Wn))
+        x = x.reshape(B, T_in, Hn, Wn, D).expand(B, T_in if still else T, Hn, Wn, D)   # :277-278
         if self.pos_embed == "learnable":                                   # :281-285
             x = x + p["pos_embed"]
         nreg = self.n_register_tokens
@@ -298,7 +302,10 @@ class SimpleCSSM:
             x = injected_features
         x = x.contiguous()
         for i, cell in enumerate(self.cells):                               # :319-496
-            y = cell.apply({"params": p[f"cssm_{i}"]}, x, injected_qkv_spatial=injected_qkv_spatial)
+            if still:
+                y = cell._apply_still({"params": p[f"cssm_{i}"]}, x, T)
+            else:
+                y = cell.apply({"params": p[f"cssm_{i}"]}, x, injected_qkv_spatial=injected_qkv_spatial)
             x = S.block_residual(x, y, x.shape[1], "none")                  # x + cssm(x), :482
             if self.depth > 1 and i < self.depth - 1:                       # :486-496
                 x = self._norm_act(x, body_norm, "pre", f"body_norm_{i}", p, bs, training)

@@ -248,6 +248,49 @@ def _gated_scan_split(u, z, gates, khat, out, max_bytes: int = 1 << 30):
     return out
 
 
+def gated_scan_last_supported(H: int, W: int) -> bool:
+    return bool(_lib.load().cssm_gated_scan_last_supported(H, W))
+
+
+def gated_scan_last(u: torch.Tensor, z: torch.Tensor, gates: torch.Tensor, khat: torch.Tensor,
+                    reps: int) -> torch.Tensor:
+    """The last frame of :func:`gated_scan` for a sequence whose n frames u (B, n, C, H, W) are followed by
+    reps - 1 more of the last one, z (B, C, H, W) being the last frame's: (B, C, H, W), float32
+    (cssm_gated_scan_last, or the transforms around cssm_gated_scan_bins_last)."""
+    for t, nm in ((u, "u"), (z, "z"), (gates, "gates")):
+        _dev(t, nm, torch.float32)
+    _dev(khat, "khat", torch.complex64)
+    B, n, C, H, W = u.shape
+    Wf = W // 2 + 1
+    if z.shape != (B, C, H, W) or gates.shape != (B, n, H, Wf, 4) or khat.shape != (C, H, Wf):
+        raise ValueError("u, z, gates and khat shapes do not match")
+    y = torch.empty_like(z)
+    if gated_scan_last_supported(H, W):
+        _lib.call("cssm_gated_scan_last", u.data_ptr(), z.data_ptr(), y.data_ptr(), B, n, C, H, W, gates.data_ptr(),
+                  khat.data_ptr(), reps, _stream())
+        return y
+    spec = rfft2_ex(u.view(B * n, C, H * W), H, W)
+    last = torch.empty((B, C, H, Wf), dtype=torch.complex64, device=u.device)
+    _lib.call("cssm_gated_scan_bins_last", spec.data_ptr(), gates.data_ptr(), khat.data_ptr(), B, n, C, H, W,
+              scan_c_scale(H, W), reps, last.data_ptr(), _stream())
+    irfft2_ex(last, W, y.view(B, C, H * W), m=z.view(B, C, H * W))
+    return y
+
+
+def short_conv_still(x: torch.Tensor, T: int, spatial, temporal):
+    """:func:`short_conv` of T equal frames x (B, C, H, W) -> (u (B, T, C, H, W), ctx (B, T, C)), float32;
+    spatial / temporal = parameter dicts or None (cssm_short_conv_still)."""
+    _dev(x, "x", torch.float32)
+    B, C, H, W = x.shape
+    ks, ws, bs, kt, wt, bt = _short_conv_ptrs(*((p["kernel"], p["bias"]) if p is not None else None
+                                                for p in (spatial, temporal)))
+    u = torch.empty((B, T, C, H, W), dtype=torch.float32, device=x.device)
+    ctx = torch.empty((B, T, C), dtype=torch.float32, device=x.device)
+    _lib.call("cssm_short_conv_still", x.data_ptr(), B, T, C, H, W, ks, ws, bs, kt, wt, bt, u.data_ptr(),
+              ctx.data_ptr(), _stream())
+    return u, ctx
+
+
 def gated_scan_backward(u: torch.Tensor, z: torch.Tensor, gates: torch.Tensor, khat: torch.Tensor,
                         dy: torch.Tensor, c_scale: float):
     """Vector-Jacobian product of :func:`gated_scan` (identity load activations) for the

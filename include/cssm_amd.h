@@ -213,6 +213,23 @@ int cssm_gated_scan_bins(float* spec, const float* gates, const float* khat, flo
                          int C, int H, int W, float c_scale, void* stream);
 
 /*
+ * The scan of a still image repeated over time, final step only (the CSSM-SHViT
+ * block and SimpleCSSM keep the cell's last frame, cssm_shvit.py:99-101, 211;
+ * simple_cssm.py:239-240, 524-527).  Only the first n steps differ (behind a causal
+ * convolution of n taps); step n repeats reps times, so T = n - 1 + reps.
+ *   cssm_gated_scan_last       u (B, n, C, H, W), gates (B, n, H, W/2+1, 4) of the distinct
+ *                              steps; z, y (B, C, H, W): y of step T as cssm_gated_scan_fwd gives it.
+ *                              H = W in 5..15 but 8 (cssm_gated_scan_last_supported)
+ *   cssm_gated_scan_bins_last  the same on spectra: spec (B, n, C, H, W/2+1) = rfft2(u), last
+ *                              (B, C, H, W/2+1) = C h of step T
+ */
+int cssm_gated_scan_last_supported(int H, int W);
+int cssm_gated_scan_last(const float* u, const float* z, float* y, int B, int n, int C, int H, int W,
+                         const float* gates, const float* khat, int reps, void* stream);
+int cssm_gated_scan_bins_last(const float* spec, const float* gates, const float* khat, int B, int n, int C, int H,
+                              int W, float c_scale, int reps, float* last, void* stream);
+
+/*
  * Backward of cssm_gated_scan_fwd (with u_act = z_act = identity): the
  * spectral-domain reverse recurrence.  Replaces the gradient jax.value_and_grad
  * takes through cssm.py:531-581 (main.py:283; the log-space scan's custom VJPs,
@@ -339,6 +356,13 @@ int cssm_proj_out(const void* y, int in_dtype, int F, int HW, int K, int N, cons
 int cssm_short_conv(const void* x, int in_dtype, int B, int T, int C, int H, int W, int ks,
                     const float* ws, const float* bs, int kt, const float* wt, const float* bt,
                     void* u, int out_dtype, float* ctx, void* stream);
+
+/*
+ * cssm_short_conv in float32 of T equal frames: x (B, C, H, W) stands for each; the
+ * sizes of cssm_short_conv_train_supported.
+ */
+int cssm_short_conv_still(const float* x, int B, int T, int C, int H, int W, int ks, const float* ws, const float* bs,
+                          int kt, const float* wt, const float* bt, float* u, float* ctx, void* stream);
 
 /*
  * Training form of cssm_short_conv in float32: o = the pre-activation the SiLU
