@@ -1081,6 +1081,27 @@ int cssm_layer_norm(const void* x, int dtype, long long M, int C, float eps, con
                     "cssm_layer_norm");
 }
 
+int cssm_stem_conv_supported(long long N, int H, int W, int Ci, int Co) {
+  return cssm::stem_conv_supported(N, H, W, Ci, Co) ? 1 : 0;
+}
+
+int cssm_stem_conv(const float* x, int N, int H, int W, int Ci, int Co, const float* kernel, const float* bias,
+                   const float* scale, const float* beta, float eps, int act, float* out, void* stream) {
+  if (!x || !kernel || !bias || !out || (scale != nullptr) != (beta != nullptr))
+    return fail(CSSM_ERR_NULL, "cssm_stem_conv: null argument (scale and beta go together)");
+  if (N <= 0 || H <= 0 || W <= 0 || Ci <= 0 || Co <= 0)
+    return fail(CSSM_ERR_SHAPE, "cssm_stem_conv: N=%d H=%d W=%d Ci=%d Co=%d", N, H, W, Ci, Co);
+  if (act < 0 || act > 3 || !(eps >= 0.0f)) return fail(CSSM_ERR_ARG, "cssm_stem_conv: act=%d, eps >= 0", act);
+  if (!cssm::stem_conv_supported(N, H, W, Ci, Co))
+    return fail(CSSM_ERR_UNSUPPORTED, "cssm_stem_conv: Co=%d (32 or 64)", Co);
+  if (!aligned(x, 4) || !aligned(kernel, 4) || !aligned(bias, 16) || !aligned(scale, 16) || !aligned(beta, 16) ||
+      !aligned(out, 16))
+    return fail(CSSM_ERR_ALIGN, "cssm_stem_conv: bias, scale, beta and out need 16-byte alignment");
+  return hip_status(cssm::launch_stem_conv(x, N, H, W, Ci, Co, kernel, bias, scale, beta, eps, act, out,
+                                           static_cast<hipStream_t>(stream)),
+                    "cssm_stem_conv");
+}
+
 int cssm_block_residual(const void* res, int T_res, const void* y, int T_y, int dtype, int B, int T_out, int H,
                         int W, int C, int act, void* out, void* stream) {
   if (!res || !y || !out) return fail(CSSM_ERR_NULL, "cssm_block_residual: res, y and out must be non-null");

@@ -281,6 +281,11 @@ hipError_t launch_block_norm_stats(const void* x, int dtype, int B, int T, int H
 hipError_t launch_block_norm_posconv(const void* x, int dtype, int B, int T_in, int T_out, int H, int W, int C,
                                      int mode, const float* stats, const float* scale, const float* bias,
                                      const float* pk, const float* pb, void* out, hipStream_t s);
+// 3 x 3 convolution, activation, LayerNorm (scale != nullptr) and 2 x 2 maximum: (N, H, W, Ci) -> (N, ceil(H/2),
+// ceil(W/2), Co), Co 32 or 64
+bool stem_conv_supported(long long N, int H, int W, int Ci, int Co);
+hipError_t launch_stem_conv(const float* x, int N, int H, int W, int Ci, int Co, const float* wt, const float* bias,
+                            const float* scale, const float* beta, float eps, int act, float* out, hipStream_t s);
 // LayerNorm over the rows of (M, C) with an activation before and / or after (0 none, 1 gelu, 2 relu,
 // 3 softplus); hipErrorInvalidValue where layer_norm_supported is false
 bool layer_norm_supported(int dtype, int C, const void* x, const float* scale, const float* bias, const void* out);

@@ -282,10 +282,17 @@ class SimpleCSSM:
                 x = norm_act(self._conv(x, p["conv1"]), "norm1")
         else:                                                               # :266-274
             for i in range(self.stem_layers):
+                conv, norm = p[f"conv{i + 1}"], p[f"norm{i + 1}"]
                 if self.stem_norm_order == "pre":
-                    x = self._conv(norm_act(x, f"norm{i + 1}"), p[f"conv{i + 1}"])
+                    x, norm, act = norm_act(x, f"norm{i + 1}"), None, "none"
                 else:
-                    x = norm_act(self._conv(x, p[f"conv{i + 1}"]), f"norm{i + 1}")
+                    act = self.act_type if self.act_type in ("gelu", "relu") else "softplus"
+                if (norm is None or stem_norm not in ("batch", "instance")) and S.stem_conv_supported(x, conv, norm):
+                    x = S.stem_conv(x, conv, norm, act)
+                    continue
+                x = self._conv(x, conv)
+                if norm is not None:
+                    x = norm_act(x, f"norm{i + 1}")
                 x = Fn.max_pool2d(x.permute(0, 3, 1, 2), 2, 2, ceil_mode=True).permute(0, 2, 3, 1)
         _, Hn, Wn, D = x.shape
         # one cell on an image's equal frames with the last one read out: the cell takes the image itself

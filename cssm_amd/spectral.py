@@ -1250,6 +1250,37 @@ def layer_norm(x: torch.Tensor, scale: torch.Tensor, bias: torch.Tensor, eps: fl
     return out
 
 
+def stem_conv_supported(x: torch.Tensor, conv: Dict[str, torch.Tensor], norm: Optional[Dict[str, torch.Tensor]]) -> bool:
+    """Layers :func:`stem_conv` takes: float32 tensors of one GPU, a 3 x 3 kernel to 32 or 64 channels."""
+    ts = [x, conv["kernel"], conv["bias"], *((norm["scale"], norm["bias"]) if norm is not None else ())]
+    if x.dim() != 4 or not x.is_cuda or any(t.dtype != torch.float32 or t.device != x.device for t in ts):
+        return False
+    N, H, W, Ci = x.shape
+    Co = conv["kernel"].shape[-1]
+    return (conv["kernel"].shape == (3, 3, Ci, Co) and all(t.shape == (Co,) for t in ts[2:])
+            and bool(_lib.load().cssm_stem_conv_supported(N, H, W, Ci, Co)))
+
+
+def stem_conv(x: torch.Tensor, conv: Dict[str, torch.Tensor], norm: Optional[Dict[str, torch.Tensor]] = None,
+              act: str = "none", eps: float = 1e-6) -> torch.Tensor:
+    """max_pool2x2(LayerNorm(act(conv3x3(x)))), the LayerNorm where norm is given (simple_cssm.py:266-274):
+    x (N, H, W, Ci) -> (N, ceil(H/2), ceil(W/2), Co), float32 (cssm_stem_conv)."""
+    x = _dev(x.contiguous(), "x", torch.float32)
+
+    def vec(t):
+        t = t.contiguous()
+        return t if t.data_ptr() % 16 == 0 else t.clone()
+    k, b = conv["kernel"].contiguous(), vec(conv["bias"])
+    sc, bt = (vec(norm["scale"]), vec(norm["bias"])) if norm is not None else (None, None)
+    N, H, W, Ci = x.shape
+    Co = k.shape[-1]
+    out = torch.empty((N, (H + 1) // 2, (W + 1) // 2, Co), dtype=torch.float32, device=x.device)
+    _lib.call("cssm_stem_conv", x.data_ptr(), N, H, W, Ci, Co, k.data_ptr(), b.data_ptr(),
+              sc.data_ptr() if sc is not None else None, bt.data_ptr() if bt is not None else None, float(eps),
+              LN_ACTS[act], out.data_ptr(), _stream())
+    return out
+
+
 def layer_norm_supported(C: int) -> bool:
     """Rows :func:`layer_norm` takes whatever the alignment of its tensors."""
     return C <= 512

@@ -851,6 +851,17 @@ int cssm_layer_norm(const void* x, int dtype, long long M, int C, float eps, con
                     int pre_act, int post_act, void* out, void* stream);
 
 /*
+ * A SimpleCSSM stem layer (simple_cssm.py:266-274), float32: 3 x 3 convolution 'SAME' of
+ * x (N, H, W, Ci) with kernel (3, 3, Ci, Co) and bias, the activation act (as
+ * cssm_layer_norm's), LayerNorm over the channels (scale and beta, or both NULL: none) and
+ * the 2 x 2 maximum, stride 2, the last row / column alone if odd:
+ * out (N, ceil(H/2), ceil(W/2), Co).  Co = 32 or 64; bias, scale, beta and out 16-byte aligned.
+ */
+int cssm_stem_conv_supported(long long N, int H, int W, int Ci, int Co);
+int cssm_stem_conv(const float* x, int N, int H, int W, int Ci, int Co, const float* kernel, const float* bias,
+                   const float* scale, const float* beta, float eps, int act, float* out, void* stream);
+
+/*
  * out = res + act(y) (cssm_shvit.py:211-228): T_out = 1 takes the last frame
  * of res (T_res frames) and of y (T_y frames), T_out > 1 frame by frame
  * (keep_time; T_res = T_y = T_out).  act 0 none, 1 gelu (tanh form, as
