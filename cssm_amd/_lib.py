@@ -152,6 +152,8 @@ SIGNATURES = {
                                                ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                                ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                                ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
+    "cssm_mlp_dwconv_supported": (_I, [_LL, _I, _I, _I]),
+    "cssm_mlp_dwconv": (_I, [_P, _I, _I, _I, _I, _P, _P, _P, _P]),
     "cssm_stem_conv_supported": (_I, [_LL, _I, _I, _I, _I]),
     "cssm_stem_conv": (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, ctypes.c_float, _I, _P, _P]),
     "cssm_layer_norm": (_I, [_P, _I, _LL, _I, ctypes.c_float, _P, _P, _I, _I, _P, _P]),

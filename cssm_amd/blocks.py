@@ -201,12 +201,16 @@ class CSSMSHViTBlock:
             h = S.block_norm_posconv(x5, S.block_norm_stats(x5, "layer"), "layer", n2["scale"], n2["bias"], None, None,
                                      x5.shape[1]).float()
         m = p["mlp"]
-        h = Fn.gelu(torch.addmm(m["fc1"]["bias"], h.reshape(-1, C), m["fc1"]["kernel"]), approximate="tanh")
+        h = torch.addmm(m["fc1"]["bias"], h.reshape(-1, C), m["fc1"]["kernel"])
         hid = h.shape[-1]
         h = h.reshape(-1, H, W, hid)
-        if self.use_dwconv:
-            dw = m["dwconv"]["dwconv"]
-            h = h + S.depthwise_conv(h, dw["kernel"], dw["bias"])
+        dw = m["dwconv"]["dwconv"] if self.use_dwconv else None
+        if dw is not None and S.mlp_dwconv_supported(h, dw["kernel"], dw["bias"]):
+            h = S.mlp_dwconv(h, dw["kernel"], dw["bias"])
+        else:
+            h = Fn.gelu(h, approximate="tanh")
+            if dw is not None:
+                h = h + S.depthwise_conv(h, dw["kernel"], dw["bias"])
         h = torch.addmm(m["fc2"]["bias"], h.reshape(-1, hid), m["fc2"]["kernel"])
         return (x.float() + h.reshape(shp)).to(x.dtype)
 

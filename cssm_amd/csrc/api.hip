@@ -1102,6 +1102,23 @@ int cssm_stem_conv(const float* x, int N, int H, int W, int Ci, int Co, const fl
                     "cssm_stem_conv");
 }
 
+int cssm_mlp_dwconv_supported(long long N, int H, int W, int C) {
+  return cssm::mlp_dwconv_supported(N, H, W, C) ? 1 : 0;
+}
+
+int cssm_mlp_dwconv(const float* x, int N, int H, int W, int C, const float* kernel, const float* bias, float* out,
+                    void* stream) {
+  if (!x || !kernel || !bias || !out) return fail(CSSM_ERR_NULL, "cssm_mlp_dwconv: null argument");
+  if (N <= 0 || H <= 0 || W <= 0 || C <= 0)
+    return fail(CSSM_ERR_SHAPE, "cssm_mlp_dwconv: N=%d H=%d W=%d C=%d", N, H, W, C);
+  if (!cssm::mlp_dwconv_supported(N, H, W, C))
+    return fail(CSSM_ERR_UNSUPPORTED, "cssm_mlp_dwconv: %dx%d planes of %d channels", H, W, C);
+  if (!aligned(x, 16) || !aligned(kernel, 16) || !aligned(bias, 16) || !aligned(out, 16) || x == out)
+    return fail(CSSM_ERR_ALIGN, "cssm_mlp_dwconv: 16-byte aligned tensors, out not x");
+  return hip_status(cssm::launch_mlp_dwconv(x, N, H, W, C, kernel, bias, out, static_cast<hipStream_t>(stream)),
+                    "cssm_mlp_dwconv");
+}
+
 int cssm_block_residual(const void* res, int T_res, const void* y, int T_y, int dtype, int B, int T_out, int H,
                         int W, int C, int act, void* out, void* stream) {
   if (!res || !y || !out) return fail(CSSM_ERR_NULL, "cssm_block_residual: res, y and out must be non-null");

@@ -281,6 +281,10 @@ hipError_t launch_block_norm_stats(const void* x, int dtype, int B, int T, int H
 hipError_t launch_block_norm_posconv(const void* x, int dtype, int B, int T_in, int T_out, int H, int W, int C,
                                      int mode, const float* stats, const float* scale, const float* bias,
                                      const float* pk, const float* pb, void* out, hipStream_t s);
+// g + conv3x3(g) + bias of g = gelu(x), channels-last, C a multiple of 32, W <= 64
+bool mlp_dwconv_supported(long long N, int H, int W, int C);
+hipError_t launch_mlp_dwconv(const float* x, int N, int H, int W, int C, const float* k3, const float* bias, float* out,
+                             hipStream_t s);
 // 3 x 3 convolution, activation, LayerNorm (scale != nullptr) and 2 x 2 maximum: (N, H, W, Ci) -> (N, ceil(H/2),
 // ceil(W/2), Co), Co 32 or 64
 bool stem_conv_supported(long long N, int H, int W, int Ci, int Co);

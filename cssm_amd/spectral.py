@@ -1250,6 +1250,24 @@ def layer_norm(x: torch.Tensor, scale: torch.Tensor, bias: torch.Tensor, eps: fl
     return out
 
 
+def mlp_dwconv_supported(x: torch.Tensor, kernel: torch.Tensor, bias: torch.Tensor) -> bool:
+    N, H, W, C = x.shape
+    return (kernel.shape == (3, 3, 1, C) and bias.shape == (C,) and kernel.is_contiguous() and bias.is_contiguous()
+            and all(t.is_cuda and t.dtype == torch.float32 and t.data_ptr() % 16 == 0 for t in (x, kernel, bias))
+            and bool(_lib.load().cssm_mlp_dwconv_supported(N, H, W, C)))
+
+
+def mlp_dwconv(x: torch.Tensor, kernel: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
+    """g + depthwise_conv(g, kernel, bias), g = gelu(x), channels-last float32 (shvit.py:156-182; cssm_mlp_dwconv)."""
+    for t, nm in ((x, "x"), (kernel, "kernel"), (bias, "bias")):
+        _dev(t, nm, torch.float32)
+    N, H, W, C = x.shape
+    out = torch.empty_like(x)
+    _lib.call("cssm_mlp_dwconv", x.data_ptr(), N, H, W, C, kernel.data_ptr(), bias.data_ptr(), out.data_ptr(),
+              _stream())
+    return out
+
+
 def stem_conv_supported(x: torch.Tensor, conv: Dict[str, torch.Tensor], norm: Optional[Dict[str, torch.Tensor]]) -> bool:
     """Layers :func:`stem_conv` takes: float32 tensors of one GPU, a 3 x 3 kernel to 32 or 64 channels."""
     ts = [x, conv["kernel"], conv["bias"], *((norm["scale"], norm["bias"]) if norm is not None else ())]

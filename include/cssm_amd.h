@@ -851,6 +851,15 @@ int cssm_layer_norm(const void* x, int dtype, long long M, int C, float eps, con
                     int pre_act, int post_act, void* out, void* stream);
 
 /*
+ * Inside the CSSM-SHViT block's MLP (cssm_shvit.py:231-266; shvit.py:156-182), float32:
+ * out = g + depthwise conv3x3 'SAME'(g) + bias, g = gelu(x) (tanh form), x and out (N, H, W, C),
+ * kernel (3, 3, 1, C).  C a multiple of 32, W <= 64, everything 16-byte aligned, out not x.
+ */
+int cssm_mlp_dwconv_supported(long long N, int H, int W, int C);
+int cssm_mlp_dwconv(const float* x, int N, int H, int W, int C, const float* kernel, const float* bias, float* out,
+                    void* stream);
+
+/*
  * A SimpleCSSM stem layer (simple_cssm.py:266-274), float32: 3 x 3 convolution 'SAME' of
  * x (N, H, W, Ci) with kernel (3, 3, Ci, Co) and bias, the activation act (as
  * cssm_layer_norm's), LayerNorm over the channels (scale and beta, or both NULL: none) and
