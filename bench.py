@@ -260,7 +260,8 @@ def gdn_step(cell, variables, x, w, S, mark):
         qkv, gv = S.gdn_qkv_gate_proj(x, p["qkv_proj"]["kernel"], p["qkv_proj"]["bias"], B, T, H, W, convs, 1, bkv,
                                       p["gate_proj"]["kernel"], p["gate_proj"]["bias"], "silu", out_dtype=f32)
         mark("qkv_gate_proj")
-    if S.gdn_core_fused_supported(H, W, cell.delta_key_dim):
+    if (S.gdn_core_fused_supported(H, W, cell.delta_key_dim)
+            and S.gdn_core_fused_pays(B, T, cell.channels, cell.delta_key_dim)):
         o = S.gdn_core_fused(qkv, True, ab, cell.gate_type, what, cell.delta_key_dim, cell.scan_variant)
         mark("core_fused")   # rfft2 -> norms -> delta rule -> irfft2 in one kernel
     else:
@@ -554,7 +555,8 @@ def run_workload(key, args, torch, cells, S, headline):
         randomise_biases(variables, torch, dev)
     step = {"gated": gated_step, "gdn": gdn_step, "stack": stack_step}[w["cell"]]
     core = ("scan",) if w["cell"] in ("gated", "stack") else (
-        ("core_fused",) if S.gdn_core_fused_supported(H, W, w["dk"]) else ("rfft2", "scan_bins", "irfft2"))
+        ("core_fused",) if S.gdn_core_fused_supported(H, W, w["dk"])
+        and S.gdn_core_fused_pays(B, T, w["C"], w["dk"]) else ("rfft2", "scan_bins", "irfft2"))
     steps = args.steps if headline else max(1, args.config_steps)
 
     per_step = 0

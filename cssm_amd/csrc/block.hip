@@ -1,7 +1,7 @@
 // Caller wiring of CSSMSHViTBlock around the cell: the token-mixer half of
 // the block (cssm_shvit.py:86-229): norm1 -> pos_conv -> cell -> frame
-// selection -> output activation -> residual.  The MLP half (:231-266) is not
-// part of this build.
+// selection -> output activation -> residual, and of the MLP half (:231-266)
+// norm2 and the gelu + depthwise convolution between the two products.
 //
 // Tensors are channels-last (B, T, H, W, C); an image input is (B, 1, H, W, C)
 // and is repeated to the cell's T frames on the way out of the pos_conv pass.
