@@ -1063,6 +1063,14 @@ def gdn_norm_gate_supported(C: int) -> bool:
     return C <= 128
 
 
+def _norm_ptrs(scale: Optional[torch.Tensor], shift: Optional[torch.Tensor], C: int):
+    """Addresses of the norm's (C,) float32 scale and shift, None where absent."""
+    for t, n in ((scale, "scale"), (shift, "shift")):
+        if t is not None and _dev(t, n, torch.float32).shape != (C,):
+            raise ValueError(f"{n} {tuple(t.shape)} does not match C={C}")
+    return (scale.data_ptr() if scale is not None else None, shift.data_ptr() if shift is not None else None)
+
+
 def gdn_norm_gate(o: torch.Tensor, g: torch.Tensor, norm: str, scale: Optional[torch.Tensor],
                   shift: Optional[torch.Tensor], act: str) -> torch.Tensor:
     """y = (norm(o) scale + shift) act(g) per pixel over the channels of plane-major o, g (F, C, HW), g a channel
@@ -1071,8 +1079,7 @@ def gdn_norm_gate(o: torch.Tensor, g: torch.Tensor, norm: str, scale: Optional[t
     F, C, HW = o.shape
     y = torch.empty_like(o)
     _lib.call("cssm_gdn_norm_gate", o.data_ptr(), g.data_ptr(), _frames(g, "g", C, HW), F, C, HW, _NORMS[norm],
-              _ACTS[act], scale.data_ptr() if scale is not None else None,
-              shift.data_ptr() if shift is not None else None, y.data_ptr(), _stream())
+              _ACTS[act], *_norm_ptrs(scale, shift, C), y.data_ptr(), _stream())
     return y
 
 
@@ -1083,12 +1090,13 @@ def gdn_norm_gate_backward(o: torch.Tensor, g: torch.Tensor, norm: str, scale: O
     _dev(o, "o", torch.float32)
     _dev(dy, "dy", torch.float32)
     F, C, HW = o.shape
+    if dy.shape != o.shape:
+        raise ValueError(f"dy {tuple(dy.shape)} does not match o {tuple(o.shape)}")
     do = torch.empty_like(o)
     n = int(_lib.load().cssm_gdn_norm_gate_blocks(F, HW))
     sums = torch.empty((n, 3, C), dtype=torch.float32, device=o.device)
     _lib.call("cssm_gdn_norm_gate_bwd", o.data_ptr(), g.data_ptr(), _frames(g, "g", C, HW), F, C, HW, _NORMS[norm],
-              _ACTS[act], scale.data_ptr() if scale is not None else None,
-              shift.data_ptr() if shift is not None else None, dy.data_ptr(), do.data_ptr(), dg.data_ptr(),
+              _ACTS[act], *_norm_ptrs(scale, shift, C), dy.data_ptr(), do.data_ptr(), dg.data_ptr(),
               _frames(dg, "dg", C, HW), sums.data_ptr(), _stream())
     return do, sums.sum(dim=0)
 

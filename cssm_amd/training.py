@@ -644,6 +644,29 @@ class _GdnFn(torch.autograd.Function):
                 ng_sums[0] if scale is not None else None, ng_sums[1] if shift is not None else None, None, *d_convs)
 
 
+def _as_read(t: torch.Tensor, dev, *shape) -> bool:
+    """Whether t, made contiguous, is what a kernel given its address reads: float32 of this shape on dev."""
+    return t.dtype == torch.float32 and t.device == dev and t.shape == shape
+
+
+def _norm_params(cell, p):
+    """(scale, shift) of the output norm, None where it has none."""
+    if cell.output_norm == "rms":
+        return p["rms_scale"], None
+    if cell.output_norm == "layer":
+        return p["output_layernorm"]["scale"], p["output_layernorm"]["bias"]
+    return None, None
+
+
+def _gdn_node_takes(cell, p, C: int, dev) -> bool:
+    """Whether _GdnFn covers the cell with these parameters: at most 128 channels and short-convolution taps its
+    kernels hold, no full-channel qkv convolution, and tensors as their addresses are read.  The torch path
+    takes the rest (a scale that broadcasts or is held in 16 bits)."""
+    if (cell.qkv_conv_size > 1 and not cell.qkv_conv_separable) or not S.gdn_norm_gate_supported(C):
+        return False
+    return cell.short_conv_size <= 8 and all(t is None or _as_read(t, dev, C) for t in _norm_params(cell, p))
+
+
 def _gdn_fused_apply(cell, p, x, ctx, what, dims):
     """gdn_train_apply through _GdnFn: the gates and W_hat on torch (small), the rest on the one node."""
     B, T, H, W, C, dk, nh = dims
@@ -674,11 +697,7 @@ def _gdn_fused_apply(cell, p, x, ctx, what, dims):
     if cell.short_conv_size > 0:
         for n in "qkv":
             convs += [p[f"short_conv_{n}"]["kernel"].contiguous(), p[f"short_conv_{n}"]["bias"].contiguous()]
-    scale = shift = None
-    if cell.output_norm == "rms":
-        scale = p["rms_scale"]
-    elif cell.output_norm == "layer":
-        scale, shift = p["output_layernorm"]["scale"], p["output_layernorm"]["bias"]
+    scale, shift = (t if t is None else t.contiguous() for t in _norm_params(cell, p))
     meta = (B, T, H, W, C, dk, gate_mode, cell.gate_type, cell.use_spectral_l2_norm, cell.scan_variant,
             cell.output_norm, "silu" if cell.output_gate_act == "silu" else "sigmoid")
     y = _GdnFn.apply(x2, xq2, p["qkv_proj"]["kernel"], p["qkv_proj"]["bias"], p["gate_proj"]["kernel"],
@@ -706,7 +725,7 @@ def gdn_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tens
     if not cell.position_independent_gates:
         ctx = ctx + _temporal_encoding(T, C, cell.rope_base, x.device)[None]
     ks = cell.qkv_conv_size
-    if not (ks > 1 and not cell.qkv_conv_separable) and S.gdn_norm_gate_supported(C) and cell.short_conv_size <= 8:
+    if _gdn_node_takes(cell, p, C, x.device):
         return _gdn_fused_apply(cell, p, x, ctx, what, (B, T, H, W, C, dk, nh))
     xq = x.reshape(F, H, W, C)
     if ks > 1 and not cell.qkv_conv_separable:

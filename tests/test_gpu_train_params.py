@@ -1,0 +1,100 @@
+"""Parameter tensors of the training entry points in other layouts than a fresh tree's: strided, broadcast and
+16-bit ones give the gradients of their contiguous float32 copies, and what no kernel may read is refused."""
+import pytest
+
+from tests.gpu_util import print_case
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mods():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from cssm_amd import cells, spectral, training
+    return cells, spectral, training
+
+
+def strided(t):
+    """t as one slice of tensors stacked on the last axis."""
+    return torch.stack([t, torch.full_like(t, 3.0)], dim=-1)[..., 0]
+
+
+def leaves(tree):
+    return [t for v in tree.values() for t in (leaves(v) if isinstance(v, dict) else [v])]
+
+
+def grads(apply, cell, variables, x, dout):
+    """Output and gradients of x and of every parameter."""
+    ls = [x.detach().requires_grad_(True)] + [t.detach().requires_grad_(True) for t in leaves(variables["params"])]
+    it = iter(ls[1:])
+
+    def put(tree):
+        return {k: put(v) if isinstance(v, dict) else next(it) for k, v in tree.items()}
+    y = apply(cell, {"params": put(variables["params"])}, ls[0])
+    return [y.detach(), *torch.autograd.grad(y, ls, dout)]
+
+
+def layer(cls, seed, shape, **kw):
+    cell = cls(channels=shape[-1], kernel_size=5, **kw)
+    v = cell.init(seed, shape)
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    for t in leaves(v["params"]):
+        t.add_(0.1 * torch.randn(t.shape, generator=gen, device="cuda"))
+    x, dout = (torch.randn(shape, generator=gen, device="cuda") for _ in range(2))
+    return cell, v, x, dout
+
+
+def close(got, ref):
+    """The same float32 arithmetic through other kernels: sums of some 1e4 O(1) terms, whose rounding stays near
+    1e-6 of the largest value."""
+    for g, r in zip(got, ref):
+        assert g.shape == r.shape
+        assert (g.double() - r.double()).abs().max() <= 1e-4 * max(1e-30, r.abs().max().item())
+
+
+@pytest.mark.parametrize("norm", ["rms", "layer"])
+@pytest.mark.parametrize("form", ["strided", "scalar", "bf16", "one"])
+def test_gdn_norm_scale_layouts(mods, norm, form):
+    """A strided slice, an expanded scalar, 16 bits and a (1,) that broadcasts."""
+    cells, _, training = mods
+    print_case(test="gdn_norm_scale", norm=norm, form=form)
+    cell, v, x, dout = layer(cells.GatedDeltaNetCSSM, 7, (2, 3, 7, 7, 12), delta_key_dim=4, gate_type="factored",
+                             output_norm=norm)
+    p = v["params"]
+    names = [(p, "rms_scale")] if norm == "rms" else [(p["output_layernorm"], n) for n in ("scale", "bias")]
+    for d, n in names:                                     # values that every form holds
+        d[n] = (d[n][:1].expand(12) if form in ("scalar", "one") else d[n]).bfloat16().float()
+    ref = grads(training.gdn_train_apply, cell, v, x, dout)
+    for d, n in names:
+        t = d[n]
+        d[n] = {"strided": strided(t), "scalar": t[:1].expand(12), "bf16": t.bfloat16(), "one": t[:1]}[form]
+        assert form in ("bf16", "one") or not d[n].is_contiguous()
+    got = grads(training.gdn_train_apply, cell, v, x, dout)
+    i = {id(t): k for k, t in enumerate(leaves(p))}
+    for d, n in names:
+        k = 2 + i[id(d[n])]
+        if form == "one":       # the sum over the channels: cancels, so its error is that of its terms, 1e-4 of each
+            assert got[k].shape == (1,)
+            assert (got[k].double() - ref[k].double().sum()).abs() <= 1e-4 * ref[k].double().abs().sum()
+            got[k] = ref[k]
+        if form == "bf16":      # rounded to 16 bits
+            assert got[k].dtype == torch.bfloat16
+            assert (got[k].double() - ref[k].double()).abs().max() <= 2 ** -8 * ref[k].abs().max()
+            got[k] = ref[k]
+    close(got, ref)
+
+
+def test_norm_gate_refuses_what_it_would_misread(mods):
+    _, S, _ = mods
+    print_case(test="norm_gate_refuses")
+    o, g = (torch.randn((2, 8, 16), device="cuda") for _ in range(2))
+    ok = torch.ones(8, device="cuda")
+    bad = [strided(ok), ok[:1].expand(8), ok.double(), ok.bfloat16(), ok.cpu(), ok[:7], torch.ones(9, device="cuda")]
+    for t in bad:
+        for scale, shift in ((t, None), (ok, t)):
+            with pytest.raises(ValueError):
+                S.gdn_norm_gate(o, g, "layer", scale, shift, "silu")
+            with pytest.raises(ValueError):
+                S.gdn_norm_gate_backward(o, g, "layer", scale, shift, "silu", torch.empty_like(o), torch.empty_like(g))
