@@ -244,6 +244,11 @@ def _causal_t(x5, p):
     return sum(terms)
 
 
+def _as_read(t: torch.Tensor, dev, *shape) -> bool:
+    """Whether t, made contiguous, is what a kernel given its address reads: float32 of this shape on dev."""
+    return t.dtype == torch.float32 and t.device == dev and t.shape == shape
+
+
 def _gate_leaves(p: Dict[str, Any], gate_type: str):
     """The gate projections' parameter tensors in a fixed order, and a function rebuilding the
     dict gate_planes reads from such a list."""
@@ -381,6 +386,19 @@ class _WhatFn(torch.autograd.Function):
                 None, None)
 
 
+def _gated_node_takes(cell, p, gate_params, T: int, H: int, W: int, Ci: int, dev) -> bool:
+    """Whether _GatedInScanFn covers the cell on these planes with these parameters: transforms with fused work,
+    short convolutions its kernels hold, and tensors as their addresses are read.  The torch path takes the rest
+    (a gate bias that broadcasts or is held in 16 bits)."""
+    ks, kt = cell.short_conv_spatial_size, cell.short_conv_size
+    if not S.fft_ex_supported(H, W) or ((ks > 0 or kt > 0) and not S.short_conv_train_supported(T, H, W, ks, kt)):
+        return False
+    sizes = (H, W // 2 + 1) if cell.gate_type == "factored" else (H * (W // 2 + 1),)
+    K = p["kernel"].shape[-1]
+    return _as_read(p["kernel"], dev, Ci, K, K) and all(
+        _as_read(t, dev, *((Ci,) if i % 2 == 0 else ()), sizes[i // 2 % len(sizes)]) for i, t in enumerate(gate_params))
+
+
 def gated_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tensor:
     """GatedCSSM forward with autograd (x (B, T, H, W, C) float32 on the GPU; params: the cell's
     tree of float32 device tensors).  Same results as ``cell.apply`` up to float32 rounding."""
@@ -391,16 +409,16 @@ def gated_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Te
     if not S.gated_scan_supported(H, W):
         raise NotImplementedError(f"no fused scan kernel for {H}x{W} planes")
     no_convs = cell.short_conv_spatial_size == 0 and cell.short_conv_size == 0
-    if S.fft_ex_supported(H, W) and (no_convs or S.short_conv_train_supported(T, H, W, cell.short_conv_spatial_size,
-                                                                               cell.short_conv_size)):
+    gps, rebuild = _gate_leaves(p, cell.gate_type)
+    if _gated_node_takes(cell, p, gps, T, H, W, Ci, x.device):
         # in_proj through the scan as one node whose backward runs on the fused HIP transforms
-        gps, rebuild = _gate_leaves(p, cell.gate_type)
         meta = (B, T, H, W, Ci, cell.gate_type, cell.gate_activation, cell.spectral_rho, rebuild)
         convs = []
         for n, size in (("short_conv_spatial", cell.short_conv_spatial_size), ("short_conv_temporal", cell.short_conv_size)):
             convs += [p[n]["kernel"].contiguous(), p[n]["bias"].contiguous()] if size > 0 else [None, None]
         y = _GatedInScanFn.apply(x.reshape(-1, cin).float().contiguous(), p["in_proj"]["kernel"],
-                                 p["in_proj"]["bias"], p["kernel"], meta, *convs, *gps)
+                                 p["in_proj"]["bias"], p["kernel"].contiguous(), meta, *convs,
+                                 *(t.contiguous() for t in gps))
         out = _ProjOutFn.apply(y.view(B * T, Ci, H * W), p["out_proj"]["kernel"], p["out_proj"]["bias"])
         return out.view(B, T, H, W, cell.channels)
     xz = _ProjPlanesFn.apply(x.reshape(-1, cin).float().contiguous(), p["in_proj"]["kernel"], p["in_proj"]["bias"],
@@ -642,11 +660,6 @@ class _GdnFn(torch.autograd.Function):
             dxq, dw_qkv = d_proj(draw, w_qkv, xq2)
         return (dx, dxq, dw_qkv, sums[:, kt + 1], dw_g, ng_sums[2], dwhat.sum(dim=0), dab, dgkv,
                 ng_sums[0] if scale is not None else None, ng_sums[1] if shift is not None else None, None, *d_convs)
-
-
-def _as_read(t: torch.Tensor, dev, *shape) -> bool:
-    """Whether t, made contiguous, is what a kernel given its address reads: float32 of this shape on dev."""
-    return t.dtype == torch.float32 and t.device == dev and t.shape == shape
 
 
 def _norm_params(cell, p):

@@ -86,6 +86,46 @@ def test_gdn_norm_scale_layouts(mods, norm, form):
     close(got, ref)
 
 
+GATED = [((2, 3, 7, 7, 6), "factored", 3), ((1, 2, 16, 16, 8), "dense", 3), ((2, 2, 9, 9, 4), "dense", 0),
+         ((1, 3, 32, 32, 2), "factored", 3)]
+
+
+@pytest.mark.parametrize("shape,gate_type,ks", GATED)
+@pytest.mark.parametrize("form", ["strided", "bf16_bias", "one_bias"])
+def test_gated_parameter_layouts(mods, shape, gate_type, ks, form):
+    """Strided spectral, gate and convolution weights; gate biases in 16 bits or one for all bins."""
+    cells, _, training = mods
+    print_case(test="gated_params", shape=shape, gates=gate_type, form=form)
+    cell, v, x, dout = layer(cells.GatedCSSM, 9, shape, gate_type=gate_type, short_conv_spatial_size=ks,
+                             short_conv_size=4 if ks else 0)
+    p = v["params"]
+    gates = [q for n, q in p.items() if n.startswith(("delta_proj", "B_proj", "C_proj"))]
+    for q in gates:
+        q["bias"] = (q["bias"][:1].expand_as(q["bias"]).contiguous() if form == "one_bias" else q["bias"] + 0.5)
+        q["bias"] = q["bias"].bfloat16().float()
+    ref = grads(training.gated_train_apply, cell, v, x, dout)
+    if form == "strided":
+        p["kernel"] = strided(p["kernel"])
+        for n, q in p.items():
+            if n not in ("kernel", "in_proj", "out_proj"):
+                p[n] = {k: strided(t) for k, t in q.items()}
+                assert not any(t.is_contiguous() for t in p[n].values() if t.numel() > 1)
+    i = {id(t): k for k, t in enumerate(leaves(p))}
+    kept = [2 + i[id(q["bias"])] for q in gates] if form != "strided" else []
+    if form != "strided":
+        for q in gates:
+            q["bias"] = q["bias"].bfloat16() if form == "bf16_bias" else q["bias"][:1].contiguous()
+    got = grads(training.gated_train_apply, cell, v, x, dout)
+    for k in kept:                                        # as test_gdn_norm_scale_layouts
+        r = ref[k].double()
+        if form == "one_bias":
+            assert (got[k].double() - r.sum()).abs() <= 1e-4 * r.abs().sum()
+        else:
+            assert got[k].dtype == torch.bfloat16 and (got[k].double() - r).abs().max() <= 2 ** -8 * r.abs().max()
+        got[k] = ref[k]
+    close(got, ref)
+
+
 def test_norm_gate_refuses_what_it_would_misread(mods):
     _, S, _ = mods
     print_case(test="norm_gate_refuses")
