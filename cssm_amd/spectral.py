@@ -283,7 +283,7 @@ def short_conv_still(x: torch.Tensor, T: int, spatial, temporal):
     _dev(x, "x", torch.float32)
     B, C, H, W = x.shape
     ks, ws, bs, kt, wt, bt = _short_conv_ptrs(*((p["kernel"], p["bias"]) if p is not None else None
-                                                for p in (spatial, temporal)))
+                                                for p in (spatial, temporal)), C)
     u = torch.empty((B, T, C, H, W), dtype=torch.float32, device=x.device)
     ctx = torch.empty((B, T, C), dtype=torch.float32, device=x.device)
     _lib.call("cssm_short_conv_still", x.data_ptr(), B, T, C, H, W, ks, ws, bs, kt, wt, bt, u.data_ptr(),
@@ -465,11 +465,21 @@ def short_conv_train_supported(T: int, H: int, W: int, ks: int, kt: int) -> bool
     return bool(_lib.load().cssm_short_conv_train_supported(T, H, W, ks, kt))
 
 
-def _short_conv_ptrs(spatial, temporal):
+def _sized(t: torch.Tensor, name: str, *shape: int) -> torch.Tensor:
+    """t, a contiguous float32 GPU tensor of this shape: what a kernel given its address reads."""
+    if _dev(t, name, torch.float32).shape != shape:
+        raise ValueError(f"{name} {tuple(t.shape)} is not {shape}")
+    return t
+
+
+def _short_conv_ptrs(spatial, temporal, C: int):
     (ws, bs), (wt, bt) = spatial or (None, None), temporal or (None, None)
-    for t, n in ((ws, "spatial kernel"), (bs, "spatial bias"), (wt, "temporal kernel"), (bt, "temporal bias")):
-        if t is not None:
-            _dev(t, f"short_conv {n}", torch.float32)
+    if ws is not None:
+        _sized(ws, "short_conv spatial kernel", ws.shape[0], ws.shape[0], 1, C)
+        _sized(bs, "short_conv spatial bias", C)
+    if wt is not None:
+        _sized(wt, "short_conv temporal kernel", wt.shape[0], 1, C)
+        _sized(bt, "short_conv temporal bias", C)
     return (ws.shape[0] if ws is not None else 0, ws.data_ptr() if ws is not None else None,
             bs.data_ptr() if bs is not None else None, wt.shape[0] if wt is not None else 0,
             wt.data_ptr() if wt is not None else None, bt.data_ptr() if bt is not None else None)
@@ -480,7 +490,7 @@ def short_conv_train(x: torch.Tensor, spatial, temporal):
     spatial / temporal = (kernel, bias) or None."""
     _dev(x, "x", torch.float32)
     B, T, C, H, W = x.shape
-    ks, ws, bs, kt, wt, bt = _short_conv_ptrs(spatial, temporal)
+    ks, ws, bs, kt, wt, bt = _short_conv_ptrs(spatial, temporal, C)
     o = torch.empty_like(x)
     ctx = torch.empty((B, T, C), dtype=torch.float32, device=x.device)
     _lib.call("cssm_short_conv_train", x.data_ptr(), B, T, C, H, W, ks, ws, bs, kt, wt, bt, o.data_ptr(),
@@ -492,13 +502,13 @@ def short_conv_backward(x: torch.Tensor, do: torch.Tensor, spatial, temporal, dx
     """Adjoint of :func:`short_conv_train`'s convolutions for the gradient do of o: writes dx (F, C, HW) (a channel
     slice of a plane-major tensor allowed) and returns the sums (C, 16) of cssm_short_conv_bwd."""
     _dev(x, "x", torch.float32)
-    _dev(do, "do", torch.float32)
     B, T, C, H, W = x.shape
-    ks, ws, bs, kt, wt, bt = _short_conv_ptrs(spatial, temporal)
+    _sized(do, "do", B, T, C, H, W)
+    ks, ws, bs, kt, wt, bt = _short_conv_ptrs(spatial, temporal, C)
     n = int(_lib.load().cssm_short_conv_bwd_chunks(B, T, C, H, W))
     sums = torch.empty((n * B, C, 16), dtype=torch.float32, device=x.device)
     _lib.call("cssm_short_conv_bwd", x.data_ptr(), do.data_ptr(), B, T, C, H, W, ks, ws, bs, kt, wt, dx.data_ptr(),
-              _frames(dx, "dx", C, H * W), sums.data_ptr(), _stream())
+              _frames(dx, "dx", B * T, C, H * W), sums.data_ptr(), _stream())
     return sums.sum(dim=0)
 
 
@@ -917,6 +927,19 @@ def _ab_strides(ab: torch.Tensor, gate_type: str):
     return {"dense": (n_ab, 0, 1), "factored": (n_ab, 0, 1), "channel": (n_ab, 1, 0), "scalar": (1, 0, 0)}[gate_type]
 
 
+def _core_sizes(spec, norms, ab, gate_type: str, what, dk: int):
+    """Shapes of the delta rule's training inputs against spec (B, T, 3C, H, Wf)."""
+    B, T, C3, H, Wf = spec.shape
+    nh = C3 // 3 // dk
+    n_ab = {"dense": H * Wf, "factored": H * Wf, "channel": nh, "scalar": 1}[gate_type]
+    if C3 != 3 * nh * dk or what.shape != (nh, H, Wf):
+        raise ValueError(f"what {tuple(what.shape)} does not match {C3} planes of {H} x {Wf} bins, d_k={dk}")
+    if ab.shape != (B, T, n_ab, 2):
+        raise ValueError(f"ab {tuple(ab.shape)} is not {(B, T, n_ab, 2)}")
+    if norms is not None:
+        _sized(norms, "norms", B, T, C3)
+
+
 def gdn_scan_bins_train(spec: torch.Tensor, ab: torch.Tensor, gate_type: str, what: torch.Tensor,
                         delta_key_dim: int, scan_variant: str = "goom"):
     """Training forward of the delta rule (cssm.py:4898-5000): spec (B, T, 3C, H, Wf) complex64 with
@@ -929,6 +952,7 @@ def gdn_scan_bins_train(spec: torch.Tensor, ab: torch.Tensor, gate_type: str, wh
     B, T, C3, H, Wf = spec.shape
     C, dk = C3 // 3, delta_key_dim
     W = 2 * (Wf - 1)
+    _core_sizes(spec, None, ab, gate_type, what, dk)
     fs, hs, bs = _ab_strides(ab, gate_type)
     ohat = torch.empty((B, T, C, H, Wf), dtype=torch.complex64, device=spec.device)
     states = torch.empty((B, T, C // dk, dk, dk, H * Wf), dtype=torch.complex64, device=spec.device)
@@ -952,6 +976,7 @@ def gdn_scan_bins_backward(spec: torch.Tensor, ab: torch.Tensor, gate_type: str,
     W = 2 * (Wf - 1)
     if tuple(dohat.shape) != (B, T, C, H, Wf) or tuple(states.shape) != (B, T, C // dk, dk, dk, H * Wf):
         raise ValueError("dohat / states shapes do not match spec")
+    _core_sizes(spec, None, ab, gate_type, what, dk)
     fs, hs, bs = _ab_strides(ab, gate_type)
     dspec = torch.empty_like(spec)
     dab = torch.empty((B, T, C // dk, H * Wf, 2), dtype=torch.float32, device=spec.device)
@@ -972,6 +997,7 @@ def gdn_core_train(spec: torch.Tensor, norms: Optional[torch.Tensor], ab: torch.
     _dev(what, "what", torch.complex64)
     B, T, C3, H, Wf = spec.shape
     C, dk = C3 // 3, delta_key_dim
+    _core_sizes(spec, norms, ab, gate_type, what, dk)
     fs, hs, bs = _ab_strides(ab, gate_type)
     ohat = torch.empty((B, T, C, H, Wf), dtype=torch.complex64, device=spec.device)
     states = torch.empty((B, T, C // dk, dk, dk, H * Wf), dtype=torch.complex64, device=spec.device)
@@ -994,6 +1020,7 @@ def gdn_core_backward(spec: torch.Tensor, norms: Optional[torch.Tensor], ab: tor
     C, dk = C3 // 3, delta_key_dim
     if tuple(dospec.shape) != (B, T, C, H, Wf) or tuple(states.shape) != (B, T, C // dk, dk, dk, H * Wf):
         raise ValueError("dospec / states shapes do not match spec")
+    _core_sizes(spec, norms, ab, gate_type, what, dk)
     fs, hs, bs = _ab_strides(ab, gate_type)
     dspec = torch.empty_like(spec)
     dab = torch.empty((B, T, C // dk, H * Wf, 2), dtype=torch.float32, device=spec.device)
@@ -1004,32 +1031,41 @@ def gdn_core_backward(spec: torch.Tensor, norms: Optional[torch.Tensor], ab: tor
     return dspec, dab, dwhat
 
 
-def _frames(t: torch.Tensor, name: str, C: int, HW: int) -> int:
+def _frames(t: torch.Tensor, name: str, F: int, C: int, HW: int) -> int:
     """Frame stride in floats of a float32 (F, C, HW) channel slice of a plane-major tensor."""
     if not isinstance(t, torch.Tensor) or t.device.type != "cuda" or t.dtype != torch.float32:
         raise ValueError(f"{name} must be a float32 GPU tensor")
-    if t.dim() != 3 or t.shape[1:] != (C, HW) or t.stride(2) != 1 or t.stride(1) != HW or t.stride(0) < C * HW:
-        raise ValueError(f"{name}: a (F, {C}, {HW}) channel slice of a plane-major tensor is needed")
+    if t.shape != (F, C, HW) or t.stride(2) != 1 or t.stride(1) != HW or t.stride(0) < C * HW:
+        raise ValueError(f"{name}: a ({F}, {C}, {HW}) channel slice of a plane-major tensor is needed")
     return t.stride(0)
 
 
-def _conv_ptrs(convs):
+def _conv_ptrs(convs, C: int):
     if not convs:
         return 0, None, None
-    ks = [_dev(convs[2 * i], "short_conv.kernel", torch.float32) for i in range(3)]
-    bs = [_dev(convs[2 * i + 1], "short_conv.bias", torch.float32) for i in range(3)]
+    ks = [_sized(convs[2 * i], "short_conv.kernel", convs[0].shape[0], 1, C) for i in range(3)]
+    bs = [_sized(convs[2 * i + 1], "short_conv.bias", C) for i in range(3)]
     return (ks[0].shape[0], (ctypes.c_void_p * 3)(*[k.data_ptr() for k in ks]),
             (ctypes.c_void_p * 3)(*[b.data_ptr() for b in bs]))
+
+
+def _qkv_gates(gates: Optional[torch.Tensor], gate_mode: int, F: int, C: int, HW: int) -> Optional[int]:
+    if not gate_mode:
+        return None
+    shapes = {1: (2, F, HW), 2: (2, F), 3: (F, 2 * C, HW)}
+    return _sized(gates, "gates", *shapes.get(gate_mode, gates.shape)).data_ptr()
 
 
 def gdn_qkv_act(raw: torch.Tensor, B: int, T: int, convs, gate_mode: int, gates: Optional[torch.Tensor]):
     """out (F, 3C, HW) = gate SiLU(short conv(raw)) of raw (F, 3C, HW), a channel slice of a plane-major tensor
     (cssm_gdn_qkv_act); convs = (kernel_q, bias_q, kernel_k, ...) or (), gates as the entry point's modes."""
     F, C3, HW = raw.shape
-    fs = _frames(raw, "raw", C3, HW)
-    kt, kern, cb = _conv_ptrs(convs)
+    if F != B * T or C3 % 3:
+        raise ValueError(f"raw {tuple(raw.shape)} does not hold q, k and v of {B} x {T} frames")
+    fs = _frames(raw, "raw", F, C3, HW)
+    kt, kern, cb = _conv_ptrs(convs, C3 // 3)
     out = torch.empty((F, C3, HW), dtype=torch.float32, device=raw.device)
-    gp = _dev(gates, "gates", torch.float32).data_ptr() if gate_mode else None
+    gp = _qkv_gates(gates, gate_mode, F, C3 // 3, HW)
     _lib.call("cssm_gdn_qkv_act", raw.data_ptr(), fs, B, T, C3 // 3, HW, kt, kern, cb, gate_mode, gp, out.data_ptr(),
               _stream())
     return out
@@ -1041,18 +1077,20 @@ def gdn_qkv_act_backward(raw: torch.Tensor, B: int, T: int, convs, gate_mode: in
     gates' shape or None, sums (3C, kt + 2): the taps', the conv bias's and draw's sums)."""
     F, C3, HW = raw.shape
     C = C3 // 3
-    fs, dfs = _frames(raw, "raw", C3, HW), _frames(draw, "draw", C3, HW)
-    _dev(dout, "dout", torch.float32)
-    kt, kern, cb = _conv_ptrs(convs)
+    if F != B * T or C3 % 3:
+        raise ValueError(f"raw {tuple(raw.shape)} does not hold q, k and v of {B} x {T} frames")
+    fs, dfs = _frames(raw, "raw", F, C3, HW), _frames(draw, "draw", F, C3, HW)
+    _sized(dout, "dout", F, C3, HW)
+    kt, kern, cb = _conv_ptrs(convs, C)
+    gp = _qkv_gates(gates, gate_mode, F, C, HW)
     n = int(_lib.load().cssm_gdn_qkv_act_bwd_blocks(B, C, HW))
     sums = torch.empty((B, n, C3, kt + 2), dtype=torch.float32, device=raw.device)
     dg = None
     if gate_mode:
-        _dev(gates, "gates", torch.float32)
         dg = torch.empty((F, 2 * C, HW) if gate_mode == 3 else (2, (C + 7) // 8, F, HW), dtype=torch.float32,
                          device=raw.device)
     _lib.call("cssm_gdn_qkv_act_bwd", raw.data_ptr(), fs, B, T, C, HW, kt, kern, cb, gate_mode,
-              gates.data_ptr() if gate_mode else None, dout.data_ptr(), draw.data_ptr(), dfs,
+              gp, dout.data_ptr(), draw.data_ptr(), dfs,
               dg.data_ptr() if dg is not None else None, sums.data_ptr(), _stream())
     if gate_mode in (1, 2):
         dg = dg.sum(dim=1) if gate_mode == 1 else dg.sum(dim=(1, 3))
@@ -1066,8 +1104,8 @@ def gdn_norm_gate_supported(C: int) -> bool:
 def _norm_ptrs(scale: Optional[torch.Tensor], shift: Optional[torch.Tensor], C: int):
     """Addresses of the norm's (C,) float32 scale and shift, None where absent."""
     for t, n in ((scale, "scale"), (shift, "shift")):
-        if t is not None and _dev(t, n, torch.float32).shape != (C,):
-            raise ValueError(f"{n} {tuple(t.shape)} does not match C={C}")
+        if t is not None:
+            _sized(t, n, C)
     return (scale.data_ptr() if scale is not None else None, shift.data_ptr() if shift is not None else None)
 
 
@@ -1078,7 +1116,7 @@ def gdn_norm_gate(o: torch.Tensor, g: torch.Tensor, norm: str, scale: Optional[t
     _dev(o, "o", torch.float32)
     F, C, HW = o.shape
     y = torch.empty_like(o)
-    _lib.call("cssm_gdn_norm_gate", o.data_ptr(), g.data_ptr(), _frames(g, "g", C, HW), F, C, HW, _NORMS[norm],
+    _lib.call("cssm_gdn_norm_gate", o.data_ptr(), g.data_ptr(), _frames(g, "g", F, C, HW), F, C, HW, _NORMS[norm],
               _ACTS[act], *_norm_ptrs(scale, shift, C), y.data_ptr(), _stream())
     return y
 
@@ -1088,16 +1126,14 @@ def gdn_norm_gate_backward(o: torch.Tensor, g: torch.Tensor, norm: str, scale: O
     """Adjoint of :func:`gdn_norm_gate`: writes dg (a channel slice allowed) and returns (do, sums (3, C): the
     gradients of scale and shift, and the sum of dg)."""
     _dev(o, "o", torch.float32)
-    _dev(dy, "dy", torch.float32)
     F, C, HW = o.shape
-    if dy.shape != o.shape:
-        raise ValueError(f"dy {tuple(dy.shape)} does not match o {tuple(o.shape)}")
+    _sized(dy, "dy", F, C, HW)
     do = torch.empty_like(o)
     n = int(_lib.load().cssm_gdn_norm_gate_blocks(F, HW))
     sums = torch.empty((n, 3, C), dtype=torch.float32, device=o.device)
-    _lib.call("cssm_gdn_norm_gate_bwd", o.data_ptr(), g.data_ptr(), _frames(g, "g", C, HW), F, C, HW, _NORMS[norm],
+    _lib.call("cssm_gdn_norm_gate_bwd", o.data_ptr(), g.data_ptr(), _frames(g, "g", F, C, HW), F, C, HW, _NORMS[norm],
               _ACTS[act], *_norm_ptrs(scale, shift, C), dy.data_ptr(), do.data_ptr(), dg.data_ptr(),
-              _frames(dg, "dg", C, HW), sums.data_ptr(), _stream())
+              _frames(dg, "dg", F, C, HW), sums.data_ptr(), _stream())
     return do, sums.sum(dim=0)
 
 

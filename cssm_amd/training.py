@@ -389,9 +389,21 @@ class _WhatFn(torch.autograd.Function):
 def _gated_node_takes(cell, p, gate_params, T: int, H: int, W: int, Ci: int, dev) -> bool:
     """Whether _GatedInScanFn covers the cell on these planes with these parameters: transforms with fused work,
     short convolutions its kernels hold, and tensors as their addresses are read.  The torch path takes the rest
-    (a gate bias that broadcasts or is held in 16 bits)."""
-    ks, kt = cell.short_conv_spatial_size, cell.short_conv_size
-    if not S.fft_ex_supported(H, W) or ((ks > 0 or kt > 0) and not S.short_conv_train_supported(T, H, W, ks, kt)):
+    (a bias that broadcasts or is held in 16 bits) and raises for shapes that do not fit."""
+    if not S.fft_ex_supported(H, W):
+        return False
+    ks = kt = 0
+    if cell.short_conv_spatial_size > 0:
+        q = p["short_conv_spatial"]
+        ks = q["kernel"].shape[0]
+        if not (_as_read(q["kernel"], dev, ks, ks, 1, Ci) and _as_read(q["bias"], dev, Ci)):
+            return False
+    if cell.short_conv_size > 0:
+        q = p["short_conv_temporal"]
+        kt = q["kernel"].shape[0]
+        if kt == 0 or not (_as_read(q["kernel"], dev, kt, 1, Ci) and _as_read(q["bias"], dev, Ci)):
+            return False
+    if (ks or kt) and not S.short_conv_train_supported(T, H, W, ks, kt):
         return False
     sizes = (H, W // 2 + 1) if cell.gate_type == "factored" else (H * (W // 2 + 1),)
     K = p["kernel"].shape[-1]
@@ -548,10 +560,15 @@ def _temporal_encoding(T: int, C: int, base: float, device) -> torch.Tensor:
     return torch.stack([torch.sin(th), torch.cos(th)], -1).reshape(T, C).float()
 
 
-def _gate_products(p, names, gate_type, ctx):
-    """{parameter name: ctx kernel + bias} of the named gates' Dense layers as one product (their kernels side
+def _gate_keys(cell):
+    """Parameter names of the GDN gates that are Dense layers of ctx."""
+    names = ["alpha", "beta"] + (["B_k", "B_v"] if cell.use_input_gates and cell.gate_type != "channel" else [])
+    return [f"{n}_{a}" for n in names for a in "hw"] if cell.gate_type == "factored" else names
+
+
+def _gate_products(p, keys, ctx):
+    """{parameter name: ctx kernel + bias} of the named Dense layers as one product (their kernels side
     by side: one GEMM forward and two backward instead of up to eight of each)."""
-    keys = [f"{n}_{a}" for n in names for a in "hw"] if gate_type == "factored" else list(names)
     out = torch.addmm(torch.cat([p[k]["bias"] for k in keys]), ctx.reshape(-1, ctx.shape[-1]),
                       torch.cat([p[k]["kernel"] for k in keys], dim=1)).view(*ctx.shape[:-1], -1)
     return dict(zip(keys, out.split([p[k]["bias"].shape[0] for k in keys], dim=-1)))
@@ -671,13 +688,27 @@ def _norm_params(cell, p):
     return None, None
 
 
-def _gdn_node_takes(cell, p, C: int, dev) -> bool:
+def _gdn_node_takes(cell, p, C: int, H: int, W: int, dev) -> bool:
     """Whether _GdnFn covers the cell with these parameters: at most 128 channels and short-convolution taps its
-    kernels hold, no full-channel qkv convolution, and tensors as their addresses are read.  The torch path
-    takes the rest (a scale that broadcasts or is held in 16 bits)."""
+    kernels hold, no full-channel qkv convolution, and tensors as their addresses are read or side by side in
+    one product.  The torch path takes the rest (a scale that broadcasts or is held in 16 bits, q, k and v with
+    taps of their own) and raises for shapes that do not fit."""
     if (cell.qkv_conv_size > 1 and not cell.qkv_conv_separable) or not S.gdn_norm_gate_supported(C):
         return False
-    return cell.short_conv_size <= 8 and all(t is None or _as_read(t, dev, C) for t in _norm_params(cell, p))
+    if not all(t is None or _as_read(t, dev, C) for t in _norm_params(cell, p)):
+        return False
+    dense = [("qkv_proj", 3 * C), ("gate_proj", C)]
+    for k in _gate_keys(cell):
+        spatial, Wf = k.startswith("B_"), W // 2 + 1
+        dense.append((k, H if k.endswith("_h") else (W if spatial else Wf) if k.endswith("_w")
+                      else {"channel": C // cell.delta_key_dim, "scalar": 1}.get(cell.gate_type, H * (W if spatial else Wf))))
+    if not all(_as_read(p[k]["kernel"], dev, C, n) and _as_read(p[k]["bias"], dev, n) for k, n in dense):
+        return False
+    if cell.short_conv_size == 0:
+        return True
+    convs = [p[f"short_conv_{n}"] for n in "qkv"]
+    kt = convs[0]["kernel"].shape[0]
+    return 0 < kt <= 8 and all(_as_read(q["kernel"], dev, kt, 1, C) and _as_read(q["bias"], dev, C) for q in convs)
 
 
 def _gdn_fused_apply(cell, p, x, ctx, what, dims):
@@ -689,12 +720,10 @@ def _gdn_fused_apply(cell, p, x, ctx, what, dims):
     if cell.qkv_conv_size > 1:
         xq2 = _dwconv_cl(x.reshape(F, H, W, C), p["qkv_dw"]).reshape(-1, C).contiguous()
 
-    names = ["alpha", "beta"] + (["B_k", "B_v"] if cell.use_input_gates and cell.gate_type != "channel" else [])
-    products = _gate_products(p, names, cell.gate_type, ctx)
+    products = _gate_products(p, _gate_keys(cell), ctx)
 
     def gate(name, **kw):
-        prods = products if name in names else None
-        return _gdn_gate(p, name, cell.gate_type, ctx, x, H, W, nh, products=prods, **kw)
+        return _gdn_gate(p, name, cell.gate_type, ctx, x, H, W, nh, products=products, **kw)
     ab = torch.stack([gate("alpha", bounded=True), gate("beta")], dim=-1).contiguous()
     gate_mode, gkv = 0, None
     if cell.use_input_gates:
@@ -738,7 +767,7 @@ def gdn_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tens
     if not cell.position_independent_gates:
         ctx = ctx + _temporal_encoding(T, C, cell.rope_base, x.device)[None]
     ks = cell.qkv_conv_size
-    if _gdn_node_takes(cell, p, C, x.device):
+    if _gdn_node_takes(cell, p, C, H, W, x.device):
         return _gdn_fused_apply(cell, p, x, ctx, what, (B, T, H, W, C, dk, nh))
     xq = x.reshape(F, H, W, C)
     if ks > 1 and not cell.qkv_conv_separable:

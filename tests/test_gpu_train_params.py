@@ -126,6 +126,79 @@ def test_gated_parameter_layouts(mods, shape, gate_type, ks, form):
     close(got, ref)
 
 
+@pytest.mark.parametrize("cls,path", [("gated", "short_conv_spatial"), ("gated", "short_conv_temporal"),
+                                      ("gated", "delta_proj_h"), ("gdn", "short_conv_k"), ("gdn", "short_conv_q"),
+                                      ("gdn", "alpha_w"), ("gdn", "gate_proj"), ("gdn", "rms_scale")])
+def test_mismatched_parameters_raise(mods, cls, path):
+    """Parameters of another channel count or plane size than the call's."""
+    cells, _, training = mods
+    print_case(test="mismatched", cls=cls, path=path)
+    kw = dict(gate_type="factored", **({"delta_key_dim": 4} if cls == "gdn" else {}))
+    cell, v, x, _ = layer(cells.GatedCSSM if cls == "gated" else cells.GatedDeltaNetCSSM, 3, (1, 2, 16, 16, 8), **kw)
+    p = v["params"]
+    p[path] = ({k: t[..., :-1].contiguous() for k, t in p[path].items()} if isinstance(p[path], dict)
+               else p[path][:-1].contiguous())
+    with pytest.raises((ValueError, RuntimeError)):
+        (training.gated_train_apply if cls == "gated" else training.gdn_train_apply)(cell, v, x)
+
+
+def test_taps_follow_the_tree(mods):
+    """q, k and v with taps of their own, and trees with fewer taps than the cell's default."""
+    cells, _, training = mods
+    print_case(test="taps_of_the_tree")
+    kw = dict(delta_key_dim=4, gate_type="factored")
+    cell, v, x, dout = layer(cells.GatedDeltaNetCSSM, 5, (2, 5, 8, 8, 8), **kw)
+    p = v["params"]
+    p["short_conv_k"]["kernel"][:2] = 0.0                  # taps a shorter kernel leaves out
+    ref = grads(training.gdn_train_apply, cell, v, x, dout)
+    i = 2 + [id(t) for t in leaves(p)].index(id(p["short_conv_k"]["kernel"]))
+    p["short_conv_k"]["kernel"] = p["short_conv_k"]["kernel"][2:].contiguous()
+    ref[i] = ref[i][2:]
+    close(grads(training.gdn_train_apply, cell, v, x, dout), ref)
+    cell, v, x, dout = layer(cells.GatedCSSM, 5, (1, 5, 16, 16, 8), gate_type="factored", short_conv_size=2)
+    ref = grads(training.gated_train_apply, cell, v, x, dout)
+    wide = cells.GatedCSSM(channels=8, kernel_size=5, gate_type="factored", short_conv_size=4)
+    close(grads(training.gated_train_apply, wide, v, x, dout), ref)
+
+
+def test_training_wrappers_refuse_other_shapes(mods):
+    _, S, _ = mods
+    print_case(test="wrappers_refuse")
+    r = lambda *s: torch.randn(s, device="cuda")
+    x, do, dx = r(1, 2, 8, 7, 7), r(1, 2, 8, 7, 7), r(2, 8, 49)
+    good = ((r(3, 3, 1, 8), r(8)), (r(4, 1, 8), r(8)))
+    for sp, tp in (((r(3, 3, 1, 7), r(8)), good[1]), ((r(3, 3, 1, 8), r(7)), good[1]), (good[0], (r(4, 1, 7), r(8))),
+                   (good[0], (r(4, 1, 8), r(7)))):
+        with pytest.raises(ValueError):
+            S.short_conv_train(x, sp, tp)
+        with pytest.raises(ValueError):
+            S.short_conv_backward(x, do, sp, tp, dx)
+    with pytest.raises(ValueError):
+        S.short_conv_backward(x, do[:, :1].contiguous(), *good, dx)
+    with pytest.raises(ValueError):
+        S.short_conv_backward(x, do, *good, dx[:1])
+    raw, g = r(2, 24, 49), r(2, 2, 49)
+    convs = [r(4, 1, 8), r(8)] * 3
+    for i, t in ((2, r(3, 1, 8)), (4, r(4, 1, 7)), (1, r(7))):
+        bad = convs[:i] + [t] + convs[i + 1:]
+        with pytest.raises(ValueError):
+            S.gdn_qkv_act(raw, 1, 2, bad, 1, g)
+        with pytest.raises(ValueError):
+            S.gdn_qkv_act_backward(raw, 1, 2, bad, 1, g, torch.empty_like(raw), torch.empty_like(raw))
+    with pytest.raises(ValueError):
+        S.gdn_qkv_act(raw, 1, 2, convs, 1, g[:, :1].contiguous())
+    with pytest.raises(ValueError):
+        S.gdn_qkv_act(raw, 1, 3, convs, 1, g)
+    spec, _ = S.rfft2(r(1, 2, 24, 8, 8))
+    ab, what = r(1, 2, 40, 2), torch.zeros((2, 8, 5), dtype=torch.complex64, device="cuda")
+    norms = r(1, 2, 24)
+    S.gdn_core_train(spec, norms, ab, "dense", what, 4, 8)
+    for a in ((spec, norms, ab[:, :, :39].contiguous(), what), (spec, norms, ab, what[:1]),
+              (spec, norms[:, :, :23].contiguous(), ab, what)):
+        with pytest.raises(ValueError):
+            S.gdn_core_train(a[0], a[1], a[2], "dense", a[3], 4, 8)
+
+
 def test_norm_gate_refuses_what_it_would_misread(mods):
     _, S, _ = mods
     print_case(test="norm_gate_refuses")
