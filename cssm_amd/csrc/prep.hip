@@ -31,20 +31,31 @@ __host__ __device__ inline SpecTaps spec_taps(int K, int H, int W) {
   return {0, K, (H - K) / 2, 0, K, (W - K) / 2};                       // zero pad
 }
 
-// LDS: tw (W), th (H) double2 tables, then R[i][j] = sum_j' k[i][j'] e^{-2 pi i v j'' / W} for the nc columns
+// e^{2 pi i m / n}: the table's entry, or (TAB false, planes too long for tables in LDS) taken each time
+template <bool TAB>
+__device__ __forceinline__ double2 twiddle(const double2* tab, int m, int n) {
+  if constexpr (TAB) return tab[m];
+  double2 w;
+  sincospi(2.0 * double(m) / double(n), &w.y, &w.x);
+  return w;
+}
+
+// LDS: tw (W), th (H) double2 tables (TAB), then R[i][j] = sum_j' k[i][j'] e^{-2 pi i v j'' / W} for the nc columns
 // v = col(j)
-template <class Col>
+template <bool TAB, class Col>
 __device__ __forceinline__ void spec_rows(const float* kc, int K, int H, int W, const SpecTaps& q, int nc, Col col,
                                           double2* tw, double2* th, double2* R) {
-  for (int m = threadIdx.x; m < W; m += blockDim.x) sincospi(2.0 * double(m) / double(W), &tw[m].y, &tw[m].x);
-  for (int m = threadIdx.x; m < H; m += blockDim.x) sincospi(2.0 * double(m) / double(H), &th[m].y, &th[m].x);
-  __syncthreads();
+  if constexpr (TAB) {
+    for (int m = threadIdx.x; m < W; m += blockDim.x) tw[m] = twiddle<false>(nullptr, m, W);
+    for (int m = threadIdx.x; m < H; m += blockDim.x) th[m] = twiddle<false>(nullptr, m, H);
+    __syncthreads();
+  }
   for (int idx = threadIdx.x; idx < q.nr * nc; idx += blockDim.x) {
     const int i = idx / nc, v = col(idx % nc);
     double re = 0.0, im = 0.0;
-    int m = v * q.ow % W;                        // v (j + ow) mod W
+    int m = TAB ? v * q.ow % W : int((long long)v * q.ow % W);   // v (j + ow) mod W
     for (int j = 0; j < q.nq; ++j, m = m + v < W ? m + v : m + v - W) {
-      const double2 w = tw[m];
+      const double2 w = twiddle<TAB>(tw, m, W);
       const double kv = double(kc[(q.r0 + i) * K + (q.q0 + j)]);
       re += kv * w.x;
       im -= kv * w.y;
@@ -54,12 +65,13 @@ __device__ __forceinline__ void spec_rows(const float* kc, int K, int H, int W, 
   __syncthreads();
 }
 // F[u][v] = sum_i R[i][j] e^{-2 pi i u i' / H}, j the column's slot of nc
+template <bool TAB>
 __device__ __forceinline__ double2 spec_bin(const double2* R, const double2* th, const SpecTaps& q, int H, int nc,
                                             int u, int j) {
   double re = 0.0, im = 0.0;
-  int m = u * q.oh % H;                          // u (i + oh) mod H
+  int m = TAB ? u * q.oh % H : int((long long)u * q.oh % H);   // u (i + oh) mod H
   for (int i = 0; i < q.nr; ++i, m = m + u < H ? m + u : m + u - H) {
-    const double2 w = th[m], a = R[i * nc + j];
+    const double2 w = twiddle<TAB>(th, m, H), a = R[i * nc + j];
     // (ar + i ai)(cs - i sn)
     re += a.x * w.x + a.y * w.y;
     im += a.y * w.x - a.x * w.y;
@@ -67,18 +79,19 @@ __device__ __forceinline__ double2 spec_bin(const double2* R, const double2* th,
   return make_double2(re, im);
 }
 
+template <bool TAB>
 __global__ void spectral_kernel_prep(const float* __restrict__ k, int K, int H, int W, float rho,
                                      int squash, int goom_floor, int scan_order, float2* __restrict__ out) {
   extern __shared__ double2 sm_d[];
   const int c = blockIdx.x, WF = W / 2 + 1;
   const SpecTaps q = spec_taps(K, H, W);
-  double2 *tw = sm_d, *th = sm_d + W, *R = sm_d + W + H;
-  spec_rows(k + size_t(c) * K * K, K, H, W, q, WF, [](int j) { return j; }, tw, th, R);
+  double2 *tw = sm_d, *th = sm_d + W, *R = TAB ? sm_d + W + H : sm_d;
+  spec_rows<TAB>(k + size_t(c) * K * K, K, H, W, q, WF, [](int j) { return j; }, tw, th, R);
   // at position (u, p) of the output with v = scan_col(p) in the scan's column order, in the scan's
   // slot khat_pos(u, p); gridDim.y workgroups share a channel's bins
   for (int idx = int(blockIdx.y) * blockDim.x + threadIdx.x; idx < H * WF; idx += gridDim.y * blockDim.x) {
     const int u = idx / WF, v = scan_order ? scan_col(H, W, idx % WF) : idx % WF;
-    double2 f = spec_bin(R, th, q, H, WF, u, v);
+    double2 f = spec_bin<TAB>(R, th, q, H, WF, u, v);
     if (squash) {
       const double mag = sqrt(f.x * f.x + f.y * f.y);
       const double g = double(rho) / (1.0 + mag);
@@ -114,7 +127,7 @@ __global__ void __launch_bounds__(256) spectral_kernel_bwd(const float* __restri
   double2 *tw = sm_d, *th = sm_d + W, *R = sm_d + W + H;
   float2* dF = reinterpret_cast<float2*>(R + q.nr * nc);
   auto col = [&](int j) { return scan_order ? scan_col(H, W, p0 + j) : p0 + j; };
-  spec_rows(k + size_t(c) * K * K, K, H, W, q, nc, col, tw, th, R);
+  spec_rows<true>(k + size_t(c) * K * K, K, H, W, q, nc, col, tw, th, R);
   for (int idx = threadIdx.x; idx < H * nc; idx += blockDim.x) {
     const int u = idx / nc, j = idx % nc;
     const size_t pos = scan_order ? khat_pos(H, W, u, p0 + j) : u * WF + p0 + j;
@@ -126,7 +139,7 @@ __global__ void __launch_bounds__(256) spectral_kernel_bwd(const float* __restri
       g.y += e.y;
     }
     if (squash || goom_floor) {
-      const double2 f = spec_bin(R, th, q, H, nc, u, j);
+      const double2 f = spec_bin<true>(R, th, q, H, nc, u, j);
       const double mag = sqrt(f.x * f.x + f.y * f.y), s = squash ? 1.0 / (1.0 + mag) : 1.0;
       const double kr = squash ? double(rho) * s : 1.0;
       const float2 o = make_float2(float(f.x * kr), float(f.y * kr));
@@ -622,9 +635,13 @@ hipError_t launch_spectral_kernel(const float* k, int C, int K, int H, int W, fl
   const int WF = W / 2 + 1;
   const SpecTaps q = spec_taps(K, H, W);
   if (size_t(q.nr) * WF * sizeof(double2) > 64 * 1024) return hipErrorInvalidValue;   // (as ever: planes refused)
-  const size_t shm = (size_t(q.nr) * WF + W + H) * sizeof(double2);
+  // the row sums fit 64 KB; the tables go beside them while all of it fits a workgroup's 160 KB (H + W to about
+  // 6000 at the most row sums, 10240 at few), longer planes take their twiddles each time
+  const size_t tab = (size_t(q.nr) * WF + W + H) * sizeof(double2);
+  const size_t shm = tab <= 160 * 1024 ? tab : size_t(q.nr) * WF * sizeof(double2);
+  const auto kern = tab <= 160 * 1024 ? spectral_kernel_prep<true> : spectral_kernel_prep<false>;
   if (shm > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(spectral_kernel_prep),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, int(shm));
     if (e != hipSuccess) return e;
   }
@@ -632,7 +649,7 @@ hipError_t launch_spectral_kernel(const float* k, int C, int K, int H, int W, fl
   int ny = (256 + C - 1) / C;
   const int most = (H * WF + 255) / 256;
   if (ny > most) ny = most;
-  hipLaunchKernelGGL(spectral_kernel_prep, dim3(C, ny), dim3(256), shm, s, k, K, H, W, rho, squash, goom_floor,
+  hipLaunchKernelGGL(kern, dim3(C, ny), dim3(256), shm, s, k, K, H, W, rho, squash, goom_floor,
                      scan_order, khat);
   return hipGetLastError();
 }

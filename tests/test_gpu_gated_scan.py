@@ -79,6 +79,18 @@ def test_spectral_kernel_matches_oracle(S, C, K, H, W):
     assert err < 1e-6 * max(1.0, np.max(np.abs(ref)))
 
 
+# the twiddle tables with the row sums at the edges of a workgroup's LDS, and planes too long for them
+@pytest.mark.parametrize("C,K,H,W", [(1, 63, 128, 128), (1, 1, 4090, 4090), (1, 1, 4096, 4096), (2, 5, 12000, 64),
+                                     (1, 1, 3000, 8000)])
+def test_spectral_kernel_of_long_planes(S, C, K, H, W):
+    print_case(test="spectral_kernel_long", C=C, K=K, H=H, W=W)
+    k = np.random.default_rng(8).standard_normal((C, K, K)) * 0.3
+    got = S.spectral_kernel(_dev(k), H, W, rho=0.999, squash=True, goom_floor=False)
+    ref = O.spectral_kernel(k, H, W, 0.999)
+    # double sums rounded once to float32, of inputs rounded to float32
+    assert np.max(np.abs(got.cpu().numpy() - ref)) < 1e-6 * max(1.0, np.max(np.abs(ref)))
+
+
 def test_spectral_kernel_goom_floor(S):
     print_case(test="spectral_kernel_floor")
     k = np.zeros((2, 3, 3))
