@@ -99,6 +99,7 @@ SIGNATURES = {
     "cssm_short_conv_train": (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P, _P, _P]),
     "cssm_short_conv_bwd_chunks": (_I, [_I, _I, _I, _I, _I]),
     "cssm_short_conv_bwd": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _LL, _P, _P]),
+    "cssm_spectral_kernel_supported": (_I, [_I, _I, _I]),
     "cssm_spectral_kernel_bwd_parts": (_I, [_I, _I, _I, _I]),
     "cssm_gated_scan_bwd_groups": (_I, [_I, _I, _I, _I]),
     "cssm_gated_scan_bwd_split": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, ctypes.c_float, _P, _P, _I, _P, _P, _P]),

@@ -79,6 +79,8 @@ int cssm_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, 
   return hip_status(e, "cssm_spectral_kernel");
 }
 
+int cssm_spectral_kernel_supported(int K, int H, int W) { return cssm::spectral_kernel_supported(K, H, W) ? 1 : 0; }
+
 int cssm_spectral_kernel_bwd_parts(int C, int K, int H, int W) {
   return cssm::spectral_kernel_bwd_supported(C, K, H, W) ? cssm::spectral_kernel_bwd_parts(C, W) : 0;
 }

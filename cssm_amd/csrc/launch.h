@@ -75,6 +75,7 @@ __device__ __forceinline__ float ctx_tile_sum(const float* __restrict__ partial,
 
 hipError_t launch_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, int squash,
                                   int goom_floor, int scan_order, float2* khat, hipStream_t s);
+bool spectral_kernel_supported(int K, int H, int W);
 bool spectral_kernel_bwd_supported(int C, int K, int H, int W);
 int spectral_kernel_bwd_parts(int C, int W);   // dk (parts, C, K, K)
 hipError_t launch_spectral_kernel_bwd(const float* k, int B, int C, int K, int H, int W, float rho, int squash,

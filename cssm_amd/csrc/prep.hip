@@ -630,12 +630,18 @@ __global__ void plane_mean_kernel(const TIN* __restrict__ x, long long nplanes, 
 
 // ----------------------------------------------------------------- launchers
 
+// the row sums fit 64 KB of LDS, and K does not lie between H and W
+bool spectral_kernel_supported(int K, int H, int W) {
+  return K > 0 && H > 0 && W > 0 && !((K > H || K > W) && (K < H || K < W)) &&
+         size_t(spec_taps(K, H, W).nr) * (W / 2 + 1) * sizeof(double2) <= 64 * 1024;
+}
+
 hipError_t launch_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, int squash,
                                   int goom_floor, int scan_order, float2* khat, hipStream_t s) {
   const int WF = W / 2 + 1;
   const SpecTaps q = spec_taps(K, H, W);
-  if (size_t(q.nr) * WF * sizeof(double2) > 64 * 1024) return hipErrorInvalidValue;   // (as ever: planes refused)
-  // the row sums fit 64 KB; the tables go beside them while all of it fits a workgroup's 160 KB (H + W to about
+  if (!spectral_kernel_supported(K, H, W)) return hipErrorInvalidValue;
+  // the tables go beside the row sums while all of it fits a workgroup's 160 KB (H + W to about
   // 6000 at the most row sums, 10240 at few), longer planes take their twiddles each time
   const size_t tab = (size_t(q.nr) * WF + W + H) * sizeof(double2);
   const size_t shm = tab <= 160 * 1024 ? tab : size_t(q.nr) * WF * sizeof(double2);

@@ -55,6 +55,10 @@ def spectral_kernel(k: torch.Tensor, H: int, W: int, rho: float = 0.999, squash:
     return out
 
 
+def spectral_kernel_supported(K: int, H: int, W: int) -> bool:
+    return bool(_lib.load().cssm_spectral_kernel_supported(K, H, W))
+
+
 def spectral_kernel_bwd_supported(C: int, K: int, H: int, W: int) -> bool:
     return bool(_lib.load().cssm_spectral_kernel_bwd_parts(C, K, H, W))
 

@@ -388,7 +388,7 @@ class _WhatFn(torch.autograd.Function):
 
 def _gated_node_takes(cell, p, gate_params, T: int, H: int, W: int, Ci: int, dev) -> bool:
     """Whether _GatedInScanFn covers the cell on these planes with these parameters: transforms with fused work,
-    short convolutions its kernels hold, and tensors as their addresses are read.  The torch path takes the rest
+    taps and short convolutions its kernels hold, and tensors as their addresses are read.  The torch path takes the rest
     (a bias that broadcasts or is held in 16 bits) and raises for shapes that do not fit."""
     if not S.fft_ex_supported(H, W):
         return False
@@ -407,7 +407,7 @@ def _gated_node_takes(cell, p, gate_params, T: int, H: int, W: int, Ci: int, dev
         return False
     sizes = (H, W // 2 + 1) if cell.gate_type == "factored" else (H * (W // 2 + 1),)
     K = p["kernel"].shape[-1]
-    return _as_read(p["kernel"], dev, Ci, K, K) and all(
+    return S.spectral_kernel_supported(K, H, W) and _as_read(p["kernel"], dev, Ci, K, K) and all(
         _as_read(t, dev, *((Ci,) if i % 2 == 0 else ()), sizes[i // 2 % len(sizes)]) for i, t in enumerate(gate_params))
 
 
@@ -759,7 +759,8 @@ def gdn_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tens
         raise NotImplementedError(f"no spectral transform kernel for {H}x{W} planes")
     x = x.float()
     squash = not cell.no_spectral_clamp
-    if S.spectral_kernel_bwd_supported(nh, p["kernel"].shape[-1], H, W):
+    K = p["kernel"].shape[-1]
+    if S.spectral_kernel_supported(K, H, W) and S.spectral_kernel_bwd_supported(nh, K, H, W):
         what = _WhatFn.apply(p["kernel"].contiguous(), H, W, cell.spectral_rho, squash)
     else:
         what = what_planes(p["kernel"], H, W, cell.spectral_rho, squash).contiguous()

@@ -113,6 +113,8 @@ const char* cssm_last_error(void);
  */
 int cssm_spectral_kernel(const float* k, int C, int K, int H, int W, float rho, int squash,
                          int goom_floor, int scan_order, float* khat, void* stream);
+/* the sizes it takes: min(K, H) (W/2+1) <= 4096, K not between H and W */
+int cssm_spectral_kernel_supported(int K, int H, int W);
 
 /*
  * Adjoint of cssm_spectral_kernel: the gradient of k from dkhat (B, C, H, W/2+1)

@@ -161,6 +161,26 @@ def test_taps_follow_the_tree(mods):
     close(grads(training.gated_train_apply, wide, v, x, dout), ref)
 
 
+@pytest.mark.parametrize("cls", ["gated", "gdn"])
+def test_more_taps_than_the_prep_kernel_holds(mods, cls):
+    """65 x 65 taps on 128 x 128 planes: K_hat by torch; zero outer taps give the gradients of the 63 x 63 ones."""
+    cells, S, training = mods
+    print_case(test="many_taps", cls=cls)
+    assert S.spectral_kernel_supported(63, 128, 128) and not S.spectral_kernel_supported(64, 128, 128)
+    kw = dict(gate_type="factored", **({"delta_key_dim": 2} if cls == "gdn" else {}))
+    apply = training.gdn_train_apply if cls == "gdn" else training.gated_train_apply
+    cell, v, x, dout = layer(cells.GatedDeltaNetCSSM if cls == "gdn" else cells.GatedCSSM, 4, (1, 2, 128, 128, 4), **kw)
+    k = v["params"]["kernel"]
+    k63 = torch.nn.functional.pad(k, (29, 29, 29, 29))
+    v["params"]["kernel"] = k63
+    i = 2 + [id(t) for t in leaves(v["params"])].index(id(k63))
+    ref = grads(apply, cell, v, x, dout)
+    v["params"]["kernel"] = torch.nn.functional.pad(k63, (1, 1, 1, 1))
+    got = grads(apply, cell, v, x, dout)
+    got[i] = got[i][:, 1:-1, 1:-1]
+    close(got, ref)
+
+
 def test_training_wrappers_refuse_other_shapes(mods):
     _, S, _ = mods
     print_case(test="wrappers_refuse")
