@@ -160,11 +160,12 @@ class _DwConvFn(torch.autograd.Function):
 
 def _dwconv_cl(x4, q):
     """Depthwise SAME conv of channels-last (F, H, W, C) frames: the HIP kernels where they apply
-    (odd ks in 3..7, C a multiple of 4 up to 1024), else torch's conv."""
+    (odd ks in 3..7, C a multiple of 4 up to 1024, taps and bias as their addresses are read), else torch's conv."""
     ks = q["kernel"].shape[0]
     F, H, W, C = x4.shape
-    if ks % 2 == 1 and S.depthwise_conv_wgrad_supported(W, C, ks):
-        return _DwConvFn.apply(x4.contiguous(), q["kernel"], q["bias"])
+    if (ks % 2 == 1 and S.depthwise_conv_wgrad_supported(W, C, ks)
+            and _as_read(q["kernel"], x4.device, ks, ks, 1, C) and _as_read(q["bias"], x4.device, C)):
+        return _DwConvFn.apply(x4.contiguous(), q["kernel"].contiguous(), q["bias"].contiguous())
     lo, hi = (ks - 1) // 2, ks // 2
     w = q["kernel"].permute(3, 2, 0, 1)                                      # (C, 1, k, k)
     return (Fn.conv2d(Fn.pad(x4.permute(0, 3, 1, 2), (lo, hi, lo, hi)), w, groups=C)

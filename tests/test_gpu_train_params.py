@@ -126,6 +126,33 @@ def test_gated_parameter_layouts(mods, shape, gate_type, ks, form):
     close(got, ref)
 
 
+@pytest.mark.parametrize("form", ["strided", "bf16_bias", "one_bias"])
+@pytest.mark.parametrize("H", [14, 16])
+def test_qkv_depthwise_layouts(mods, form, H):
+    """Rows of eight pixels and others: taps and bias strided, the bias in 16 bits or one for all channels."""
+    cells, _, training = mods
+    print_case(test="qkv_dw_params", form=form, H=H)
+    cell, v, x, dout = layer(cells.GatedDeltaNetCSSM, 6, (1, 2, H, H, 8), delta_key_dim=4, gate_type="factored",
+                             qkv_conv_size=3)
+    q = v["params"]["qkv_dw"]
+    q["bias"] = (q["bias"][:1].expand(8).contiguous() if form == "one_bias" else q["bias"]).bfloat16().float()
+    i = 2 + [id(t) for t in leaves(v["params"])].index(id(q["bias"]))
+    ref = grads(training.gdn_train_apply, cell, v, x, dout)
+    if form == "strided":
+        q["kernel"], q["bias"] = strided(q["kernel"]), strided(q["bias"])
+    else:
+        q["bias"] = q["bias"].bfloat16() if form == "bf16_bias" else q["bias"][:1].contiguous()
+    got = grads(training.gdn_train_apply, cell, v, x, dout)
+    if form != "strided":                                  # as test_gdn_norm_scale_layouts
+        r = ref[i].double()
+        if form == "one_bias":
+            assert (got[i].double() - r.sum()).abs() <= 1e-4 * r.abs().sum()
+        else:
+            assert got[i].dtype == torch.bfloat16 and (got[i].double() - r).abs().max() <= 2 ** -8 * r.abs().max()
+        got[i] = ref[i]
+    close(got, ref)
+
+
 @pytest.mark.parametrize("cls,path", [("gated", "short_conv_spatial"), ("gated", "short_conv_temporal"),
                                       ("gated", "delta_proj_h"), ("gdn", "short_conv_k"), ("gdn", "short_conv_q"),
                                       ("gdn", "alpha_w"), ("gdn", "gate_proj"), ("gdn", "rms_scale")])
