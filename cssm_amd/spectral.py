@@ -200,7 +200,9 @@ def gated_scan(u: torch.Tensor, z: torch.Tensor, gates: torch.Tensor, khat: torc
     if out is None:
         out = torch.empty_like(u)
     _dev(out, "out", u.dtype)
-    if u.dtype == torch.float32 and not (u_silu or z_silu) and gated_split_rule(B * C, T, H, W):
+    # (what the fused kernel refuses, no planes, channels or alignment, stays with it)
+    if (u.dtype == torch.float32 and not (u_silu or z_silu) and gated_split_rule(B * C, T, H, W)
+            and C % gated_scan_min_group(H, W) == 0 and not (u.data_ptr() | z.data_ptr() | out.data_ptr()) % 16):
         return _gated_scan_split(u, z, gates, khat, out)
     _lib.call("cssm_gated_scan_fwd", u.data_ptr(), z.data_ptr(), out.data_ptr(), _DTYPES[u.dtype],
               B, T, C, H, W, gates.data_ptr(), khat.data_ptr(), int(u_silu), int(z_silu), _stream())
@@ -226,7 +228,7 @@ def gated_split_rule(planes: int, T: int, H: int, W: int) -> bool:
     23 / 21."""
     step = _FUSED_STEP_US.get(H) if H == W else None
     per_sample = 6.2e-6 if H >= 8 and (H & (H - 1)) == 0 else 12e-6
-    return step is not None and 24.0 + per_sample * planes * T * H * W < 0.9 * step * T
+    return step is not None and planes > 0 and 24.0 + per_sample * planes * T * H * W < 0.9 * step * T
 
 
 def _gated_scan_split(u, z, gates, khat, out, max_bytes: int = 1 << 30):

@@ -55,6 +55,23 @@ def test_rule_picks_the_split_form_for_few_planes(S):
     assert not S.gated_split_rule(64, 64, 16, 32)
 
 
+def test_what_the_fused_scan_refuses_stays_refused(S):
+    """Channels that are no whole group and planes off 16 bytes, at sizes where the rule takes the split form."""
+    from cssm_amd._lib import CssmError
+    print_case(test="split_refuses")
+    assert S.gated_split_rule(4, 64, 16, 16) and S.gated_split_rule(5, 64, 7, 7)
+    u, z, gates, khat = _case(S, 1, 64, 4, 16)
+    with pytest.raises(CssmError, match="multiple of 8"):
+        S.gated_scan(u, z, gates, khat)
+    u, z, gates, khat = _case(S, 1, 64, 5, 7)
+    with pytest.raises(CssmError, match="B=0"):
+        S.gated_scan(u[:0], z[:0], gates[:0], khat)
+    off = torch.zeros(u.numel() + 1, device="cuda")[1:].view(u.shape)
+    for a in ((off, z, None), (u, off, None), (u, z, off)):
+        with pytest.raises(CssmError, match="misaligned"):
+            S.gated_scan(a[0], a[1], gates, khat, out=a[2])
+
+
 @pytest.mark.parametrize("H", [3, 7, 12, 14, 15])
 def test_small_plane_transforms_with_fused_work(S, H):
     """cssm_rfft2_ex / cssm_irfft2_ex on small planes: strided halves of a (F, 2C, HW) tensor, activations,
