@@ -64,7 +64,7 @@ def test_what_the_fused_scan_refuses_stays_refused(S):
     with pytest.raises(CssmError, match="multiple of 8"):
         S.gated_scan(u, z, gates, khat)
     u, z, gates, khat = _case(S, 1, 64, 5, 7)
-    with pytest.raises(CssmError, match="B=0"):
+    with pytest.raises(CssmError, match="non-null"):        # an empty tensor has no address
         S.gated_scan(u[:0], z[:0], gates[:0], khat)
     off = torch.zeros(u.numel() + 1, device="cuda")[1:].view(u.shape)
     for a in ((off, z, None), (u, off, None), (u, z, off)):
