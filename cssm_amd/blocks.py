@@ -156,7 +156,7 @@ class CSSMSHViTBlock:
         pc = p.get("pos_conv") if self.use_pos_conv else None
         # of an image's equal frames only the cell's last is kept (without the timestep gate): one frame in
         still = (is_image and not self.timestep_gate and self.cssm_type != "gdn"
-                 and self.cell._still_pays(B, T, H, W))
+                 and self.cell._still_pays(B, T, H, W, p["cssm"]))
         xc = S.block_norm_posconv(x5, stats, self.block_norm, n1["scale"], n1["bias"],
                                   pc["kernel"] if pc is not None else None, pc["bias"] if pc is not None else None,
                                   1 if still else T)

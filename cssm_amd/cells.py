@@ -205,7 +205,16 @@ class GatedCSSM:
                          out_dtype=out_dtype or x.dtype)
         return out.view(B, T, H, W, self.channels)
 
-    def _still_pays(self, B: int, T: int, H: int, W: int) -> bool:
+    def _conv_sizes(self, p: Optional[Dict[str, Any]]):
+        """(pixels, frames) of the short convolutions: the parameters' own, which :meth:`apply` takes, or without
+        them the attributes'."""
+        ks, kt = self.short_conv_spatial_size, self.short_conv_size
+        if p is not None:
+            ks = p["short_conv_spatial"]["kernel"].shape[0] if ks > 0 else 0
+            kt = p["short_conv_temporal"]["kernel"].shape[0] if kt > 0 else 0
+        return ks, kt
+
+    def _still_pays(self, B: int, T: int, H: int, W: int, p: Optional[Dict[str, Any]] = None) -> bool:
         """Whether :meth:`_apply_still` covers B images of H x W (square planes that the batched transforms take,
         a short convolution of at most 4 frames and 3 x 3 pixels) and is the faster form: always where the scan
         itself ends in one frame (64 images of 14 x 14, C = 256, T = 2: 160 -> 123 us), behind the batched
@@ -213,12 +222,13 @@ class GatedCSSM:
         1405 -> 623 us, T = 2 439 -> 453; 512 of 4 x 4, C = 128: T = 8 130 -> 110, T = 5 99 -> 112; one of
         64 x 64, C = 64, no taps, T = 2: 58 -> 64)."""
         Ci = self.channels * self.expand
-        saved = T - min(T, max(1, self.short_conv_size))
+        ks, kt = self._conv_sizes(p)
+        saved = T - min(T, max(1, kt))
         if T <= 1 or not (S.gated_scan_last_supported(H, W) or B * Ci * H * W * saved > 1 << 20):
             return False
         return (S.gated_scan_supported(H, W) and Ci % S.gated_scan_min_group(H, W) == 0
                 and H >= 3 and S.fft_ex_supported(H, W) and B <= 65535
-                and S.short_conv_train_supported(1, H, W, self.short_conv_spatial_size, self.short_conv_size))
+                and S.short_conv_train_supported(1, H, W, ks, kt))
 
     def _apply_still(self, variables: Params, x: torch.Tensor, T: int,
                      out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
@@ -232,7 +242,7 @@ class GatedCSSM:
         HW, f32 = H * W, torch.float32
         x = x.contiguous()
         c_scale = S.scan_c_scale(H, W)
-        n = min(T, max(1, self.short_conv_size))
+        n = min(T, max(1, self._conv_sizes(p)[1]))
         if self.short_conv_spatial_size > 0 or self.short_conv_size > 0:
             xm, z, _ = S.proj_in(x, p["in_proj"]["kernel"], p["in_proj"]["bias"], B, HW, silu_hi=True, out_dtype=f32)
             u, ctx = S.short_conv_still(xm.view(B, Ci, H, W), n,

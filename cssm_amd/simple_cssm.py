@@ -298,7 +298,7 @@ class SimpleCSSM:
         # one cell on an image's equal frames with the last one read out: the cell takes the image itself
         still = (T_in == 1 and self.depth == 1 and self.cssm_type == "gated" and self.frame_readout == "last"
                  and self.n_register_tokens == 0 and injected_features is None and injected_post_cssm is None
-                 and not return_features and not return_spatial and self.cells[0]._still_pays(B, T, Hn, Wn))
+                 and not return_features and not return_spatial and self.cells[0]._still_pays(B, T, Hn, Wn, p["cssm_0"]))
         x = x.reshape(B, T_in, Hn, Wn, D).expand(B, T_in if still else T, Hn, Wn, D)   # :277-278
         if self.pos_embed == "learnable":                                   # :281-285
             x = x + p["pos_embed"]

@@ -35,6 +35,28 @@ def test_still_equals_repeated_frames(B, T, C, H, kt, ks, dtype):
     assert (got - ref).abs().max() <= 2e-5 * ref.pow(2).mean().sqrt()
 
 
+@pytest.mark.parametrize("size,kt", [(2, 4), (4, 2), (4, 6), (1, 3)])
+def test_block_image_with_other_taps_than_the_cell_names(size, kt):
+    """The cell convolves with the taps of its parameters; a block's image gives the last frame of that."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from cssm_amd import blocks, spectral as S
+    print_case(test="still_taps", size=size, kt=kt)
+    C, T, shape = 32, 8, (2, 14, 14, 32)
+    v = blocks.CSSMSHViTBlock(dim=C, num_timesteps=T, kernel_size=5, short_conv_size=kt).init(1, shape)
+    block = blocks.CSSMSHViTBlock(dim=C, num_timesteps=T, kernel_size=5, short_conv_size=size)
+    assert block.cell._still_pays(2, T, 14, 14, v["params"]["cssm"]) == (kt <= 4)
+    gen = torch.Generator(device="cuda").manual_seed(kt)
+    x = torch.randn(shape, generator=gen, device="cuda")
+    got = block.token_mixer(v, x)
+    p, x5 = v["params"], x.unsqueeze(1)
+    n, pc = p["norm1"], p["pos_conv"]
+    xc = S.block_norm_posconv(x5, S.block_norm_stats(x5, "global_layer"), "global_layer", n["scale"], n["bias"],
+                              pc["kernel"], pc["bias"], T)
+    ref = x + block.cell.apply({"params": p["cssm"]}, xc)[:, -1]
+    assert (got - ref).abs().max() <= 2e-5 * ref.pow(2).mean().sqrt()      # as above
+
+
 def test_still_rule():
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
