@@ -295,13 +295,15 @@ class SimpleCSSM:
                     x = norm_act(x, f"norm{i + 1}")
                 x = Fn.max_pool2d(x.permute(0, 3, 1, 2), 2, 2, ceil_mode=True).permute(0, 2, 3, 1)
         _, Hn, Wn, D = x.shape
-        # one cell on an image's equal frames with the last one read out: the cell takes the image itself
-        still = (T_in == 1 and self.depth == 1 and self.cssm_type == "gated" and self.frame_readout == "last"
-                 and self.n_register_tokens == 0 and injected_features is None and injected_post_cssm is None
-                 and not return_features and not return_spatial and self.cells[0]._still_pays(B, T, Hn, Wn, p["cssm_0"]))
-        x = x.reshape(B, T_in, Hn, Wn, D).expand(B, T_in if still else T, Hn, Wn, D)   # :277-278
+        x = x.reshape(B, T_in, Hn, Wn, D)                                   # :277-278
         if self.pos_embed == "learnable":                                   # :281-285
             x = x + p["pos_embed"]
+        # one cell on an image's equal frames with the last one read out: the cell takes the image itself
+        still = (x.shape[1] == 1 and self.depth == 1 and self.cssm_type == "gated" and self.frame_readout == "last"
+                 and self.n_register_tokens == 0 and injected_features is None and injected_post_cssm is None
+                 and not return_features and not return_spatial and self.cells[0]._still_pays(B, T, Hn, Wn, p["cssm_0"]))
+        if not still and T != T_in:
+            x = x.expand(B, T, Hn, Wn, D)
         nreg = self.n_register_tokens
         if nreg > 0:                                                        # :302-306
             x = torch.cat([p["register_tokens"].expand(B, -1, -1, -1, -1), x], dim=1)

@@ -63,6 +63,24 @@ def test_simple_cssm_matches_oracle(simple, name, shape, kw, call):
     assert rel_err(to_np(y), ref) <= TOL_F32
 
 
+def test_position_embedding_per_frame(simple):
+    """A position embedding with a frame axis broadcasts over an image's repeated frames, which then differ."""
+    print_case(test="pos_embed_per_frame")
+    kw = dict(num_classes=3, embed_dim=32, depth=1, cssm_type="gated", kernel_size=5, seq_len=6, pos_embed="learnable",
+              norm_type="layer", frame_readout="last")
+    rng = np.random.default_rng(12)
+    cfg = O.SimpleConfig(**kw)
+    p = init_simple(O.simple_param_shapes(cfg, (2, 56, 56, 3))[0], rng)
+    p["pos_embed"] = rng.standard_normal((1, 6, 14, 14, 32))
+    x = rng.standard_normal((2, 56, 56, 3))
+    model, dev = simple(**kw), torch.from_numpy(x).to("cuda", torch.float32)
+    y = model.apply(simple.load_params({"params": p}), dev)
+    assert rel_err(to_np(y), O.simple_cssm_forward(p, x, cfg)) <= TOL_F32
+    p["pos_embed"] = p["pos_embed"][:, :4]
+    with pytest.raises(RuntimeError):                      # four frames of positions for six
+        model.apply(simple.load_params({"params": p}), dev)
+
+
 def test_simple_cssm_from_checkpoint_file(simple, tmp_path):
     """A SimpleCheckpointer-format pickle (written here) read by the weights-only loader runs
     the model with the same result as the in-memory parameters."""
