@@ -323,7 +323,7 @@ class _GatedInScanFn(torch.autograd.Function):
         dfac = S.gated_gates_backward(cx3, gps, H, W, dgates, gate_type, activation, c_scale).view(F, -1)
         del dgates
         wcat = torch.cat(gate_params[0::2], dim=1)
-        dcx = dfac @ wcat.t()
+        dcx = (dfac @ wcat.t()).float()                # (16 bits where the backward runs under autocast)
         dwcat = cx.view(F, Ci).t() @ dfac
         dbcat = dfac.sum(dim=0)
         gp_grads, off = [], 0
@@ -569,9 +569,10 @@ def _gate_keys(cell):
 
 def _gate_products(p, keys, ctx):
     """{parameter name: ctx kernel + bias} of the named Dense layers as one product (their kernels side
-    by side: one GEMM forward and two backward instead of up to eight of each)."""
-    out = torch.addmm(torch.cat([p[k]["bias"] for k in keys]), ctx.reshape(-1, ctx.shape[-1]),
-                      torch.cat([p[k]["kernel"] for k in keys], dim=1)).view(*ctx.shape[:-1], -1)
+    by side: one GEMM forward and two backward instead of up to eight of each), in float32 under autocast too."""
+    with torch.autocast("cuda", enabled=False):
+        out = torch.addmm(torch.cat([p[k]["bias"] for k in keys]), ctx.reshape(-1, ctx.shape[-1]),
+                          torch.cat([p[k]["kernel"] for k in keys], dim=1)).view(*ctx.shape[:-1], -1)
     return dict(zip(keys, out.split([p[k]["bias"].shape[0] for k in keys], dim=-1)))
 
 

@@ -153,6 +153,23 @@ def test_qkv_depthwise_layouts(mods, form, H):
     close(got, ref)
 
 
+@pytest.mark.parametrize("cls,gate_type", [("gated", "factored"), ("gated", "dense"), ("gdn", "factored"),
+                                           ("gdn", "dense"), ("gdn", "channel"), ("gdn", "scalar")])
+def test_training_under_autocast(mods, cls, gate_type):
+    """A forward and backward inside autocast: the layer computes in float32, torch's products in bf16."""
+    cells, _, training = mods
+    print_case(test="autocast", cls=cls, gates=gate_type)
+    kw = dict(gate_type=gate_type, **({"delta_key_dim": 4} if cls == "gdn" else {}))
+    apply = training.gdn_train_apply if cls == "gdn" else training.gated_train_apply
+    cell, v, x, dout = layer(cells.GatedDeltaNetCSSM if cls == "gdn" else cells.GatedCSSM, 8, (1, 2, 16, 16, 8), **kw)
+    ref = grads(apply, cell, v, x, dout)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        got = grads(apply, cell, v, x, dout)
+    for g, r in zip(got, ref):                             # bf16 operands: 2^-9 each, sums that cancel some
+        assert g.dtype == r.dtype
+        assert (g - r).pow(2).sum() <= (5e-2) ** 2 * r.pow(2).sum()
+
+
 @pytest.mark.parametrize("cls,path", [("gated", "short_conv_spatial"), ("gated", "short_conv_temporal"),
                                       ("gated", "delta_proj_h"), ("gdn", "short_conv_k"), ("gdn", "short_conv_q"),
                                       ("gdn", "alpha_w"), ("gdn", "gate_proj"), ("gdn", "rms_scale")])
