@@ -738,7 +738,8 @@ def gdn_qkv_gate_proj(x: torch.Tensor, kernel: torch.Tensor, bias: torch.Tensor,
 
 
 def gdn_qkv_fused(T: int, H: int, W: int, K: int, kt: int) -> bool:
-    """True when gdn_qkv_proj runs as one fused kernel for this shape and short-conv length."""
+    """True when gdn_qkv_proj has one fused kernel for this shape and short-conv length (few sequences, B H W <= 4096
+    from 4 frames, run as projection and post pass all the same)."""
     return bool(_lib.load().cssm_gdn_qkv_fused(T, H, W, K, kt))
 
 

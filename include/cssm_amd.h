@@ -487,7 +487,9 @@ int cssm_gdn_qkv_post(void* qkv, int dtype, int B, int T, int C, int H, int W, i
  * and input gates of cssm_gdn_qkv_post fused into the GEMM's epilogue:
  *   qkv = post(proj(x)),  proj = cssm_proj_planes with N = 3C (identity act).
  * Replaces cssm.py:4753-4758 (qkv_proj), :4763-4780 and :4844-4848 in one pass
- * over qkv instead of three.  Fused when cssm_gdn_qkv_fused(T, H, W, K, kt)
+ * over qkv instead of three.  Up to 64 sequences of 64 pixels (B*H*W <= 4096) and
+ * from 4 frames, fp32 qkv, it runs the two calls it replaces, faster there and with the
+ * same results.  Else fused when cssm_gdn_qkv_fused(T, H, W, K, kt)
  * (K <= 64, K % 4 == 0): any T with kt <= 4 or T <= 4 and H*W a multiple of 64
  * (tiles of 64 pixels of one frame, a workgroup walking the frames in order with
  * the three previous frames' projections in registers; 3C*H*W elements of
@@ -525,7 +527,8 @@ int cssm_gdn_qkv_gate_proj(const void* x, int in_dtype, int B, int T, int H, int
                            const float* gate_kernel, const float* gate_bias, int gate_act, void* qkv, void* gv,
                            int out_dtype, void* stream);
 
-/* 1 if cssm_gdn_qkv_proj runs fused for (T, H, W, K, kt), else 0 (it then runs two kernels). */
+/* 1 if cssm_gdn_qkv_proj has a fused kernel for (T, H, W, K, kt), which it runs but for few sequences (above), else 0
+ * (it then runs two kernels). */
 int cssm_gdn_qkv_fused(int T, int H, int W, int K, int kt);
 
 /*

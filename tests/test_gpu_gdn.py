@@ -219,13 +219,15 @@ def test_gdn_qkv_post_matches_oracle(mods, kt):
 
 
 # (B, T, H, W, K, C): with H*W a multiple of 64 and kt <= 4 (or T <= 4) one frame-sequential kernel
-# (any T); else T = 4 or a multiple of 8 (chunks of 8 frames carrying 3, kt <= 4) with H*W a
+# (any T) where T < 4 or B H W is past 64 * 64, up to there (fp32 planes) proj_planes + qkv_post; else T = 4 or a multiple of 8 (chunks of 8 frames carrying 3, kt <= 4) with H*W a
 # multiple of 128 / min(T, 8) the tiled kernel ((1, 4, 4, 8): T = 4; (1, 8, 4, 4): T = 8;
 # (2, 24, 4, 4): chunks); the rest (kt = 6 at T = 8 or 16; T = 3 at 4 x 4) through proj_planes +
-# qkv_post
+# qkv_post.  The last row's cases are the frame-sequential kernel from T = 4 on, with its carry over 3 frames
 QKV_CASES = [(2, 8, 16, 16, 64, 16), (1, 4, 8, 8, 32, 8), (3, 2, 8, 8, 64, 12), (2, 1, 16, 8, 48, 8),
              (2, 3, 8, 8, 64, 16), (1, 16, 8, 8, 32, 8), (2, 1, 8, 8, 64, 8), (1, 32, 8, 8, 64, 8),
-             (2, 24, 4, 4, 32, 8), (1, 4, 4, 8, 32, 8), (1, 8, 4, 4, 32, 8), (2, 3, 4, 4, 32, 8)]
+             (2, 24, 4, 4, 32, 8), (1, 4, 4, 8, 32, 8), (1, 8, 4, 4, 32, 8), (2, 3, 4, 4, 32, 8),
+             (17, 8, 16, 16, 64, 16), (65, 4, 8, 8, 32, 8), (66, 16, 8, 8, 32, 8), (65, 24, 8, 8, 64, 16),
+             (65, 32, 8, 8, 64, 8), (22, 5, 8, 24, 40, 8)]
 
 
 @pytest.mark.parametrize("shape", QKV_CASES)
@@ -618,7 +620,7 @@ LAYER_CASES = [
     ("small_12_dense_T1", (2, 1, 12, 12, 8), dict(delta_key_dim=4, gate_type="dense", kernel_size=5)),
     # the k x k full-channel qkv conv (qkv_conv_separable=False): the fused 32 x 32 core, an even tap
     # count on 14 x 14 planes with d_k = 3, channel input gates
-    ("full_qkv_conv3_fused32", (1, 3, 32, 32, 16),
+    ("full_qkv_conv3_fused32", (17, 3, 32, 32, 16),
      dict(delta_key_dim=4, gate_type="factored", qkv_conv_size=3, qkv_conv_separable=False)),
     ("full_qkv_conv4_14_dk3", (2, 3, 14, 14, 12),
      dict(delta_key_dim=3, gate_type="factored", qkv_conv_size=4, qkv_conv_separable=False, kernel_size=3)),
@@ -639,9 +641,11 @@ def _layer(kw, shape, seed):
 
 @pytest.mark.parametrize("name,shape,kw", LAYER_CASES, ids=[c[0] for c in LAYER_CASES])
 def test_gdn_layer_matches_oracle(mods, name, shape, kw):
-    cells, _ = mods
+    cells, S = mods
     print_case(test="gdn_layer", case=name)
     cfg, p, x = _layer(kw, shape, 21)
+    assert "fused32" not in name or S.gdn_core_fused_pays(shape[0], shape[1], shape[4], 4)
+    some = sorted({0, shape[0] // 2, shape[0] - 1})       # batch elements the oracle computes
     if kw.get("position_independent_gates"):
         # no temporal encoding of ctx: compare against the oracle with the table cancelled
         T, C = shape[1], shape[4]
@@ -649,22 +653,24 @@ def test_gdn_layer_matches_oracle(mods, name, shape, kw):
         orig = O.temporal_context_encoding
         O.temporal_context_encoding = lambda T_, C_, base=10000.0: np.zeros((T_, C_))
         try:
-            ref = O.gdn_forward(p, x, cfg)
+            ref = O.gdn_forward(p, x[some], cfg)
         finally:
             O.temporal_context_encoding = orig
         assert enc.shape == (T, C)
     else:
-        ref = O.gdn_forward(p, x, cfg)
+        ref = O.gdn_forward(p, x[some], cfg)
     cell = cells.GatedDeltaNetCSSM(channels=shape[4], **kw)
     y = cell.apply(cells.GatedDeltaNetCSSM.load_params(p), _dev(x))
     torch.cuda.synchronize()
     assert tuple(y.shape) == shape
-    assert rel_err(to_np(y), ref) <= TOL_F32
+    assert rel_err(to_np(y[some]), ref) <= TOL_F32
 
 
 ZERO_FRAME_CASES = [
-    # name, (B, T, H, W, C), cfg kwargs: the fused 32 x 32 core, the three-kernel core, a small plane
-    ("fused32", (2, 6, 32, 32, 16), dict(delta_key_dim=4, gate_type="factored", kernel_size=11)),
+    # name, (B, T, H, W, C), cfg kwargs: the fused 32 x 32 core (from 257 workgroups), the three-kernel core at
+    # 32 x 32 and 16 x 16, a small plane
+    ("fused32", (65, 6, 32, 32, 16), dict(delta_key_dim=4, gate_type="factored", kernel_size=11)),
+    ("planes32", (2, 6, 32, 32, 16), dict(delta_key_dim=4, gate_type="factored", kernel_size=11)),
     ("planes16_dk2", (2, 5, 16, 16, 8), dict(delta_key_dim=2, gate_type="channel", kernel_size=5)),
     ("small14", (1, 4, 14, 14, 8), dict(delta_key_dim=4, gate_type="dense", kernel_size=5, short_conv_size=0)),
 ]
@@ -678,7 +684,7 @@ def test_gdn_layer_zero_masked_frames_per_scan_variant(mods, name, shape, kw, va
     (main.py:1429-1438): those frames' q / k / v planes are constant (bias only), so every
     non-DC bin of their spectra is zero up to the transform's rounding, the entries the scan
     variants map differently.  Against the oracle under the same flags."""
-    cells, _ = mods
+    cells, S = mods
     flags = dict(VARIANT_FLAGS.get(variant, {}))
     kw = dict(kw)
     if variant == "pallas_d2":
@@ -690,8 +696,12 @@ def test_gdn_layer_zero_masked_frames_per_scan_variant(mods, name, shape, kw, va
     cell = cells.GatedDeltaNetCSSM(channels=shape[4], **kw)
     expect = ("linear" if kw["delta_key_dim"] == 2 else "goom") if variant == "pallas_d2" else variant
     assert cell.scan_variant == O.gdn_scan_variant(cfg) == expect
-    ref = O.gdn_forward(p, x, cfg)
-    y = cell.apply(cells.GatedDeltaNetCSSM.load_params(p), _dev(x))
+    fused = S.gdn_core_fused_supported(*shape[2:4], kw["delta_key_dim"]) and S.gdn_core_fused_pays(
+        shape[0], shape[1], shape[4], kw["delta_key_dim"])
+    assert fused == (name == "fused32")
+    some = [0, shape[0] - 1]                              # batch elements the oracle computes
+    ref = O.gdn_forward(p, x[some], cfg)
+    y = cell.apply(cells.GatedDeltaNetCSSM.load_params(p), _dev(x))[some]
     torch.cuda.synchronize()
     assert rel_err(to_np(y), ref) <= TOL_F32
     # the masked frames alone, against their own RMS
@@ -744,25 +754,25 @@ def _moving_dots(rng, shape):
 
 
 def test_gdn_layer_c4_shape_bf16_chunk_carry(mods):
-    """C4's frame shape at full width (T = 32, 32 x 32, C = 64, d_k = 4, bf16 I/O) on moving dots:
-    the frame-sequential qkv projection walks the 32 frames carrying the short conv's three
-    previous frames in registers, with gate_proj's columns in the same launch, inside the layer."""
+    """C4's frame shape at full width (T = 32, 32 x 32, C = 64, d_k = 4, bf16 I/O) on moving dots, of
+    enough batch elements that the layer runs the frame-sequential qkv projection (32 frames walked with
+    the short conv's three previous frames in registers) and the fused core."""
     cells, S = mods
     print_case(test="gdn_layer_c4_T32_bf16")
     kw = dict(delta_key_dim=4, gate_type="factored", kernel_size=11, short_conv_size=4)
-    shape = (1, 32, 32, 32, 64)
-    assert S.gdn_qkv_fused(32, 32, 32, 64, 4)
+    shape = (17, 32, 32, 32, 64)
+    assert S.gdn_qkv_fused(32, 32, 32, 64, 4) and 17 * 32 * 32 > 64 * 64 and S.gdn_core_fused_pays(17, 32, 64, 4)
     cfg, p, _ = _layer(kw, shape, 27)
     x = _moving_dots(np.random.default_rng(28), shape)
     xb = _dev(x, torch.bfloat16)
     y = cells.GatedDeltaNetCSSM(channels=64, **kw).apply(cells.GatedDeltaNetCSSM.load_params(p), xb)
     assert y.dtype == torch.bfloat16
-    ref = O.gdn_forward(p, to_np(xb), cfg)
-    assert bf16_excess_err(to_np(y), ref) <= TOL_BF16
+    ref = O.gdn_forward(p, to_np(xb[-1:]), cfg)           # the last element
+    assert bf16_excess_err(to_np(y[-1:]), ref) <= TOL_BF16
     # the same layer in fp32 I/O holds the fp32 bar (the carry is exact)
     y32 = cells.GatedDeltaNetCSSM(channels=64, **kw).apply(cells.GatedDeltaNetCSSM.load_params(p),
                                                            _dev(to_np(xb)))
-    assert rel_err(to_np(y32), ref) <= TOL_F32
+    assert rel_err(to_np(y32[-1:]), ref) <= TOL_F32
 
 
 def test_gdn_layer_two_parameter_trees(mods):

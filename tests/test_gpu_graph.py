@@ -25,13 +25,17 @@ def cells():
     return c
 
 
-# (name, cell kwargs, input shape, input dtype): the power-of-two and the small-plane gated scans,
-# the fused 32 x 32 GDN core with the frame-sequential qkv projection, and the three-kernel GDN core
+# (name, cell kwargs, input shape, input dtype): the power-of-two and the small-plane gated scans and the gated
+# scan through spectra, the fused 32 x 32 GDN core with the frame-sequential qkv projection, and the three-kernel
+# GDN core with the projection of all frames (few sequences) and at 16 x 16
 CASES = [
     ("gated_32", dict(channels=16, kernel_size=7), (2, 3, 32, 32, 16), torch.float32),
+    ("gated_split_32", dict(channels=16, kernel_size=7), (2, 9, 32, 32, 16), torch.float32),
     ("gated_14_bf16", dict(channels=32, kernel_size=5, expand=2, short_conv_size=0, short_conv_spatial_size=0),
      (4, 1, 14, 14, 32), torch.bfloat16),
     ("gdn_32", dict(channels=16, delta_key_dim=4, gate_type="factored", kernel_size=7, short_conv_size=4),
+     (65, 8, 32, 32, 16), torch.float32),
+    ("gdn_few_32", dict(channels=16, delta_key_dim=4, gate_type="factored", kernel_size=7, short_conv_size=4),
      (1, 8, 32, 32, 16), torch.float32),
     ("gdn_16", dict(channels=8, delta_key_dim=2, gate_type="channel", kernel_size=5, short_conv_size=3),
      (2, 3, 16, 16, 8), torch.float32),
@@ -40,7 +44,13 @@ CASES = [
 
 @pytest.mark.parametrize("name,kw,shape,dtype", CASES, ids=[c[0] for c in CASES])
 def test_cell_forward_replays_from_a_graph(cells, name, kw, shape, dtype):
+    from cssm_amd import spectral as S
     print_case(test="graph_replay", case=name, shape=shape)
+    B, T, H, _, C = shape
+    if name.startswith("gated"):
+        assert S.gated_split_rule(B * C, T, H, H) == (name == "gated_split_32")
+    elif H == 32:
+        assert S.gdn_core_fused_pays(B, T, C, 4) == (B * H * H > 64 * 64) == (name == "gdn_32")
     cls = cells.GatedCSSM if name.startswith("gated") else cells.GatedDeltaNetCSSM
     cell = cls(**kw)
     variables = cell.init(3, shape)
