@@ -240,9 +240,12 @@ def test_gated_scan_matches_oracle(S, B, T, C, H, W):
 
 
 @pytest.mark.parametrize("H", [8, 32, 128, 14])
-def test_gated_scan_goom_floor_zero_inputs(S, H):
-    """Exact zeros (a zero frame, a zero B row) take to_goom's 1e-7 floor."""
-    print_case(test="gated_scan_floor", H=H)
+@pytest.mark.parametrize("form", ["fused", "split"])
+def test_gated_scan_goom_floor_zero_inputs(S, monkeypatch, H, form):
+    """Exact zeros (a zero frame, a zero B row) take to_goom's 1e-7 floor, in the fused kernel and through
+    spectra."""
+    print_case(test="gated_scan_floor", H=H, form=form)
+    monkeypatch.setattr(S, "gated_split_rule", lambda *a: form == "split")
     rng = np.random.default_rng(5)
     B, T, W = 1, 4, H
     C = {8: 32, 32: 8, 128: 2, 14: 4}[H]

@@ -63,6 +63,57 @@ def test_simple_cssm_matches_oracle(simple, name, shape, kw, call):
     assert rel_err(to_np(y), ref) <= TOL_F32
 
 
+IMAGE = dict(num_classes=3, embed_dim=32, depth=1, cssm_type="gated", kernel_size=5, seq_len=6, pos_embed="none",
+             norm_type="layer", frame_readout="last", stem_mode="default", stem_layers=2)
+IMAGE_CASES = [
+    # name, x shape, changes to IMAGE, whether the cell takes the image as one frame
+    ("seq6", (2, 56, 56, 3), dict(), True),
+    ("seq2_pos", (2, 56, 56, 3), dict(seq_len=2, pos_embed="learnable"), True),
+    ("seq3_pre_order_64", (1, 51, 52, 3), dict(seq_len=3, embed_dim=64, stem_norm_order="pre"), True),    # 13 x 13
+    ("seq8_pre_order_pos_gelu", (2, 25, 28, 3), dict(seq_len=8, stem_norm_order="pre", pos_embed="learnable",
+                                                    act_type="gelu", gate_type="factored"), True),        # 7 x 7
+    ("seq5_64_relu_max", (3, 53, 54, 4), dict(seq_len=5, embed_dim=64, act_type="relu", pool_type="max",
+                                              readout_norm="post"), True),                                # 14 x 14
+    ("seq4_one_layer", (2, 9, 9, 3), dict(seq_len=4, stem_layers=1, short_conv_size=0), True),            # 5 x 5
+    ("seq21_spectra_64", (4, 64, 64, 3), dict(seq_len=21, embed_dim=64), True),                           # 16 x 16
+    ("seq8_batch_norm", (2, 28, 28, 3), dict(seq_len=8, norm_type="batch"), True),
+    ("all_frames", (2, 28, 28, 3), dict(frame_readout="all"), False),
+    ("registers", (2, 28, 28, 3), dict(n_register_tokens=2), False),
+    ("depth2", (2, 28, 28, 3), dict(depth=2), False),
+    ("gdn", (2, 28, 28, 3), dict(cssm_type="gdn", delta_key_dim=2), False),
+    ("taps5", (2, 28, 28, 3), dict(short_conv_size=5), False),
+    ("one_frame", (2, 28, 28, 3), dict(seq_len=1), False),
+]
+
+
+@pytest.mark.parametrize("call", [{}, dict(return_features=True), dict(return_spatial=True)])
+@pytest.mark.parametrize("name,shape,kw,one", IMAGE_CASES, ids=[c[0] for c in IMAGE_CASES])
+def test_images_match_oracle(simple, monkeypatch, name, shape, kw, one, call):
+    """Images through the stem once and, where only the cell's last frame is read, the cell on one frame: against
+    the oracle, which repeats the image to seq_len frames first."""
+    if call and (name.startswith("seq21") or "spatial" in str(call) and name == "registers"):
+        pytest.skip("covered by the other cases")
+    print_case(test="simple_image", case=name, call=call)
+    kw = {**IMAGE, **kw}
+    rng = np.random.default_rng(15)
+    model, cfg = simple(**kw), O.SimpleConfig(**kw)
+    shapes, bss = O.simple_param_shapes(cfg, shape)
+    p = init_simple(shapes, rng)
+    bs = {n: {"mean": rng.standard_normal(v["mean"]) * 0.1, "var": 1 + rng.random(v["var"])} for n, v in bss.items()}
+    x = rng.standard_normal(shape)
+    took = []
+    for c in model.cells:
+        if hasattr(c, "_apply_still"):
+            orig = c._apply_still
+            monkeypatch.setattr(c, "_apply_still", lambda *a, orig=orig, **k: took.append(1) or orig(*a, **k))
+    y = model.apply(simple.load_params({"params": p, "batch_stats": bs}),
+                    torch.from_numpy(x).to("cuda", torch.float32), **call)
+    assert len(took) == int(one and not call)
+    ref = O.simple_cssm_forward(p, x, cfg, batch_stats=bs, **call)
+    assert tuple(y.shape) == ref.shape
+    assert rel_err(to_np(y), ref) <= TOL_F32
+
+
 def test_position_embedding_per_frame(simple):
     """A position embedding with a frame axis broadcasts over an image's repeated frames, which then differ."""
     print_case(test="pos_embed_per_frame")
