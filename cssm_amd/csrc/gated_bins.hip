@@ -12,7 +12,7 @@
 // Bound by the latency of its loads at few bins, so U and the gates of the next eight
 // frames are in flight while eight are advanced (64-thread workgroups, so that few bins
 // still reach every CU).  1024 frames x 256 planes of 16 x 16: transforms and recurrence
-// 566 us, the fused kernel 7830 us.
+// 637 us, the fused kernel 7300 us.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

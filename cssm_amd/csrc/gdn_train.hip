@@ -5,7 +5,8 @@
 // (main.py:283) through cssm.py:4763-4859, 4890-4897 and 5026-5141.
 // Each is one pass over its planes where a chain of elementwise, padding, slicing and
 // reduction launches made ten to thirty (training step of 256 frames x 64 channels of 32 x 32,
-// T = 8: 9.1 ms with them, 2.2 ms here).  Bound by HBM; times at that size (fwd / adjoint):
+// T = 8: 9.1 ms with them, 2.1 ms here).  Bound by HBM, but norm_gate's adjoint by its loads' latency between
+// barriers; times at that size (fwd / adjoint):
 // qkv_act 86 / 143 us (4.7 / 4.2 TB/s), norm_gate 46 / 180 us (4.4 / 1.9 TB/s), spec_norm_bwd
 // 90 us (4.8 TB/s).
 #include <hip/hip_runtime.h>

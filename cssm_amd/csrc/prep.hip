@@ -17,7 +17,7 @@ namespace cssm {
 // pad rule: K <= H -> zero pad with pad_before = (H-K)//2 (the tap (i,j) lands
 // at (i + ph, j + pw)); K > H -> centre crop starting at (K-H)//2.  The DFT of
 // the padded plane only needs the K x K (or cropped) taps, evaluated separably
-// in double precision.  One block per channel.
+// in double precision.  One block per channel, several where the channels are few.
 // out: (C, H, W/2+1) complex, optionally GOOM-floored (|x| < 1e-7 -> 1e-7+0j).
 // ---------------------------------------------------------------------------
 // The twiddles cos / sin (2 pi m / N) are taken once per workgroup into LDS (one sincospi per table entry

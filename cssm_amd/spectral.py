@@ -221,7 +221,7 @@ def gated_split_rule(planes: int, T: int, H: int, W: int) -> bool:
     measured at 64 planes, T = 16..1024); the split form takes three launches (24 us) and its traffic, 6.2e-6
     us per sample of a power-of-two plane from 8x8 up and 12e-6 of the others (measured at 3..128, 64..4096
     planes).  Split where that estimate is at least a tenth lower; measured fused / split us: 16x16, 256
-    planes, T = 8 58 / 25, T = 1024 7830 / 570; 32x32, 512 planes, T = 8 61 / 38; 64x64, 256 planes, T = 8
+    planes, T = 8 58 / 25, T = 1024 7300 / 637; 32x32, 512 planes, T = 8 61 / 38; 64x64, 256 planes, T = 8
     108 / 65; 128x128, 64 planes, T = 8 91 / 61; 13x13, 4096 planes, T = 8 124 / 71; 14x14, 512 planes, T = 32
     137 / 44; and on the other side of the line 16x16, 4096 planes, T = 16 131 / 127; 32x32, 2048 planes, T = 8
     78 / 106; 128x128, 128 planes, T = 8 100 / 107; 14x14, 4096 planes, T = 32 155 / 322; 7x7, 512 planes, T = 8
@@ -235,7 +235,7 @@ def _gated_scan_split(u, z, gates, khat, out, max_bytes: int = 1 << 30):
     """:func:`gated_scan` as batched rfft2 -> recurrence per bin (cssm_gated_scan_bins) -> irfft2 x z
     through spectra in HBM, at most ``max_bytes`` of them at a time: batch elements in groups, or one
     element's frames in pieces with the state carried over.  (1024 frames x 256 planes of 16x16 in pieces of
-    64 / 128 / 256 / 512 MiB: 640 / 588 / 585 / 566 us.)"""
+    64 / 128 / 256 / 512 MiB: 699 / 636 / 659 / 638 us.)"""
     B, T, C, H, W = u.shape
     Wf = W // 2 + 1
     frames = max(1, max_bytes // (C * H * Wf * 8))

@@ -1,16 +1,17 @@
-"""Training path of the gated cell: forward and backward through the HIP scan.
+"""Training paths of the two cells: forward and backward through the HIP kernels.
 
 The reference trains through the layer with ``jax.value_and_grad``
-(main.py:283).  Here the spectral core -- rfft2, the GOOM-gated complex
-recurrence over T, irfft2, x SiLU(z), the part of the layer that costs the
-time -- runs forward in ``cssm_gated_scan_fwd`` and backward in the reverse
-recurrence ``cssm_gated_scan_bwd`` between batched FFTs (``_ScanFn``).  The
-rest of the layer is a handful of small or GEMM-shaped ops that torch
-differentiates on the same stream: in_proj / out_proj (library GEMMs), the
-short convolutions, SiLU, the spatial mean ctx, and the construction of the
-per-bin gate planes and the floored K_hat, written here exactly as the HIP
-prep kernels lay them out (columns in the scan's order, the GOOM floor
-terms folded in).
+(main.py:283).  Here a layer up to its output projection is one autograd node
+whose forward and backward run on HIP kernels (``_GatedInScanFn``, ``_GdnFn``):
+projections, short convolutions, gates, transforms, recurrence and their
+adjoints, with the weight gradients as library GEMMs.  Sizes without such
+kernels and parameters that they would not read as torch does (16 bits,
+broadcast shapes, taps that q, k and v do not share) take the composite: the
+spectral core in ``_ScanFn`` / ``_GdnBinsFn`` between batched transforms, and
+around it the short convolutions, SiLU, the mean ctx, the per-bin gate planes
+and the floored K_hat as torch expressions that torch differentiates, laid out
+exactly as the HIP prep kernels lay them out (columns in the scan's order, the
+GOOM floor terms folded in).
 
 ``gated_train_apply(cell, params, x)`` returns the layer output with the
 autograd graph attached; ``params`` is the cell's parameter tree of leaf

@@ -622,6 +622,8 @@ LAYER_CASES = [
     # count on 14 x 14 planes with d_k = 3, channel input gates
     ("full_qkv_conv3_fused32", (17, 3, 32, 32, 16),
      dict(delta_key_dim=4, gate_type="factored", qkv_conv_size=3, qkv_conv_separable=False)),
+    ("full_qkv_conv3_few32", (1, 3, 32, 32, 16),
+     dict(delta_key_dim=4, gate_type="factored", qkv_conv_size=3, qkv_conv_separable=False)),
     ("full_qkv_conv4_14_dk3", (2, 3, 14, 14, 12),
      dict(delta_key_dim=3, gate_type="factored", qkv_conv_size=4, qkv_conv_separable=False, kernel_size=3)),
     ("full_qkv_conv5_channel_16", (2, 2, 16, 16, 8),
@@ -753,15 +755,17 @@ def _moving_dots(rng, shape):
     return x
 
 
-def test_gdn_layer_c4_shape_bf16_chunk_carry(mods):
-    """C4's frame shape at full width (T = 32, 32 x 32, C = 64, d_k = 4, bf16 I/O) on moving dots, of
-    enough batch elements that the layer runs the frame-sequential qkv projection (32 frames walked with
-    the short conv's three previous frames in registers) and the fused core."""
+@pytest.mark.parametrize("B", [17, 1])
+def test_gdn_layer_c4_shape_bf16_chunk_carry(mods, B):
+    """C4's frame shape at full width (T = 32, 32 x 32, C = 64, d_k = 4, bf16 I/O) on moving dots: 17
+    elements, where the layer runs the frame-sequential qkv projection (32 frames walked with the short
+    conv's three previous frames in registers) and the fused core, and one, where it runs neither."""
     cells, S = mods
-    print_case(test="gdn_layer_c4_T32_bf16")
+    print_case(test="gdn_layer_c4_T32_bf16", B=B)
     kw = dict(delta_key_dim=4, gate_type="factored", kernel_size=11, short_conv_size=4)
-    shape = (17, 32, 32, 32, 64)
-    assert S.gdn_qkv_fused(32, 32, 32, 64, 4) and 17 * 32 * 32 > 64 * 64 and S.gdn_core_fused_pays(17, 32, 64, 4)
+    shape = (B, 32, 32, 32, 64)
+    assert S.gdn_qkv_fused(32, 32, 32, 64, 4)
+    assert (B * 32 * 32 > 64 * 64) == S.gdn_core_fused_pays(B, 32, 64, 4) == (B == 17)
     cfg, p, _ = _layer(kw, shape, 27)
     x = _moving_dots(np.random.default_rng(28), shape)
     xb = _dev(x, torch.bfloat16)
