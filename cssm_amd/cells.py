@@ -210,8 +210,8 @@ class GatedCSSM:
         them the attributes'."""
         ks, kt = self.short_conv_spatial_size, self.short_conv_size
         if p is not None:
-            ks = p["short_conv_spatial"]["kernel"].shape[0] if ks > 0 else 0
-            kt = p["short_conv_temporal"]["kernel"].shape[0] if kt > 0 else 0
+            ks, kt = (p[n]["kernel"].shape[0] if size > 0 and p.get(n) is not None else 0
+                      for n, size in (("short_conv_spatial", ks), ("short_conv_temporal", kt)))
         return ks, kt
 
     def _still_pays(self, B: int, T: int, H: int, W: int, p: Optional[Dict[str, Any]] = None) -> bool:

@@ -35,7 +35,7 @@ def test_still_equals_repeated_frames(B, T, C, H, kt, ks, dtype):
     assert (got - ref).abs().max() <= 2e-5 * ref.pow(2).mean().sqrt()
 
 
-@pytest.mark.parametrize("size,kt", [(2, 4), (4, 2), (4, 6), (1, 3)])
+@pytest.mark.parametrize("size,kt", [(2, 4), (4, 2), (4, 6), (1, 3), (4, 0)])
 def test_block_image_with_other_taps_than_the_cell_names(size, kt):
     """The cell convolves with the taps of its parameters; a block's image gives the last frame of that."""
     if not torch.cuda.is_available():
