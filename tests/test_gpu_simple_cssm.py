@@ -91,8 +91,6 @@ IMAGE_CASES = [
 def test_images_match_oracle(simple, monkeypatch, name, shape, kw, one, call):
     """Images through the stem once and, where only the cell's last frame is read, the cell on one frame: against
     the oracle, which repeats the image to seq_len frames first."""
-    if call and (name.startswith("seq21") or "spatial" in str(call) and name == "registers"):
-        pytest.skip("covered by the other cases")
     print_case(test="simple_image", case=name, call=call)
     kw = {**IMAGE, **kw}
     rng = np.random.default_rng(15)
