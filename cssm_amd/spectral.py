@@ -28,7 +28,7 @@ def _stream() -> int:
 
 
 def _dev(t: torch.Tensor, name: str, dtype=None) -> torch.Tensor:
-    if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
+    if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise ValueError(f"{name} must be a GPU tensor")
     if dtype is not None and t.dtype != dtype:
         raise ValueError(f"{name} must be {dtype}, got {t.dtype}")
@@ -809,7 +809,7 @@ def _plane_set(t: Optional[torch.Tensor], C: int, HW: int, name: str):
     contiguous (F, S, HW) tensor, S >= C (a channel slice of a plane-major tensor)."""
     if t is None:
         return None, C
-    if not isinstance(t, torch.Tensor) or t.device.type != "cuda" or t.dtype != torch.float32:
+    if not isinstance(t, torch.Tensor) or not t.is_cuda or t.dtype != torch.float32:
         raise ValueError(f"{name} must be a float32 GPU tensor")
     F = t.shape[0]
     if t.dim() != 3 or t.shape[1] != C or t.shape[2] != HW or t.stride(2) != 1 or t.stride(1) != HW \
@@ -1040,7 +1040,7 @@ def gdn_core_backward(spec: torch.Tensor, norms: Optional[torch.Tensor], ab: tor
 
 def _frames(t: torch.Tensor, name: str, F: int, C: int, HW: int) -> int:
     """Frame stride in floats of a float32 (F, C, HW) channel slice of a plane-major tensor."""
-    if not isinstance(t, torch.Tensor) or t.device.type != "cuda" or t.dtype != torch.float32:
+    if not isinstance(t, torch.Tensor) or not t.is_cuda or t.dtype != torch.float32:
         raise ValueError(f"{name} must be a float32 GPU tensor")
     if t.shape != (F, C, HW) or t.stride(2) != 1 or t.stride(1) != HW or t.stride(0) < C * HW:
         raise ValueError(f"{name}: a ({F}, {C}, {HW}) channel slice of a plane-major tensor is needed")

@@ -165,7 +165,7 @@ def _dwconv_cl(x4, q):
     ks = q["kernel"].shape[0]
     F, H, W, C = x4.shape
     if (ks % 2 == 1 and S.depthwise_conv_wgrad_supported(W, C, ks)
-            and _as_read(q["kernel"], x4.device, ks, ks, 1, C) and _as_read(q["bias"], x4.device, C)):
+            and _as_read(x4.get_device(), (q["kernel"], (ks, ks, 1, C)), (q["bias"], (C,)))):
         return _DwConvFn.apply(x4.contiguous(), q["kernel"].contiguous(), q["bias"].contiguous())
     lo, hi = (ks - 1) // 2, ks // 2
     w = q["kernel"].permute(3, 2, 0, 1)                                      # (C, 1, k, k)
@@ -246,9 +246,13 @@ def _causal_t(x5, p):
     return sum(terms)
 
 
-def _as_read(t: torch.Tensor, dev, *shape) -> bool:
-    """Whether t, made contiguous, is what a kernel given its address reads: float32 of this shape on dev."""
-    return t.dtype == torch.float32 and t.device == dev and t.shape == shape
+def _as_read(dev: int, *sized) -> bool:
+    """Whether every tensor of the (tensor, shape) pairs, made contiguous, is what a kernel given its address reads:
+    float32 of the shape on the device of this index (a few attributes each: small steps are bound by the host)."""
+    for t, shape in sized:
+        if t.dtype is not torch.float32 or t.get_device() != dev or t.shape != shape:
+            return False
+    return True
 
 
 def _gate_leaves(p: Dict[str, Any], gate_type: str):
@@ -388,7 +392,7 @@ class _WhatFn(torch.autograd.Function):
                 None, None)
 
 
-def _gated_node_takes(cell, p, gate_params, T: int, H: int, W: int, Ci: int, dev) -> bool:
+def _gated_node_takes(cell, p, gate_params, T: int, H: int, W: int, Ci: int, dev: int) -> bool:
     """Whether _GatedInScanFn covers the cell on these planes with these parameters: transforms with fused work,
     taps and short convolutions its kernels hold, and tensors as their addresses are read.  The torch path takes the rest
     (a bias that broadcasts or is held in 16 bits) and raises for shapes that do not fit."""
@@ -398,19 +402,19 @@ def _gated_node_takes(cell, p, gate_params, T: int, H: int, W: int, Ci: int, dev
     if cell.short_conv_spatial_size > 0:
         q = p["short_conv_spatial"]
         ks = q["kernel"].shape[0]
-        if not (_as_read(q["kernel"], dev, ks, ks, 1, Ci) and _as_read(q["bias"], dev, Ci)):
+        if not _as_read(dev, (q["kernel"], (ks, ks, 1, Ci)), (q["bias"], (Ci,))):
             return False
     if cell.short_conv_size > 0:
         q = p["short_conv_temporal"]
         kt = q["kernel"].shape[0]
-        if kt == 0 or not (_as_read(q["kernel"], dev, kt, 1, Ci) and _as_read(q["bias"], dev, Ci)):
+        if kt == 0 or not _as_read(dev, (q["kernel"], (kt, 1, Ci)), (q["bias"], (Ci,))):
             return False
     if (ks or kt) and not S.short_conv_train_supported(T, H, W, ks, kt):
         return False
-    sizes = (H, W // 2 + 1) if cell.gate_type == "factored" else (H * (W // 2 + 1),)
-    K = p["kernel"].shape[-1]
-    return S.spectral_kernel_supported(K, H, W) and _as_read(p["kernel"], dev, Ci, K, K) and all(
-        _as_read(t, dev, *((Ci,) if i % 2 == 0 else ()), sizes[i // 2 % len(sizes)]) for i, t in enumerate(gate_params))
+    Wf, K = W // 2 + 1, p["kernel"].shape[-1]
+    shapes = [(Ci, H), (H,), (Ci, Wf), (Wf,)] if cell.gate_type == "factored" else [(Ci, H * Wf), (H * Wf,)]
+    return (S.spectral_kernel_supported(K, H, W)
+            and _as_read(dev, (p["kernel"], (Ci, K, K)), *zip(gate_params, shapes * 3)))
 
 
 def gated_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tensor:
@@ -424,7 +428,7 @@ def gated_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Te
         raise NotImplementedError(f"no fused scan kernel for {H}x{W} planes")
     no_convs = cell.short_conv_spatial_size == 0 and cell.short_conv_size == 0
     gps, rebuild = _gate_leaves(p, cell.gate_type)
-    if _gated_node_takes(cell, p, gps, T, H, W, Ci, x.device):
+    if _gated_node_takes(cell, p, gps, T, H, W, Ci, x.get_device()):
         # in_proj through the scan as one node whose backward runs on the fused HIP transforms
         meta = (B, T, H, W, Ci, cell.gate_type, cell.gate_activation, cell.spectral_rho, rebuild)
         convs = []
@@ -571,9 +575,11 @@ def _gate_keys(cell):
 def _gate_products(p, keys, ctx):
     """{parameter name: ctx kernel + bias} of the named Dense layers as one product (their kernels side
     by side: one GEMM forward and two backward instead of up to eight of each), in float32 under autocast too."""
-    with torch.autocast("cuda", enabled=False):
-        out = torch.addmm(torch.cat([p[k]["bias"] for k in keys]), ctx.reshape(-1, ctx.shape[-1]),
-                          torch.cat([p[k]["kernel"] for k in keys], dim=1)).view(*ctx.shape[:-1], -1)
+    if torch.is_autocast_enabled("cuda"):
+        with torch.autocast("cuda", enabled=False):
+            return _gate_products(p, keys, ctx)
+    out = torch.addmm(torch.cat([p[k]["bias"] for k in keys]), ctx.reshape(-1, ctx.shape[-1]),
+                      torch.cat([p[k]["kernel"] for k in keys], dim=1)).view(*ctx.shape[:-1], -1)
     return dict(zip(keys, out.split([p[k]["bias"].shape[0] for k in keys], dim=-1)))
 
 
@@ -691,27 +697,30 @@ def _norm_params(cell, p):
     return None, None
 
 
-def _gdn_node_takes(cell, p, C: int, H: int, W: int, dev) -> bool:
+def _gdn_node_takes(cell, p, C: int, H: int, W: int, dev: int) -> bool:
     """Whether _GdnFn covers the cell with these parameters: at most 128 channels and short-convolution taps its
     kernels hold, no full-channel qkv convolution, and tensors as their addresses are read or side by side in
     one product.  The torch path takes the rest (a scale that broadcasts or is held in 16 bits, q, k and v with
     taps of their own) and raises for shapes that do not fit."""
     if (cell.qkv_conv_size > 1 and not cell.qkv_conv_separable) or not S.gdn_norm_gate_supported(C):
         return False
-    if not all(t is None or _as_read(t, dev, C) for t in _norm_params(cell, p)):
-        return False
+    sized = [(t, (C,)) for t in _norm_params(cell, p) if t is not None]
     dense = [("qkv_proj", 3 * C), ("gate_proj", C)]
-    for k in _gate_keys(cell):
-        spatial, Wf = k.startswith("B_"), W // 2 + 1
-        dense.append((k, H if k.endswith("_h") else (W if spatial else Wf) if k.endswith("_w")
-                      else {"channel": C // cell.delta_key_dim, "scalar": 1}.get(cell.gate_type, H * (W if spatial else Wf))))
-    if not all(_as_read(p[k]["kernel"], dev, C, n) and _as_read(p[k]["bias"], dev, n) for k, n in dense):
-        return False
-    if cell.short_conv_size == 0:
-        return True
-    convs = [p[f"short_conv_{n}"] for n in "qkv"]
-    kt = convs[0]["kernel"].shape[0]
-    return 0 < kt <= 8 and all(_as_read(q["kernel"], dev, kt, 1, C) and _as_read(q["bias"], dev, C) for q in convs)
+    for k in _gate_keys(cell):                          # outputs of each gate's Dense layer
+        cols = W if k[0] == "B" else W // 2 + 1
+        if cell.gate_type == "factored":
+            dense.append((k, H if k[-1] == "h" else cols))
+        else:
+            dense.append((k, {"channel": C // cell.delta_key_dim, "scalar": 1}.get(cell.gate_type, H * cols)))
+    for k, n in dense:
+        sized += [(p[k]["kernel"], (C, n)), (p[k]["bias"], (n,))]
+    if cell.short_conv_size > 0:
+        kt = p["short_conv_q"]["kernel"].shape[0]
+        if not 0 < kt <= 8:
+            return False
+        for n in ("short_conv_q", "short_conv_k", "short_conv_v"):
+            sized += [(p[n]["kernel"], (kt, 1, C)), (p[n]["bias"], (C,))]
+    return _as_read(dev, *sized)
 
 
 def _gdn_fused_apply(cell, p, x, ctx, what, dims):
@@ -771,7 +780,7 @@ def gdn_train_apply(cell, params: Dict[str, Any], x: torch.Tensor) -> torch.Tens
     if not cell.position_independent_gates:
         ctx = ctx + _temporal_encoding(T, C, cell.rope_base, x.device)[None]
     ks = cell.qkv_conv_size
-    if _gdn_node_takes(cell, p, C, H, W, x.device):
+    if _gdn_node_takes(cell, p, C, H, W, x.get_device()):
         return _gdn_fused_apply(cell, p, x, ctx, what, (B, T, H, W, C, dk, nh))
     xq = x.reshape(F, H, W, C)
     if ks > 1 and not cell.qkv_conv_separable:
